@@ -276,6 +276,110 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
     dense_epilogue<__bf16, EPI, SN, MI, NI>(a, tm * BM + wm * TM, tn * BN + wn * TN, lane, blockIdx.y, acc);
 }
 
+// 1 KB of global memory straight into LDS: lane i's 16 bytes at base + off_lane land at lds + 16 i.  Inline assembly: with
+// the compiler's form of this load every later wait on an LDS read is a wait for all loads in flight.  A vector instruction
+// may have written the scalar registers of base (readfirstlane, a reload of a spilled one): the five wait states that a load
+// needs behind such a write stand in the block, since the compiler does not look into it.
+__device__ __forceinline__ void dense_dma_1k(uint64_t base, uint32_t off_lane, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off_lane), "s"(base), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t dense_lds_addr(const void* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(p)));
+}
+// an address that is the same in every lane, in scalar registers
+__device__ __forceinline__ uint64_t dense_uniform(uint64_t v) {
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32)));
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
+
+// 256 x 256 tile, eight wavefronts as 2 x 4, each 128 rows x 64 tokens: 24 KB of fragments per wavefront and K step of 64
+// against 32 KB of the same work on 128 x 128 tiles, whose four wavefronts read LDS for as long as they multiply.  One
+// barrier a K step, in its middle: behind it the step's second half is in registers, so its buffer takes the K step after
+// next while that half is multiplied.  What bounds it: LDS (2048 of the 2660 clocks that a K step of a workgroup takes alone)
+// beside the matrix cores (2048), and the clock, which a full chip lowers to 2.2 GHz.  28672 x 4096 times 2048 / 512 tokens:
+// 1100 / 1040 TFLOP/s, 128 x 128 tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
+template <int EPI, int SN>
+__global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
+    constexpr int B = 256, BK = 64, MI = 8, NI = 4, HALF = B * BK, BUF = 2 * HALF;
+    __shared__ __align__(1024) __bf16 lds[2][BUF];
+    uint32_t tm, tn, group;
+    if (!dense_tile(a, tm, tn, group)) return;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t k0 = blockIdx.y * a.k_chunk, k1 = min(a.kp, k0 + a.k_chunk), steps = (k1 - k0) / BK;
+    // wavefronts 0 - 3 bring the weight rows in, 4 - 7 the tokens, 64 rows each; rows past the end re-read the last one
+    const bool toks = wave >= 4;
+    const uint32_t first = toks ? tn * B : tm * B, last = (toks ? a.n : a.m) - 1 - first;
+    const uint64_t ld = (toks ? a.ldx : a.kp) * 2;
+    const char* const base = toks ? static_cast<const char*>(a.x) + group * a.gx * 2 : reinterpret_cast<const char*>(a.w + group * a.gw);
+    uint64_t src = dense_uniform(reinterpret_cast<uint64_t>(base) + first * ld + k0 * 2);
+    const uint32_t sub = lane >> 3, slot = lane & 7;
+    uint32_t off[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) off[s] = min((wave & 3) * 64 + s * 8 + sub, last) * static_cast<uint32_t>(ld) + (slot ^ sub) * 16;
+    const uint32_t dst = dense_lds_addr(&lds[0][0]) + wave * 8192;
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) dense_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
+        src = dense_uniform(src + BK * 2);
+    };
+    const uint32_t wm = wave >> 2, wn = wave & 3, fr = lane & 15, fg = lane >> 4;
+    bf16x8 fa[2][MI], fb[2][NI];
+    auto frags = [&](int buf, int kk) {
+        const uint32_t o = ((kk * 4 + fg) ^ (fr & 7)) * 8;
+        const __bf16* const aw = &lds[buf][(wm * 128 + fr) * BK + o];
+        const __bf16* const bx = &lds[buf][HALF + (wn * 64 + fr) * BK + o];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) fa[kk][mi] = *reinterpret_cast<const bf16x8*>(aw + mi * 16 * BK);
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) fb[kk][ni] = *reinterpret_cast<const bf16x8*>(bx + ni * 16 * BK);
+    };
+    f32x4 acc[MI][NI];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int kk) {
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[kk][mi], fb[kk][ni], acc[mi][ni], 0, 0, 0);
+        // the reads of the next fragments between the matrix instructions
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    };
+    auto step = [&](uint32_t s, int buf) {
+        frags(buf, 1);
+        multiply(0);
+        // the next step's pieces are in, and no wavefront reads this buffer any more
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 2 < steps) stage(buf);
+        if (s + 1 < steps) frags(buf ^ 1, 0);
+        multiply(1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    stage(0);
+    if (steps > 1) {
+        stage(1);
+        asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    frags(0, 0);
+    for (uint32_t s = 0; s < steps; s += 2) {
+        step(s, 0);
+        if (s + 1 < steps) step(s + 1, 1);
+    }
+    a.out = static_cast<char*>(a.out) + group * a.go;
+    dense_epilogue<__bf16, EPI, SN, MI, NI>(a, tm * B + wm * 128, tn * B + wn * 64, lane, blockIdx.y, acc);
+}
+
 // 64 x 64 tile in true f32: weights widened on their way into LDS, K in steps of 32.  A lane's four
 // consecutive k of a 16-wide block feed four MFMA steps (the same k order in both operands).
 template <int EPI, int SN> __global__ __launch_bounds__(256) void dense_gemm_f32_kernel(GemmDArgs a) {
@@ -590,11 +694,15 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     a.u = o.u;
     if (o.streams) a.st = *o.streams;
     a.epi = o.epi; a.out = o.out; a.ldo = o.ld; a.bias = o.bias; a.mult = o.mult; a.out_rows = o.rows;
-    // tile: large where it fills the chip, else smaller, else K is split
+    // tile: large where it fills the chip, else smaller, else K is split.  256 x 256 from 60 % of a round of one workgroup per CU on:
+    // 5120 x 3072 times 2048 tokens (160 tiles, 62 %) 77 us against 86 on 128 x 128 tiles, 6176 x 4096 times 1900 (78 %) 98 / 119;
+    // below, 4096 x 18432 times 1900 (128 tiles, 50 %) 337 / 268, 3072 x 3072 times 2048 (38 %) 75 / 51
     int shape = 2;
     uint32_t bm = 64, bn = 32;
     auto count = [&](uint32_t tm, uint32_t tn) { return static_cast<uint64_t>((a.m + tm - 1) / tm) * ((n + tn - 1) / tn) * groups.count; };
+    const uint64_t wide = count(256, 256), rounds = (wide + ctx->n_cu - 1) / ctx->n_cu;
     if (f32) { bm = bn = 64; }
+    else if (n > 128 && wide * 5 >= rounds * ctx->n_cu * 3) { shape = 3; bm = bn = 256; }
     else if (n > 64 && (count(128, 128) >= ctx->n_cu || (a.kp >= 8192 && count(128, 128) * 4 >= ctx->n_cu))) { shape = 0; bm = bn = 128; }
     else if (n > 32) { shape = 1; bm = bn = 64; }
     a.tiles_m = (a.m + bm - 1) / bm;
@@ -603,7 +711,7 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     const uint32_t steps = a.kp / DENSE_PAD;
     uint32_t split = 1;
     const uint32_t want_wgs = 2 * ctx->n_cu;
-    if (wgs < want_wgs && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
+    if (shape != 3 && wgs < want_wgs && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
     if (split < 1) split = 1;
     const uint32_t per = (steps + split - 1) / split;
     split = (steps + per - 1) / per;
@@ -622,6 +730,7 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
         constexpr int E = decltype(epi)::value, SN = decltype(streams)::value;
         constexpr int EG = E == DENSE_STREAMS && SN == 0 ? DENSE_STORE : E;   // leaves partial sums, whatever it is
         if (f32) hipLaunchKernelGGL((dense_gemm_f32_kernel<EG, SN>), grid, block, 0, ctx->stream, a);
+        else if (shape == 3) hipLaunchKernelGGL((dense_gemm_wide_kernel<EG, SN>), grid, dim3(512), 0, ctx->stream, a);
         else if (shape == 0) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 128, 128, 2, 2>), grid, block, 0, ctx->stream, a);
         else if (shape == 1) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 64, 2, 2>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 32, 2, 2>), grid, block, 0, ctx->stream, a);

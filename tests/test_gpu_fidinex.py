@@ -321,6 +321,19 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
+@pytest.mark.parametrize("width, ff, n, streams", [(70, 41000, 129, 2), (5200, 64, 1800, 4), (5200, 64, 1800, 3)])
+def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
+    """From 60 % of a round of 256 x 256 tiles on: the feed-forward's first product, and the residual streams' epilogue."""
+    cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=ff)], width=width, vocab=64, streams=streams)
+    w = U.random_model(cfg, 47)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 5)
+    err = U.rel(m.forward_prefill_logits_all(toks, 0), U.reference(cfg, w, toks))
+    print(f"width={width} ff={ff} n={n} streams={streams}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 @DTYPES
 def test_steps_behind_a_very_long_context(tmp_path, f32):
     """Thousands of visible keys: decode steps and short portions split them over many workgroups."""

@@ -289,6 +289,20 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
+@pytest.mark.parametrize("width, ff, n", [(60, 20500, 129), (130, 20480, 257), (200, 20500, 300), (5200, 64, 1800)])
+def test_products_on_the_widest_tiles(tmp_path, width, ff, n):
+    """From 60 % of a round of 256 x 256 tiles on: one, two, three and four K steps, a ragged last tile of rows and of
+    tokens, a token more than one tile; the last has the residual products there."""
+    cfg = U.config([U.attention(2, 1, 32, 32, 700, 32, 10000.0, ff=ff)], width=width, vocab=64, taps=2, positions=n)
+    w = R.random_model(cfg, 47)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 5)
+    err = U.rel(m.forward_prefill_logits_all(toks, 0), U.reference(cfg, w, toks))
+    print(f"width={width} ff={ff} n={n}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 @DTYPES
 def test_steps_behind_a_very_long_context(tmp_path, f32):
     """Thousands of visible keys: decode steps and short portions split them over many workgroups."""
