@@ -694,15 +694,15 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     a.u = o.u;
     if (o.streams) a.st = *o.streams;
     a.epi = o.epi; a.out = o.out; a.ldo = o.ld; a.bias = o.bias; a.mult = o.mult; a.out_rows = o.rows;
-    // tile: large where it fills the chip, else smaller, else K is split.  256 x 256 from 60 % of a round of one workgroup per CU on:
-    // 5120 x 3072 times 2048 tokens (160 tiles, 62 %) 77 us against 86 on 128 x 128 tiles, 6176 x 4096 times 1900 (78 %) 98 / 119;
-    // below, 4096 x 18432 times 1900 (128 tiles, 50 %) 337 / 268, 3072 x 3072 times 2048 (38 %) 75 / 51
+    // tile: large where it fills the chip, else smaller, else K is split.  256 x 256 where the outputs are at least 55 % of
+    // the rounds of one workgroup per CU: 5120 x 3072 times 2048 tokens (62 %) 77 us against 86 on 128 x 128 tiles, 6176 x 4096
+    // times 1900 (70 %) 98 / 119; below, 4096 x 18432 times 1900 (46 %) 337 / 268, 3072 x 3072 times 2048 (38 %) 75 / 51
     int shape = 2;
     uint32_t bm = 64, bn = 32;
     auto count = [&](uint32_t tm, uint32_t tn) { return static_cast<uint64_t>((a.m + tm - 1) / tm) * ((n + tn - 1) / tn) * groups.count; };
-    const uint64_t wide = count(256, 256), rounds = (wide + ctx->n_cu - 1) / ctx->n_cu;
+    const uint64_t rounds = (count(256, 256) + ctx->n_cu - 1) / ctx->n_cu, area = static_cast<uint64_t>(w.rows) * n;
     if (f32) { bm = bn = 64; }
-    else if (n > 128 && wide * 5 >= rounds * ctx->n_cu * 3) { shape = 3; bm = bn = 256; }
+    else if (n > 128 && area * 20 >= rounds * ctx->n_cu * 65536 * 11) { shape = 3; bm = bn = 256; }
     else if (n > 64 && (count(128, 128) >= ctx->n_cu || (a.kp >= 8192 && count(128, 128) * 4 >= ctx->n_cu))) { shape = 0; bm = bn = 128; }
     else if (n > 32) { shape = 1; bm = bn = 64; }
     a.tiles_m = (a.m + bm - 1) / bm;
@@ -710,14 +710,17 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     const uint64_t wgs = count(bm, bn);
     const uint32_t steps = a.kp / DENSE_PAD;
     uint32_t split = 1;
+    // two workgroups per CU; three quarters of that are left alone on large tiles, whose partial sums cost more than the idle
+    // quarter: 3072 x 3072 times 2048 tokens (384) 51 us whole, 50 + 24 in two parts
     const uint32_t want_wgs = 2 * ctx->n_cu;
-    if (shape != 3 && wgs < want_wgs && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
+    if (shape != 3 && wgs * 4 < want_wgs * (shape == 0 ? 3ull : 4ull) && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
     if (split < 1) split = 1;
     const uint32_t per = (steps + split - 1) / split;
     split = (steps + per - 1) / per;
     a.k_chunk = per * DENSE_PAD;
-    // any number of streams but four: through the reduction, whose threads hold little else
-    const bool apart = o.epi == DENSE_STREAMS && o.streams->count != 4;
+    // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
+    // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
+    const bool apart = o.epi == DENSE_STREAMS && (o.streams->count != 4 || shape == 0 || shape == 3);
     if (split > 1 || apart) {
         void* part;
         CERA_TRY(cera_scratch(ctx, 9, static_cast<uint64_t>(split) * n * a.m * sizeof(float), &part));
@@ -728,10 +731,10 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     const dim3 rg(static_cast<uint32_t>((quads + 255) / 256)), block(256);
     auto go = [&](auto epi, auto streams) {
         constexpr int E = decltype(epi)::value, SN = decltype(streams)::value;
-        constexpr int EG = E == DENSE_STREAMS && SN == 0 ? DENSE_STORE : E;   // leaves partial sums, whatever it is
+        constexpr int EG = E == DENSE_STREAMS && SN == 0 ? DENSE_STORE : E, EL = E == DENSE_STREAMS ? DENSE_STORE : E;   // leave partial sums, whatever it is
         if (f32) hipLaunchKernelGGL((dense_gemm_f32_kernel<EG, SN>), grid, block, 0, ctx->stream, a);
-        else if (shape == 3) hipLaunchKernelGGL((dense_gemm_wide_kernel<EG, SN>), grid, dim3(512), 0, ctx->stream, a);
-        else if (shape == 0) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 128, 128, 2, 2>), grid, block, 0, ctx->stream, a);
+        else if (shape == 3) hipLaunchKernelGGL((dense_gemm_wide_kernel<EL, 0>), grid, dim3(512), 0, ctx->stream, a);
+        else if (shape == 0) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EL, 0, 128, 128, 2, 2>), grid, block, 0, ctx->stream, a);
         else if (shape == 1) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 64, 2, 2>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 32, 2, 2>), grid, block, 0, ctx->stream, a);
         if (!a.part) return;

@@ -145,6 +145,17 @@ cera_hip_status layered_rotation(cera_hip_model* m, const cera_hip_attn_spec& s,
     return CERA_HIP_OK;
 }
 
+cera_hip_status layered_row_logits(cera_hip_model* m, const float* x) {
+    CeraLayered& g = *m->layered;
+    DenseIn in;
+    in.kind = DenseIn::NORM; in.x = x; in.n_mean = g.cfg.width; in.eps = g.cfg.eps; in.scale_a = g.final_norm;
+    DenseOut out;
+    out.out = m->logits; out.rows = g.cfg.vocab;
+    bool ok = false;
+    CERA_TRY(cera_launch_dense_gemv(m->ctx, in, g.head, out, nullptr, nullptr, g.f32, &ok));
+    return ok ? CERA_HIP_OK : cera_fail(m->ctx, CERA_HIP_ERR_SHAPE, "logits: the row does not fit the GEMV");
+}
+
 namespace {
 
 // ---- the decode step ------------------------------------------------------------------------------
@@ -209,14 +220,7 @@ cera_hip_status decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool wan
     g.hist_pos = pos + 1;
     advance_ring(g, pos, pos + 1);
     m->hidden = g.x;
-    if (want_logits) {
-        DenseIn in;
-        in.kind = DenseIn::NORM; in.x = g.x; in.n_mean = width; in.eps = g.cfg.eps; in.scale_a = g.final_norm;
-        DenseOut out;
-        out.out = m->logits; out.rows = g.cfg.vocab;
-        CERA_TRY(gemv(in, g.head, out));
-    }
-    return CERA_HIP_OK;
+    return want_logits ? layered_row_logits(m, g.x) : CERA_HIP_OK;
 }
 
 // ---- the batched pass -----------------------------------------------------------------------------
@@ -298,6 +302,7 @@ cera_hip_status batch_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n
     advance_ring(g, start, start + n);
     m->hidden = g.bx + static_cast<uint64_t>(n - 1) * g.ld;
     if (!last && !all) return CERA_HIP_OK;
+    if (!all && g.step_fits) return layered_row_logits(m, m->hidden);
     NormConv nc;
     nc.x = all ? g.bx : m->hidden; nc.ld = g.ld; nc.n = all ? n : 1; nc.width = width; nc.eps = g.cfg.eps; nc.w = g.final_norm; nc.out_a = g.ba;
     CERA_TRY(cera_launch_norm_conv(ctx, nc, g.f32));

@@ -29,18 +29,6 @@ DenseOut to_streams(const DenseStreams& st, float* x, float* u, uint64_t ld, uin
 
 cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, uint32_t start, bool last, float* all);
 
-// logits of the row u through the final norm
-cera_hip_status row_logits(cera_hip_model* m, const float* u) {
-    L& g = *m->layered;
-    DenseIn in;
-    in.kind = DenseIn::NORM; in.x = u; in.n_mean = g.cfg.width; in.eps = g.cfg.eps; in.scale_a = g.final_norm;
-    DenseOut out;
-    out.out = m->logits; out.rows = g.cfg.vocab;
-    bool ok = false;
-    CERA_TRY(cera_launch_dense_gemv(m->ctx, in, g.head, out, nullptr, nullptr, g.f32, &ok));
-    return ok ? CERA_HIP_OK : cera_fail(m->ctx, CERA_HIP_ERR_SHAPE, "logits: the row does not fit the GEMV");
-}
-
 // ---- the decode step ------------------------------------------------------------------------------
 cera_hip_status seq_decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool want_logits) {
     L& g = *m->layered;
@@ -95,7 +83,7 @@ cera_hip_status seq_decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool
         CERA_TRY(gemv(down, W.down, streams(W.st_ffn)));
     }
     m->hidden = g.u;
-    return want_logits ? row_logits(m, g.u) : CERA_HIP_OK;
+    return want_logits ? layered_row_logits(m, g.u) : CERA_HIP_OK;
 }
 
 // ---- the batched pass -----------------------------------------------------------------------------
@@ -227,7 +215,7 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
     }
     m->hidden = g.bu + static_cast<uint64_t>(n - 1) * g.ld;
     if (!last && !all) return CERA_HIP_OK;
-    if (!all && cera_dense_gemv_fits(g.ld, g.f32)) return row_logits(m, m->hidden);
+    if (!all && cera_dense_gemv_fits(g.ld, g.f32)) return layered_row_logits(m, m->hidden);
     const uint32_t rows = all ? n : 1;
     CERA_TRY(norm(all ? g.bu : m->hidden, rows, g.final_norm));
     DenseOut out;
