@@ -1,0 +1,385 @@
+// Products of Q4_K and Q6_K matrices with a few tokens at once (2 to 48: drafted tokens to verify, a chat turn), read from
+// their decode copies or, with the same bits, from the native blocks.
+//
+// A wavefront owns 16 weight rows and streams their super-blocks straight into registers, two to four of them ahead; the tokens, in
+// tiles of 16, come from LDS, where the workgroup's four wavefronts put them as f16 (the Q8_0 codes are whole numbers, exact
+// in f16), a chunk of super-blocks ahead.  One v_mfma_f32_16x16x32_f16 is one 32-weight block: Q4_K weights enter as
+// scale * code, at most 945 and exact in f16; Q6_K weights, at most 4064, as two f16 parts whose sum they are.  So a block's
+// result is the exact whole number sum(scale * code * quant), below 2^24, and what the vector ALU adds is one FMA with the
+// token's block scale per output and block, one with the row's d per super-block, and for Q4_K one with dmin on the mins'
+// own product (mins times the tokens' block sums in three bf16 parts).  Sums over K go in order within a slice.
+//
+// What bounds it: up to 16 tokens the weights' way from HBM, above that the vector ALU, about 130 (Q4_K) and 225 (Q6_K)
+// instructions per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens.
+#include <algorithm>
+
+#include "gemv.hip.h"
+#include "gemm_few.h"
+
+namespace {
+
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+struct FewArgs {
+    FewMat a, b;               // b: a second matrix of the same type and k, or m = 0
+    uint32_t tiles_a;          // workgroups of a
+    const int8_t* xq;
+    const float *xs, *bsum;
+    uint32_t n, k, row_bytes, sb_per;
+    uint64_t part_stride;      // floats between the slices of a split K; 0: no split
+    const float* resid;        // added to segment 0 of a (unsplit)
+    float resid_scale;
+};
+
+constexpr int FEW_WAVES = 4, FEW_ROWS = 16 * FEW_WAVES;
+// LDS of one tile of 16 tokens and one super-block: a block's operand fragments (64 lanes x 16 bytes, the blocks 16 bytes
+// further apart than that, so that the eight blocks of a token do not share their banks when they are written), the block
+// scales, the mins' operand
+constexpr uint32_t FEW_BLOCK = 1040, FEW_XS = 8 * FEW_BLOCK, FEW_MIN = FEW_XS + 512, FEW_TILE = FEW_MIN + 1024;
+
+__device__ __forceinline__ h2v as_h2(uint32_t v) { return __builtin_bit_cast(h2v, v); }
+__device__ __forceinline__ h2v fma2(h2v a, h2v b, h2v c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ h2v both(float v) { return h2v{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
+// bytes 0 and 2, or 1 and 3, of v as 1024 + byte
+__device__ __forceinline__ h2v bytes02(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)); }
+__device__ __forceinline__ h2v bytes13(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
+// byte j of v, twice, as 1024 + byte
+template <int J> __device__ __forceinline__ h2v byte_twice(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | J | J << 16)); }
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {   // a's upper 32 lanes with b's lower 32
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0]; b = r[1];
+}
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {   // a's odd rows of 16 lanes with b's even ones
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0]; b = r[1];
+}
+
+// ---- Q4_K -----------------------------------------------------------------------------------------
+// Lane group g (of 16 lanes, one per row) loads unit g of the super-block, the blocks 2g and 2g + 1, in two 16-byte halves,
+// and after the exchange holds dword g of both halves of every unit: codes 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3 of a block.
+struct FewQ4 {
+    static constexpr bool MINS = true;
+    struct W { uint4 h, f, s; };
+    static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * e + g; }   // e-th dword of a block's quants in lane group g
+    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* row, uint32_t sb, uint32_t g, uint32_t nsb) {
+        if (COPY) {
+            w.h = ld_u128(row + sb * 16);
+            w.f = ld_u128(row + Q4K::stream_q0(4 * nsb) + (sb * 4 + g) * 16);
+            w.s = ld_u128(row + Q4K::stream_q1(4 * nsb) + (sb * 4 + g) * 16);
+        } else {
+            const uint8_t* const blk = row + sb * 144;
+            w.h = ld_u128(blk);
+            w.f = ld_u128(blk + 16 + g * 32);
+            w.s = ld_u128(blk + 32 + g * 32);
+        }
+    }
+    template <int T>
+    static __device__ __forceinline__ void multiply(const W& w, const unsigned char* st, uint32_t lane, f4v (&acc)[T]) {
+        uint32_t f[4] = {w.f.x, w.f.y, w.f.z, w.f.w}, s[4] = {w.s.x, w.s.y, w.s.z, w.s.w};
+        swap32(f[0], f[2]); swap32(f[1], f[3]); swap32(s[0], s[2]); swap32(s[1], s[3]);
+        swap16(f[0], f[1]); swap16(f[2], f[3]); swap16(s[0], s[1]); swap16(s[2], s[3]);   // now by unit
+        const uint32_t sc[2] = {w.h.y & 0x3F3F3F3Fu, (w.h.w & 0x0F0F0F0Fu) | ((w.h.y >> 2) & 0x30303030u)};
+        const uint32_t mn[2] = {w.h.z & 0x3F3F3F3Fu, ((w.h.w >> 4) & 0x0F0F0F0Fu) | ((w.h.z >> 2) & 0x30303030u)};
+        const f4v zero{0.f, 0.f, 0.f, 0.f};
+        f4v sum[T];
+        auto unit = [&](auto u_) {
+            constexpr int u = decltype(u_)::value;
+            // 1024 + code, and for the upper nibbles 1024 + 16 code in place; the FMA leaves scale * code
+            const h2v s0 = byte_twice<2 * (u & 1)>(sc[u >> 1]) - both(1024.f), s1 = (byte_twice<2 * (u & 1) + 1>(sc[u >> 1]) - both(1024.f)) * both(0.0625f);
+            const h2v o0 = s0 * both(-1024.f), o1 = s1 * both(-1024.f);
+            h8v lo, hi;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t q = e ? s[u] : f[u], r = q >> 8;
+                const h2v a = fma2(as_h2((q & 0x000F000Fu) | 0x64006400u), s0, o0), b = fma2(as_h2((r & 0x000F000Fu) | 0x64006400u), s0, o0);
+                const h2v c = fma2(as_h2((q & 0x00F000F0u) | 0x64006400u), s1, o1), d = fma2(as_h2((r & 0x00F000F0u) | 0x64006400u), s1, o1);
+                lo[4 * e] = a[0]; lo[4 * e + 1] = a[1]; lo[4 * e + 2] = b[0]; lo[4 * e + 3] = b[1];
+                hi[4 * e] = c[0]; hi[4 * e + 1] = c[1]; hi[4 * e + 2] = d[0]; hi[4 * e + 3] = d[1];
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const unsigned char* const p = st + t * FEW_TILE;
+#pragma unroll
+                for (int z = 0; z < 2; ++z) {
+                    const int b = 2 * u + z;
+                    const f4v r = __builtin_amdgcn_mfma_f32_16x16x32_f16(z ? hi : lo, *reinterpret_cast<const h8v*>(p + b * FEW_BLOCK + lane * 16), zero, 0, 0, 0);
+                    const float xs = *reinterpret_cast<const float*>(p + FEW_XS + b * 64 + (lane & 15) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum[t][i] = b ? fmaf(r[i], xs, sum[t][i]) : r[i] * xs;
+                }
+                if (T > 2 && (t & 1)) __builtin_amdgcn_sched_barrier(0);   // else the fragments of all tiles and units are read at once, and spilled
+            }
+        };
+        unit(std::integral_constant<int, 0>{}); unit(std::integral_constant<int, 1>{});
+        unit(std::integral_constant<int, 2>{}); unit(std::integral_constant<int, 3>{});
+        b8v am;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) am[b] = static_cast<__bf16>(static_cast<float>((mn[b >> 2] >> (8 * (b & 3))) & 0xFF));
+        float d[4], dm[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.h.x)));
+            d[i] = h2f(v & 0xFFFF); dm[i] = -h2f(v >> 16);
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const f4v m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, *reinterpret_cast<const b8v*>(st + t * FEW_TILE + FEW_MIN + lane * 16), zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(dm[i], m[i], fmaf(d[i], sum[t][i], acc[t][i]));
+        }
+    }
+};
+
+// ---- Q6_K -----------------------------------------------------------------------------------------
+// Unit (h, j): run j of 16 codes of the four blocks of half h.  Lane group 2h + j loads it and after the exchange holds, as
+// group 2a + j, dwords 2a and 2a + 1 of the runs j of both halves: codes 16j + 8a .. 16j + 8a + 7 of a block.
+struct FewQ6 {
+    static constexpr bool MINS = false;
+    struct W { uint4 a, b, q, sc; uint32_t d; };
+    static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * (g & 1) + 2 * (g >> 1) + e; }
+    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* row, uint32_t sb, uint32_t g, uint32_t nsb) {
+        if (!COPY) {
+            const uint8_t* const blk = row + sb * 210;
+            w.a = ld_u128_a2(blk + (g >> 1) * 64 + (g & 1) * 16);
+            w.b = ld_u128_a2(blk + (g >> 1) * 64 + 32 + (g & 1) * 16);
+            w.q = ld_u128_a2(blk + 128 + (g >> 1) * 32 + (g & 1) * 16);
+            w.sc = ld_u128_a2(blk + 192);
+            w.d = ld_u16(blk + 208);
+            return;
+        }
+        const uint32_t plane = Q6K::up128(64 * nsb), at = (sb * 4 + g) * 16;
+        w.a = ld_u128(row + at);
+        w.b = ld_u128(row + plane + at);
+        w.q = ld_u128(row + 2 * plane + at);
+        w.sc = ld_u128(row + Q6K::stream_sc(4 * nsb) + sb * 16);
+        w.d = ld_u16(row + Q6K::stream_d(4 * nsb) + sb * 2);
+    }
+    template <int T>
+    static __device__ __forceinline__ void multiply(const W& w, const unsigned char* st, uint32_t lane, f4v (&acc)[T]) {
+        uint32_t a[4] = {w.a.x, w.a.y, w.a.z, w.a.w}, b[4] = {w.b.x, w.b.y, w.b.z, w.b.w}, q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
+        swap32(a[0], a[2]); swap32(a[1], a[3]); swap32(b[0], b[2]); swap32(b[1], b[3]); swap32(q[0], q[2]); swap32(q[1], q[3]);   // now [half][dword]
+        const uint32_t sh = 8 * ((lane >> 4) & 1);
+        const f4v zero{0.f, 0.f, 0.f, 0.f};
+        f4v sum[T];
+        auto half = [&](auto h_) {
+            constexpr int h = decltype(h_)::value;
+            h8v hi[4], lo[4];
+            const uint32_t s01 = ((h ? w.sc.z : w.sc.x) ^ 0x80808080u) >> sh, s23 = ((h ? w.sc.w : w.sc.y) ^ 0x80808080u) >> sh;
+            const h2v sc[4] = {byte_twice<0>(s01) - both(1152.f), byte_twice<2>(s01) - both(1152.f), byte_twice<0>(s23) - both(1152.f), byte_twice<2>(s23) - both(1152.f)};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t qa = a[2 * h + e], qb = b[2 * h + e], qh = q[2 * h + e];
+                const uint32_t c[4] = {(qa & 0x0F0F0F0Fu) | ((qh << 4) & 0x30303030u), (qb & 0x0F0F0F0Fu) | ((qh << 2) & 0x30303030u),
+                                       ((qa >> 4) & 0x0F0F0F0Fu) | (qh & 0x30303030u), ((qb >> 4) & 0x0F0F0F0Fu) | ((qh >> 2) & 0x30303030u)};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    // code - 32, times the scale: rounded to f16, and the remainder
+                    const h2v x = bytes02(c[t]) - both(1056.f), y = bytes13(c[t]) - both(1056.f);
+                    const h2v xh = x * sc[t], yh = y * sc[t], xl = fma2(x, sc[t], -xh), yl = fma2(y, sc[t], -yh);
+                    hi[t][4 * e] = xh[0]; hi[t][4 * e + 1] = xh[1]; hi[t][4 * e + 2] = yh[0]; hi[t][4 * e + 3] = yh[1];
+                    lo[t][4 * e] = xl[0]; lo[t][4 * e + 1] = xl[1]; lo[t][4 * e + 2] = yl[0]; lo[t][4 * e + 3] = yl[1];
+                }
+            }
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const int blk = 4 * h + z;
+                    const unsigned char* const p = st + t * FEW_TILE;
+                    const h8v x = *reinterpret_cast<const h8v*>(p + blk * FEW_BLOCK + lane * 16);
+                    f4v r = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[z], x, zero, 0, 0, 0);
+                    r = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[z], x, r, 0, 0, 0);
+                    const float xs = *reinterpret_cast<const float*>(p + FEW_XS + blk * 64 + (lane & 15) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum[t][i] = blk ? fmaf(r[i], xs, sum[t][i]) : r[i] * xs;
+                }
+                if (T > 2) __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        half(std::integral_constant<int, 0>{}); half(std::integral_constant<int, 1>{});
+        float d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = h2f(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.d))));
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[i], sum[t][i], acc[t][i]);
+    }
+};
+
+// T tiles of 16 tokens; S super-blocks a chunk, so that a chunk is four tiles (three for T = 3) and two of them fill half the
+// LDS.  Four tiles of tokens would spill registers.
+template <typename W, int T, bool COPY>
+__global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) {
+    constexpr int S = T == 1 ? 4 : T == 2 ? 2 : 1, AHEAD = T > 2 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+    __shared__ __align__(16) unsigned char lds[2][S * T * FEW_TILE];
+    const bool second = blockIdx.x >= a.tiles_a;
+    const FewMat& M = second ? a.b : a.a;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nsb = a.k / 256;
+    const uint32_t row0 = (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
+    const uint32_t sb0 = blockIdx.y * a.sb_per, sb1 = min(nsb, sb0 + a.sb_per);
+    const uint8_t* const row = M.w + static_cast<uint64_t>(min(row0 + (lane & 15), M.m - 1)) * a.row_bytes;   // rows past the end: the last one again
+    // the tokens of a chunk: a thread takes the 32 quants of one block of one token
+    uint4 q0[NP], q1[NP];
+    float xs[NP], bs[NP];
+    auto act_load = [&](uint32_t sb) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x, tile = p >> 7, tok = min((tile % T) * 16 + ((p >> 3) & 15), a.n - 1);
+            const uint32_t blk = min(sb + tile / T, sb1 - 1) * 8 + (p & 7);
+            if (PAIRS % (FEW_WAVES * 64) && p >= PAIRS) break;
+            const int8_t* const x = a.xq + static_cast<uint64_t>(tok) * a.k + blk * 32;
+            q0[i] = *reinterpret_cast<const uint4*>(x);
+            q1[i] = *reinterpret_cast<const uint4*>(x + 16);
+            xs[i] = a.xs[static_cast<uint64_t>(tok) * (a.k / 32) + blk];
+            if (W::MINS) bs[i] = a.bsum[static_cast<uint64_t>(tok) * (a.k / 32) + blk];
+        }
+    };
+    auto act_store = [&](uint32_t buf) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x, tok = (p >> 3) & 15, b = p & 7;
+            if (PAIRS % (FEW_WAVES * 64) && p >= PAIRS) break;
+            unsigned char* const t = &lds[buf][(p >> 7) * FEW_TILE];
+            const uint32_t q[8] = {q0[i].x, q0[i].y, q0[i].z, q0[i].w, q1[i].x, q1[i].y, q1[i].z, q1[i].w};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                h2v v[4];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t u = q[W::dword(g, e)] ^ 0x80808080u;
+                    v[2 * e] = bytes02(u) - both(1152.f);
+                    v[2 * e + 1] = bytes13(u) - both(1152.f);
+                }
+                *reinterpret_cast<h8v*>(t + b * FEW_BLOCK + (g * 16 + tok) * 16) = h8v{v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
+            }
+            *reinterpret_cast<float*>(t + FEW_XS + b * 64 + tok * 4) = xs[i];
+            if (W::MINS) {   // three bf16 parts that add up to the block sum, and a zero
+                float rest = bs[i];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const uint32_t top = g < 3 ? __builtin_bit_cast(uint32_t, rest) & 0xFFFF0000u : 0u;
+                    rest -= __builtin_bit_cast(float, top);
+                    *reinterpret_cast<uint16_t*>(t + FEW_MIN + (g * 16 + tok) * 16 + b * 2) = static_cast<uint16_t>(top >> 16);
+                }
+            }
+        }
+    };
+    typename W::W w[AHEAD];
+    act_load(sb0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+        if (sb0 + i < sb1) W::template load<COPY>(w[i], row, sb0 + i, lane >> 4, nsb);
+    f4v acc[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
+    act_store(0);
+    uint32_t buf = 0;
+    for (uint32_t base = sb0; base < sb1; base += AHEAD) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const uint32_t sb = base + i;
+            if (sb < sb1) {
+                const uint32_t next = sb - i % S + S;   // the chunk behind this one
+                if (i % S == 0) {
+                    // this chunk is written, and no wavefront reads the other buffer any more
+                    lds_barrier();
+                    if (next < sb1) act_load(next);
+                }
+                W::template multiply<T>(w[i], &lds[buf][(i % S) * T * FEW_TILE], lane, acc);
+                if (sb + AHEAD < sb1) W::template load<COPY>(w[i], row, sb + AHEAD, lane >> 4, nsb);
+                if (i % S == S - 1 && next < sb1) {
+                    buf ^= 1;
+                    act_store(buf);
+                }
+            }
+        }
+    }
+    // four consecutive rows of one token per lane and tile
+    const uint32_t r0 = row0 + (lane >> 4) * 4;
+    if (r0 >= M.m) return;
+    const int seg = r0 < M.cut[0] ? 0 : r0 < M.cut[1] ? 1 : 2;   // the cuts are multiples of four
+    float* const out = M.out[seg] + blockIdx.y * a.part_stride + (r0 - (seg ? M.cut[seg - 1] : 0));
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const uint32_t tok = t * 16 + (lane & 15);
+        if (tok >= a.n) continue;
+        const uint64_t at = static_cast<uint64_t>(tok) * M.ld[seg];
+        f4v v = acc[t];
+        if (a.resid && !second && seg == 0) {
+            const f4v r = *reinterpret_cast<const f4v*>(a.resid + at + r0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = r[i] + (a.resid_scale != 1.0f ? v[i] * a.resid_scale : v[i]);
+        }
+        *reinterpret_cast<f4v*>(out + at) = v;
+    }
+}
+
+}  // namespace
+
+bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n) {
+    return w && (w->dtype == CERA_HIP_Q6_K || (reinterpret_cast<uintptr_t>(w->dev) & 15) == 0) && (w->dtype == CERA_HIP_Q4_K || w->dtype == CERA_HIP_Q6_K) && w->k >= FEW_MIN_K && w->k % 256 == 0 && w->m % 4 == 0 && w->m < (1u << 30) && n >= 2 &&
+           n <= FEW_MAX_TOKENS;
+}
+
+cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const FewOut* ob, const float* xs, const int8_t* xq, const float* bsum, uint32_t n,
+                                     const float* resid, float resid_scale, int part_slot, FewParts* parts) {
+    const cera_hip_dtensor* w = oa.w;
+    if (!cera_gemm_few_supports(w, n) || (ob && (!cera_gemm_few_supports(ob->w, n) || ob->w->dtype != w->dtype || ob->w->k != w->k)))
+        return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "gemm_few: bad shape");
+    FewArgs a{};
+    const bool copy = w->dev_stream && (!ob || ob->w->dev_stream);
+    a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k); a.row_bytes = static_cast<uint32_t>(copy ? w->stream_row_bytes : w->row_bytes);
+    auto tiles = [](const cera_hip_dtensor* t) { return static_cast<uint32_t>((t->m + FEW_ROWS - 1) / FEW_ROWS); };
+    a.tiles_a = tiles(w);
+    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = 2 * ctx->n_cu;
+    // K is split where the rows leave more than a quarter of two workgroups per CU idle, down to two super-blocks a slice
+    uint32_t split = wgs * 4 >= want * 3 ? 1 : std::min({(want + wgs - 1) / wgs, std::max(nsb / 2, 1u), 8u});
+    a.sb_per = (nsb + split - 1) / split;
+    split = (nsb + a.sb_per - 1) / a.sb_per;
+    uint64_t rows = 0;
+    float* part = nullptr;
+    auto set = [&](FewMat& m, const FewOut& o) {
+        m.w = copy ? o.w->dev_stream : o.w->dev;
+        m.m = static_cast<uint32_t>(o.w->m);
+        uint32_t at = 0;
+        for (int s = 0; s < 3; ++s) {   // segments lie side by side in a slice, as outputs of their own would
+            const uint32_t len = std::min(s < 2 && o.len[s] ? o.len[s] : m.m - at, m.m - at);
+            m.out[s] = split > 1 ? part + (rows + at) * n : o.out[s];
+            m.ld[s] = len;
+            at += len;
+            if (s < 2) m.cut[s] = at;
+        }
+        rows += m.m;
+    };
+    if (split > 1) {
+        void* p;
+        CERA_TRY(cera_scratch(ctx, part_slot, split * (w->m + (ob ? ob->w->m : 0)) * static_cast<uint64_t>(n) * 4, &p));
+        part = static_cast<float*>(p);
+    } else {
+        a.resid = resid; a.resid_scale = resid_scale;
+    }
+    set(a.a, oa);
+    if (ob) set(a.b, *ob);
+    a.part_stride = split > 1 ? rows * n : 0;
+    *parts = FewParts{part, split, a.part_stride};
+    const dim3 grid(wgs, split), block(FEW_WAVES * 64);
+    auto go = [&](auto type, auto from_copy) {
+        using W = decltype(type);
+        constexpr bool COPY = decltype(from_copy)::value;
+        if (n <= 16) hipLaunchKernelGGL((gemm_few_kernel<W, 1, COPY>), grid, block, 0, ctx->stream, a);
+        else if (n <= 32) hipLaunchKernelGGL((gemm_few_kernel<W, 2, COPY>), grid, block, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((gemm_few_kernel<W, 3, COPY>), grid, block, 0, ctx->stream, a);
+    };
+    auto of_type = [&](auto from_copy) {
+        if (w->dtype == CERA_HIP_Q4_K) go(FewQ4{}, from_copy);
+        else go(FewQ6{}, from_copy);
+    };
+    if (copy) of_type(std::true_type{});
+    else of_type(std::false_type{});
+    HIP_TRY(ctx, hipGetLastError());
+    return CERA_HIP_OK;
+}

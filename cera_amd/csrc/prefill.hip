@@ -9,6 +9,7 @@
 #include "gemm_q5k_f16.hip.h"
 #include "gemm_q6k_f16.hip.h"
 #include "gemm_fp8.hip.h"
+#include "gemm_few.h"
 #include "glue.hip.h"
 #include "model.h"
 
@@ -343,6 +344,26 @@ extern "C" cera_hip_status cera_hip_gemm_pair(cera_hip_ctx* ctx, const cera_hip_
         CERA_TRY(cera_hip_upload(ctx, dx, x, n * k * 4));
         CERA_TRY(quantize_rows(ctx, static_cast<float*>(dx), n, k, static_cast<float*>(ds), static_cast<int8_t*>(dq),
                                static_cast<float*>(db)));
+        if (n >= 2 && n <= FEW_MAX_TOKENS && cera_gemm_few_supports(wa, static_cast<uint32_t>(n)) && cera_gemm_few_supports(wb, static_cast<uint32_t>(n))) {
+            // as the forward pass does, whose matrices have decode copies
+            CERA_TRY(cera_tensor_prepare_stream(ctx, wa));
+            CERA_TRY(cera_tensor_prepare_stream(ctx, wb));
+            FewOut oa, ob;
+            oa.w = wa; oa.out[0] = static_cast<float*>(dya);
+            ob.w = wb; ob.out[0] = static_cast<float*>(dyb);
+            FewParts p;
+            CERA_TRY(cera_launch_gemm_few(ctx, oa, &ob, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
+                                          static_cast<uint32_t>(n), nullptr, 1.0f, 9, &p));
+            if (p.n_split > 1) {
+                const uint64_t n4 = wa->m * n / 4, all4 = n4 + wb->m * n / 4;
+                hipLaunchKernelGGL(gemm_reduce_kernel, dim3(static_cast<uint32_t>((all4 + 255) / 256)), dim3(256), 0, ctx->stream, p.part,
+                                   p.n_split, p.stride, all4, static_cast<float*>(dya), static_cast<const float*>(nullptr), 1.0f, n4,
+                                   static_cast<float*>(dyb));
+                HIP_TRY(ctx, hipGetLastError());
+            }
+            CERA_TRY(cera_hip_download(ctx, out_a, dya, n * wa->m * 4));
+            return cera_hip_download(ctx, out_b, dyb, n * wb->m * 4);
+        }
         bool paired = false;
         CERA_TRY(cera_launch_gemm(ctx, wa, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
                                   static_cast<uint32_t>(n), static_cast<float*>(dya), 1, wa->m, nullptr, 1.0f, wb,
@@ -508,6 +529,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
 
     // whether pf_xh holds the f16 form of the quants now in pf_xq; cleared wherever those are rewritten
     bool staged = false;
+    const bool few_tokens = n <= FEW_MAX_TOKENS;
     // the same for pf_x8, the fp8 split copy the Q4_K GEMMs read
     bool staged8 = false;
     // the f32 activations whose hi / lo split (Q5_K GEMMs) the context's workspace holds now
@@ -531,10 +553,31 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         HIP_TRY(ctx, hipGetLastError());
         return CERA_HIP_OK;
     };
+    // the kernel for a few tokens: o (and o2) of the quantized activations; sums over a split K are added up here unless
+    // `pending` takes them
+    auto few = [&](const FewOut& o, const FewOut* o2, const float* resid, RowsPending* pending, int part_slot) -> cera_hip_status {
+        FewParts p;
+        CERA_TRY(cera_launch_gemm_few(ctx, o, o2, m->pf_xs, m->pf_xq, m->pf_bsum, n, resid, c.residual_scale, part_slot, &p));
+        if (p.n_split == 1) return CERA_HIP_OK;
+        if (pending) {
+            *pending = RowsPending{p.part, p.n_split, p.stride, resid, c.residual_scale, o.out[0]};
+            return CERA_HIP_OK;
+        }
+        const uint64_t n4 = o.w->m * n / 4, all4 = n4 + (o2 ? o2->w->m * n / 4 : 0);
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3(static_cast<uint32_t>((all4 + 255) / 256)), dim3(256), 0, s, p.part, p.n_split, p.stride, all4,
+                           o.out[0], resid, c.residual_scale, n4, o2 ? o2->out[0] : static_cast<float*>(nullptr));
+        HIP_TRY(ctx, hipGetLastError());
+        return CERA_HIP_OK;
+    };
     // out[n][w->m] (token-major rows) = B . W^T, optionally added onto resid
     // xf: the f32 activations the quantized ones in pf_xs / pf_xq were made from (what a Q5_K matrix reads)
     auto gemm = [&](const cera_hip_dtensor* w, float* out, const float* resid, const float* xf,
                     RowsPending* pending = nullptr, int part_slot = 9) -> cera_hip_status {
+        if (few_tokens && cera_gemm_few_supports(w, n)) {
+            FewOut o;
+            o.w = w; o.out[0] = out;
+            return few(o, nullptr, resid, pending, part_slot);
+        }
         // a short batch streams the weights once per 8 tokens through the multi-token GEMV (an
         // int8-MFMA tile would be mostly empty); its residual add is unscaled
         if ((n <= PREFILL_SMALL_BATCH || !gemm_batched(w->dtype, w->k)) && (!resid || c.residual_scale == 1.0f)) {
@@ -557,6 +600,12 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     // pending (nullable): filled when the two went out as one launch whose split-K partial sums the caller adds up
     auto gemm2 = [&](const cera_hip_dtensor* wa, float* outa, const cera_hip_dtensor* wb, float* outb, const float* xf,
                      RowsPending* pending = nullptr) -> cera_hip_status {
+        if (few_tokens && cera_gemm_few_supports(wa, n) && cera_gemm_few_supports(wb, n) && wa->dtype == wb->dtype && wa->k == wb->k) {
+            FewOut oa, ob;
+            oa.w = wa; oa.out[0] = outa;
+            ob.w = wb; ob.out[0] = outb;
+            return few(oa, &ob, nullptr, pending, 9);
+        }
         if (n > PREFILL_SMALL_BATCH && gemm_batched(wa->dtype, wa->k) && gemm_batched(wb->dtype, wb->k)) {
             bool paired = false;
             bool split_held = split_of == xf;
@@ -583,8 +632,10 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     for (uint32_t i = 0; i < c.n_layers; ++i) {
         LayerDev& L = m->layers[i];
         CERA_TRY(norm_rows(m->pf_hidden, L.attn_norm, m->pf_normed));
+        // the joint Q | K (| V) matrix in one launch
+        const bool few_qkv = few_tokens && cera_gemm_few_supports(L.qkv, n);
         // Q4_K Q and K next to a Q6_K V (the Q4_K_M mix): both re-laid copies of the activations in one launch
-        if (n > PREFILL_SMALL_BATCH && L.q->dtype == CERA_HIP_Q4_K && L.k->dtype == CERA_HIP_Q4_K && L.v->dtype == CERA_HIP_Q6_K &&
+        if (n > PREFILL_SMALL_BATCH && !few_qkv && L.q->dtype == CERA_HIP_Q4_K && L.k->dtype == CERA_HIP_Q4_K && L.v->dtype == CERA_HIP_Q6_K &&
             gemm_batched(CERA_HIP_Q4_K, hs) && gemm_batched(CERA_HIP_Q6_K, hs)) {
             hipLaunchKernelGGL(gemm_act_fp8_kernel, dim3((n + G8_BN - 1) / G8_BN * 2 * (hs / 256)), dim3(256), 0, s, m->pf_xq, m->pf_xs,
                                m->pf_bsum, static_cast<uint8_t*>(m->pf_x8), n, hs, static_cast<uint4*>(m->pf_xh));
@@ -596,8 +647,21 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         // the split-K partial sums of Q | K and of V itself: two reduction launches less.
         RowsPending pqk{}, pvv{};
         const bool rope_adds = !L.q_bias && !L.q_norm;
-        CERA_TRY(gemm2(L.q, m->pf_q, L.k, m->pf_k, m->pf_normed, rope_adds ? &pqk : nullptr));
-        CERA_TRY(gemm(L.v, m->pf_v, nullptr, m->pf_normed, rope_adds ? &pvv : nullptr, 14));
+        if (few_qkv && rope_adds) {
+            FewOut o;
+            o.w = L.qkv;
+            o.len[0] = q_dim; o.len[1] = kv_dim;
+            o.out[0] = m->pf_q; o.out[1] = m->pf_k; o.out[2] = m->pf_v;
+            CERA_TRY(few(o, nullptr, nullptr, &pqk, 9));
+            if (L.qkv_rows > q_dim + kv_dim) {
+                if (pqk.n_split) pvv = RowsPending{pqk.part + static_cast<uint64_t>(n) * (q_dim + kv_dim), pqk.n_split, pqk.stride, nullptr, 1.0f, m->pf_v};
+            } else {
+                CERA_TRY(gemm(L.v, m->pf_v, nullptr, m->pf_normed, &pvv, 14));
+            }
+        } else {
+            CERA_TRY(gemm2(L.q, m->pf_q, L.k, m->pf_k, m->pf_normed, rope_adds ? &pqk : nullptr));
+            CERA_TRY(gemm(L.v, m->pf_v, nullptr, m->pf_normed, rope_adds ? &pvv : nullptr, 14));
+        }
         if (L.q_bias) {
             // bias rows: one launch per token keeps the kernel trivial; models with biases are rare here
             for (uint32_t t = 0; t < n; ++t) {
@@ -651,7 +715,8 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         float *const hs = m->pf_up, *const hb = m->pf_up + static_cast<uint64_t>(n) * (c.ffn / 32);
         // a Q6_K down projection reads its activations as f16: the SwiGLU epilogue of the fp8 kernel writes them too
         const bool hh = L.gate->dtype == CERA_HIP_Q4_K && L.down->dtype == CERA_HIP_Q6_K;
-        if (n > PREFILL_SMALL_BATCH && L.down->dtype != CERA_HIP_Q5_K)   // a Q5_K down projection reads the f32 SwiGLU output
+        const bool few_gate_up = few_tokens && cera_gemm_few_supports(L.gate, n) && cera_gemm_few_supports(L.up, n);
+        if (n > PREFILL_SMALL_BATCH && !few_gate_up && L.down->dtype != CERA_HIP_Q5_K)   // a Q5_K down projection reads the f32 SwiGLU output
             CERA_TRY(cera_launch_gemm_swiglu(ctx, L.gate, L.up, m->pf_xs, m->pf_xq, m->pf_bsum, n, hq, hs, hb, &fused, m->pf_x8, &staged8,
                                              hh ? m->pf_xh : nullptr));
         staged = fused && hh;   // pf_xh: the down projection's activations, or stale

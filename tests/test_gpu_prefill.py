@@ -104,6 +104,34 @@ def test_gemm_pair_matches_single_launches(hip, orc, dtype, ma, mb, n, k):
     assert np.abs(ob[:, rows].T.astype(np.float64) - ref).max() <= GEMM_TOL * util.rms(ref)
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("ma,mb,k", [(300, 68, 2048), (64, 4, 2304), (132, 1024, 14336)])
+@pytest.mark.parametrize("n", [2, 5, 16, 17, 32, 33, 48])
+def test_gemm_pair_of_a_few_tokens(hip, orc, dtype, ma, mb, k, n):
+    """Two to 48 tokens against the exact product of the dequantized weights and quantized tokens: block results are whole
+    numbers, so what is left is the rounding of k / 32 sums, sqrt(448) 2^-24 of a partial sum or about 1.3e-6 of the outputs'
+    rms at the longest row, and 2e-5 is fifteen times that.  Last tiles of rows and tokens, one to four tokens of a last tile,
+    slices of K that do not divide into the chunks read ahead; the native
+    bytes give the same bits as the decode copy."""
+    _say(f"few tokens {util.NAMES[dtype]} ma={ma} mb={mb} k={k} n={n}")
+    wa, _ = util.make_weights(dtype, ma, k, seed=51)
+    wb, _ = util.make_weights(dtype, mb, k, seed=52)
+    x = util.rng(n + k).standard_normal((n, k)).astype(np.float32) * np.exp2(util.rng(n).integers(-6, 7, (n, 1))).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    oa, ob = hip.gemm_pair(dtype, wa, ma, dtype, wb, mb, x, n, k)
+    hip.set_decode_copies(False)
+    try:
+        native = hip.gemm_pair(dtype, wa, ma, dtype, wb, mb, x, n, k)
+    finally:
+        hip.set_decode_copies(True)
+    assert np.array_equal(oa, native[0]) and np.array_equal(ob, native[1])
+    for got, w, m in ((oa, wa, ma), (ob, wb, mb)):
+        want = xd @ util.dequant_np(dtype, w, m, k).astype(np.float64).T
+        rms = np.sqrt(np.mean(want * want, axis=1, keepdims=True))
+        assert (np.abs(got - want) / rms).max() <= 2e-5
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q4_0, Q4_1, Q8_0])
 @pytest.mark.parametrize("m,k,n,want_fused", [(2048, 512, 1040, True), (1056, 256, 2000, True), (512, 256, 70, False)])
 def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n, want_fused):
