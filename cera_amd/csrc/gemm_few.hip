@@ -34,7 +34,7 @@ struct FewArgs {
     float resid_scale;
 };
 
-constexpr int FEW_WAVES = 4, FEW_ROWS = 16 * FEW_WAVES;
+constexpr int FEW_WAVES = 8, FEW_ROWS = 16 * FEW_WAVES;
 // LDS of one tile of 16 tokens and one super-block: a block's operand fragments (64 lanes x 16 bytes, the blocks 16 bytes
 // further apart than that, so that the eight blocks of a token do not share their banks when they are written), the block
 // scales, the mins' operand
@@ -57,6 +57,14 @@ __device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {   // a's odd 
     a = r[0]; b = r[1];
 }
 
+// Masks and biases in registers of their own: an instruction of this kind takes no literal, and two steps otherwise.
+struct Consts { uint32_t lo, hi, bias; };
+__device__ __forceinline__ Consts consts() {
+    Consts c{0x000F000Fu, 0x00F000F0u, 0x64006400u};
+    asm("" : "+s"(c.lo)); asm("" : "+s"(c.hi)); asm("" : "+v"(c.bias));
+    return c;
+}
+
 // ---- Q4_K -----------------------------------------------------------------------------------------
 // Lane group g (of 16 lanes, one per row) loads unit g of the super-block, the blocks 2g and 2g + 1, in two 16-byte halves,
 // and after the exchange holds dword g of both halves of every unit: codes 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3 of a block.
@@ -64,20 +72,38 @@ struct FewQ4 {
     static constexpr bool MINS = true;
     struct W { uint4 h, f, s; };
     static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * e + g; }   // e-th dword of a block's quants in lane group g
-    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* row, uint32_t sb, uint32_t g, uint32_t nsb) {
-        if (COPY) {
-            w.h = ld_u128(row + sb * 16);
-            w.f = ld_u128(row + Q4K::stream_q0(4 * nsb) + (sb * 4 + g) * 16);
-            w.s = ld_u128(row + Q4K::stream_q1(4 * nsb) + (sb * 4 + g) * 16);
-        } else {
-            const uint8_t* const blk = row + sb * 144;
-            w.h = ld_u128(blk);
-            w.f = ld_u128(blk + 16 + g * 32);
-            w.s = ld_u128(blk + 32 + g * 32);
-        }
+    // a lane's offsets from the matrix's first byte, and the super-block's three loads at them: the base that moves is scalar
+    struct At { uint32_t h, f, s; };
+    template <bool COPY> static __device__ __forceinline__ At at(uint32_t row, uint32_t g, uint32_t nsb) {
+        if (COPY) return At{row, row + Q4K::stream_q0(4 * nsb) + g * 16, row + Q4K::stream_q1(4 * nsb) + g * 16};
+        return At{row, row + 16 + g * 32, row + 32 + g * 32};
+    }
+    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* m, uint32_t sb, const At& o) {
+        const uint8_t *const h = m + sb * (COPY ? 16u : 144u), *const q = m + sb * (COPY ? 64u : 144u);
+        w.h = ld_u128(h + o.h);
+        w.f = ld_u128(q + o.f);
+        w.s = ld_u128(q + o.s);
     }
     template <int T>
     static __device__ __forceinline__ void multiply(const W& w, const unsigned char* st, uint32_t lane, f4v (&acc)[T]) {
+        // the tokens' fragments and scales of a unit's two blocks, read a unit ahead
+        h8v x[2][T][2];
+        float xs[2][T][2];
+        auto read = [&](int u) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int z = 0; z < 2; ++z) {
+                    const unsigned char* const p = st + t * FEW_TILE;
+                    x[u & 1][t][z] = *reinterpret_cast<const h8v*>(p + (2 * u + z) * FEW_BLOCK + lane * 16);
+                    xs[u & 1][t][z] = *reinterpret_cast<const float*>(p + FEW_XS + (2 * u + z) * 64 + (lane & 15) * 4);
+                }
+        };
+        read(0);
+        uint32_t dd[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dd[i] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.h.x)));
+        const Consts k = consts();
         uint32_t f[4] = {w.f.x, w.f.y, w.f.z, w.f.w}, s[4] = {w.s.x, w.s.y, w.s.z, w.s.w};
         swap32(f[0], f[2]); swap32(f[1], f[3]); swap32(s[0], s[2]); swap32(s[1], s[3]);
         swap16(f[0], f[1]); swap16(f[2], f[3]); swap16(s[0], s[1]); swap16(s[2], s[3]);   // now by unit
@@ -85,50 +111,54 @@ struct FewQ4 {
         const uint32_t mn[2] = {w.h.z & 0x3F3F3F3Fu, ((w.h.w >> 4) & 0x0F0F0F0Fu) | ((w.h.z >> 2) & 0x30303030u)};
         const f4v zero{0.f, 0.f, 0.f, 0.f};
         f4v sum[T];
+        b8v xm[T];
+        f4v r[T][2];
+        auto fold = [&](int u) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int z = 0; z < 2; ++z)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sum[t][i] = u + z ? fmaf(r[t][z][i], xs[u & 1][t][z], sum[t][i]) : r[t][z][i] * xs[u & 1][t][z];
+        };
+        // a unit's weights are unpacked while the matrix cores are at the unit before
         auto unit = [&](auto u_) {
             constexpr int u = decltype(u_)::value;
             // 1024 + code, and for the upper nibbles 1024 + 16 code in place; the FMA leaves scale * code
-            const h2v s0 = byte_twice<2 * (u & 1)>(sc[u >> 1]) - both(1024.f), s1 = (byte_twice<2 * (u & 1) + 1>(sc[u >> 1]) - both(1024.f)) * both(0.0625f);
+            const h2v s0 = byte_twice<2 * (u & 1)>(sc[u >> 1]) - both(1024.f), s1 = fma2(byte_twice<2 * (u & 1) + 1>(sc[u >> 1]), both(0.0625f), both(-64.f));
             const h2v o0 = s0 * both(-1024.f), o1 = s1 * both(-1024.f);
-            h8v lo, hi;
+            h8v wt[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const uint32_t q = e ? s[u] : f[u], r = q >> 8;
-                const h2v a = fma2(as_h2((q & 0x000F000Fu) | 0x64006400u), s0, o0), b = fma2(as_h2((r & 0x000F000Fu) | 0x64006400u), s0, o0);
-                const h2v c = fma2(as_h2((q & 0x00F000F0u) | 0x64006400u), s1, o1), d = fma2(as_h2((r & 0x00F000F0u) | 0x64006400u), s1, o1);
-                lo[4 * e] = a[0]; lo[4 * e + 1] = a[1]; lo[4 * e + 2] = b[0]; lo[4 * e + 3] = b[1];
-                hi[4 * e] = c[0]; hi[4 * e + 1] = c[1]; hi[4 * e + 2] = d[0]; hi[4 * e + 3] = d[1];
+                const uint32_t q = e ? s[u] : f[u], q8 = q >> 8;
+                const h2v a = fma2(as_h2((q & k.lo) | k.bias), s0, o0), b = fma2(as_h2((q8 & k.lo) | k.bias), s0, o0);
+                const h2v c = fma2(as_h2((q & k.hi) | k.bias), s1, o1), d = fma2(as_h2((q8 & k.hi) | k.bias), s1, o1);
+                wt[0][4 * e] = a[0]; wt[0][4 * e + 1] = a[1]; wt[0][4 * e + 2] = b[0]; wt[0][4 * e + 3] = b[1];
+                wt[1][4 * e] = c[0]; wt[1][4 * e + 1] = c[1]; wt[1][4 * e + 2] = d[0]; wt[1][4 * e + 3] = d[1];
             }
+            if (u) fold(u - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (u < 3) read(u + 1);
+            else
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const unsigned char* const p = st + t * FEW_TILE;
+                for (int t = 0; t < T; ++t) xm[t] = *reinterpret_cast<const b8v*>(st + t * FEW_TILE + FEW_MIN + lane * 16);
 #pragma unroll
-                for (int z = 0; z < 2; ++z) {
-                    const int b = 2 * u + z;
-                    const f4v r = __builtin_amdgcn_mfma_f32_16x16x32_f16(z ? hi : lo, *reinterpret_cast<const h8v*>(p + b * FEW_BLOCK + lane * 16), zero, 0, 0, 0);
-                    const float xs = *reinterpret_cast<const float*>(p + FEW_XS + b * 64 + (lane & 15) * 4);
+            for (int t = 0; t < T; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) sum[t][i] = b ? fmaf(r[i], xs, sum[t][i]) : r[i] * xs;
-                }
-                if (T > 2 && (t & 1)) __builtin_amdgcn_sched_barrier(0);   // else the fragments of all tiles and units are read at once, and spilled
-            }
+                for (int z = 0; z < 2; ++z) r[t][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wt[z], x[u & 1][t][z], zero, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         };
         unit(std::integral_constant<int, 0>{}); unit(std::integral_constant<int, 1>{});
         unit(std::integral_constant<int, 2>{}); unit(std::integral_constant<int, 3>{});
         b8v am;
 #pragma unroll
         for (int b = 0; b < 8; ++b) am[b] = static_cast<__bf16>(static_cast<float>((mn[b >> 2] >> (8 * (b & 3))) & 0xFF));
-        float d[4], dm[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.h.x)));
-            d[i] = h2f(v & 0xFFFF); dm[i] = -h2f(v >> 16);
-        }
+        fold(3);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            const f4v m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, *reinterpret_cast<const b8v*>(st + t * FEW_TILE + FEW_MIN + lane * 16), zero, 0, 0, 0);
+            const f4v m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, xm[t], zero, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(dm[i], m[i], fmaf(d[i], sum[t][i], acc[t][i]));
+            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(-h2f(dd[i] >> 16), m[i], fmaf(h2f(dd[i] & 0xFFFF), sum[t][i], acc[t][i]));
         }
     }
 };
@@ -140,73 +170,91 @@ struct FewQ6 {
     static constexpr bool MINS = false;
     struct W { uint4 a, b, q, sc; uint32_t d; };
     static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * (g & 1) + 2 * (g >> 1) + e; }
-    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* row, uint32_t sb, uint32_t g, uint32_t nsb) {
-        if (!COPY) {
-            const uint8_t* const blk = row + sb * 210;
-            w.a = ld_u128_a2(blk + (g >> 1) * 64 + (g & 1) * 16);
-            w.b = ld_u128_a2(blk + (g >> 1) * 64 + 32 + (g & 1) * 16);
-            w.q = ld_u128_a2(blk + 128 + (g >> 1) * 32 + (g & 1) * 16);
-            w.sc = ld_u128_a2(blk + 192);
-            w.d = ld_u16(blk + 208);
-            return;
+    struct At { uint32_t a, b, q, sc, d; };
+    template <bool COPY> static __device__ __forceinline__ At at(uint32_t row, uint32_t g, uint32_t nsb) {
+        const uint32_t plane = Q6K::up128(64 * nsb), h = g >> 1, j = (g & 1) * 16;
+        if (COPY) return At{row + g * 16, row + plane + g * 16, row + 2 * plane + g * 16, row + Q6K::stream_sc(4 * nsb), row + Q6K::stream_d(4 * nsb)};
+        return At{row + h * 64 + j, row + h * 64 + 32 + j, row + 128 + h * 32 + j, row + 192, row + 208};
+    }
+    template <bool COPY> static __device__ __forceinline__ void load(W& w, const uint8_t* m, uint32_t sb, const At& o) {
+        const uint8_t* const q = m + sb * (COPY ? 64u : 210u);
+        if (COPY) {
+            w.a = ld_u128(q + o.a);
+            w.b = ld_u128(q + o.b);
+            w.q = ld_u128(q + o.q);
+            w.sc = ld_u128(m + sb * 16u + o.sc);
+            w.d = ld_u16(m + sb * 2u + o.d);
+        } else {
+            w.a = ld_u128_a2(q + o.a);
+            w.b = ld_u128_a2(q + o.b);
+            w.q = ld_u128_a2(q + o.q);
+            w.sc = ld_u128_a2(q + o.sc);
+            w.d = ld_u16(q + o.d);
         }
-        const uint32_t plane = Q6K::up128(64 * nsb), at = (sb * 4 + g) * 16;
-        w.a = ld_u128(row + at);
-        w.b = ld_u128(row + plane + at);
-        w.q = ld_u128(row + 2 * plane + at);
-        w.sc = ld_u128(row + Q6K::stream_sc(4 * nsb) + sb * 16);
-        w.d = ld_u16(row + Q6K::stream_d(4 * nsb) + sb * 2);
     }
     template <int T>
     static __device__ __forceinline__ void multiply(const W& w, const unsigned char* st, uint32_t lane, f4v (&acc)[T]) {
+        h8v x[2][T];   // a block ahead
+        float xs[2][T];
+        auto read = [&](int b) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                x[b & 1][t] = *reinterpret_cast<const h8v*>(st + t * FEW_TILE + b * FEW_BLOCK + lane * 16);
+                xs[b & 1][t] = *reinterpret_cast<const float*>(st + t * FEW_TILE + FEW_XS + b * 64 + (lane & 15) * 4);
+            }
+        };
+        read(0);
+        uint32_t dd[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dd[i] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.d)));
         uint32_t a[4] = {w.a.x, w.a.y, w.a.z, w.a.w}, b[4] = {w.b.x, w.b.y, w.b.z, w.b.w}, q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
         swap32(a[0], a[2]); swap32(a[1], a[3]); swap32(b[0], b[2]); swap32(b[1], b[3]); swap32(q[0], q[2]); swap32(q[1], q[3]);   // now [half][dword]
         const uint32_t sh = 8 * ((lane >> 4) & 1);
+        uint32_t lo4 = 0x0F0F0F0Fu, hi2 = 0x30303030u;
+        asm("" : "+s"(lo4)); asm("" : "+s"(hi2));
         const f4v zero{0.f, 0.f, 0.f, 0.f};
         f4v sum[T];
-        auto half = [&](auto h_) {
-            constexpr int h = decltype(h_)::value;
-            h8v hi[4], lo[4];
-            const uint32_t s01 = ((h ? w.sc.z : w.sc.x) ^ 0x80808080u) >> sh, s23 = ((h ? w.sc.w : w.sc.y) ^ 0x80808080u) >> sh;
-            const h2v sc[4] = {byte_twice<0>(s01) - both(1152.f), byte_twice<2>(s01) - both(1152.f), byte_twice<0>(s23) - both(1152.f), byte_twice<2>(s23) - both(1152.f)};
+        f4v r[T];
+        auto fold = [&](int blk) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[t][i] = blk ? fmaf(r[t][i], xs[blk & 1][t], sum[t][i]) : r[t][i] * xs[blk & 1][t];
+        };
+        auto block = [&](auto b_) {
+            constexpr int blk = decltype(b_)::value, h = blk >> 2, z = blk & 3;
+            const uint32_t sv = ((z < 2 ? (h ? w.sc.z : w.sc.x) : (h ? w.sc.w : w.sc.y)) ^ 0x80808080u) >> sh;
+            const h2v sc = byte_twice<2 * (z & 1)>(sv) - both(1152.f);
+            h8v hi, lo;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const uint32_t qa = a[2 * h + e], qb = b[2 * h + e], qh = q[2 * h + e];
-                const uint32_t c[4] = {(qa & 0x0F0F0F0Fu) | ((qh << 4) & 0x30303030u), (qb & 0x0F0F0F0Fu) | ((qh << 2) & 0x30303030u),
-                                       ((qa >> 4) & 0x0F0F0F0Fu) | (qh & 0x30303030u), ((qb >> 4) & 0x0F0F0F0Fu) | ((qh >> 2) & 0x30303030u)};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    // code - 32, times the scale: rounded to f16, and the remainder
-                    const h2v x = bytes02(c[t]) - both(1056.f), y = bytes13(c[t]) - both(1056.f);
-                    const h2v xh = x * sc[t], yh = y * sc[t], xl = fma2(x, sc[t], -xh), yl = fma2(y, sc[t], -yh);
-                    hi[t][4 * e] = xh[0]; hi[t][4 * e + 1] = xh[1]; hi[t][4 * e + 2] = yh[0]; hi[t][4 * e + 3] = yh[1];
-                    lo[t][4 * e] = xl[0]; lo[t][4 * e + 1] = xl[1]; lo[t][4 * e + 2] = yl[0]; lo[t][4 * e + 3] = yl[1];
-                }
+                const uint32_t ql = z & 1 ? b[2 * h + e] : a[2 * h + e], qh = q[2 * h + e];
+                const uint32_t top = (z == 0 ? qh << 4 : z == 1 ? qh << 2 : z == 2 ? qh : qh >> 2) & hi2;
+                const uint32_t c = ((z < 2 ? ql : ql >> 4) & lo4) | top;
+                // code - 32, times the scale: rounded to f16, and the remainder
+                const h2v u = bytes02(c) - both(1056.f), v = bytes13(c) - both(1056.f);
+                const h2v uh = u * sc, vh = v * sc, ul = fma2(u, sc, -uh), vl = fma2(v, sc, -vh);
+                hi[4 * e] = uh[0]; hi[4 * e + 1] = uh[1]; hi[4 * e + 2] = vh[0]; hi[4 * e + 3] = vh[1];
+                lo[4 * e] = ul[0]; lo[4 * e + 1] = ul[1]; lo[4 * e + 2] = vl[0]; lo[4 * e + 3] = vl[1];
             }
+            if (blk) fold(blk - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (blk < 7) read(blk + 1);
 #pragma unroll
-            for (int z = 0; z < 4; ++z) {
+            for (int t = 0; t < T; ++t) r[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, x[blk & 1][t], zero, 0, 0, 0);
 #pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    const int blk = 4 * h + z;
-                    const unsigned char* const p = st + t * FEW_TILE;
-                    const h8v x = *reinterpret_cast<const h8v*>(p + blk * FEW_BLOCK + lane * 16);
-                    f4v r = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[z], x, zero, 0, 0, 0);
-                    r = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[z], x, r, 0, 0, 0);
-                    const float xs = *reinterpret_cast<const float*>(p + FEW_XS + blk * 64 + (lane & 15) * 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) sum[t][i] = blk ? fmaf(r[i], xs, sum[t][i]) : r[i] * xs;
-                }
-                if (T > 2) __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int t = 0; t < T; ++t) r[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, x[blk & 1][t], r[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         };
-        half(std::integral_constant<int, 0>{}); half(std::integral_constant<int, 1>{});
-        float d[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = h2f(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.d))));
+        block(std::integral_constant<int, 0>{}); block(std::integral_constant<int, 1>{});
+        block(std::integral_constant<int, 2>{}); block(std::integral_constant<int, 3>{});
+        block(std::integral_constant<int, 4>{}); block(std::integral_constant<int, 5>{});
+        block(std::integral_constant<int, 6>{}); block(std::integral_constant<int, 7>{});
+        fold(7);
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[i], sum[t][i], acc[t][i]);
+            for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(h2f(dd[i] & 0xFFFF), sum[t][i], acc[t][i]);
     }
 };
 
@@ -214,35 +262,44 @@ struct FewQ6 {
 // LDS.  Four tiles of tokens would spill registers.
 template <typename W, int T, bool COPY>
 __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) {
-    constexpr int S = T == 1 ? 4 : T == 2 ? 2 : 1, AHEAD = T > 2 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+    constexpr int S = T == 1 ? 4 : T == 2 ? 2 : 1, AHEAD = T > 1 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
     __shared__ __align__(16) unsigned char lds[2][S * T * FEW_TILE];
     const bool second = blockIdx.x >= a.tiles_a;
     const FewMat& M = second ? a.b : a.a;
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nsb = a.k / 256;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nsb = a.k / 256;
     const uint32_t row0 = (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
     const uint32_t sb0 = blockIdx.y * a.sb_per, sb1 = min(nsb, sb0 + a.sb_per);
-    const uint8_t* const row = M.w + static_cast<uint64_t>(min(row0 + (lane & 15), M.m - 1)) * a.row_bytes;   // rows past the end: the last one again
-    // the tokens of a chunk: a thread takes the 32 quants of one block of one token
+    const uint8_t* const m0 = M.w;
+    const typename W::At at = W::template at<COPY>(min(row0 + (lane & 15), M.m - 1) * a.row_bytes, lane >> 4, nsb);   // rows past the end: the last one again
+    // the tokens of a chunk: a thread takes the 32 quants of one block of one token (of three tiles some twice)
+    auto pair = [](int i) {
+        const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x;
+        return p - (p >= PAIRS ? 128 : 0);
+    };
     uint4 q0[NP], q1[NP];
     float xs[NP], bs[NP];
+    uint32_t oq[NP], os[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const uint32_t p = pair(i), tok = min((p >> 7) % T * 16 + ((p >> 3) & 15), a.n - 1);
+        oq[i] = tok * a.k + (p & 7) * 32;
+        os[i] = (tok * (a.k / 32) + (p & 7)) * 4;
+    }
     auto act_load = [&](uint32_t sb) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x, tile = p >> 7, tok = min((tile % T) * 16 + ((p >> 3) & 15), a.n - 1);
-            const uint32_t blk = min(sb + tile / T, sb1 - 1) * 8 + (p & 7);
-            if (PAIRS % (FEW_WAVES * 64) && p >= PAIRS) break;
-            const int8_t* const x = a.xq + static_cast<uint64_t>(tok) * a.k + blk * 32;
-            q0[i] = *reinterpret_cast<const uint4*>(x);
-            q1[i] = *reinterpret_cast<const uint4*>(x + 16);
-            xs[i] = a.xs[static_cast<uint64_t>(tok) * (a.k / 32) + blk];
-            if (W::MINS) bs[i] = a.bsum[static_cast<uint64_t>(tok) * (a.k / 32) + blk];
+            const uint32_t s = min(sb + min(i * (FEW_WAVES / 2) + (wave >> 1), S * T - 1u) / T, sb1 - 1);   // the super-block of the pair's tile
+            const int8_t* const x = a.xq + s * 256;
+            q0[i] = *reinterpret_cast<const uint4*>(x + oq[i]);
+            q1[i] = *reinterpret_cast<const uint4*>(x + oq[i] + 16);
+            xs[i] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.xs + s * 8) + os[i]);
+            if (W::MINS) bs[i] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(a.bsum + s * 8) + os[i]);
         }
     };
     auto act_store = [&](uint32_t buf) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x, tok = (p >> 3) & 15, b = p & 7;
-            if (PAIRS % (FEW_WAVES * 64) && p >= PAIRS) break;
+            const uint32_t p = pair(i), tok = (p >> 3) & 15, b = p & 7;
             unsigned char* const t = &lds[buf][(p >> 7) * FEW_TILE];
             const uint32_t q[8] = {q0[i].x, q0[i].y, q0[i].z, q0[i].w, q1[i].x, q1[i].y, q1[i].z, q1[i].w};
 #pragma unroll
@@ -268,34 +325,40 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) 
             }
         }
     };
+    // The loads stand outside every condition, past the end the last super-block again: where paths with and without a load
+    // meet, the compiler's wait for an older one is a wait for all.
     typename W::W w[AHEAD];
     act_load(sb0);
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i)
-        if (sb0 + i < sb1) W::template load<COPY>(w[i], row, sb0 + i, lane >> 4, nsb);
+    for (int i = 0; i < AHEAD; ++i) W::template load<COPY>(w[i], m0, min(sb0 + i, sb1 - 1), at);
     f4v acc[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
     act_store(0);
-    uint32_t buf = 0;
-    for (uint32_t base = sb0; base < sb1; base += AHEAD) {
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            const uint32_t sb = base + i;
-            if (sb < sb1) {
-                const uint32_t next = sb - i % S + S;   // the chunk behind this one
-                if (i % S == 0) {
-                    // this chunk is written, and no wavefront reads the other buffer any more
-                    lds_barrier();
-                    if (next < sb1) act_load(next);
-                }
-                W::template multiply<T>(w[i], &lds[buf][(i % S) * T * FEW_TILE], lane, acc);
-                if (sb + AHEAD < sb1) W::template load<COPY>(w[i], row, sb + AHEAD, lane >> 4, nsb);
-                if (i % S == S - 1 && next < sb1) {
-                    buf ^= 1;
-                    act_store(buf);
-                }
-            }
+    uint32_t buf = 0, sb = sb0;
+    auto step = [&](auto i_) {   // one super-block; whether it was the last
+        constexpr int i = decltype(i_)::value;
+        if (i % S == 0) {
+            // this chunk is written, and no wavefront reads the other buffer any more
+            lds_barrier();
+            act_load(min(sb + S, sb1 - 1));
+        }
+        W::template multiply<T>(w[i], &lds[buf][(i % S) * T * FEW_TILE], lane, acc);
+        __builtin_amdgcn_sched_barrier(0);   // the next load into the registers it has left, not into others and then copied, with a wait
+        W::template load<COPY>(w[i], m0, min(sb + AHEAD, sb1 - 1), at);
+        if (++sb == sb1) return true;
+        if (i % S == S - 1) {
+            buf ^= 1;
+            act_store(buf);
+        }
+        return false;
+    };
+    while (true) {
+        if (step(std::integral_constant<int, 0>{})) break;
+        if (step(std::integral_constant<int, 1>{})) break;
+        if constexpr (AHEAD > 2) {
+            if (step(std::integral_constant<int, 2>{})) break;
+            if (step(std::integral_constant<int, 3>{})) break;
         }
     }
     // four consecutive rows of one token per lane and tile
@@ -321,7 +384,8 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) 
 }  // namespace
 
 bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n) {
-    return w && (w->dtype == CERA_HIP_Q6_K || (reinterpret_cast<uintptr_t>(w->dev) & 15) == 0) && (w->dtype == CERA_HIP_Q4_K || w->dtype == CERA_HIP_Q6_K) && w->k >= FEW_MIN_K && w->k % 256 == 0 && w->m % 4 == 0 && w->m < (1u << 30) && n >= 2 &&
+    return w && (w->dtype == CERA_HIP_Q6_K || (reinterpret_cast<uintptr_t>(w->dev) & 15) == 0) && (w->dtype == CERA_HIP_Q4_K || w->dtype == CERA_HIP_Q6_K) && w->k >= FEW_MIN_K && w->k % 256 == 0 && w->m % 4 == 0 &&
+           w->m * std::max(w->row_bytes, w->stream_row_bytes) < (1ull << 32) && n >= 2 &&
            n <= FEW_MAX_TOKENS;
 }
 
@@ -335,7 +399,7 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k); a.row_bytes = static_cast<uint32_t>(copy ? w->stream_row_bytes : w->row_bytes);
     auto tiles = [](const cera_hip_dtensor* t) { return static_cast<uint32_t>((t->m + FEW_ROWS - 1) / FEW_ROWS); };
     a.tiles_a = tiles(w);
-    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = 2 * ctx->n_cu;
+    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = 8 / FEW_WAVES * ctx->n_cu;
     // K is split where the rows leave more than a quarter of two workgroups per CU idle, down to two super-blocks a slice
     uint32_t split = wgs * 4 >= want * 3 ? 1 : std::min({(want + wgs - 1) / wgs, std::max(nsb / 2, 1u), 8u});
     a.sb_per = (nsb + split - 1) / split;
