@@ -8,23 +8,24 @@ namespace {
 
 __device__ __forceinline__ float bf16_at(const uint16_t* p, uint64_t i) { return __builtin_bit_cast(float, static_cast<uint32_t>(p[i]) << 16); }
 
-__global__ __launch_bounds__(256) void embed_pos_kernel(const uint16_t* __restrict__ embed, const uint16_t* __restrict__ pos,
-                                                        const uint32_t* __restrict__ tokens, uint32_t token, uint32_t start,
-                                                        uint32_t width, uint64_t ld, float* __restrict__ x, float* __restrict__ x0) {
-    const uint32_t t = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+template <int N>
+__global__ __launch_bounds__(256) void embed_pos_kernel(const uint16_t* __restrict__ embed, const uint16_t* __restrict__ pos, CeraIds<N> tokens, uint32_t first,
+                                                        uint32_t start, uint32_t width, uint64_t ld, float* __restrict__ x, float* __restrict__ x0) {
+    const uint32_t t = first + blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
     if (c >= ld) return;
-    const uint64_t tok = tokens ? tokens[t] : token;
+    const uint64_t tok = tokens.id[blockIdx.y];
     const float v = c < width ? bf16_at(embed, tok * width + c) + bf16_at(pos, static_cast<uint64_t>(start + t) * width + c) : 0.0f;
     x[t * ld + c] = v;
     x0[t * ld + c] = v;
 }
 
-__global__ __launch_bounds__(256) void embed_streams_kernel(const uint16_t* __restrict__ embed, const uint32_t* __restrict__ tokens, uint32_t token,
-                                                            uint32_t width, uint64_t ld, float* __restrict__ x, uint32_t streams, uint64_t stride,
-                                                            float u_scale, float* __restrict__ u) {
-    const uint32_t t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;   // ld is a multiple of 4
+template <int N>
+__global__ __launch_bounds__(256) void embed_streams_kernel(const uint16_t* __restrict__ embed, CeraIds<N> tokens, uint32_t first, uint32_t width, uint64_t ld,
+                                                            float* __restrict__ x, uint32_t streams, uint64_t stride, float u_scale,
+                                                            float* __restrict__ u) {
+    const uint32_t t = first + blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;   // ld is a multiple of 4
     if (c >= ld) return;
-    const uint16_t* const row = embed + static_cast<uint64_t>(tokens ? tokens[t] : token) * width;
+    const uint16_t* const row = embed + static_cast<uint64_t>(tokens.id[blockIdx.y]) * width;
     const float4 v = make_float4(c < width ? bf16_at(row, c) : 0.0f, c + 1 < width ? bf16_at(row, c + 1) : 0.0f,
                                  c + 2 < width ? bf16_at(row, c + 2) : 0.0f, c + 3 < width ? bf16_at(row, c + 3) : 0.0f);
     for (uint32_t s = 0; s < streams; ++s) *reinterpret_cast<float4*>(x + s * stride + t * ld + c) = v;
@@ -124,19 +125,23 @@ __global__ __launch_bounds__(256) void concat2_kernel(const float* __restrict__ 
 
 }  // namespace
 
-cera_hip_status cera_launch_embed_pos(cera_hip_ctx* ctx, const void* embed, const void* pos, const uint32_t* tokens, uint32_t token,
-                                      uint32_t n, uint32_t start, uint32_t width, uint64_t ld, float* x, float* x0) {
-    hipLaunchKernelGGL(embed_pos_kernel, dim3(static_cast<uint32_t>((ld + 255) / 256), n), dim3(256), 0, ctx->stream,
-                       static_cast<const uint16_t*>(embed), static_cast<const uint16_t*>(pos), tokens, token, start, width, ld, x, x0);
+cera_hip_status cera_launch_embed_pos(cera_hip_ctx* ctx, const void* embed, const void* pos, const uint32_t* tokens, uint32_t n, uint32_t start, uint32_t width,
+                                      uint64_t ld, float* x, float* x0) {
+    cera_by_ids(tokens, n, [&](const auto& ids, uint32_t first, uint32_t count) {
+        hipLaunchKernelGGL(embed_pos_kernel, dim3(static_cast<uint32_t>((ld + 255) / 256), count), dim3(256), 0, ctx->stream,
+                           static_cast<const uint16_t*>(embed), static_cast<const uint16_t*>(pos), ids, first, start, width, ld, x, x0);
+    });
     HIP_TRY(ctx, hipGetLastError());
     return CERA_HIP_OK;
 }
 
-cera_hip_status cera_launch_embed_streams(cera_hip_ctx* ctx, const void* embed, const uint32_t* tokens, uint32_t token, uint32_t n, uint32_t width,
-                                          uint64_t ld, float* x, uint32_t streams, uint64_t stride, float u_scale, float* u) {
+cera_hip_status cera_launch_embed_streams(cera_hip_ctx* ctx, const void* embed, const uint32_t* tokens, uint32_t n, uint32_t width, uint64_t ld, float* x,
+                                          uint32_t streams, uint64_t stride, float u_scale, float* u) {
     if (ld % 4 || stride % 4) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "embed_streams: rows in whole vectors");
-    hipLaunchKernelGGL(embed_streams_kernel, dim3(static_cast<uint32_t>((ld + 1023) / 1024), n), dim3(256), 0, ctx->stream,
-                       static_cast<const uint16_t*>(embed), tokens, token, width, ld, x, streams, stride, u_scale, u);
+    cera_by_ids(tokens, n, [&](const auto& ids, uint32_t first, uint32_t count) {
+        hipLaunchKernelGGL(embed_streams_kernel, dim3(static_cast<uint32_t>((ld + 1023) / 1024), count), dim3(256), 0, ctx->stream,
+                           static_cast<const uint16_t*>(embed), ids, first, width, ld, x, streams, stride, u_scale, u);
+    });
     HIP_TRY(ctx, hipGetLastError());
     return CERA_HIP_OK;
 }

@@ -83,6 +83,20 @@ hipFunction_t cera_module_fn(cera_hip_ctx* ctx, const std::string& name);
 // launch a one-struct-argument kernel of the loaded code object
 cera_hip_status cera_module_launch(cera_hip_ctx* ctx, hipFunction_t f, uint32_t grid, uint32_t block, void* args);
 
+// Token ids as a kernel argument: a pass's first launch takes them along, where a copy to device memory of its own would make
+// the host wait for the device before it queues the pass.  Small passes carry small arguments; a launch takes at most as many
+// as fit the 4 KB of its arguments, with room for the others.
+template <int N> struct CeraIds { uint32_t id[N]; };
+template <class F> void cera_by_ids(const uint32_t* tokens, uint32_t n, F launch) {   // launch(ids, first, count)
+    constexpr int FEW = 64, MANY = 896;
+    auto part = [&](auto ids, uint32_t first, uint32_t count) {
+        for (uint32_t i = 0; i < count; ++i) ids.id[i] = tokens[first + i];
+        launch(ids, first, count);
+    };
+    if (n <= FEW) return part(CeraIds<FEW>{}, 0u, n);
+    for (uint32_t at = 0; at < n; at += MANY) part(CeraIds<MANY>{}, at, n - at < MANY ? n - at : MANY);
+}
+
 // ---- launchers (defined next to their kernels) --------------------------------
 enum CeraEpilogue { CERA_EPI_STORE = 0, CERA_EPI_ADD = 1, CERA_EPI_SILU_MUL = 2 };
 

@@ -70,7 +70,6 @@ struct CeraLayered {
     uint32_t cap_n = 0;
     float *bx = nullptr, *bx0 = nullptr, *bqkvg = nullptr, *binv = nullptr;
     void *ba = nullptr, *bb = nullptr, *bq = nullptr, *bcat = nullptr, *bcat2 = nullptr;
-    uint32_t* btok = nullptr;
     float* blogits = nullptr;
     uint32_t logits_cap = 0;
     uint64_t b_bytes = 0;

@@ -185,7 +185,7 @@ cera_hip_status decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool wan
         if (st == CERA_HIP_OK && !ok) st = cera_fail(ctx, CERA_HIP_ERR_SHAPE, "decode: a product's input does not fit the GEMV");
         return st;
     };
-    CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, nullptr, token, 1, pos, width, g.ld, g.x, g.x0));
+    CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, &token, 1, pos, width, g.ld, g.x, g.x0));
     for (Run& R : g.runs) {
         const LayerW& W = g.layers[R.layer];
         if (R.step >= 0) {
@@ -247,8 +247,7 @@ cera_hip_status ensure_batch(cera_hip_model* m, uint32_t n, bool logits) {
             CERA_TRY(layered_batch_alloc(m, N * g.ld * g.esz, &g.bb));
             CERA_TRY(layered_batch_alloc(m, N * q * g.esz, &g.bq));
             CERA_TRY(layered_batch_alloc(m, N * cat * g.esz, &g.bcat));
-            if (g.loop_in.w) CERA_TRY(layered_batch_alloc(m, N * 2 * g.ld * g.esz, &g.bcat2));
-            return layered_batch_alloc(m, N * 4, reinterpret_cast<void**>(&g.btok));
+            return g.loop_in.w ? layered_batch_alloc(m, N * 2 * g.ld * g.esz, &g.bcat2) : CERA_HIP_OK;
         };
         const cera_hip_status st = all();
         if (st != CERA_HIP_OK) { layered_batch_free(m); return st; }
@@ -265,8 +264,7 @@ cera_hip_status batch_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n
     cera_hip_ctx* ctx = m->ctx;
     const uint32_t width = g.cfg.width;
     CERA_TRY(ensure_batch(m, n, all != nullptr));
-    CERA_TRY(cera_hip_upload(ctx, g.btok, tokens, n * 4ull));
-    CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, g.btok, 0, n, start, width, g.ld, g.bx, g.bx0));
+    CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, tokens, n, start, width, g.ld, g.bx, g.bx0));
     for (const Run& R : g.runs) {
         const LayerW& W = g.layers[R.layer];
         if (R.step >= 0) {

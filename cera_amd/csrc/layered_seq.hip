@@ -45,7 +45,7 @@ cera_hip_status seq_decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool
         st.stride = g.ld;
         return to_streams(st, g.x, g.u, g.ld, width);
     };
-    CERA_TRY(cera_launch_embed_streams(ctx, g.embed, nullptr, token, 1, width, g.ld, g.x, g.cfg.streams, g.ld, g.u_scale, g.u));
+    CERA_TRY(cera_launch_embed_streams(ctx, g.embed, &token, 1, width, g.ld, g.x, g.cfg.streams, g.ld, g.u_scale, g.u));
     for (SeqLayer& W : g.seq) {
         DenseIn in;
         in.kind = DenseIn::NORM; in.x = g.u; in.n_mean = width; in.eps = g.cfg.eps; in.scale_a = W.norm;
@@ -117,8 +117,7 @@ cera_hip_status ensure_batch(cera_hip_model* m, uint32_t n, bool logits) {
             CERA_TRY(el(N * att, &g.bcat));
             CERA_TRY(el(N * q, &g.bq));
             CERA_TRY(el(N * qn, &g.bqn));
-            CERA_TRY(el(N * lat, &g.bo));
-            return layered_batch_alloc(m, N * 4, reinterpret_cast<void**>(&g.btok));
+            return el(N * lat, &g.bo);
         };
         const cera_hip_status st = get();
         if (st != CERA_HIP_OK) { layered_batch_free(m); return st; }
@@ -177,9 +176,8 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
     cera_hip_ctx* ctx = m->ctx;
     const uint32_t width = g.cfg.width;
     CERA_TRY(ensure_batch(m, n, all != nullptr));
-    CERA_TRY(cera_hip_upload(ctx, g.btok, tokens, n * 4ull));
     const uint64_t stride = g.cap_n * g.ld;
-    CERA_TRY(cera_launch_embed_streams(ctx, g.embed, g.btok, 0, n, width, g.ld, g.bx, g.cfg.streams, stride, g.u_scale, g.bu));
+    CERA_TRY(cera_launch_embed_streams(ctx, g.embed, tokens, n, width, g.ld, g.bx, g.cfg.streams, stride, g.u_scale, g.bu));
     auto norm = [&](const float* x, uint32_t rows, const float* w) {
         NormConv nc;
         nc.x = x; nc.ld = g.ld; nc.n = rows; nc.width = width; nc.eps = g.cfg.eps; nc.w = w; nc.out_a = g.ba;
