@@ -7,7 +7,7 @@ constexpr uint32_t FEW_MAX_TOKENS = 48, FEW_MIN_K = 2048;
 // One matrix as the kernel sees it: its rows in up to three segments, each with an output [n][ld] of its own.
 struct FewMat {
     const uint8_t* w = nullptr;
-    uint32_t m = 0;
+    uint32_t m = 0, row_bytes = 0;
     uint32_t cut[2] = {}, ld[3] = {};
     float* out[3] = {};
 };
@@ -30,6 +30,6 @@ struct FewParts {
 // rows long enough (FEW_MIN_K) for a wavefront's loads to run ahead
 bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n);
 // y[t][row] = W . x_t (+ resid, of oa's first segment and unless K is split) for n tokens quantized to xs / xq / bsum; ob
-// (nullable): a second matrix of the same type and k in the same launch.
+// (nullable): a second matrix of the same k in the same launch, of the same type or Q6_K beside Q4_K.
 cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const FewOut* ob, const float* xs, const int8_t* xq, const float* bsum, uint32_t n,
                                      const float* resid, float resid_scale, int part_slot, FewParts* parts);

@@ -24,11 +24,11 @@ typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 struct FewArgs {
-    FewMat a, b;               // b: a second matrix of the same type and k, or m = 0
+    FewMat a, b;               // b: a second matrix of the same k, or m = 0
     uint32_t tiles_a;          // workgroups of a
     const int8_t* xq;
     const float *xs, *bsum;
-    uint32_t n, k, row_bytes, sb_per;
+    uint32_t n, k, sb_per;
     uint64_t part_stride;      // floats between the slices of a split K; 0: no split
     const float* resid;        // added to segment 0 of a (unsplit)
     float resid_scale;
@@ -260,17 +260,16 @@ struct FewQ6 {
 
 // T tiles of 16 tokens; S super-blocks a chunk, so that a chunk is four tiles (three for T = 3) and two of them fill half the
 // LDS.  Four tiles of tokens would spill registers.
+template <int T> constexpr int FEW_CHUNK = T == 1 ? 4 : T == 2 ? 2 : 1;
 template <typename W, int T, bool COPY>
-__global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) {
-    constexpr int S = T == 1 ? 4 : T == 2 ? 2 : 1, AHEAD = T > 1 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
-    __shared__ __align__(16) unsigned char lds[2][S * T * FEW_TILE];
-    const bool second = blockIdx.x >= a.tiles_a;
+__device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned char (*lds)[FEW_CHUNK<T> * T * FEW_TILE]) {
+    constexpr int S = FEW_CHUNK<T>, AHEAD = T > 1 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
     const FewMat& M = second ? a.b : a.a;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nsb = a.k / 256;
     const uint32_t row0 = (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
     const uint32_t sb0 = blockIdx.y * a.sb_per, sb1 = min(nsb, sb0 + a.sb_per);
     const uint8_t* const m0 = M.w;
-    const typename W::At at = W::template at<COPY>(min(row0 + (lane & 15), M.m - 1) * a.row_bytes, lane >> 4, nsb);   // rows past the end: the last one again
+    const typename W::At at = W::template at<COPY>(min(row0 + (lane & 15), M.m - 1) * M.row_bytes, lane >> 4, nsb);   // rows past the end: the last one again
     // the tokens of a chunk: a thread takes the 32 quants of one block of one token (of three tiles some twice)
     auto pair = [](int i) {
         const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x;
@@ -380,6 +379,14 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) 
         *reinterpret_cast<f4v*>(out + at) = v;
     }
 }
+// WA, WB: the types of the two matrices
+template <typename WA, typename WB, int T, bool COPY>
+__global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) {
+    __shared__ __align__(16) unsigned char lds[2][FEW_CHUNK<T> * T * FEW_TILE];
+    const bool second = blockIdx.x >= a.tiles_a;
+    if (std::is_same<WA, WB>::value || !second) few_body<WA, T, COPY>(a, second, lds);
+    else few_body<WB, T, COPY>(a, second, lds);
+}
 
 }  // namespace
 
@@ -392,11 +399,11 @@ bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n) {
 cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const FewOut* ob, const float* xs, const int8_t* xq, const float* bsum, uint32_t n,
                                      const float* resid, float resid_scale, int part_slot, FewParts* parts) {
     const cera_hip_dtensor* w = oa.w;
-    if (!cera_gemm_few_supports(w, n) || (ob && (!cera_gemm_few_supports(ob->w, n) || ob->w->dtype != w->dtype || ob->w->k != w->k)))
+    if (!cera_gemm_few_supports(w, n) || (ob && (!cera_gemm_few_supports(ob->w, n) || ob->w->k != w->k || (ob->w->dtype != w->dtype && w->dtype != CERA_HIP_Q4_K))))
         return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "gemm_few: bad shape");
     FewArgs a{};
     const bool copy = w->dev_stream && (!ob || ob->w->dev_stream);
-    a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k); a.row_bytes = static_cast<uint32_t>(copy ? w->stream_row_bytes : w->row_bytes);
+    a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k);
     auto tiles = [](const cera_hip_dtensor* t) { return static_cast<uint32_t>((t->m + FEW_ROWS - 1) / FEW_ROWS); };
     a.tiles_a = tiles(w);
     const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = 8 / FEW_WAVES * ctx->n_cu;
@@ -408,6 +415,7 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     float* part = nullptr;
     auto set = [&](FewMat& m, const FewOut& o) {
         m.w = copy ? o.w->dev_stream : o.w->dev;
+        m.row_bytes = static_cast<uint32_t>(copy ? o.w->stream_row_bytes : o.w->row_bytes);
         m.m = static_cast<uint32_t>(o.w->m);
         uint32_t at = 0;
         for (int s = 0; s < 3; ++s) {   // segments lie side by side in a slice, as outputs of their own would
@@ -431,16 +439,18 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     a.part_stride = split > 1 ? rows * n : 0;
     *parts = FewParts{part, split, a.part_stride};
     const dim3 grid(wgs, split), block(FEW_WAVES * 64);
-    auto go = [&](auto type, auto from_copy) {
-        using W = decltype(type);
+    auto go = [&](auto type_a, auto type_b, auto from_copy) {
+        using WA = decltype(type_a);
+        using WB = decltype(type_b);
         constexpr bool COPY = decltype(from_copy)::value;
-        if (n <= 16) hipLaunchKernelGGL((gemm_few_kernel<W, 1, COPY>), grid, block, 0, ctx->stream, a);
-        else if (n <= 32) hipLaunchKernelGGL((gemm_few_kernel<W, 2, COPY>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((gemm_few_kernel<W, 3, COPY>), grid, block, 0, ctx->stream, a);
+        if (n <= 16) hipLaunchKernelGGL((gemm_few_kernel<WA, WB, 1, COPY>), grid, block, 0, ctx->stream, a);
+        else if (n <= 32) hipLaunchKernelGGL((gemm_few_kernel<WA, WB, 2, COPY>), grid, block, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((gemm_few_kernel<WA, WB, 3, COPY>), grid, block, 0, ctx->stream, a);
     };
     auto of_type = [&](auto from_copy) {
-        if (w->dtype == CERA_HIP_Q4_K) go(FewQ4{}, from_copy);
-        else go(FewQ6{}, from_copy);
+        if (w->dtype == CERA_HIP_Q6_K) go(FewQ6{}, FewQ6{}, from_copy);
+        else if (ob && ob->w->dtype == CERA_HIP_Q6_K) go(FewQ4{}, FewQ6{}, from_copy);
+        else go(FewQ4{}, FewQ4{}, from_copy);
     };
     if (copy) of_type(std::true_type{});
     else of_type(std::false_type{});

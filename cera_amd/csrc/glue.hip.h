@@ -259,6 +259,71 @@ static __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(const float* _
     rmsnorm_row_body<QUANT>(x, w, n, eps, y, scales, quants, part);
 }
 
+// The same for each of a few rows, which may still be split-K partial sums (pd.n_split, as rmsnorm_pending_kernel adds them
+// up).  16 to 48 rows of 4096 with eight slices: 6 us, against 4.5 us for the reduction launch and 5.7 us for the norm behind it.
+static __global__ __launch_bounds__(1024) void rmsnorm_few_kernel(const float* x, const float* __restrict__ w, uint32_t n, float eps, float* __restrict__ y,
+                                                                  float* __restrict__ scales, int8_t* __restrict__ quants, float* __restrict__ bsum,
+                                                                  RowsPending pd) {
+    __shared__ double part[16];
+    const uint64_t row = static_cast<uint64_t>(blockIdx.x) * n;
+    float4 v[4], g[4];
+    double s = 0.0;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const uint32_t i = threadIdx.x * 4 + 4096 * it;
+        if (i >= n) continue;
+        g[it] = *reinterpret_cast<const float4*>(w + i);
+        if (pd.n_split) {
+            float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (pd.resid) r = *reinterpret_cast<const float4*>(pd.resid + row + i);
+            float4 t = *reinterpret_cast<const float4*>(pd.part + row + i);
+#pragma unroll 8
+            for (uint32_t z = 1; z < pd.n_split; ++z) {
+                const float4 a = *reinterpret_cast<const float4*>(pd.part + z * pd.stride + row + i);
+                t.x += a.x; t.y += a.y; t.z += a.z; t.w += a.w;
+            }
+            if (pd.resid) {
+                if (pd.resid_scale != 1.0f) { t.x *= pd.resid_scale; t.y *= pd.resid_scale; t.z *= pd.resid_scale; t.w *= pd.resid_scale; }
+                t.x = r.x + t.x; t.y = r.y + t.y; t.z = r.z + t.z; t.w = r.w + t.w;
+            }
+            *reinterpret_cast<float4*>(pd.x_out + row + i) = t;
+            v[it] = t;
+        } else {
+            v[it] = *reinterpret_cast<const float4*>(x + row + i);
+        }
+        s += static_cast<double>(v[it].x) * v[it].x;
+        s += static_cast<double>(v[it].y) * v[it].y;
+        s += static_cast<double>(v[it].z) * v[it].z;
+        s += static_cast<double>(v[it].w) * v[it].w;
+    }
+    s = wave_sum_f64(s);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    double tot = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tot += part[i];
+    const float inv = static_cast<float>(1.0 / sqrt(tot / static_cast<double>(n) + static_cast<double>(eps)));
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const uint32_t i = threadIdx.x * 4 + 4096 * it;
+        if (i >= n) continue;
+        float4 o;
+        o.x = __fmul_rn(__fmul_rn(v[it].x, inv), g[it].x);
+        o.y = __fmul_rn(__fmul_rn(v[it].y, inv), g[it].y);
+        o.z = __fmul_rn(__fmul_rn(v[it].z, inv), g[it].z);
+        o.w = __fmul_rn(__fmul_rn(v[it].w, inv), g[it].w);
+        *reinterpret_cast<float4*>(y + row + i) = o;
+        float sc;
+        const uint32_t packed = q8_quantize_quad(o, sc);
+        const float ssum = q8_block_scaled_sum(packed, sc);
+        reinterpret_cast<uint32_t*>(quants)[(row + i) >> 2] = packed;
+        if ((threadIdx.x & 7) == 0) {
+            scales[(row + i) >> 5] = sc;
+            bsum[(row + i) >> 5] = ssum;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // RoPE on q and k in place + append k, v to the head-major KV cache.
 // cos/sin come from a host-built table [max_seq][head_dim/2] computed with the

@@ -509,7 +509,16 @@ cera_hip_status cera_model_ensure_prefill_buffers(cera_hip_model* m, uint32_t n)
     return CERA_HIP_OK;
 }
 
-static __global__ void set_pos_kernel(uint32_t* scalars, uint32_t pos) { scalars[1] = pos; }
+// The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.
+template <int N>
+static __global__ __launch_bounds__(256) void embed_ids_kernel(uint32_t dtype, const uint8_t* __restrict__ w, uint64_t row_bytes, CeraIds<N> tokens, uint32_t first,
+                                                               uint32_t pos, uint32_t* __restrict__ scalars, uint32_t k, float scale, float* __restrict__ out) {
+    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    if (e == 0 && first + blockIdx.y == 0) scalars[1] = pos;
+    if (e >= k) return;
+    const float v = dequant_elem(dtype, w + static_cast<uint64_t>(tokens.id[blockIdx.y]) * row_bytes, e);
+    out[static_cast<uint64_t>(first + blockIdx.y) * k + e] = scale != 1.0f ? __fmul_rn(v, scale) : v;
+}
 
 // all_logits (host, [n][vocab]): when set, every position is projected through the LM head in one
 // GEMM (project_logits_batched, cera/src/model/llama.rs:645-722) instead of the last one only.
@@ -521,10 +530,10 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     const uint32_t hs = c.hidden, q_dim = c.n_heads * c.head_dim, kv_dim = c.n_kv_heads * c.head_dim;
     const float scale = c.attn_scale != 0.0f ? c.attn_scale : 1.0f / std::sqrt(static_cast<float>(c.head_dim));
     CERA_TRY(cera_model_ensure_prefill_buffers(m, n));
-    CERA_TRY(cera_hip_upload(ctx, m->pf_tokens, tokens, n * 4ull));
-    hipLaunchKernelGGL(set_pos_kernel, dim3(1), dim3(1), 0, s, m->scalars, start_pos);
-    hipLaunchKernelGGL(embed_row_kernel, dim3((hs + 255) / 256, n), dim3(256), 0, s, m->embd->dtype, m->embd->dev,
-                       m->embd->row_bytes, m->pf_tokens, hs, c.embed_scale, m->pf_hidden);
+    cera_by_ids(tokens, n, [&](const auto& ids, uint32_t first, uint32_t count) {
+        hipLaunchKernelGGL(embed_ids_kernel, dim3((hs + 255) / 256, count), dim3(256), 0, s, m->embd->dtype, m->embd->dev, m->embd->row_bytes, ids, first,
+                           start_pos, m->scalars, hs, c.embed_scale, m->pf_hidden);
+    });
     HIP_TRY(ctx, hipGetLastError());
 
     // whether pf_xh holds the f16 form of the quants now in pf_xq; cleared wherever those are rewritten
@@ -538,12 +547,16 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     // the norm runs one workgroup per row, and a few dozen workgroups adding up partial sums take longer than
     // the reduction launch they save (12.8 against 4.8 + 5.7 us at 16 rows, 11.3 against 6.3 + 7.4 at 512).
     RowsPending pend{};
-    const bool norm_adds = n >= 128;
+    // A few rows take a workgroup of 1024 threads each that keeps its row in registers and has all slices on their way at once.
+    const bool norm_row = few_tokens && hs <= 16384, norm_adds = n >= 128 || norm_row;
     auto norm_rows = [&](const float* x, const float* w, float* y) -> cera_hip_status {
         staged = false;
         staged8 = false;
         split_of = nullptr;
-        if (pend.n_split && pend.x_out == x)
+        if (norm_row)
+            hipLaunchKernelGGL(rmsnorm_few_kernel, dim3(n), dim3(1024), 0, s, x, w, hs, c.rms_eps, y, m->pf_xs, m->pf_xq, m->pf_bsum,
+                               pend.n_split && pend.x_out == x ? pend : RowsPending{});
+        else if (pend.n_split && pend.x_out == x)
             hipLaunchKernelGGL(rmsnorm_pending_kernel, dim3(n), dim3(256), 0, s, x, w, hs, c.rms_eps, y, m->pf_xs, m->pf_xq,
                                m->pf_bsum, pend);
         else
@@ -652,10 +665,14 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             o.w = L.qkv;
             o.len[0] = q_dim; o.len[1] = kv_dim;
             o.out[0] = m->pf_q; o.out[1] = m->pf_k; o.out[2] = m->pf_v;
-            CERA_TRY(few(o, nullptr, nullptr, &pqk, 9));
-            if (L.qkv_rows > q_dim + kv_dim) {
+            const bool whole = L.qkv_rows > q_dim + kv_dim;
+            if (whole || (cera_gemm_few_supports(L.v, n) && (L.v->dtype == L.qkv->dtype || L.qkv->dtype == CERA_HIP_Q4_K))) {
+                FewOut ov;
+                ov.w = L.v; ov.out[0] = m->pf_v;
+                CERA_TRY(few(o, whole ? nullptr : &ov, nullptr, &pqk, 9));
                 if (pqk.n_split) pvv = RowsPending{pqk.part + static_cast<uint64_t>(n) * (q_dim + kv_dim), pqk.n_split, pqk.stride, nullptr, 1.0f, m->pf_v};
             } else {
+                CERA_TRY(few(o, nullptr, nullptr, &pqk, 9));
                 CERA_TRY(gemm(L.v, m->pf_v, nullptr, m->pf_normed, &pvv, 14));
             }
         } else {
@@ -780,8 +797,13 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
                            m->xs, m->xq, static_cast<float*>(nullptr));
         HIP_TRY(ctx, hipGetLastError());
         const cera_hip_dtensor* o = m->output ? m->output : m->embd;
-        if (o->dtype == CERA_HIP_Q5_K) CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, m->logits));
-        else CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, m->logits, nullptr, CERA_EPI_STORE));
+        if (o->dtype == CERA_HIP_Q5_K) {
+            CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, m->logits));
+        } else {   // from the decode copy where the head has one, as the decode step
+            bool done = false;
+            CERA_TRY(cera_launch_row_gemv_store(ctx, o, m->xs, m->xq, m->logits, &done));
+            if (!done) CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, m->logits, nullptr, CERA_EPI_STORE));
+        }
         if (c.logit_scale != 1.0f) {
             hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, m->logits, 1.0f / c.logit_scale, c.vocab);
             HIP_TRY(ctx, hipGetLastError());
