@@ -9,6 +9,7 @@
 #include "gemm_q5k_f16.hip.h"
 #include "gemm_q6k_f16.hip.h"
 #include "gemm_fp8.hip.h"
+#include "gemm_kq.h"
 #include "gemm_few.h"
 #include "glue.hip.h"
 #include "model.h"
@@ -29,6 +30,9 @@ static bool gemm_batched(uint32_t dtype, uint64_t k) { return cera_gemm_supports
 static_assert(G8_BN == 64 && G8_REC == 21504, "cera_fp8_split_bytes (copy_budget.h) restates this record geometry");
 uint64_t cera_gemm_fp8_ws_bytes(uint64_t n, uint64_t k) { return cera_fp8_split_bytes(n, k); }
 
+// which f16 form of the quants a workspace holds for Q6_K matrices: row-major (gemm_act_f16_kernel) or in gemm_kq.h's records
+enum class ActForm { none, rows, records };
+
 // out[i*ld_m + j*ld_n] = (W . B)[i][j] (+ resid)
 // w2 / out2 (nullable): a second matrix of the same type and k multiplied by the same activations
 // in the same launch, out2[i*ld_m + j*ld_n2]; *paired says whether that happened (if not, the
@@ -37,7 +41,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
                                  const float* bsum, uint32_t n, float* out, uint64_t ld_m, uint64_t ld_n,
                                  const float* resid, float resid_scale, const cera_hip_dtensor* w2 = nullptr,
                                  float* out2 = nullptr, uint64_t ld_n2 = 0, bool* paired = nullptr, void* bh_ws = nullptr,
-                                 bool* staged = nullptr, int32_t* dbg_dots = nullptr, const float* x_f32 = nullptr,
+                                 ActForm* staged = nullptr, int32_t* dbg_dots = nullptr, const float* x_f32 = nullptr,
                                  bool* staged_f32 = nullptr, void* b8_ws = nullptr, bool* staged8 = nullptr,
                                  RowsPending* pending = nullptr, int part_slot = 9) {
     // pending (nullable): a caller whose next launch can add split-K partial sums itself (the row norm or the
@@ -61,19 +65,28 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     a.row_bytes = static_cast<uint32_t>(w->row_bytes);
     a.ld_m = ld_m; a.ld_n = ld_n; a.resid = resid; a.resid_scale = resid_scale;
     a.hq = nullptr; a.hs = nullptr; a.hbsum = nullptr; a.hh = nullptr; a.dbg_dots = dbg_dots;
+    // a pair is taken when both outputs are token-major and dense (what the split-K reduction needs)
+    const bool pair = w2 && !resid && w2->dtype == w->dtype && w2->k == w->k && w2->row_bytes == w->row_bytes && ld_m == 1 &&
+                      ld_n == w->m && ld_n2 == w2->m && (w->m * n) % 4 == 0 && (w2->m * n) % 4 == 0;
+    // the outputs must be dense in m*n floats for a split K's elementwise reduction
+    const bool dense = ((ld_m == 1 && ld_n == a.m) || (ld_n == 1 && ld_m == n)) && (static_cast<uint64_t>(a.m) * n) % 4 == 0;
+    // Q6_K with many tokens: gemm_kq.hip, in this many slices of K (0: not there)
+    const uint32_t kq = dbg_dots || !dense ? 0 : kq_slices(w->dtype, a.m, pair ? w2->m : 0, n, a.k, ctx->n_cu);
     // Q6_K runs its block dots on the f16 matrix cores and reads the quants as f16: converted here
-    // unless the caller says its workspace (bh_ws) still holds these activations (*staged)
+    // unless the caller says its workspace (bh_ws) still holds these activations in that form (*staged)
     a.bh = nullptr;
     if (w->dtype == CERA_HIP_Q6_K) {
+        const ActForm form = kq ? ActForm::records : ActForm::rows;
         if (!bh_ws) {
-            CERA_TRY(cera_scratch(ctx, 10, static_cast<uint64_t>(n) * a.k * 2, &bh_ws));
+            CERA_TRY(cera_scratch(ctx, 10, kq ? cera_kq_act_bytes(n, a.k) : static_cast<uint64_t>(n) * a.k * 2, &bh_ws));
             staged = nullptr;
         }
-        if (!staged || !*staged) {
+        if (!staged || *staged != form) {
             const uint64_t words = static_cast<uint64_t>(n) * a.k / 16;
-            hipLaunchKernelGGL(gemm_act_f16_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0,
-                               ctx->stream, reinterpret_cast<const uint4*>(bq), static_cast<uint4*>(bh_ws), words);
-            if (staged) *staged = true;
+            if (kq) CERA_TRY(cera_launch_kq_act(ctx, bs, bq, n, a.k, bh_ws));
+            else hipLaunchKernelGGL(gemm_act_f16_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0,
+                                    ctx->stream, reinterpret_cast<const uint4*>(bq), static_cast<uint4*>(bh_ws), words);
+            if (staged) *staged = form;
         }
         a.bh = bh_ws;
     }
@@ -95,12 +108,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         }
         a.bf8 = static_cast<const uint8_t*>(b8_ws);
     }
-    // Q6_K: 128-token tiles (eight wavefronts) once there is more than one 64-token tile, where they round the
-    // token count up by at most a tenth more than 64-token tiles do (down projection of the 8B shapes: 71 -> 62 us
-    // at 128 tokens, 243 -> 207 at 512, 828 -> 727 at 2048)
-    const bool q6_wide = w->dtype == CERA_HIP_Q6_K && !dbg_dots && n > 64 &&
-                         (n + 127) / 128 * 128 * 10 <= (n + 63) / 64 * 64 * 11;
-    const uint32_t BM = fp8 ? G8_BM : GEMM_BM, BN = fp8 ? G8_BN : (q6_wide ? 2 * GEMM_BN : GEMM_BN);
+    const uint32_t BM = kq ? KQ_ROWS : fp8 ? G8_BM : GEMM_BM, BN = kq ? KQ_TOKENS : fp8 ? G8_BN : GEMM_BN;
     if (q5) {
         // hi | lo f16 halves of x and its f32 block sums, in one scratch allocation
         const uint64_t nk = static_cast<uint64_t>(n) * a.k;
@@ -122,23 +130,18 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     dim3 grid((n + BN - 1) / BN, (a.m + BM - 1) / BM);
     a.w2 = nullptr; a.out2 = nullptr; a.m2 = 0; a.tiles1 = grid.y; a.ld_n2 = 0;
     if (paired) *paired = false;
-    // a pair is taken when both outputs are token-major and dense (what the split-K reduction needs)
-    if (w2 && !resid && w2->dtype == w->dtype && w2->k == w->k && w2->row_bytes == w->row_bytes && ld_m == 1 &&
-        ld_n == w->m && ld_n2 == w2->m && (w->m * n) % 4 == 0 && (w2->m * n) % 4 == 0) {
+    if (pair) {
         a.w2 = w2->dev; a.out2 = out2; a.m2 = static_cast<uint32_t>(w2->m); a.ld_n2 = ld_n2;
         grid.y += static_cast<uint32_t>((w2->m + BM - 1) / BM);
         if (paired) *paired = true;
     }
     // Few output tiles and a long K (the down projection at a few hundred tokens): split K over
     // grid.z so the chip is filled, partial sums to scratch, then one fixed-order reduction.
-    // The outputs must be dense in m*n floats for the elementwise reduction.
-    uint32_t split = 1;
+    uint32_t split = kq ? kq : 1;
     const uint32_t wgs = grid.x * grid.y, nsb = a.k / GEMM_KSUPER;
-    const bool dense = (ld_m == 1 && ld_n == a.m) || (ld_n == 1 && ld_m == n);
-    const uint32_t per_cu = q6_wide ? 1 : 2;   // workgroups a CU holds at once
-    if (!dbg_dots && wgs < per_cu * ctx->n_cu && nsb >= 8 && dense && (static_cast<uint64_t>(a.m) * n) % 4 == 0) {
+    if (!kq && !dbg_dots && wgs < 2 * ctx->n_cu && nsb >= 8 && dense) {   // (a CU holds two workgroups)
         // smallest divisor of the super-block count that fills every CU
-        const uint32_t want = std::min<uint32_t>(8, (per_cu * ctx->n_cu + wgs - 1) / wgs);
+        const uint32_t want = std::min<uint32_t>(8, (2 * ctx->n_cu + wgs - 1) / wgs);
         // (a slice keeps at least two super-blocks: below that the tile's prologue outweighs its K loop)
         for (uint32_t d = 2; d <= 8 && split < want; ++d)
             if (nsb % d == 0 && nsb / d >= 2) split = d;
@@ -171,7 +174,9 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     switch (w->dtype) {
         case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false>), grid, dim3(256), 0, ctx->stream, a); break;
         case CERA_HIP_Q6_K:
-            if (q6_wide) hipLaunchKernelGGL((gemm_q6k_f16_kernel<false, 2>), grid, dim3(512), 0, ctx->stream, a);
+            if (kq)
+                CERA_TRY(cera_launch_kq(ctx, KqArgs{a.w, a.w2, static_cast<const uint8_t*>(a.bh), a.out, a.out2, a.m, a.m2, n, a.k, a.row_bytes, a.tiles1,
+                                                    a.k_chunk, ld_m, ld_n, ld_n2, a.part_stride, a.resid, resid_scale}, split));
             else hipLaunchKernelGGL(gemm_q6k_f16_kernel<false>, grid, dim3(256), 0, ctx->stream, a);
             break;
         case CERA_HIP_Q5_K: hipLaunchKernelGGL(gemm_q5k_f16_kernel, grid, dim3(256), 0, ctx->stream, a); break;
@@ -509,6 +514,13 @@ cera_hip_status cera_model_ensure_prefill_buffers(cera_hip_model* m, uint32_t n)
     return CERA_HIP_OK;
 }
 
+// both re-laid copies of the activations: the first fp8_records workgroups gemm_fp8.hip.h's, the others gemm_kq.h's
+static __global__ __launch_bounds__(256) void act_fp8_records_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xs, const float* __restrict__ bsum,
+                                                                     uint8_t* __restrict__ x8, uint32_t fp8_records, uint8_t* __restrict__ records, uint32_t n, uint32_t k) {
+    if (blockIdx.x < fp8_records) gemm_act_fp8_body(xq, xs, bsum, x8, n, k);
+    else kq_act_record(blockIdx.x - fp8_records, xq, xs, records, n, k);
+}
+
 // The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.
 template <int N>
 static __global__ __launch_bounds__(256) void embed_ids_kernel(uint32_t dtype, const uint8_t* __restrict__ w, uint64_t row_bytes, CeraIds<N> tokens, uint32_t first,
@@ -536,8 +548,8 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     });
     HIP_TRY(ctx, hipGetLastError());
 
-    // whether pf_xh holds the f16 form of the quants now in pf_xq; cleared wherever those are rewritten
-    bool staged = false;
+    // which f16 form of the quants now in pf_xq pf_xh holds; cleared wherever those are rewritten
+    ActForm staged = ActForm::none;
     const bool few_tokens = n <= FEW_MAX_TOKENS;
     // the same for pf_x8, the fp8 split copy the Q4_K GEMMs read
     bool staged8 = false;
@@ -550,7 +562,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     // A few rows take a workgroup of 1024 threads each that keeps its row in registers and has all slices on their way at once.
     const bool norm_row = few_tokens && hs <= 16384, norm_adds = n >= 128 || norm_row;
     auto norm_rows = [&](const float* x, const float* w, float* y) -> cera_hip_status {
-        staged = false;
+        staged = ActForm::none;
         staged8 = false;
         split_of = nullptr;
         if (norm_row)
@@ -650,10 +662,17 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         // Q4_K Q and K next to a Q6_K V (the Q4_K_M mix): both re-laid copies of the activations in one launch
         if (n > PREFILL_SMALL_BATCH && !few_qkv && L.q->dtype == CERA_HIP_Q4_K && L.k->dtype == CERA_HIP_Q4_K && L.v->dtype == CERA_HIP_Q6_K &&
             gemm_batched(CERA_HIP_Q4_K, hs) && gemm_batched(CERA_HIP_Q6_K, hs)) {
-            hipLaunchKernelGGL(gemm_act_fp8_kernel, dim3((n + G8_BN - 1) / G8_BN * 2 * (hs / 256)), dim3(256), 0, s, m->pf_xq, m->pf_xs,
-                               m->pf_bsum, static_cast<uint8_t*>(m->pf_x8), n, hs, static_cast<uint4*>(m->pf_xh));
+            const uint32_t fp8 = (n + G8_BN - 1) / G8_BN * 2 * (hs / 256);
+            if (kq_slices(CERA_HIP_Q6_K, L.v->m, 0, n, hs, ctx->n_cu)) {
+                hipLaunchKernelGGL(act_fp8_records_kernel, dim3(fp8 + kq_act_records(n, hs)), dim3(256), 0, s, m->pf_xq, m->pf_xs, m->pf_bsum,
+                                   static_cast<uint8_t*>(m->pf_x8), fp8, static_cast<uint8_t*>(m->pf_xh), n, hs);
+                staged = ActForm::records;
+            } else {
+                hipLaunchKernelGGL(gemm_act_fp8_kernel, dim3(fp8), dim3(256), 0, s, m->pf_xq, m->pf_xs, m->pf_bsum,
+                                   static_cast<uint8_t*>(m->pf_x8), n, hs, static_cast<uint4*>(m->pf_xh));
+                staged = ActForm::rows;
+            }
             HIP_TRY(ctx, hipGetLastError());
-            staged = true;
             staged8 = true;
         }
         // With nothing between the projections and RoPE (no biases, no QK norm) the RoPE / append kernel adds up
@@ -717,7 +736,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         // causal attention: query t sees positions 0 .. start_pos + t
         CERA_TRY(cera_launch_attn(ctx, m->pf_q, L.kc, L.vc, c.n_heads, c.n_kv_heads, c.head_dim, start_pos + 1ull,
                                   c.max_seq_len, scale, 0, n, m->pf_attn, m->pf_xs, m->pf_xq, m->pf_bsum, nullptr, m->kv_f16));
-        staged = false;   // the attention merge rewrote the quants
+        staged = ActForm::none;   // the attention merge rewrote the quants
         staged8 = false;
         split_of = nullptr;
         // (the row norm that follows adds the O projection's split-K partial sums itself)
@@ -730,20 +749,21 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         bool fused = false;
         int8_t* const hq = reinterpret_cast<int8_t*>(m->pf_gate);
         float *const hs = m->pf_up, *const hb = m->pf_up + static_cast<uint64_t>(n) * (c.ffn / 32);
-        // a Q6_K down projection reads its activations as f16: the SwiGLU epilogue of the fp8 kernel writes them too
-        const bool hh = L.gate->dtype == CERA_HIP_Q4_K && L.down->dtype == CERA_HIP_Q6_K;
+        // a Q6_K down projection reads its activations as f16: where it takes the rows, the SwiGLU epilogue of the fp8 kernel writes them too
+        const bool hh = L.gate->dtype == CERA_HIP_Q4_K && L.down->dtype == CERA_HIP_Q6_K &&
+                        !kq_slices(L.down->dtype, L.down->m, 0, n, L.down->k, ctx->n_cu);
         const bool few_gate_up = few_tokens && cera_gemm_few_supports(L.gate, n) && cera_gemm_few_supports(L.up, n);
         if (n > PREFILL_SMALL_BATCH && !few_gate_up && L.down->dtype != CERA_HIP_Q5_K)   // a Q5_K down projection reads the f32 SwiGLU output
             CERA_TRY(cera_launch_gemm_swiglu(ctx, L.gate, L.up, m->pf_xs, m->pf_xq, m->pf_bsum, n, hq, hs, hb, &fused, m->pf_x8, &staged8,
                                              hh ? m->pf_xh : nullptr));
-        staged = fused && hh;   // pf_xh: the down projection's activations, or stale
+        staged = fused && hh ? ActForm::rows : ActForm::none;   // pf_xh: the down projection's activations, or stale
         if (fused) staged8 = false;
         if (fused && cera_gemm_supports(L.down->dtype, L.down->k)) {
             // (all layers but the last: the next layer's first row norm adds the partial sums)
             CERA_TRY(cera_launch_gemm(ctx, L.down, hs, hq, hb, n, m->pf_hidden, 1, L.down->m, m->pf_hidden, c.residual_scale,
                                       nullptr, nullptr, 0, nullptr, m->pf_xh, &staged, nullptr, nullptr, nullptr, m->pf_x8, &staged8,
                                       norm_adds && i + 1 < c.n_layers ? &pend : nullptr));
-            staged = false;   // pf_xh / pf_x8 now mirror hq, not pf_xq
+            staged = ActForm::none;   // pf_xh / pf_x8 now mirror hq, not pf_xq
             staged8 = false;
             continue;
         }

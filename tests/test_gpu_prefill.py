@@ -132,6 +132,32 @@ def test_gemm_pair_of_a_few_tokens(hip, orc, dtype, ma, mb, k, n):
         assert (np.abs(got - want) / rms).max() <= 2e-5
 
 
+@pytest.mark.parametrize("ma,mb,n,k", [(200, 56, 66, 14336), (1, 4, 68, 14336), (256, 256, 128, 4352), (260, 17, 132, 14336),
+                                       (1028, 4, 257, 2304), (1028, 300, 256, 4096), (2052, 256, 2049, 1024)])
+def test_gemm_q6k_of_many_tokens(hip, orc, ma, mb, n, k):
+    """Q6_K with more than 64 tokens against the exact product of the dequantized weights and quantized tokens, alone (one
+    output row after the other) and as a pair (one token after the other): last tiles of rows and tokens, one row, one to
+    sixteen slices of K from one super-block on.  Scales and codes of random bytes take the whole range, -128 times -32
+    included, so both parts of a weight count; the bound is that of the products of a few tokens above, of an output's rms
+    over random signs."""
+    _say(f"many tokens Q6_K ma={ma} mb={mb} n={n} k={k}")
+    r = util.rng(ma + n + k)
+    def weights(m):
+        w = r.integers(0, 256, (m, k // 256, 210), dtype=np.uint8)
+        w[:, :, 208:] = (r.uniform(0.5, 2.0, (m, k // 256, 1)) * 1e-3).astype(np.float16).view(np.uint8)
+        return w.reshape(-1)
+    wa, wb = weights(ma), weights(mb)
+    x = r.standard_normal((n, k)).astype(np.float32) * np.exp2(r.integers(-6, 7, (n, 1))).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    alone = hip.gemm(Q6_K, wa, x, ma, n, k)
+    oa, ob = hip.gemm_pair(Q6_K, wa, ma, Q6_K, wb, mb, x, n, k)
+    for got, w, m in ((alone.reshape(ma, n).T, wa, ma), (oa, wa, ma), (ob, wb, mb)):
+        wd = util.dequant_np(Q6_K, w, m, k).astype(np.float64)
+        rms = np.sqrt((xd * xd).sum(1, keepdims=True) * (wd * wd).sum(1) / k)
+        assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q4_0, Q4_1, Q8_0])
 @pytest.mark.parametrize("m,k,n,want_fused", [(2048, 512, 1040, True), (1056, 256, 2000, True), (512, 256, 70, False)])
 def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n, want_fused):
