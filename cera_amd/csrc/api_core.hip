@@ -190,6 +190,7 @@ struct AttnLaunch {
     bool batch, fused_new_kv;
     AttnNewKV nk;
     float *acc, *ml;   // split-K partials: (o) and (m, l) per (query, head, part)
+    uint8_t* records;  // nullable: room for the split tiles of all visible keys (attn_records_kernel)
 };
 
 // G = heads per wavefront; a.G = heads per kv head (G or 2 G)
@@ -234,7 +235,27 @@ static void attn_launch_decode_g(cera_hip_ctx* ctx, const AttnLaunch& a, const K
 template <typename KV, int HD>
 static void attn_launch_partials(cera_hip_ctx* ctx, const AttnLaunch& a, const KV* kc, const KV* vc) {
     if (a.batch) {
-        // heaviest query blocks (most visible keys) first
+        if (a.records) {
+            const uint32_t n_keys = a.seq_len + a.n_queries - 1, tiles = (n_keys + 31) / 32;
+            hipLaunchKernelGGL((attn_records_kernel<KV, HD>), dim3(tiles, a.n_kv_heads), dim3(256), 0, ctx->stream, kc, vc, a.max_seq, n_keys, a.records);
+            auto launch = [&](auto g_) {
+                constexpr int GG = decltype(g_)::value;
+                if constexpr (attn_records_fit(attn_record_bytes<KV, HD>(), GG))
+                    hipLaunchKernelGGL((attn_prefill_records_kernel<KV, HD, GG>), dim3(a.n_kv_heads, (a.n_queries + 31) / 32, a.n_parts), dim3(64 * GG), 0,
+                                       ctx->stream, a.q, a.records, tiles, a.seq_len, a.n_queries, a.scale, a.part_keys, a.n_parts, a.q_stride, a.acc, a.ml);
+            };
+            switch (a.G) {
+                case 1: launch(std::integral_constant<int, 1>{}); break;
+                case 2: launch(std::integral_constant<int, 2>{}); break;
+                case 3: launch(std::integral_constant<int, 3>{}); break;
+                case 4: launch(std::integral_constant<int, 4>{}); break;
+                case 5: launch(std::integral_constant<int, 5>{}); break;
+                case 6: launch(std::integral_constant<int, 6>{}); break;
+                case 7: launch(std::integral_constant<int, 7>{}); break;
+                default: launch(std::integral_constant<int, 8>{}); break;
+            }
+            return;
+        }
         const dim3 pgrid((a.n_queries + 31) / 32, a.n_kv_heads, a.n_parts);
 #define ATTN_PF(GG)                                                                                                        \
     hipLaunchKernelGGL((attn_prefill_partial_kernel<KV, HD, GG>), pgrid, dim3(64 * GG), 0, ctx->stream, a.q, kc, vc, a.seq_len, \
@@ -273,6 +294,13 @@ static void attn_launch_partials(cera_hip_ctx* ctx, const AttnLaunch& a, const K
         default: attn_launch_decode_g<8, KV, HD>(ctx, a, kc, vc); break;
     }
 }
+
+// From this many pairs of a query and a key on, a batch splits the cache's tiles once: the pass over the cache has to be
+// earned back.  Below, at 256 queries behind 1024 keys (295 k pairs), the two are equal (32 / 8 heads of 128: 34.0 against
+// 36.4 us; 24 / 8: 33.9, 33.6); above, 1001 queries (501 k) take 87.5 -> 57.6 and 88.1 -> 55.0 us, 128 behind 4096 (532 k)
+// 59.9 -> 56.7 and 71.9 -> 55.2, 2048 queries 205.7 -> 143.1 and 208.8 -> 132.5; heads of 64 45.3 -> 35.2 at 1001 queries.
+static constexpr uint64_t ATTN_RECORDS_MIN_PAIRS = 448 * 1024;
+static constexpr uint64_t ATTN_RECORDS_MAX_BYTES = 128ull << 20;   // of the 512 MB that are kept free for workspaces
 
 cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* kc, const void* vc,
                                  uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint64_t seq_len,
@@ -399,8 +427,15 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
         acc = ctx->attn_acc;
         ml = ctx->attn_ml;
     }
+    // Many queries: the tiles split once (attn_prefill_records_kernel), where the context may allocate and the records of all
+    // visible keys are a bounded part of what is kept free for its workspaces.
+    void* records = nullptr;
+    const uint64_t rec = head_dim * 128ull * (kv_f16 ? 1 : 2), rec_bytes = (last_len + 31) / 32 * n_kv_heads * rec;
+    if (batch && !ws && n_queries * (seq_len + last_len) / 2 >= ATTN_RECORDS_MIN_PAIRS && rec_bytes <= ATTN_RECORDS_MAX_BYTES && attn_records_fit(static_cast<uint32_t>(rec), G))
+        CERA_TRY(cera_scratch(ctx, 13, rec_bytes, &records));
     AttnLaunch a{q, static_cast<uint32_t>(seq_len), static_cast<uint32_t>(max_seq), scale, n_heads, n_kv_heads, n_queries,
-                 n_heads * head_dim, G, S, n_parts, part_keys, chunks_per_part, Gw, batch, new_kv != nullptr, nk, acc, ml};
+                 n_heads * head_dim, G, S, n_parts, part_keys, chunks_per_part, Gw, batch, new_kv != nullptr, nk, acc, ml,
+                 static_cast<uint8_t*>(records)};
     const kv_half *kh = static_cast<const kv_half*>(kc), *vh = static_cast<const kv_half*>(vc);
     const float *kf = static_cast<const float*>(kc), *vf = static_cast<const float*>(vc);
     if (head_dim == 128) {

@@ -23,6 +23,7 @@
 // reduction at the end of the part.
 #pragma once
 #include "common.hip.h"
+#include "lds_dma.hip.h"
 #include "attn_types.h"
 #include "quantize.hip.h"
 
@@ -497,6 +498,152 @@ __device__ __forceinline__ attn_v16f attn_mfma(const uint4& a, const uint4& b, a
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(attn_v8h, a), __builtin_bit_cast(attn_v8h, b), c, 0, 0, 0);
 }
 
+// the value of the lane 32 away
+__device__ __forceinline__ float attn_other_half(float v) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    const uint32_t x = __float_as_uint(v);
+    const u2 r = __builtin_amdgcn_permlane32_swap(x, x, false, false);   // (low, low), (high, high)
+    return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+}
+// One tile of 32 keys for the wavefront's 32 queries.  f: the tile's operands, this lane's 16-byte words of them.  whole_to: the
+// keys that every query of the block sees.
+// AHEAD: the operands' LDS reads run this many steps before their use (0: where the registers are taken).
+template <int HD, bool LOW, int AHEAD, class F>
+__device__ __forceinline__ void attn_prefill_tile(const F& f, const uint4 (&qh)[HD / 16], const uint4 (&ql)[HD / 16], attn_v16f (&acc)[HD / 32], float& m, double& l,
+                                                  float* sX, uint32_t k0, uint32_t key_hi, uint32_t whole_to, bool q_live, uint32_t my_len, float scale2,
+                                                  uint32_t col, uint32_t half) {
+    constexpr int NJ = HD / 16, NDT = HD / 32;
+    // ---- scores, transposed: c[4blk + r] = <K[k0 + 8blk + 4half + r], Q[qidx]>; the cross terms
+    // (scaled low parts) collect in c2
+    attn_v16f c, c2;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) c[e] = c2[e] = 0.0f;
+    uint4 oh[AHEAD + 1], ol[AHEAD + 1];
+    auto read_k = [&](int j) {
+        oh[j % (AHEAD + 1)] = f.kh(j);
+        if (LOW) ol[j % (AHEAD + 1)] = f.kl(j);
+    };
+    auto read_v = [&](int i) {   // step i: 16 keys i / NDT, 32 dims i % NDT
+        oh[i % (AHEAD + 1)] = f.vh(i / NDT, i % NDT);
+        if (LOW) ol[i % (AHEAD + 1)] = f.vl(i / NDT, i % NDT);
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) read_k(j);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        if (j + AHEAD < NJ) read_k(j + AHEAD);
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+        c = attn_mfma(oh[j % (AHEAD + 1)], qh[j], c);
+        c2 = attn_mfma(oh[j % (AHEAD + 1)], ql[j], c2);
+        if (LOW) c2 = attn_mfma(ol[j % (AHEAD + 1)], qh[j], c2);
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) read_v(i);   // on their way while the scores become weights
+    if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+    // scores in the base-2 domain (scale * log2 e folded into one factor); a tile that every
+    // query of the block sees whole skips the masking
+    float mx = -__builtin_inff();
+    if (k0 + 32 <= min(key_hi, whole_to)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            c[e] = fmaf(c2[e], 1.0f / ATTN_LO_SCALE, c[e]) * scale2;
+            mx = fmaxf(mx, c[e]);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const uint32_t kg = k0 + 8 * (e >> 2) + 4 * half + (e & 3);
+            const bool ok = q_live && kg < my_len && kg < key_hi;
+            c[e] = ok ? fmaf(c2[e], 1.0f / ATTN_LO_SCALE, c[e]) * scale2 : -__builtin_inff();
+            mx = fmaxf(mx, c[e]);
+        }
+    }
+    mx = fmaxf(mx, attn_other_half(mx));
+    const float m_new = fmaxf(m, mx);
+    // a query with nothing visible yet keeps m = -inf: weights and correction are then 0 / 1
+    const float corr = m_new == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+    const float m_sub = m_new == -__builtin_inff() ? 0.0f : m_new;   // -inf is then a weight of 0 without a look at every score
+    float ps = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        c[e] = __builtin_amdgcn_exp2f(c[e] - m_sub);
+        ps += c[e];
+    }
+    ps += attn_other_half(ps);
+    l = l * static_cast<double>(corr) + static_cast<double>(ps);
+    m = m_new;
+    // ---- the correction factors, re-laid out by output row (query 8blk + 4half + r); once the
+    // running maxima have settled they are all exactly 1
+    if (__builtin_amdgcn_ballot_w64(corr != 1.0f) != 0) {
+        if (half == 0) sX[col] = corr;
+        __builtin_amdgcn_wave_barrier();   // sX is this wavefront's own: LDS operations of one wavefront complete in order
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
+            const float4 cr = *reinterpret_cast<const float4*>(sX + 8 * blk + 4 * half);
+            const float crv[4] = {cr.x, cr.y, cr.z, cr.w};
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[dt][4 * blk + r] *= crv[r];
+        }
+    }
+    // ---- O += P . V: the weights split like everything else; slot s of step kk is c[8kk + s]
+    uint4 ph[2], pl[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+        attn_split2<false>(c[8 * kk + 0], c[8 * kk + 1], ph[kk].x, pl[kk].x);
+        attn_split2<false>(c[8 * kk + 2], c[8 * kk + 3], ph[kk].y, pl[kk].y);
+        attn_split2<false>(c[8 * kk + 4], c[8 * kk + 5], ph[kk].z, pl[kk].z);
+        attn_split2<false>(c[8 * kk + 6], c[8 * kk + 7], ph[kk].w, pl[kk].w);
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * NDT; ++i) {
+        const int kk = i / NDT, dt = i % NDT;
+        if (i + AHEAD < 2 * NDT) read_v(i + AHEAD);
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+        acc[dt] = attn_mfma(ph[kk], oh[i % (AHEAD + 1)], acc[dt]);
+        acc[dt] = attn_mfma(pl[kk], oh[i % (AHEAD + 1)], acc[dt]);
+        if (LOW) acc[dt] = attn_mfma(ph[kk], ol[i % (AHEAD + 1)], acc[dt]);
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int HD>
+__device__ __forceinline__ void attn_prefill_query(const float* qp, uint4 (&qh)[HD / 16], uint4 (&ql)[HD / 16]) {
+#pragma unroll
+    for (int j = 0; j < HD / 16; ++j) {
+        const float4 a = *reinterpret_cast<const float4*>(qp + 16 * j), b = *reinterpret_cast<const float4*>(qp + 16 * j + 4);
+        attn_split2<true>(a.x, a.y, qh[j].x, ql[j].x);
+        attn_split2<true>(a.z, a.w, qh[j].y, ql[j].y);
+        attn_split2<true>(b.x, b.y, qh[j].z, ql[j].z);
+        attn_split2<true>(b.z, b.w, qh[j].w, ql[j].w);
+    }
+}
+template <int HD, int G>
+__device__ __forceinline__ void attn_prefill_out(const attn_v16f (&acc)[HD / 32], float m, double l, uint32_t q0, uint32_t n_queries, uint32_t kvh, uint32_t n_kv,
+                                                 uint32_t part, uint32_t n_parts, uint32_t hg, bool q_live, uint32_t col, uint32_t half,
+                                                 float* __restrict__ part_acc, float* __restrict__ part_ml) {
+    constexpr int NDT = HD / 32;
+    const uint32_t qidx = q0 + col;
+    // ---- partial out: rows of acc are queries 8blk + 4half + r, columns 32dt + col
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t qi = q0 + 8 * blk + 4 * half + r;
+            if (qi < n_queries) {
+                float* dst = part_acc + (((static_cast<uint64_t>(qi) * n_kv + kvh) * n_parts + part) * G + hg) * HD + col;
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) dst[32 * dt] = acc[dt][4 * blk + r];
+            }
+        }
+    if (half == 0 && q_live) {
+        float* ml = part_ml + (((static_cast<uint64_t>(qidx) * n_kv + kvh) * n_parts + part) * G + hg) * 2;
+        ml[0] = m * 0.69314718055994530942f;   // back to the natural-log domain the merge works in
+        ml[1] = static_cast<float>(l);
+    }
+}
+
 template <typename KV, int HD, int G>
 __device__ __forceinline__ void attn_prefill_partial_body(
     const float* __restrict__ q,       // [n_queries][q_stride], rows 16-byte aligned
@@ -538,17 +685,7 @@ __device__ __forceinline__ void attn_prefill_partial_body(
 
     // this lane's query, split: step j holds dims 16j + 8half .. +7
     uint4 qh[NJ], ql[NJ];
-    {
-        const float* qp = q + static_cast<uint64_t>(min(qidx, n_queries - 1)) * q_stride + head * HD + 8 * half;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const float4 a = *reinterpret_cast<const float4*>(qp + 16 * j), b = *reinterpret_cast<const float4*>(qp + 16 * j + 4);
-            attn_split2<true>(a.x, a.y, qh[j].x, ql[j].x);
-            attn_split2<true>(a.z, a.w, qh[j].y, ql[j].y);
-            attn_split2<true>(b.x, b.y, qh[j].z, ql[j].z);
-            attn_split2<true>(b.z, b.w, qh[j].w, ql[j].w);
-        }
-    }
+    attn_prefill_query<HD>(q + static_cast<uint64_t>(min(qidx, n_queries - 1)) * q_stride + head * HD + 8 * half, qh, ql);
     attn_v16f acc[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -615,108 +752,20 @@ __device__ __forceinline__ void attn_prefill_partial_body(
         stage();
         __syncthreads();
         if (PREFETCH && k0 + 32 < key_hi) fetch(k0 + 32);
-        // ---- scores, transposed: c[4blk + r] = <K[k0 + 8blk + 4half + r], Q[qidx]>; the cross terms
-        // (scaled low parts) collect in c2
-        attn_v16f c, c2;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) c[e] = c2[e] = 0.0f;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const uint4 kh = *reinterpret_cast<const uint4*>(sKh + col * KLD + 16 * j + 8 * half);
-            c = attn_mfma(kh, qh[j], c);
-            c2 = attn_mfma(kh, ql[j], c2);
-            if (LOW) {
-                const uint4 kl = *reinterpret_cast<const uint4*>(sKl + col * KLD + 16 * j + 8 * half);
-                c2 = attn_mfma(kl, qh[j], c2);
-            }
-        }
-        // scores in the base-2 domain (scale * log2 e folded into one factor); a tile that every
-        // query of the block sees whole skips the masking
-        float mx = -__builtin_inff();
-        if (k0 + 32 <= min(key_hi, first_len + q0)) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                c[e] = fmaf(c2[e], 1.0f / ATTN_LO_SCALE, c[e]) * scale2;
-                mx = fmaxf(mx, c[e]);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const uint32_t kg = k0 + 8 * (e >> 2) + 4 * half + (e & 3);
-                const bool ok = q_live && kg < my_len && kg < key_hi;
-                c[e] = ok ? fmaf(c2[e], 1.0f / ATTN_LO_SCALE, c[e]) * scale2 : -__builtin_inff();
-                mx = fmaxf(mx, c[e]);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m, mx);
-        // a query with nothing visible yet keeps m = -inf: weights and correction are then 0 / 1
-        const float corr = m_new == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
-        float ps = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            c[e] = c[e] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(c[e] - m_new);
-            ps += c[e];
-        }
-        ps += __shfl_xor(ps, 32, 64);
-        l = l * static_cast<double>(corr) + static_cast<double>(ps);
-        m = m_new;
-        // ---- the correction factors, re-laid out by output row (query 8blk + 4half + r); once the
-        // running maxima have settled they are all exactly 1
-        if (__builtin_amdgcn_ballot_w64(corr != 1.0f) != 0) {
-            if (half == 0) sX[col] = corr;
-            __builtin_amdgcn_wave_barrier();   // sX is this wavefront's own: LDS operations of one wavefront complete in order
-#pragma unroll
-            for (int blk = 0; blk < 4; ++blk) {
-                const float4 cr = *reinterpret_cast<const float4*>(sX + 8 * blk + 4 * half);
-                const float crv[4] = {cr.x, cr.y, cr.z, cr.w};
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[dt][4 * blk + r] *= crv[r];
-            }
-        }
-        // ---- O += P . V: the weights split like everything else; slot s of step kk is c[8kk + s]
-        uint4 ph[2], pl[2];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            attn_split2<false>(c[8 * kk + 0], c[8 * kk + 1], ph[kk].x, pl[kk].x);
-            attn_split2<false>(c[8 * kk + 2], c[8 * kk + 3], ph[kk].y, pl[kk].y);
-            attn_split2<false>(c[8 * kk + 4], c[8 * kk + 5], ph[kk].z, pl[kk].z);
-            attn_split2<false>(c[8 * kk + 6], c[8 * kk + 7], ph[kk].w, pl[kk].w);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                const uint4 vh = *reinterpret_cast<const uint4*>(sVh + (32 * dt + col) * VTLD + 16 * kk + 8 * half);
-                acc[dt] = attn_mfma(ph[kk], vh, acc[dt]);
-                acc[dt] = attn_mfma(pl[kk], vh, acc[dt]);
-                if (LOW) {
-                    const uint4 vl = *reinterpret_cast<const uint4*>(sVl + (32 * dt + col) * VTLD + 16 * kk + 8 * half);
-                    acc[dt] = attn_mfma(ph[kk], vl, acc[dt]);
-                }
-            }
+        struct Frags {
+            const _Float16 *kh_, *kl_, *vh_, *vl_;
+            __device__ __forceinline__ uint4 kh(int j) const { return *reinterpret_cast<const uint4*>(kh_ + 16 * j); }
+            __device__ __forceinline__ uint4 kl(int j) const { return *reinterpret_cast<const uint4*>(kl_ + 16 * j); }
+            __device__ __forceinline__ uint4 vh(int kk, int dt) const { return *reinterpret_cast<const uint4*>(vh_ + 32 * dt * VTLD + 16 * kk); }
+            __device__ __forceinline__ uint4 vl(int kk, int dt) const { return *reinterpret_cast<const uint4*>(vl_ + 32 * dt * VTLD + 16 * kk); }
+        };
+        const uint32_t ko = col * KLD + 8 * half, vo = col * VTLD + 8 * half;
+        attn_prefill_tile<HD, LOW, 0>(Frags{sKh + ko, LOW ? sKl + ko : nullptr, sVh + vo, LOW ? sVl + vo : nullptr}, qh, ql, acc, m, l, sX, k0, key_hi,
+                                   first_len + q0, q_live, my_len, scale2, col, half);
         __syncthreads();   // the K and V tiles are rewritten by the next tile
     }
 
-    // ---- partial out: rows of acc are queries 8blk + 4half + r, columns 32dt + col
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t qi = q0 + 8 * blk + 4 * half + r;
-            if (qi < n_queries) {
-                float* dst = part_acc + (((static_cast<uint64_t>(qi) * n_kv + kvh) * n_parts + part) * G + hg) * HD + col;
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) dst[32 * dt] = acc[dt][4 * blk + r];
-            }
-        }
-    if (half == 0 && q_live) {
-        float* ml = part_ml + (((static_cast<uint64_t>(qidx) * n_kv + kvh) * n_parts + part) * G + hg) * 2;
-        ml[0] = m * 0.69314718055994530942f;   // back to the natural-log domain the merge works in
-        ml[1] = static_cast<float>(l);
-    }
+    attn_prefill_out<HD, G>(acc, m, l, q0, n_queries, kvh, n_kv, part, n_parts, hg, q_live, col, half, part_acc, part_ml);
 }
 template <typename KV, int HD, int G>
 __global__ __launch_bounds__(64 * G) void attn_prefill_partial_kernel(
@@ -728,6 +777,142 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_partial_kernel(
     float* __restrict__ part_acc,      // [n_queries][n_kv][n_parts][G][128]
     float* __restrict__ part_ml) {
     attn_prefill_partial_body<KV, HD, G>(q, kc, vc, first_len, n_queries, max_seq, scale, part_keys, n_parts, q_stride, part_acc, part_ml);
+}
+
+// ---- many queries: the K / V tiles split and laid out once ----------------------------------------------------
+//
+// The kernel above splits, transposes and stages every K / V tile anew for each block of 32 queries: more than half of its
+// vector instructions for 4 heads a workgroup.  Here a pass over the visible cache writes one record per KV head and tile of
+// 32 keys, the tile's operands in the order in which the wavefronts' lanes take them -- K by steps of 16 dims, V by 16 keys and
+// 32 dims, the high parts of each in 1 KB and the low ones behind it -- and the workgroups load records straight into LDS, the
+// next tile's while this one is multiplied: one barrier a tile, no vector instruction for staging, LDS read without conflicts.
+// What is multiplied and its order are the same.  Workgroups of a KV head lie on one XCD where there are eight of them (the
+// head is the grid's fastest index), whose L2 then holds that head's records only; the blocks with the most keys start first.
+// What bounds it is the order of a wavefront's own instructions: LDS reads run three steps ahead of the products, and the first
+// values' reads go out before the scores become weights.  2048 queries behind 4096 keys, 32 / 8 heads of 128, f32 cache: 615 ->
+// 464 us with the pass over the cache (18); the products alone take 205.  Reads at their use: 520.  Two accumulators
+// for the cross terms and two output tiles in turn, against waits between dependent products: no gain.
+template <typename KV, int HD> constexpr uint32_t attn_record_bytes() { return 32 * HD * 2 * 2 * (sizeof(KV) == 4 ? 2 : 1); }
+// grid = (tiles, KV heads); keys from n_keys on are zeros
+template <typename KV, int HD>
+__global__ __launch_bounds__(256) void attn_records_kernel(const KV* __restrict__ kc, const KV* __restrict__ vc, uint32_t max_seq, uint32_t n_keys,
+                                                           uint8_t* __restrict__ records) {
+    constexpr bool LOW = sizeof(KV) == 4;
+    constexpr int PARTS = LOW ? 2 : 1, NJ = HD / 16, NDT = HD / 32;
+    const uint32_t k0 = blockIdx.x * 32;
+    const uint64_t head = static_cast<uint64_t>(blockIdx.y) * max_seq * HD;
+    uint8_t* const rec = records + (static_cast<uint64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * attn_record_bytes<KV, HD>();
+    for (uint32_t i = threadIdx.x; i < 64 * NJ; i += 256) {   // K: (step, lane), eight dims of a key
+        const uint32_t lane = i & 63, key = k0 + (lane & 31), d = (i >> 6) * 16 + (lane >> 5) * 8;
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+        if (key < n_keys) {
+            const KV* const p = kc + head + static_cast<uint64_t>(key) * HD;
+            a = KvOps<KV>::ld4(p, d / 4);
+            b = KvOps<KV>::ld4(p, d / 4 + 1);
+        }
+        uint4 hi, lo;
+        attn_split2<true>(a.x, a.y, hi.x, lo.x);
+        attn_split2<true>(a.z, a.w, hi.y, lo.y);
+        attn_split2<true>(b.x, b.y, hi.z, lo.z);
+        attn_split2<true>(b.z, b.w, hi.w, lo.w);
+        uint8_t* const dst = rec + (i >> 6) * (PARTS * 1024) + lane * 16;
+        *reinterpret_cast<uint4*>(dst) = hi;
+        if (LOW) *reinterpret_cast<uint4*>(dst + 1024) = lo;
+    }
+    for (uint32_t i = threadIdx.x; i < 64 * 2 * NDT; i += 256) {   // V: (16 keys, 32 dims, lane), the half's eight keys of a dim in slot order
+        const uint32_t lane = i & 63, kk = (i >> 6) / NDT, dt = (i >> 6) % NDT, key = k0 + 16 * kk + 4 * (lane >> 5);
+        const KV* const p = vc + head + 32 * dt + (lane & 31);
+        float v[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t at = key + 8 * (s >> 2) + (s & 3);
+            v[s] = at < n_keys ? static_cast<float>(p[static_cast<uint64_t>(at) * HD]) : 0.0f;
+        }
+        uint4 hi, lo;
+        attn_split2<false>(v[0], v[1], hi.x, lo.x);
+        attn_split2<false>(v[2], v[3], hi.y, lo.y);
+        attn_split2<false>(v[4], v[5], hi.z, lo.z);
+        attn_split2<false>(v[6], v[7], hi.w, lo.w);
+        uint8_t* const dst = rec + (NJ + (i >> 6)) * (PARTS * 1024) + lane * 16;
+        *reinterpret_cast<uint4*>(dst) = hi;
+        if (LOW) *reinterpret_cast<uint4*>(dst + 1024) = lo;
+    }
+}
+
+// Two records in LDS have to leave room for six wavefronts a CU: with four (two heads of 128 a workgroup, f32 cache) the kernel
+// above, which holds eight, stays the better one.
+constexpr bool attn_records_fit(uint32_t record_bytes, uint32_t G) { return 163840 / (2 * record_bytes + 128 * G) * G >= 6; }
+// grid = (KV heads, query blocks, parts), 64 * G threads; part_keys is a multiple of 32
+template <typename KV, int HD, int G>
+__global__ __launch_bounds__(64 * G, 2) void attn_prefill_records_kernel(
+    const float* __restrict__ q, const uint8_t* __restrict__ records, uint32_t n_tiles, uint32_t first_len, uint32_t n_queries, float scale, uint32_t part_keys,
+    uint32_t n_parts, uint32_t q_stride, float* __restrict__ part_acc, float* __restrict__ part_ml) {
+    constexpr bool LOW = sizeof(KV) == 4;
+    constexpr int PARTS = LOW ? 2 : 1, NJ = HD / 16, NDT = HD / 32;
+    constexpr uint32_t REC = attn_record_bytes<KV, HD>(), PIECES = REC / 1024;
+    constexpr int AHEAD = 3;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[2][REC];
+    __shared__ __attribute__((aligned(16))) float sXall[G * 32];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5, hg = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t kvh = blockIdx.x, n_kv = gridDim.x, head = kvh * G + hg, part = blockIdx.z;
+    float* const sX = sXall + 32 * hg;
+    const uint32_t q0 = (gridDim.y - 1 - blockIdx.y) * 32, qidx = q0 + col;
+    const bool q_live = qidx < n_queries;
+    const uint32_t my_len = first_len + qidx, block_len = first_len + min(n_queries, q0 + 32) - 1;
+    const uint32_t key_lo = part * part_keys, key_hi = min(key_lo + part_keys, block_len);
+    uint4 qh[NJ], ql[NJ];
+    attn_prefill_query<HD>(q + static_cast<uint64_t>(min(qidx, n_queries - 1)) * q_stride + head * HD + 8 * half, qh, ql);
+    attn_v16f acc[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[dt][e] = 0.0f;
+    float m = -__builtin_inff();
+    double l = 0.0;
+    const float scale2 = scale * 1.44269504088896340736f;
+
+    const uint8_t* const mine = records + static_cast<uint64_t>(kvh) * n_tiles * REC;
+    const uint32_t lds = lds_addr(&tile[0][0]);
+    auto fetch = [&](uint32_t k0, uint32_t buf) {
+        const uint8_t* const src = lds_dma_base(mine + static_cast<uint64_t>(k0 / 32) * REC + hg * 1024);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds + buf * REC + hg * 1024);
+#pragma unroll
+        for (uint32_t p = 0; p < (PIECES + G - 1) / G; ++p)
+            if (p * G + hg < PIECES) lds_dma_1k(src + p * G * 1024, lane * 16, dst + p * G * 1024);
+    };
+    uint32_t buf = 0;
+    if (key_lo < key_hi) fetch(key_lo, 0);
+    for (uint32_t k0 = key_lo; k0 < key_hi; k0 += 32, buf ^= 1) {
+        // this tile is in, and no wavefront reads the other buffer any more
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (k0 + 32 < key_hi) fetch(k0 + 32, buf ^ 1);
+        uint8_t* const t = tile[buf];
+        if (k0 + 32 > key_hi) {
+            // the block's last tile: the values of keys that none of its queries sees become zeros, as their weights are (a later
+            // query's infinity or NaN would come through)
+            for (uint32_t i = tid; i < 64 * 2 * NDT; i += 64 * G) {
+                const uint32_t ln = i & 63, key = k0 + 16 * ((i >> 6) / NDT) + 4 * (ln >> 5);
+                uint16_t* const v = reinterpret_cast<uint16_t*>(t + (NJ + (i >> 6)) * (PARTS * 1024) + ln * 16);
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    if (key + 8 * (s >> 2) + (s & 3) >= key_hi) {
+                        v[s] = 0;
+                        if (LOW) v[512 + s] = 0;
+                    }
+            }
+            __syncthreads();
+        }
+        struct Frags {
+            const uint8_t* p;
+            __device__ __forceinline__ uint4 at(int piece) const { return *reinterpret_cast<const uint4*>(p + piece * 1024); }
+            __device__ __forceinline__ uint4 kh(int j) const { return at(PARTS * j); }
+            __device__ __forceinline__ uint4 kl(int j) const { return at(PARTS * j + 1); }
+            __device__ __forceinline__ uint4 vh(int kk, int dt) const { return at(PARTS * (NJ + kk * NDT + dt)); }
+            __device__ __forceinline__ uint4 vl(int kk, int dt) const { return at(PARTS * (NJ + kk * NDT + dt) + 1); }
+        };
+        attn_prefill_tile<HD, LOW, AHEAD>(Frags{t + lane * 16}, qh, ql, acc, m, l, sX, k0, key_hi, first_len + q0, q_live, my_len, scale2, col, half);
+    }
+    attn_prefill_out<HD, G>(acc, m, l, q0, n_queries, kvh, n_kv, part, n_parts, hg, q_live, col, half, part_acc, part_ml);
 }
 
 // Merge the parts of one query head: out = sum_p e^{m_p - M} acc_p / sum_p e^{m_p - M} l_p.

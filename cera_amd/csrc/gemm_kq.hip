@@ -17,6 +17,7 @@
 // folds 70, the unpacking 45 and the rows' loads, 210 bytes apart by super-block, 60.
 #include "gemm_kq.h"
 #include "gemv.hip.h"
+#include "lds_dma.hip.h"
 
 namespace {
 
@@ -34,17 +35,6 @@ template <int J> __device__ __forceinline__ h2v byte_twice(uint32_t v) { return 
 
 __global__ __launch_bounds__(256) void kq_act_kernel(const int8_t* __restrict__ bq, const float* __restrict__ bs, uint8_t* __restrict__ act, uint32_t n, uint32_t k) {
     kq_act_record(blockIdx.x, bq, bs, act, n, k);
-}
-
-// 1 KB (256 B) straight into LDS, as dense.hip's: with the wait states that scalar registers written by a vector instruction need
-__device__ __forceinline__ void kq_dma_1k(const uint8_t* base, uint32_t off_lane, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off_lane), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void kq_dma_256(const uint8_t* base, uint32_t off_lane, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(off_lane), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t kq_lds_addr(const void* p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(p)));
 }
 
 // ---- Q6_K: half h of a super-block is two runs j of 16 codes of each of its four blocks --------------------------
@@ -109,7 +99,7 @@ __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
     const uint8_t* const wrow = wmat + static_cast<uint64_t>(min(m0 + wr, rows - 1)) * p.row_bytes;
     // this wavefront's share of a stage's tokens: one tile of 16
     const uint8_t* const rec = p.act + static_cast<uint64_t>(blockIdx.x * T + wave) * nsb * KQ_REC;
-    const uint32_t act_lds = kq_lds_addr(&act[0][0]) + wave * KQ_HALF;
+    const uint32_t act_lds = lds_addr(&act[0][0]) + wave * KQ_HALF;
     // piece p of a stage's loads: the rows' first, then the tokens'
     typename W::Stage st;
     auto load = [&](auto p_, uint32_t stage, uint32_t buf) {
@@ -118,8 +108,8 @@ __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
         else if constexpr (p < W::LOADS + 5) {
             const uint8_t* const r = rec + static_cast<uint64_t>(stage >> 1) * KQ_REC + (stage & 1) * KQ_HALF + (p - W::LOADS) * 1024;
             const uint32_t l = act_lds + buf * (T * KQ_HALF) + (p - W::LOADS) * 1024;
-            if constexpr (p < W::LOADS + 4) kq_dma_1k(r, lane * 16, l);
-            else kq_dma_256(r, lane * 4, l);
+            if constexpr (p < W::LOADS + 4) lds_dma_1k(r, lane * 16, l);
+            else lds_dma_256(r, lane * 4, l);
         }
     };
     f4v acc[RT][T], sum[RT][T];

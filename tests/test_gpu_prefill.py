@@ -465,6 +465,41 @@ def test_attn_prefill_batch_head_dim_64(hip, orc, kv_f16, nh, nkv, start, n):
         assert err <= 2e-3 * util.rms(ref), (i, err, util.rms(ref))
 
 
+@pytest.mark.parametrize("nh,nkv,hd,kv_f16,start,n", [(8, 2, 128, False, 1500, 290), (3, 1, 128, False, 0, 961), (14, 2, 128, True, 900, 481),
+                                                       (8, 1, 128, False, 31, 970), (2, 2, 64, True, 1200, 353), (6, 3, 64, False, 3001, 161),
+                                                       (16, 8, 128, False, 1500, 290)])
+def test_attn_prefill_of_many_queries(hip, orc, nh, nkv, hd, kv_f16, start, n):
+    """Batches large enough that the cache's tiles are split once and read as records (and one shape, two heads a group, that
+    keeps the other kernel): blocks that end inside a tile of 32 keys, last blocks of one query and of all 32, each group size's
+    way of dividing a record.  A value that is not finite at a later position must not come through to a block of queries
+    before it, though its tile is read there; the bound is that of the smaller batches."""
+    _say(f"attn_prefill many nh={nh} nkv={nkv} hd={hd} start={start} n={n} f16={kv_f16}")
+    r = util.rng(17 * n + start)
+    L = start + n
+    q = r.standard_normal((n, nh * hd), dtype=np.float32)
+    k = r.standard_normal((L, nkv * hd), dtype=np.float32)
+    v = r.standard_normal((L, nkv * hd), dtype=np.float32)
+    bad = start + 64   # the first key behind the first two blocks of queries
+    v[bad] = np.nan
+    if kv_f16:
+        k = k.astype(np.float16).astype(np.float32); v = v.astype(np.float16).astype(np.float32)
+    scale = 1.0 / np.sqrt(hd)
+    fn = hip.attn_f16kv if kv_f16 else hip.attn_prefill
+    picks = sorted({0, 31, 32, 63, 64, n // 2, n - 2, n - 1})
+    for poison in (True, False):
+        if not poison:
+            v[bad] = 0.5
+        out = fn(q, k.reshape(-1), v.reshape(-1), nh, nkv, hd, start, n, scale)
+        for i in picks:
+            if poison and i >= 64:
+                continue
+            Li = start + i + 1
+            ref = orc.decode_attention(q[i], k[:Li].reshape(-1), v[:Li].reshape(-1), nh, nkv, hd, scale, Li)
+            err = np.abs(out[i].astype(np.float64) - ref).max()
+            assert err <= 2e-3 * util.rms(ref), (poison, i, err, util.rms(ref))
+        assert np.isfinite(out[:64] if poison else out).all()
+
+
 def test_prefill_longer_than_one_pass(hip, orc):
     """A prompt beyond the 2048-token pass size is cut into passes; logits and the cache rows on
     both sides of the cut track the oracle's single batched prefill."""
