@@ -20,10 +20,6 @@ static constexpr uint64_t CERA_COPY_HEADROOM = 512ull << 20;  // left for scratc
 // (64-token tiles in two halves, one 21504-byte record per half tile and 256-element super-block)
 static inline uint64_t cera_fp8_split_bytes(uint64_t n, uint64_t k) { return (n + 63) / 64 * 2 * (k / 256) * 21504ull; }
 
-// bytes of the fragment-ordered f16 copy of the same that the Q6_K products with many tokens read (tiles of 128 tokens, one
-// 8704-byte record per 16 tokens and super-block)
-static inline uint64_t cera_kq_act_bytes(uint64_t n, uint64_t k) { return (n + 127) / 128 * 8 * (k / 256) * 8704ull; }
-
 // sizes of the buffers one batched prefill pass over `cap` tokens holds, in allocation order
 struct CeraPrefillSizes {
     uint64_t hidden, normed, q, k, v, attn, gate, up, xq, xh, x8, xs, bsum, tokens;
@@ -39,7 +35,7 @@ static inline CeraPrefillSizes cera_prefill_sizes(const cera_hip_config& c, uint
     s.k = s.v = n * kv_dim * 4;
     s.gate = s.up = n * c.ffn * 4;
     s.xq = n * maxk;
-    s.xh = std::max(n * maxk * 2, cera_kq_act_bytes(n, maxk));   // one of the two f16 forms
+    s.xh = (n + 15) / 16 * 16 * maxk * 2;   // records of 16 tokens
     s.x8 = cera_fp8_split_bytes(n, maxk);
     s.xs = s.bsum = n * (maxk / 32) * 4;
     s.tokens = n * 4;

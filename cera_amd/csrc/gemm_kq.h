@@ -1,20 +1,18 @@
 // Products of Q6_K matrices with many tokens (gemm_kq.hip): the tokens' operand and the launcher.
 #pragma once
-#include "copy_budget.h"
 #include "host_common.h"
 
-// The tokens' operand: one record per 16 tokens and super-block of 256, its two halves of four blocks one behind the other --
-// per block 64 lanes x 16 bytes of f16 quants, then the four blocks' 16 scales each.  Tokens up to a whole tile repeat the last.
-constexpr uint32_t KQ_HALF = 4 * 1024 + 4 * 64, KQ_REC = 2 * KQ_HALF, KQ_TOKENS = 128, KQ_ROWS = 256;
-static_assert(KQ_TOKENS == 128 && KQ_REC == 8704, "cera_kq_act_bytes (copy_budget.h) restates this record geometry");
-static inline uint32_t kq_act_records(uint32_t n, uint32_t k) { return (n + KQ_TOKENS - 1) / KQ_TOKENS * (KQ_TOKENS / 16) * (k / 256); }
+// The tokens' operand: one record per 16 tokens and super-block of 256, per block 64 lanes x 16 bytes of f16 quants; as many bytes
+// as the row-major form where the tokens are a multiple of 16.  Tokens up to a whole tile repeat the last.
+constexpr uint32_t KQ_HALF = 4 * 1024, KQ_REC = 2 * KQ_HALF, KQ_TOKENS = 128, KQ_ROWS = 256;
+static inline uint32_t kq_act_records(uint32_t n, uint32_t k) { return (n + 15) / 16 * (k / 256); }
+static inline uint64_t kq_act_bytes(uint64_t n, uint64_t k) { return (n + 15) / 16 * (k / 256) * KQ_REC; }
 
 // Of the eight dwords of a block's 32 quants, lane group g holds this one and the next: groups with an even number the first
 // sixteen quants, with an odd one the others.
 __device__ __forceinline__ constexpr uint32_t kq_dword(uint32_t g) { return 4 * (g & 1) + 2 * (g >> 1); }
 // One workgroup of 256 per record: a thread takes 8 of the 16 x 128 quants of each half.
-__device__ __forceinline__ void kq_act_record(uint32_t index, const int8_t* __restrict__ bq, const float* __restrict__ bs, uint8_t* __restrict__ act,
-                                              uint32_t n, uint32_t k) {
+__device__ __forceinline__ void kq_act_record(uint32_t index, const int8_t* __restrict__ bq, uint8_t* __restrict__ act, uint32_t n, uint32_t k) {
     typedef _Float16 v2 __attribute__((ext_vector_type(2)));
     const uint32_t nsb = k / 256, tile = index / nsb, sb = index - tile * nsb;
     uint8_t* const rec = act + static_cast<uint64_t>(index) * KQ_REC;
@@ -29,10 +27,6 @@ __device__ __forceinline__ void kq_act_record(uint32_t index, const int8_t* __re
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2, w[i] | 0x64006400u) + off);
         *reinterpret_cast<uint4*>(rec + h * KQ_HALF + wave * 1024 + lane * 16) = make_uint4(o[0], o[1], o[2], o[3]);
-    }
-    if (threadIdx.x < 128) {
-        const uint32_t b = threadIdx.x >> 4, t = min(tile * 16 + (threadIdx.x & 15), n - 1);
-        *reinterpret_cast<float*>(rec + (b >> 2) * KQ_HALF + 4096 + (b & 3) * 64 + (threadIdx.x & 15) * 4) = bs[static_cast<uint64_t>(t) * (k / 32) + sb * 8 + b];
     }
 }
 
@@ -54,7 +48,8 @@ static inline uint32_t kq_slices(uint32_t dtype, uint64_t m, uint64_t m2, uint32
 
 struct KqArgs {
     const uint8_t *w, *w2;   // native blocks; w2 (nullable): a second matrix of the same type and k
-    const uint8_t* act;
+    const uint8_t* act;      // records
+    const float* bs;         // [n][k / 32] the tokens' block scales
     float *out, *out2;
     uint32_t m, m2, n, k, row_bytes, tiles1, k_chunk;   // tiles1: row tiles of the first matrix
     uint64_t ld_m, ld_n, ld_n2;                         // out[i * ld_m + j * ld_n], out2[i * ld_m + j * ld_n2]
@@ -63,6 +58,6 @@ struct KqArgs {
     float resid_scale;
 };
 
-cera_hip_status cera_launch_kq_act(cera_hip_ctx* ctx, const float* bs, const int8_t* bq, uint32_t n, uint32_t k, void* act);
+cera_hip_status cera_launch_kq_act(cera_hip_ctx* ctx, const int8_t* bq, uint32_t n, uint32_t k, void* act);
 // grid (token tiles, row tiles, slices of k_chunk)
 cera_hip_status cera_launch_kq(cera_hip_ctx* ctx, const KqArgs& a, uint32_t split);

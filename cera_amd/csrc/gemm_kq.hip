@@ -33,8 +33,8 @@ __device__ __forceinline__ h2v bytes02(uint32_t v) { return as_h2(__builtin_amdg
 __device__ __forceinline__ h2v bytes13(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
 template <int J> __device__ __forceinline__ h2v byte_twice(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | J | J << 16)); }
 
-__global__ __launch_bounds__(256) void kq_act_kernel(const int8_t* __restrict__ bq, const float* __restrict__ bs, uint8_t* __restrict__ act, uint32_t n, uint32_t k) {
-    kq_act_record(blockIdx.x, bq, bs, act, n, k);
+__global__ __launch_bounds__(256) void kq_act_kernel(const int8_t* __restrict__ bq, uint8_t* __restrict__ act, uint32_t n, uint32_t k) {
+    kq_act_record(blockIdx.x, bq, act, n, k);
 }
 
 // ---- Q6_K: half h of a super-block is two runs j of 16 codes of each of its four blocks --------------------------
@@ -87,7 +87,8 @@ struct KqQ6 {
 template <typename W>
 __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
     constexpr int RT = 2, T = KQ_TOKENS / 16;   // 16-row and 16-token tiles of a wavefront
-    __shared__ __align__(16) uint8_t act[2][T * KQ_HALF];
+    constexpr uint32_t TILE = KQ_HALF + 256;    // a tile's half record, and behind it the four blocks' 16 scales each
+    __shared__ __align__(16) uint8_t act[2][T * TILE];
     __shared__ __align__(16) uint8_t wts[2][W::BYTES];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
     const bool second = p.w2 != nullptr && blockIdx.y >= p.tiles1;
@@ -98,18 +99,21 @@ __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
     const uint32_t wr = threadIdx.x >> 1, wj = threadIdx.x & 1;
     const uint8_t* const wrow = wmat + static_cast<uint64_t>(min(m0 + wr, rows - 1)) * p.row_bytes;
     // this wavefront's share of a stage's tokens: one tile of 16
-    const uint8_t* const rec = p.act + static_cast<uint64_t>(blockIdx.x * T + wave) * nsb * KQ_REC;
-    const uint32_t act_lds = lds_addr(&act[0][0]) + wave * KQ_HALF;
+    // (tiles past the end are the last one again: their products are not stored)
+    const uint32_t tile = min(blockIdx.x * T + wave, (p.n - 1) / 16);
+    const uint8_t* const rec = p.act + static_cast<uint64_t>(tile) * nsb * KQ_REC;
+    const float* const bs = p.bs + static_cast<uint64_t>(tile) * 16 * (p.k / 32);
+    const uint32_t bs_lane = (min(col, p.n - 1 - tile * 16) * (p.k / 32) + g) * 4;
+    const uint32_t act_lds = lds_addr(&act[0][0]) + wave * TILE;
     // piece p of a stage's loads: the rows' first, then the tokens'
     typename W::Stage st;
     auto load = [&](auto p_, uint32_t stage, uint32_t buf) {
         constexpr int p = decltype(p_)::value;
         if constexpr (p < W::LOADS) W::template load<p>(st, wrow, stage, wj);
         else if constexpr (p < W::LOADS + 5) {
-            const uint8_t* const r = rec + static_cast<uint64_t>(stage >> 1) * KQ_REC + (stage & 1) * KQ_HALF + (p - W::LOADS) * 1024;
-            const uint32_t l = act_lds + buf * (T * KQ_HALF) + (p - W::LOADS) * 1024;
-            if constexpr (p < W::LOADS + 4) lds_dma_1k(r, lane * 16, l);
-            else lds_dma_256(r, lane * 4, l);
+            const uint32_t l = act_lds + buf * (T * TILE) + (p - W::LOADS) * 1024;
+            if constexpr (p < W::LOADS + 4) lds_dma_1k(rec + static_cast<uint64_t>(stage) * KQ_HALF + (p - W::LOADS) * 1024, lane * 16, l);
+            else lds_dma_256(bs + stage * 4, bs_lane, l);
         }
     };
     f4v acc[RT][T], sum[RT][T];
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
         h8v x[3];        // tokens' fragments and scales, two steps ahead
         float xs[4];
         auto read = [&](int i) {
-            const uint8_t* const a = al + (i & 7) * KQ_HALF;
+            const uint8_t* const a = al + (i & 7) * TILE;
             x[i % 3] = *reinterpret_cast<const h8v*>(a + (i >> 3) * 1024 + lane * 16);
             xs[i & 3] = *reinterpret_cast<const float*>(a + 4096 + (i >> 3) * 64 + col * 4);
         };
@@ -227,8 +231,8 @@ __global__ __launch_bounds__(512, 2) void gemm_kq_kernel(KqArgs p) {
 
 }  // namespace
 
-cera_hip_status cera_launch_kq_act(cera_hip_ctx* ctx, const float* bs, const int8_t* bq, uint32_t n, uint32_t k, void* act) {
-    hipLaunchKernelGGL(kq_act_kernel, dim3(kq_act_records(n, k)), dim3(256), 0, ctx->stream, bq, bs, static_cast<uint8_t*>(act), n, k);
+cera_hip_status cera_launch_kq_act(cera_hip_ctx* ctx, const int8_t* bq, uint32_t n, uint32_t k, void* act) {
+    hipLaunchKernelGGL(kq_act_kernel, dim3(kq_act_records(n, k)), dim3(256), 0, ctx->stream, bq, static_cast<uint8_t*>(act), n, k);
     HIP_TRY(ctx, hipGetLastError());
     return CERA_HIP_OK;
 }

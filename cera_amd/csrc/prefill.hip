@@ -78,12 +78,12 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     if (w->dtype == CERA_HIP_Q6_K) {
         const ActForm form = kq ? ActForm::records : ActForm::rows;
         if (!bh_ws) {
-            CERA_TRY(cera_scratch(ctx, 10, kq ? cera_kq_act_bytes(n, a.k) : static_cast<uint64_t>(n) * a.k * 2, &bh_ws));
+            CERA_TRY(cera_scratch(ctx, 10, kq ? kq_act_bytes(n, a.k) : static_cast<uint64_t>(n) * a.k * 2, &bh_ws));
             staged = nullptr;
         }
         if (!staged || *staged != form) {
             const uint64_t words = static_cast<uint64_t>(n) * a.k / 16;
-            if (kq) CERA_TRY(cera_launch_kq_act(ctx, bs, bq, n, a.k, bh_ws));
+            if (kq) CERA_TRY(cera_launch_kq_act(ctx, bq, n, a.k, bh_ws));
             else hipLaunchKernelGGL(gemm_act_f16_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0,
                                     ctx->stream, reinterpret_cast<const uint4*>(bq), static_cast<uint4*>(bh_ws), words);
             if (staged) *staged = form;
@@ -175,7 +175,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false>), grid, dim3(256), 0, ctx->stream, a); break;
         case CERA_HIP_Q6_K:
             if (kq)
-                CERA_TRY(cera_launch_kq(ctx, KqArgs{a.w, a.w2, static_cast<const uint8_t*>(a.bh), a.out, a.out2, a.m, a.m2, n, a.k, a.row_bytes, a.tiles1,
+                CERA_TRY(cera_launch_kq(ctx, KqArgs{a.w, a.w2, static_cast<const uint8_t*>(a.bh), bs, a.out, a.out2, a.m, a.m2, n, a.k, a.row_bytes, a.tiles1,
                                                     a.k_chunk, ld_m, ld_n, ld_n2, a.part_stride, a.resid, resid_scale}, split));
             else hipLaunchKernelGGL(gemm_q6k_f16_kernel<false>, grid, dim3(256), 0, ctx->stream, a);
             break;
@@ -518,7 +518,7 @@ cera_hip_status cera_model_ensure_prefill_buffers(cera_hip_model* m, uint32_t n)
 static __global__ __launch_bounds__(256) void act_fp8_records_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xs, const float* __restrict__ bsum,
                                                                      uint8_t* __restrict__ x8, uint32_t fp8_records, uint8_t* __restrict__ records, uint32_t n, uint32_t k) {
     if (blockIdx.x < fp8_records) gemm_act_fp8_body(xq, xs, bsum, x8, n, k);
-    else kq_act_record(blockIdx.x - fp8_records, xq, xs, records, n, k);
+    else kq_act_record(blockIdx.x - fp8_records, xq, records, n, k);
 }
 
 // The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.
