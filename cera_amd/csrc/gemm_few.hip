@@ -2,7 +2,7 @@
 // their decode copies or, with the same bits, from the native blocks.
 //
 // A wavefront owns 16 weight rows and streams their super-blocks straight into registers, two to four of them ahead; the tokens, in
-// tiles of 16, come from LDS, where the workgroup's four wavefronts put them as f16 (the Q8_0 codes are whole numbers, exact
+// tiles of 16, come from LDS, where the workgroup's eight wavefronts put them as f16 (the Q8_0 codes are whole numbers, exact
 // in f16), a chunk of super-blocks ahead.  One v_mfma_f32_16x16x32_f16 is one 32-weight block: Q4_K weights enter as
 // scale * code, at most 945 and exact in f16; Q6_K weights, at most 4064, as two f16 parts whose sum they are.  So a block's
 // result is the exact whole number sum(scale * code * quant), below 2^24, and what the vector ALU adds is one FMA with the
@@ -10,7 +10,10 @@
 // own product (mins times the tokens' block sums in three bf16 parts).  Sums over K go in order within a slice.
 //
 // What bounds it: up to 16 tokens the weights' way from HBM, above that the vector ALU, about 130 (Q4_K) and 225 (Q6_K)
-// instructions per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens.
+// instructions per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens (45 tokens: vector ALU 56 % busy, matrix cores
+// 15 %).  Gate | up, 14336 x 4096 Q4_K as a pair: 22 us at 5 tokens, 37 at 45; down, 4096 x 14336 Q6_K: 20 and 25.  The 64-token
+// tiles before it took 36 us for a down product and 50 for a pair, with a launch for the tokens' copy before and one for the sums
+// behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 289 us, 45 tokens 466 -> 322.
 #include <algorithm>
 
 #include "gemv.hip.h"
