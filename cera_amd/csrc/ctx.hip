@@ -61,6 +61,8 @@ bool cera_type_geometry(uint32_t t, uint32_t* e, uint32_t* b) {
 cera_hip_status cera_scratch(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out) {
     if (nbytes == 0) nbytes = 256;
     if (ctx->scratch_bytes[slot] < nbytes) {
+        if (ctx->scratch_limit && nbytes > ctx->scratch_limit)
+            return cera_fail(ctx, CERA_HIP_ERR_OOM, "workspace of " + std::to_string(nbytes) + " bytes: over the context's limit of " + std::to_string(ctx->scratch_limit));
         if (ctx->scratch[slot]) {
             HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
             HIP_TRY(ctx, hipFree(ctx->scratch[slot]));
@@ -72,6 +74,14 @@ cera_hip_status cera_scratch(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void*
         ctx->scratch_bytes[slot] = want;
     }
     *out = ctx->scratch[slot];
+    return CERA_HIP_OK;
+}
+
+cera_hip_status cera_scratch_if_room(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out) {
+    *out = nullptr;
+    const cera_hip_status st = cera_scratch(ctx, slot, nbytes, out);
+    if (st != CERA_HIP_ERR_OOM) return st;
+    (void)hipGetLastError();   // or the next launch would report it
     return CERA_HIP_OK;
 }
 
@@ -193,6 +203,13 @@ cera_hip_status cera_hip_ctx_set_decode_copies(cera_hip_ctx* ctx, int enabled) {
     if (!ctx) return CERA_HIP_ERR_ARGUMENT;
     std::lock_guard<std::recursive_mutex> lk(ctx->op_mu);
     ctx->decode_copies = enabled != 0;
+    return CERA_HIP_OK;
+}
+
+cera_hip_status cera_hip_ctx_set_workspace_limit(cera_hip_ctx* ctx, uint64_t bytes) {
+    if (!ctx) return CERA_HIP_ERR_ARGUMENT;
+    std::lock_guard<std::recursive_mutex> lk(ctx->op_mu);
+    ctx->scratch_limit = bytes;
     return CERA_HIP_OK;
 }
 

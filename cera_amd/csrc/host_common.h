@@ -38,6 +38,7 @@ struct cera_hip_ctx {
     // grow-only device scratch for the host-pointer entry points
     void* scratch[16] = {nullptr};
     uint64_t scratch_bytes[16] = {0};
+    uint64_t scratch_limit = 0;       // cera_hip_ctx_set_workspace_limit; 0: none
     void* static_scratch = nullptr;   // this device's copy of the library's fixed workspace (resolved at creation)
     // optional standalone code object (cera_hip_ctx_create with an hsaco_path): the quantizer and the
     // GEMV instances it exports are then launched from it with hipModuleLaunchKernel
@@ -78,6 +79,8 @@ bool cera_type_geometry(uint32_t t, uint32_t* block_elems, uint32_t* block_bytes
 // type, shape and byte count of a caller's tensor; *row_bytes: bytes of one row
 cera_hip_status cera_check_tensor(cera_hip_ctx* ctx, const cera_hip_tensor* t, uint64_t* row_bytes);
 cera_hip_status cera_scratch(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out);
+// a workspace that a call is faster with but can do without: *out = nullptr where there is no room for it
+cera_hip_status cera_scratch_if_room(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out);
 // kernel `name` of the context's loaded code object, nullptr when there is no module or no such kernel
 hipFunction_t cera_module_fn(cera_hip_ctx* ctx, const std::string& name);
 // launch a one-struct-argument kernel of the loaded code object

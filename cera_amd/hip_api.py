@@ -18,7 +18,7 @@ STATUS = {0: "OK", 1: "ERR_DEVICE", 2: "ERR_OOM", 3: "ERR_UNSUPPORTED_DTYPE", 4:
 
 # every symbol include/cera_hip.h declares
 SYMBOLS = [
-    "cera_hip_ctx_create", "cera_hip_ctx_destroy", "cera_hip_ctx_set_decode_copies", "cera_hip_decode_copy_reserve_bytes", "cera_hip_decode_copy_plan", "cera_hip_drop_decode_copies", "cera_hip_last_error", "cera_hip_sync", "cera_hip_device_info",
+    "cera_hip_ctx_create", "cera_hip_ctx_destroy", "cera_hip_ctx_set_decode_copies", "cera_hip_ctx_set_workspace_limit", "cera_hip_decode_copy_reserve_bytes", "cera_hip_decode_copy_plan", "cera_hip_drop_decode_copies", "cera_hip_last_error", "cera_hip_sync", "cera_hip_device_info",
     "cera_hip_malloc", "cera_hip_free", "cera_hip_upload", "cera_hip_download", "cera_hip_copy_dev", "cera_hip_copy_kernel",
     "cera_hip_event_create", "cera_hip_event_destroy", "cera_hip_event_record", "cera_hip_event_elapsed_ms",
     "cera_hip_tensor_upload", "cera_hip_tensor_clone", "cera_hip_tensor_free", "cera_hip_tensor_nbytes",
@@ -122,6 +122,7 @@ def load_library() -> C.CDLL:
     sig = {
         "cera_hip_ctx_create": (i32, [i32, C.c_char_p, pp]), "cera_hip_ctx_destroy": (None, [vp]),
         "cera_hip_ctx_set_decode_copies": (i32, [vp, i32]),
+        "cera_hip_ctx_set_workspace_limit": (i32, [vp, u64]),
         "cera_hip_decode_copy_reserve_bytes": (u64, [vp]),
         "cera_hip_decode_copy_plan": (u64, [vp, u32, u64, u64, vp]),
         "cera_hip_drop_decode_copies": (i32, [vp, vp]),
@@ -268,6 +269,10 @@ class Context:
     def set_decode_copies(self, enabled: bool):
         """Whether matrices prepared from now on get the permuted second copy the decode GEMVs stream."""
         self.check(self.lib.cera_hip_ctx_set_decode_copies(self.h, 1 if enabled else 0))
+
+    def set_workspace_limit(self, nbytes: int):
+        """Most bytes one of this context's workspaces may grow to (0: no limit)."""
+        self.check(self.lib.cera_hip_ctx_set_workspace_limit(self.h, nbytes))
 
     def device_info(self):
         name = C.create_string_buffer(256)

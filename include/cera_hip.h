@@ -111,6 +111,11 @@ CERA_HIP_API cera_hip_status cera_hip_sync(cera_hip_ctx*);
  * for one kernel, as the reference's x86 path does with repack_q4_k_8x8
  * (cera/src/backend/cpu.rs:1282-1358); it has no switch there. */
 CERA_HIP_API cera_hip_status cera_hip_ctx_set_decode_copies(cera_hip_ctx* ctx, int enabled);
+/* The most bytes one of the context's workspaces may grow to (0, the default: no limit).  A call that
+ * cannot do without more fails with CERA_HIP_ERR_OOM, as it does where the device has no more memory; one
+ * that is only faster with it (key and value tiles of a large attention batch laid out once) runs without
+ * it.  Workspaces that are already larger stay. */
+CERA_HIP_API cera_hip_status cera_hip_ctx_set_workspace_limit(cera_hip_ctx* ctx, uint64_t bytes);
 /* The rule by which cera_hip_model_create hands out decode copies, as plain arithmetic (no device
  * is touched; callable without a GPU).  A model's copies are built last -- after every native
  * upload, the KV caches and the single-token buffers -- and only while the device keeps

@@ -258,6 +258,7 @@ pub fn cera_hip_ctx_create(
     ) -> cera_hip_status;
     pub fn cera_hip_ctx_destroy(ctx: *mut cera_hip_ctx);
     pub fn cera_hip_ctx_set_decode_copies(ctx: *mut cera_hip_ctx, enabled: c_int) -> cera_hip_status;
+    pub fn cera_hip_ctx_set_workspace_limit(ctx: *mut cera_hip_ctx, bytes: u64) -> cera_hip_status;
     pub fn cera_hip_decode_copy_reserve_bytes(cfg: *const cera_hip_config) -> u64;
     pub fn cera_hip_decode_copy_plan(
         copy_bytes: *const u64,

@@ -500,6 +500,24 @@ def test_attn_prefill_of_many_queries(hip, orc, nh, nkv, hd, kv_f16, start, n):
         assert np.isfinite(out[:64] if poison else out).all()
 
 
+def test_attn_prefill_without_room_for_records():
+    """The split tiles of the cache are a workspace that the pass can do without: where it cannot be had (here by a limit
+    that the inputs fit and the records do not), the kernel without it runs, with the same products in the same order."""
+    nh, nkv, hd, start, n = 8, 2, 128, 1500, 290
+    r = util.rng(3)
+    L = start + n
+    q = r.standard_normal((n, nh * hd), dtype=np.float32)
+    k, v = (r.standard_normal(L * nkv * hd, dtype=np.float32) for _ in range(2))
+    out = []
+    for limit in (0, 5 << 19):
+        ctx = hip_api.Context(0)
+        ctx.set_workspace_limit(limit)
+        _say(f"attn_prefill many, workspace limit {limit}")
+        out.append(ctx.attn_prefill(q, k, v, nh, nkv, hd, start, n, 1.0 / np.sqrt(hd)))
+        ctx.close()
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
 def test_prefill_longer_than_one_pass(hip, orc):
     """A prompt beyond the 2048-token pass size is cut into passes; logits and the cache rows on
     both sides of the cut track the oracle's single batched prefill."""
