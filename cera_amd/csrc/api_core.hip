@@ -431,8 +431,13 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
     // visible keys are a bounded part of what is kept free for its workspaces.
     void* records = nullptr;
     const uint64_t rec = head_dim * 128ull * (kv_f16 ? 1 : 2), rec_bytes = (last_len + 31) / 32 * n_kv_heads * rec;
-    if (batch && !ws && n_queries * (seq_len + last_len) / 2 >= ATTN_RECORDS_MIN_PAIRS && rec_bytes <= ATTN_RECORDS_MAX_BYTES && attn_records_fit(static_cast<uint32_t>(rec), G))
-        CERA_TRY(cera_scratch_if_room(ctx, 13, rec_bytes, &records));   // without room the other kernel, which needs none
+    if (batch && !ws && n_queries * (seq_len + last_len) / 2 >= ATTN_RECORDS_MIN_PAIRS && rec_bytes <= ATTN_RECORDS_MAX_BYTES && attn_records_fit(static_cast<uint32_t>(rec), G)) {
+        // room for the whole cache as far as that is bounded, so that a context that grows does not free and allocate in every
+        // pass; without room for that, room for this pass, and without that the other kernel, which needs none
+        const uint64_t whole = std::min(ATTN_RECORDS_MAX_BYTES, (max_seq + 31) / 32 * n_kv_heads * rec);
+        if (ctx->scratch_bytes[13] < rec_bytes) CERA_TRY(cera_scratch_if_room(ctx, 13, whole, &records));
+        if (!records) CERA_TRY(cera_scratch_if_room(ctx, 13, rec_bytes, &records));
+    }
     AttnLaunch a{q, static_cast<uint32_t>(seq_len), static_cast<uint32_t>(max_seq), scale, n_heads, n_kv_heads, n_queries,
                  n_heads * head_dim, G, S, n_parts, part_keys, chunks_per_part, Gw, batch, new_kv != nullptr, nk, acc, ml,
                  static_cast<uint8_t*>(records)};

@@ -518,6 +518,23 @@ def test_attn_prefill_without_room_for_records():
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
 
 
+def test_records_of_a_growing_context_take_their_room_once():
+    """Passes further and further into a context split more and more tiles: the room for them is that of the whole cache from
+    the first pass on, so that no later one stops to allocate."""
+    cfg = dict(synth.TINY, hidden=512, ffn=512, n_heads=24, n_kv_heads=8, head_dim=128, n_layers=1, max_seq_len=4096)
+    ctx = hip_api.Context(0)
+    m = hip_api.Model(ctx, cfg, synth.make_llama(cfg, seed=5, sigma=0.05))
+    toks = [int(t) for t in util.rng(6).integers(0, cfg["vocab"], 4000)]
+    free = []
+    for at in range(0, 4000, 1000):
+        m.forward_prefill(toks[at:at + 1000], at)
+        free.append(util.free_device_bytes())
+        _say(f"prefill of 1000 tokens behind {at}: {free[-1]} bytes free")
+    m.close()
+    ctx.close()
+    assert len(set(free)) == 1
+
+
 def test_prefill_longer_than_one_pass(hip, orc):
     """A prompt beyond the 2048-token pass size is cut into passes; logits and the cache rows on
     both sides of the cut track the oracle's single batched prefill."""

@@ -3,6 +3,8 @@ dequantizer written from the GGUF block-format definition (used to check the
 oracle, never the other way round)."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 
 from cera_amd import host_api as H
@@ -147,3 +149,10 @@ def unpack_ints_np(dtype: int, blocks: np.ndarray, m: int, k: int) -> np.ndarray
 def rms(a) -> float:
     a = np.asarray(a, np.float64)
     return float(np.sqrt(np.mean(a * a)))
+
+
+def free_device_bytes() -> int:
+    rt = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
