@@ -705,8 +705,6 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     else if (n > 128 && area * 20 >= rounds * ctx->n_cu * 65536 * 11) { shape = 3; bm = bn = 256; }
     else if (n > 64 && (count(128, 128) >= ctx->n_cu || (a.kp >= 8192 && count(128, 128) * 4 >= ctx->n_cu))) { shape = 0; bm = bn = 128; }
     else if (n > 32) { shape = 1; bm = bn = 64; }
-    a.tiles_m = (a.m + bm - 1) / bm;
-    a.tiles_n = (n + bn - 1) / bn;
     const uint64_t wgs = count(bm, bn);
     const uint32_t steps = a.kp / DENSE_PAD;
     uint32_t split = 1;
@@ -717,15 +715,23 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     if (split < 1) split = 1;
     const uint32_t per = (steps + split - 1) / split;
     split = (steps + per - 1) / per;
-    a.k_chunk = per * DENSE_PAD;
     // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
     // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
     const bool apart = o.epi == DENSE_STREAMS && (o.streams->count != 4 || shape == 0 || shape == 3);
     if (split > 1 || apart) {
-        void* part;
-        CERA_TRY(cera_scratch(ctx, 9, static_cast<uint64_t>(split) * n * a.m * sizeof(float), &part));
+        void* part = nullptr;
+        CERA_TRY(cera_scratch_if_room(ctx, 9, static_cast<uint64_t>(split) * n * a.m * sizeof(float), &part));
+        // without room: the whole of K in one workgroup, four streams by small tiles' own lanes
+        if (!part) {
+            split = 1;
+            if (apart && o.streams->count != 4) CERA_TRY(cera_scratch(ctx, 9, static_cast<uint64_t>(n) * a.m * sizeof(float), &part));
+            else if (apart) { shape = 1; bm = bn = 64; }
+        }
         a.part = static_cast<float*>(part);
     }
+    a.k_chunk = (steps + split - 1) / split * DENSE_PAD;
+    a.tiles_m = (a.m + bm - 1) / bm;
+    a.tiles_n = (n + bn - 1) / bn;
     const dim3 grid((a.tiles_m * groups.count + 7) / 8 * 8 * a.tiles_n, split);
     const uint64_t quads = (a.epi == DENSE_SWIGLU ? (a.m / 2 + 3) / 4 : (a.m + 3) / 4) * static_cast<uint64_t>(n);
     const dim3 rg(static_cast<uint32_t>((quads + 255) / 256)), block(256);

@@ -334,6 +334,26 @@ def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
     m.close()
 
 
+def test_streams_of_large_tiles_without_room_for_partial_sums():
+    """Large tiles hand the streams' products to the reduction, which needs room for them; where there is none (here by a
+    limit), smaller tiles update the four streams themselves."""
+    cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=200)], width=5200, vocab=64, streams=4)
+    w = U.random_model(cfg, 47)
+    bits = {name: U.bf16_bits(a) if a.ndim == 2 and ".hc" not in name else a for name, a in w.items()}
+    toks = U.tokens(cfg, 1800, 5)
+    out = []
+    for limit in (0, 16 << 20):   # the products are 37 MB
+        ctx = hip_api.Context(0)
+        ctx.set_workspace_limit(limit)
+        m = hip_api.LayeredModel(ctx, cfg, bits, 1800)
+        out.append(m.forward_prefill_logits_all(np.asarray(toks, np.uint32), 0))
+        print(f"limit {limit}: {U.rel(out[-1], U.reference(cfg, w, toks)):.2e}", flush=True)
+        m.close()
+        ctx.close()
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+    assert U.rel(out[1], U.reference(cfg, w, toks)) < TOL[False]
+
+
 @DTYPES
 def test_steps_behind_a_very_long_context(tmp_path, f32):
     """Thousands of visible keys: decode steps and short portions split them over many workgroups."""
