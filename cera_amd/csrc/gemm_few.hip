@@ -415,7 +415,13 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     a.sb_per = (nsb + split - 1) / split;
     split = (nsb + a.sb_per - 1) / a.sb_per;
     uint64_t rows = 0;
-    float* part = nullptr;
+    void* part_room = nullptr;
+    if (split > 1) CERA_TRY(cera_scratch_if_room(ctx, part_slot, split * (w->m + (ob ? ob->w->m : 0)) * static_cast<uint64_t>(n) * 4, &part_room));
+    if (!part_room) {   // the whole of K in one workgroup
+        split = 1;
+        a.sb_per = nsb;
+    }
+    float* const part = static_cast<float*>(part_room);
     auto set = [&](FewMat& m, const FewOut& o) {
         m.w = copy ? o.w->dev_stream : o.w->dev;
         m.row_bytes = static_cast<uint32_t>(copy ? o.w->stream_row_bytes : o.w->row_bytes);
@@ -430,11 +436,7 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
         }
         rows += m.m;
     };
-    if (split > 1) {
-        void* p;
-        CERA_TRY(cera_scratch(ctx, part_slot, split * (w->m + (ob ? ob->w->m : 0)) * static_cast<uint64_t>(n) * 4, &p));
-        part = static_cast<float*>(p);
-    } else {
+    if (split == 1) {
         a.resid = resid; a.resid_scale = resid_scale;
     }
     set(a.a, oa);

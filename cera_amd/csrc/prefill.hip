@@ -146,13 +146,14 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         for (uint32_t d = 2; d <= 8 && split < want; ++d)
             if (nsb % d == 0 && nsb / d >= 2) split = d;
     }
-    a.k_chunk = a.k / split;
-    a.part_stride = 0;
     // a pair's partials lie side by side: [split][m*n | m2*n]
     const uint64_t mn = static_cast<uint64_t>(a.m) * n, mn2 = static_cast<uint64_t>(a.m2) * n;
+    void* part = nullptr;
+    if (split > 1) CERA_TRY(cera_scratch_if_room(ctx, part_slot, split * (mn + mn2) * sizeof(float), &part));
+    if (!part) split = 1;   // without room: the whole of K in one workgroup
+    a.k_chunk = a.k / split;
+    a.part_stride = 0;
     if (split > 1) {
-        void* part;
-        CERA_TRY(cera_scratch(ctx, part_slot, split * (mn + mn2) * sizeof(float), &part));
         a.out = static_cast<float*>(part);
         if (a.w2) a.out2 = a.out + mn;
         a.part_stride = mn + mn2;

@@ -113,8 +113,8 @@ CERA_HIP_API cera_hip_status cera_hip_sync(cera_hip_ctx*);
 CERA_HIP_API cera_hip_status cera_hip_ctx_set_decode_copies(cera_hip_ctx* ctx, int enabled);
 /* The most bytes one of the context's workspaces may grow to (0, the default: no limit).  A call that
  * cannot do without more fails with CERA_HIP_ERR_OOM, as it does where the device has no more memory; one
- * that is only faster with it (key and value tiles of a large attention batch laid out once) runs without
- * it.  Workspaces that are already larger stay. */
+ * that is only faster with it (key and value tiles of a large attention batch laid out once, sums over
+ * parts of K) runs without it.  Workspaces that are already larger stay. */
 CERA_HIP_API cera_hip_status cera_hip_ctx_set_workspace_limit(cera_hip_ctx* ctx, uint64_t bytes);
 /* The rule by which cera_hip_model_create hands out decode copies, as plain arithmetic (no device
  * is touched; callable without a GPU).  A model's copies are built last -- after every native

@@ -158,6 +158,24 @@ def test_gemm_q6k_of_many_tokens(hip, orc, ma, mb, n, k):
         assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
 
 
+@pytest.mark.parametrize("dtype,n,m,k,limit", [(Q4_K, 48, 4096, 2048, 2 << 20), (Q6_K, 5, 4096, 2048, 1 << 18), (Q6_K, 128, 4096, 2048, 4 << 20)])
+def test_products_without_room_for_partial_sums(dtype, n, m, k, limit):
+    """Sums over parts of K are a workspace that a product can do without: where it cannot be had (here by a limit that the
+    inputs and outputs fit and the parts do not), one workgroup takes the whole of K.  Both are within 2e-5 of the outputs' rms
+    of the exact product, as test_gemm_pair_of_a_few_tokens has it."""
+    w, _ = util.make_weights(dtype, m, k, seed=3)
+    x = util.rng(n).standard_normal((n, k)).astype(np.float32)
+    out = []
+    for room in (0, limit):
+        ctx = hip_api.Context(0)
+        ctx.set_workspace_limit(room)
+        _say(f"gemm_pair {util.NAMES[dtype]} {m}x{k} n={n} limit {room}")
+        out.append(ctx.gemm_pair(dtype, w, m, dtype, w, m, x, n, k))
+        ctx.close()
+    assert np.array_equal(out[1][0], out[1][1])
+    assert np.abs(out[0][0] - out[1][0]).max() <= 4e-5 * util.rms(out[0][0])
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q4_0, Q4_1, Q8_0])
 @pytest.mark.parametrize("m,k,n,want_fused", [(2048, 512, 1040, True), (1056, 256, 2000, True), (512, 256, 70, False)])
 def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n, want_fused):
