@@ -780,6 +780,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             hipLaunchKernelGGL((silu_mul_kernel<true>), dim3(static_cast<uint32_t>((tot / 4 + 255) / 256)), dim3(256), 0, s,
                                m->pf_gate, m->pf_up, tot, m->pf_gate, m->pf_xs, m->pf_xq, m->pf_bsum);
             HIP_TRY(ctx, hipGetLastError());
+            staged = ActForm::none;   // pf_xh holds what a Q6_K gate and up have read
             split_of = nullptr;
         }
         staged8 = false;   // pf_xq holds the SwiGLU output now

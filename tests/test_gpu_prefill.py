@@ -402,6 +402,20 @@ def test_prefill_where_the_norm_adds_split_k_partial_sums(hip, orc, rope_type, k
     gm.close(); om.close()
 
 
+@pytest.mark.parametrize("n", [12, 49, 70, 200])
+def test_prefill_of_a_model_all_in_q6_k(hip, orc, n):
+    """Q6_K gate and up in front of a Q6_K down projection: the f16 form of the normed activations, which gate and up
+    leave behind, is not the down projection's input.  A pass of 64-token tiles, and of the records of more tokens."""
+    cfg = dict(synth.TINY, max_seq_len=256)
+    weights = synth.make_llama(cfg, seed=84, sigma=0.05, norm_jitter=0.1, type_of=lambda name: Q6_K)
+    gm, om = hip_api.Model(hip, cfg, weights), orc.Llama(cfg, weights)
+    toks = [int(t) for t in util.rng(n).integers(0, cfg["vocab"], n)]
+    lg, lo = gm.forward_prefill(toks, 0), om.forward_prefill_batched(toks, 0)
+    _say(f"q6_k model, {n} tokens: cos {_cos(lg, lo):.8f}")
+    assert _cos(lg, lo) > 0.999
+    gm.close(); om.close()
+
+
 @pytest.mark.parametrize("nh,nkv,start,n", [(32, 8, 0, 512), (8, 2, 0, 40), (8, 8, 300, 100), (16, 2, 1000, 33),
                                              (4, 1, 0, 16), (32, 8, 4000, 96), (32, 8, 2048, 2048)])
 def test_attn_prefill_batch_vs_oracle(hip, orc, nh, nkv, start, n):
