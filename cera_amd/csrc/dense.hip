@@ -680,6 +680,23 @@ static uint64_t gemv_stage_len(uint64_t kp, int r) {
 }
 bool cera_dense_gemv_fits(uint64_t kp, bool f32) { return gemv_stage_len(kp, 1) * (f32 ? 4 : 2) <= GEMV_LDS_MAX; }
 
+// the bf16 tiles, and which one a product of `groups` times m rows with n tokens takes
+static constexpr uint32_t DENSE_BM[] = {128, 64, 64, 256}, DENSE_BN[] = {128, 64, 32, 256};
+static int dense_shape(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uint32_t n_cu) {
+    // 256 x 256 where the outputs are at least 55 % of the rounds of one workgroup per CU: 5120 x 3072 times 2048 tokens
+    // (62 %) 77 us against 86 on 128 x 128 tiles, 6176 x 4096 times 1900 (70 %) 98 / 119; below, 4096 x 18432 times 1900 (46 %)
+    // 337 / 268, 3072 x 3072 times 2048 (38 %) 75 / 51.  An XCD takes whole weight tiles (dense_tile), so the rounds are those
+    // of the XCD with the most: 21504 rows times 640 tokens are 252 tiles, but 33 of them on most of the XCDs' 32 CUs.
+    const uint64_t per_xcd = std::max<uint64_t>(n_cu / 8, 1), most = ((m + 255) / 256 * groups + 7) / 8 * ((n + 255) / 256);
+    const uint64_t rounds = (most + per_xcd - 1) / per_xcd, large = (m + 127) / 128 * ((n + 127) / 128) * groups;
+    if (n > 128 && m * groups * n * 20 >= rounds * per_xcd * 8 * 65536 * 11) return 3;
+    if (n > 64 && (large >= n_cu || (kp >= 8192 && large * 4 >= n_cu))) return 0;
+    return n > 32 ? 1 : 2;
+}
+extern "C" uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu) {
+    return DENSE_BM[dense_shape(rows, (k + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD, n, 1, n_cu)];
+}
+
 cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, const void* x, uint64_t ldx, uint32_t n,
                                        const DenseOut& o, bool f32, const DenseGroups& groups) {
     if (n == 0 || w.rows == 0 || groups.count == 0 || w.rows % groups.count || w.kp == 0 || w.kp % DENSE_PAD || ldx < w.kp || ldx % 8)
@@ -694,18 +711,10 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     a.u = o.u;
     if (o.streams) a.st = *o.streams;
     a.epi = o.epi; a.out = o.out; a.ldo = o.ld; a.bias = o.bias; a.mult = o.mult; a.out_rows = o.rows;
-    // tile: large where it fills the chip, else smaller, else K is split.  256 x 256 where the outputs are at least 55 % of
-    // the rounds of one workgroup per CU: 5120 x 3072 times 2048 tokens (62 %) 77 us against 86 on 128 x 128 tiles, 6176 x 4096
-    // times 1900 (70 %) 98 / 119; below, 4096 x 18432 times 1900 (46 %) 337 / 268, 3072 x 3072 times 2048 (38 %) 75 / 51
-    int shape = 2;
-    uint32_t bm = 64, bn = 32;
-    auto count = [&](uint32_t tm, uint32_t tn) { return static_cast<uint64_t>((a.m + tm - 1) / tm) * ((n + tn - 1) / tn) * groups.count; };
-    const uint64_t rounds = (count(256, 256) + ctx->n_cu - 1) / ctx->n_cu, area = static_cast<uint64_t>(w.rows) * n;
-    if (f32) { bm = bn = 64; }
-    else if (n > 128 && area * 20 >= rounds * ctx->n_cu * 65536 * 11) { shape = 3; bm = bn = 256; }
-    else if (n > 64 && (count(128, 128) >= ctx->n_cu || (a.kp >= 8192 && count(128, 128) * 4 >= ctx->n_cu))) { shape = 0; bm = bn = 128; }
-    else if (n > 32) { shape = 1; bm = bn = 64; }
-    const uint64_t wgs = count(bm, bn);
+    // tile: large where it fills the chip, else smaller, else K is split
+    int shape = f32 ? 2 : dense_shape(a.m, a.kp, n, groups.count, ctx->n_cu);
+    uint32_t bm = f32 ? 64 : DENSE_BM[shape], bn = f32 ? 64 : DENSE_BN[shape];
+    const uint64_t wgs = static_cast<uint64_t>((a.m + bm - 1) / bm) * ((n + bn - 1) / bn) * groups.count;
     const uint32_t steps = a.kp / DENSE_PAD;
     uint32_t split = 1;
     // two workgroups per CU; three quarters of that are left alone on large tiles, whose partial sums cost more than the idle

@@ -546,6 +546,9 @@ typedef struct {
  * layers in execution order, every pass of the loop counted. */
 CERA_HIP_API cera_hip_status cera_hip_layered_create(cera_hip_ctx*, const cera_hip_layered_config*,
                                                      const cera_hip_layered_layer* layers, cera_hip_model** out);
+/* The rule by which a bf16 product [rows][k] times n tokens of such a model takes its tile, as plain arithmetic (no device
+ * is touched): weight rows of the tile -- 256 (times 256 tokens), 128 (128) or 64 (64 or 32) -- on a device of n_cu CUs. */
+CERA_HIP_API uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu);
 CERA_HIP_API void cera_hip_model_destroy(cera_hip_model*);
 /* Model::forward (cera/src/model/mod.rs:200-606; LlamaModel::forward,
  * cera/src/model/llama.rs:1585-1605): one token at `pos` -> vocab logits.
