@@ -321,9 +321,12 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
-@pytest.mark.parametrize("width, ff, n, streams", [(70, 41000, 129, 2), (5200, 64, 1800, 4), (5200, 64, 1800, 3)])
+@pytest.mark.parametrize("width, ff, n, streams", [(70, 32768, 300, 2), (130, 5200, 1800, 2), (200, 5300, 1777, 1), (260, 32700, 287, 2),
+                                                   (5200, 64, 1800, 4), (5200, 130, 1800, 3), (5203, 200, 1799, 4), (5200, 330, 1800, 2)])
 def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
-    """From 60 % of a round of 256 x 256 tiles on: the feed-forward's first product, and the residual streams' epilogue."""
+    """256 x 256 tiles: the feed-forward's first product (width < ff) over two to five K steps of 64, the residual streams'
+    products (ff < width) over one to six, ragged last tiles of rows and tokens."""
+    assert hip_api.dense_tile(max(width, ff), min(width, ff), n) == 256
     cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=ff)], width=width, vocab=64, streams=streams)
     w = U.random_model(cfg, 47)
     m = _open(U.save(tmp_path / "m", cfg, w), False, n)

@@ -289,11 +289,14 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
-@pytest.mark.parametrize("width, ff, n", [(60, 20500, 129), (130, 20480, 257), (200, 20500, 300), (5200, 64, 1800)])
-def test_products_on_the_widest_tiles(tmp_path, width, ff, n):
-    """From 60 % of a round of 256 x 256 tiles on: one, two, three and four K steps, a ragged last tile of rows and of
-    tokens, a token more than one tile; the last has the residual products there."""
-    cfg = U.config([U.attention(2, 1, 32, 32, 700, 32, 10000.0, ff=ff)], width=width, vocab=64, taps=2, positions=n)
+@pytest.mark.parametrize("width, ff, n, vocab", [(60, 16384, 300, 64), (130, 2600, 1800, 64), (200, 16300, 290, 64), (260, 2700, 1777, 64),
+                                                 (330, 64, 1800, 5203), (5200, 64, 1800, 64), (5201, 200, 1799, 64)])
+def test_products_on_the_widest_tiles(tmp_path, width, ff, n, vocab):
+    """256 x 256 tiles over one, three, four and five K steps of 64 for gate | up, six for the head of all positions, two and five for the
+    residual products, ragged last tiles of rows and tokens."""
+    wide, k = max((2 * ff, width), (vocab, width), (width, 64 + ff))
+    assert hip_api.dense_tile(wide, k, n) == 256
+    cfg = U.config([U.attention(2, 1, 32, 32, 700, 32, 10000.0, ff=ff)], width=width, vocab=vocab, taps=2, positions=n)
     w = R.random_model(cfg, 47)
     m = _open(U.save(tmp_path / "m", cfg, w), False, n)
     toks = U.tokens(cfg, n, 5)
