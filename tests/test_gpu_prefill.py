@@ -158,6 +158,43 @@ def test_gemm_q6k_of_many_tokens(hip, orc, ma, mb, n, k):
         assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
 
 
+@pytest.mark.parametrize("dtype,m,k,n", [(Q4_K, 132, 2304, 5), (Q4_K, 300, 4096, 48), (Q6_K, 132, 2304, 3), (Q6_K, 300, 4096, 33),
+                                         (Q6_K, 300, 4096, 160), (Q6_K, 516, 2304, 384)])
+def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
+    """The products of a few and of many tokens in the kernels that passes run: tokens of a single block each and scales
+    that are powers of two leave one block's whole number in every output, so any rounding on the way would show.  Weights
+    of random bytes take the whole range; the last row's scales and codes and the first token's quants are the largest, 32
+    of -128 * -32 * 127 for Q6_K, 1 % below 2^24."""
+    _say(f"whole numbers {util.NAMES[dtype]} m={m} k={k} n={n}")
+    r = util.rng(m + n)
+    bytes_ = 144 if dtype == Q4_K else 210
+    w = r.integers(0, 256, (m, k // 256, bytes_), dtype=np.uint8)
+    w[-1] = 255 if dtype == Q4_K else 0     # the largest scales, mins and codes; for Q6_K code 0 is -32
+    if dtype == Q6_K:
+        w[-1, :, 192:208] = 128
+    d = np.exp2(r.integers(-12, -5, (m, k // 256, 1))).astype(np.float16).view(np.uint8)
+    if dtype == Q4_K:
+        w[:, :, 0:2], w[:, :, 2:4] = d, d
+    else:
+        w[:, :, 208:210] = d
+    x = np.zeros((n, k // 32, 32), np.float32)
+    for t in range(n):
+        q = r.integers(-127, 128, 32) if t else np.full(32, 127)
+        q[t % 32] = 127                     # so that the block's scale is a power of two
+        x[t, t * 7 % (k // 32)] = q * np.exp2(int(r.integers(-8, 9)))
+    x = x.reshape(n, k)
+    want = (x.astype(np.float64) @ util.dequant_np(dtype, w.reshape(-1), m, k).astype(np.float64).T).astype(np.float32)
+    for copies in (True, False):
+        hip.set_decode_copies(copies)
+        try:
+            got = hip.gemm_pair(dtype, w.reshape(-1), m, dtype, w.reshape(-1), m, x, n, k)
+        finally:
+            hip.set_decode_copies(True)
+        assert np.array_equal(got[0], want) and np.array_equal(got[1], want), copies
+    if n > 64:
+        assert np.array_equal(hip.gemm(dtype, w.reshape(-1), x, m, n, k).reshape(m, n).T, want)
+
+
 @pytest.mark.parametrize("dtype,n,m,k,limit", [(Q4_K, 48, 4096, 2048, 2 << 20), (Q6_K, 5, 4096, 2048, 1 << 18), (Q6_K, 128, 4096, 2048, 4 << 20)])
 def test_products_without_room_for_partial_sums(dtype, n, m, k, limit):
     """Sums over parts of K are a workspace that a product can do without: where it cannot be had (here by a limit that the
@@ -399,6 +436,68 @@ def test_prefill_where_the_norm_adds_split_k_partial_sums(hip, orc, rope_type, k
     lg2 = gm.forward(7, 130)
     lo2 = om.forward(7, 130)
     assert _cos(lg2, lo2) > 0.999
+    gm.close(); om.close()
+
+
+# a pass of a few tokens: (config, make_llama's arguments, biases, QK norm, f16 cache)
+FEW_MODELS = {
+    "q4_k_m": (dict(), dict(), False, False, False),                                        # Q | K and a Q6_K V in one launch
+    "q4_k_m_neox_f16": (dict(rope_type=0), dict(), False, False, True),
+    "q4_k": (dict(), dict(type_of=lambda name: Q4_K), False, False, False),                 # one joint Q | K | V
+    "q6_k_f16": (dict(), dict(type_of=lambda name: Q6_K), False, False, True),
+    "q4_k_m_bias": (dict(rope_type=0), dict(), True, False, False),                         # RoPE cannot add the sums up
+    "q4_k_qknorm": (dict(rope_type=0), dict(type_of=lambda name: Q4_K), False, True, False),
+    "granite_scalars": (dict(embed_scale=12.0, residual_scale=0.22, attn_scale=0.0078125, logit_scale=8.0), dict(), False, False, False),
+    "q5_k_m": (dict(), dict(type_of=lambda name: Q5_K if synth.q4_k_m_type(name) == Q4_K else synth.q4_k_m_type(name)), False, False, False),
+    "q8_0": (dict(), dict(type_of=lambda name: Q8_0), False, False, False),                 # only the norm of a few rows is another
+}
+
+
+@pytest.mark.parametrize("name", list(FEW_MODELS))
+def test_passes_of_a_few_tokens_vs_oracle(hip, orc, name):
+    """Portions of 2 to 49 tokens of a 2048-wide model, one behind the other, against the oracle fed the same portions:
+    joint Q | K (| V) outputs in their segments, sums over slices of K left to RoPE and to the row norm with the residual
+    and its scale, both caches, and the same behind biases and QK norms, which keep RoPE from adding up.  The first layer's
+    cache rows have only one product behind them.  Beyond it codes flip: a difference d in front of a rounding to steps of s
+    leaves sqrt(d s) behind it, so last bits grow to the rounding's own noise within a layer.  A step is 2.3 / 127 of a
+    block's rms, two routes' noise 2 / 12 of its square per rounded input, four of them lie in front of the second layer's
+    rows (1.5 % of the rms together), and the largest of their 1e5 differences is 4.6 times that: 7e-2."""
+    over, mk, bias, qk_norm, kv_f16 = FEW_MODELS[name]
+    cfg = dict(synth.TINY, hidden=2048, ffn=2304, n_heads=16, n_kv_heads=4, head_dim=128, max_seq_len=256, **over)
+    weights = synth.make_llama(cfg, seed=83, sigma=0.03, norm_jitter=0.1, **mk)
+    r = util.rng(8)
+    for i in range(cfg["n_layers"]):
+        for part, rows in (("q", 2048), ("k", 512), ("v", 512)):
+            if bias:
+                weights[f"blk.{i}.attn_{part}.bias"] = (r.standard_normal(rows) * 0.5).astype(np.float32)
+            if qk_norm and part != "v":
+                weights[f"blk.{i}.attn_{part}_norm.weight"] = (1.0 + 0.3 * r.standard_normal(128)).astype(np.float32)
+    gm, om = hip_api.Model(hip, cfg, weights), orc.Llama(cfg, weights)
+    if kv_f16:
+        gm.configure_kv(True); om.set_kv_f16(True)
+    at = 0
+    for n in (5, 17) if name == "q5_k_m" else (5, 48, 3, 33, 16, 17, 2, 32, 49):
+        toks = [int(t) for t in r.integers(0, cfg["vocab"], n)]
+        if n == 33:   # all positions' logits: the last row is the oracle's, the others what a shorter portion ends in
+            got = gm.forward_prefill_logits_all(toks, at)
+            gm.truncate_kv(at)
+            short = gm.forward_prefill(toks[:20], at)
+            gm.truncate_kv(at)
+            lg = gm.forward_prefill(toks, at)
+            assert _cos(got[19], short) > 0.999 and _cos(got[-1], lg) > 0.999
+        else:
+            lg = gm.forward_prefill(toks, at)
+        # (the oracle has no batched Q5_K)
+        lo = (om.forward_prefill_per_token if name == "q5_k_m" else om.forward_prefill_batched)(toks, at)
+        _say(f"{name}: {n} tokens behind {at}: cos {_cos(lg, lo):.8f} max|err| {np.abs(lg - lo).max():.3e} of rms {util.rms(lo):.3e}")
+        assert _cos(lg, lo) > 0.999, (n, at)
+        at += n
+    for layer in range(cfg["n_layers"]):
+        for got, want in zip(gm.read_kv(layer), om.kv(layer)):
+            err = np.abs(got - want).max() / util.rms(want)
+            _say(f"  layer {layer}: {err:.2e}")
+            # (an f16 cache: a value next to a rounding boundary is 2^-11 of itself off, of six times the rms at most)
+            assert err <= (7e-2 if layer else 3e-3 if kv_f16 else 2e-3), layer
     gm.close(); om.close()
 
 
