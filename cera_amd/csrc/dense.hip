@@ -13,6 +13,7 @@
 
 #include "bf16.hip.h"
 #include "dense.h"
+#include "lds_dma.hip.h"
 #include "partials.hip.h"
 
 namespace {
@@ -276,23 +277,6 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
     dense_epilogue<__bf16, EPI, SN, MI, NI>(a, tm * BM + wm * TM, tn * BN + wn * TN, lane, blockIdx.y, acc);
 }
 
-// 1 KB of global memory straight into LDS: lane i's 16 bytes at base + off_lane land at lds + 16 i.  Inline assembly: with
-// the compiler's form of this load every later wait on an LDS read is a wait for all loads in flight.  A vector instruction
-// may have written the scalar registers of base (readfirstlane, a reload of a spilled one): the five wait states that a load
-// needs behind such a write stand in the block, since the compiler does not look into it.
-__device__ __forceinline__ void dense_dma_1k(uint64_t base, uint32_t off_lane, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off_lane), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t dense_lds_addr(const void* p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(p)));
-}
-// an address that is the same in every lane, in scalar registers
-__device__ __forceinline__ uint64_t dense_uniform(uint64_t v) {
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32)));
-    return static_cast<uint64_t>(hi) << 32 | lo;
-}
-
 // 256 x 256 tile, eight wavefronts as 2 x 4, each 128 rows x 64 tokens: 24 KB of fragments per wavefront and K step of 64
 // against 32 KB of the same work on 128 x 128 tiles, whose four wavefronts read LDS for as long as they multiply.  One
 // barrier a K step, in its middle: behind it the step's second half is in registers, so its buffer takes the K step after
@@ -311,17 +295,17 @@ __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
     const bool toks = wave >= 4;
     const uint32_t first = toks ? tn * B : tm * B, last = (toks ? a.n : a.m) - 1 - first;
     const uint64_t ld = (toks ? a.ldx : a.kp) * 2;
-    const char* const base = toks ? static_cast<const char*>(a.x) + group * a.gx * 2 : reinterpret_cast<const char*>(a.w + group * a.gw);
-    uint64_t src = dense_uniform(reinterpret_cast<uint64_t>(base) + first * ld + k0 * 2);
+    const uint8_t* const base = toks ? static_cast<const uint8_t*>(a.x) + group * a.gx * 2 : reinterpret_cast<const uint8_t*>(a.w + group * a.gw);
+    const uint8_t* src = lds_dma_base(base + first * ld + k0 * 2);
     const uint32_t sub = lane >> 3, slot = lane & 7;
     uint32_t off[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) off[s] = min((wave & 3) * 64 + s * 8 + sub, last) * static_cast<uint32_t>(ld) + (slot ^ sub) * 16;
-    const uint32_t dst = dense_lds_addr(&lds[0][0]) + wave * 8192;
+    const uint32_t dst = lds_addr(&lds[0][0]) + wave * 8192;
     auto stage = [&](int buf) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) dense_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
-        src = dense_uniform(src + BK * 2);
+        for (int s = 0; s < 8; ++s) lds_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
+        src = lds_dma_base(src + BK * 2);
     };
     const uint32_t wm = wave >> 2, wn = wave & 3, fr = lane & 15, fg = lane >> 4;
     bf16x8 fa[2][MI], fb[2][NI];

@@ -2,8 +2,10 @@
 #pragma once
 #include <cstdint>
 
-// 64 lanes x 16 (4) bytes: base + off_lane of every lane to lds, lane after lane.  Behind m0's write, and for a base that a
-// vector instruction has put into scalar registers, wait states are needed that the compiler does not see into here.
+// 64 lanes x 16 (4) bytes: base + off_lane of every lane to lds, lane after lane.  Inline assembly: with the compiler's form of
+// these loads every later wait on an LDS read is a wait for all loads in flight.  Behind m0's write, and for a base that a
+// vector instruction has put into scalar registers (readfirstlane, a reload of a spilled one: five wait states), the waits
+// stand in the block, since the compiler does not look into it.
 __device__ __forceinline__ void lds_dma_1k(const void* base, uint32_t off_lane, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off_lane), "s"(base), "s"(lds) : "memory", "m0");
 }
