@@ -16,15 +16,13 @@
 // behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 289 us, 45 tokens 466 -> 322.
 #include <algorithm>
 
+#include "f16_codes.hip.h"
 #include "gemv.hip.h"
 #include "gemm_few.h"
 
 namespace {
 
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef __bf16 b8v __attribute__((ext_vector_type(8)));
-typedef float f4v __attribute__((ext_vector_type(4)));
 
 struct FewArgs {
     FewMat a, b;               // b: a second matrix of the same k, or m = 0
@@ -43,14 +41,6 @@ constexpr int FEW_WAVES = 8, FEW_ROWS = 16 * FEW_WAVES;
 // scales, the mins' operand
 constexpr uint32_t FEW_BLOCK = 1040, FEW_XS = 8 * FEW_BLOCK, FEW_MIN = FEW_XS + 512, FEW_TILE = FEW_MIN + 1024;
 
-__device__ __forceinline__ h2v as_h2(uint32_t v) { return __builtin_bit_cast(h2v, v); }
-__device__ __forceinline__ h2v fma2(h2v a, h2v b, h2v c) { return __builtin_elementwise_fma(a, b, c); }
-__device__ __forceinline__ h2v both(float v) { return h2v{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
-// bytes 0 and 2, or 1 and 3, of v as 1024 + byte
-__device__ __forceinline__ h2v bytes02(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)); }
-__device__ __forceinline__ h2v bytes13(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
-// byte j of v, twice, as 1024 + byte
-template <int J> __device__ __forceinline__ h2v byte_twice(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | J | J << 16)); }
 __device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {   // a's upper 32 lanes with b's lower 32
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     a = r[0]; b = r[1];

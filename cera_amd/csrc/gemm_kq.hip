@@ -15,23 +15,12 @@
 // 4096 x 14336 (with the tokens' operand and the sum of the slices): 512 tokens 172 -> 139 us, 2048 tokens 617 -> 440 us;
 // 4096 x 4096 with 512 tokens 66 -> 56 us, 128 tokens 33 -> 29 us.  Of the 440 us the matrix instructions alone take 222, the
 // folds 70, the unpacking 45 and the rows' loads, 210 bytes apart by super-block, 60.
+#include "f16_codes.hip.h"
 #include "gemm_kq.h"
 #include "gemv.hip.h"
 #include "lds_dma.hip.h"
 
 namespace {
-
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ h2v as_h2(uint32_t v) { return __builtin_bit_cast(h2v, v); }
-__device__ __forceinline__ h2v fma2(h2v a, h2v b, h2v c) { return __builtin_elementwise_fma(a, b, c); }
-__device__ __forceinline__ h2v both(float v) { return h2v{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
-// bytes 0 and 2, or 1 and 3, of v as 1024 + byte
-__device__ __forceinline__ h2v bytes02(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)); }
-__device__ __forceinline__ h2v bytes13(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
-template <int J> __device__ __forceinline__ h2v byte_twice(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | J | J << 16)); }
 
 __global__ __launch_bounds__(256) void kq_act_kernel(const int8_t* __restrict__ bq, uint8_t* __restrict__ act, uint32_t n, uint32_t k) {
     kq_act_record(blockIdx.x, bq, act, n, k);
@@ -39,7 +28,6 @@ __global__ __launch_bounds__(256) void kq_act_kernel(const int8_t* __restrict__ 
 
 // ---- Q6_K: half h of a super-block is two runs j of 16 codes of each of its four blocks --------------------------
 struct KqQ6 {
-    static constexpr int PARTS = 2;
     // a row's bytes of a stage in LDS: two 16-byte runs of ql, of ql + 32 and of qh; eight scales; d as f32
     static constexpr uint32_t A = 0, B = KQ_ROWS * 32, Q = 2 * KQ_ROWS * 32, SC = 3 * KQ_ROWS * 32, D = SC + KQ_ROWS * 8, BYTES = D + KQ_ROWS * 4;
     struct Stage { uint4 a, b, q; uint2 sc; uint32_t d; };   // what a thread brings in: run j of its row
