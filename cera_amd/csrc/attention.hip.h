@@ -787,11 +787,12 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_partial_kernel(
 // 32 dims, the high parts of each in 1 KB and the low ones behind it -- and the workgroups load records straight into LDS, the
 // next tile's while this one is multiplied: one barrier a tile, no vector instruction for staging, LDS read without conflicts.
 // What is multiplied and its order are the same.  Workgroups of a KV head lie on one XCD where there are eight of them (the
-// head is the grid's fastest index), whose L2 then holds that head's records only; the blocks with the most keys start first.
-// What bounds it is the order of a wavefront's own instructions: LDS reads run three steps ahead of the products, and the first
-// values' reads go out before the scores become weights.  2048 queries behind 4096 keys, 32 / 8 heads of 128, f32 cache: 615 ->
-// 464 us with the pass over the cache (18); the products alone take 205.  Reads at their use: 520.  Two accumulators
-// for the cross terms and two output tiles in turn, against waits between dependent products: no gain.
+// head is the grid's fastest index), whose L2 then holds that head's records only (445 us in place of 486 with the query blocks
+// fastest); the blocks with the most keys start first.  What bounds it is the order of a wavefront's own instructions: matrix
+// cores busy for 55 % of the time and the vector ALU for 39 %, in turns.  LDS reads run three steps ahead of the products, and
+// the first values' reads go out before the scores become weights.  2048 queries behind 4096 keys, 32 / 8 heads of 128, f32
+// cache: 615 -> 464 us with the pass over the cache (18); reads at their use: 520.  Two accumulators for the cross terms and two
+// output tiles in turn, against waits between dependent products: no gain.
 template <typename KV, int HD> constexpr uint32_t attn_record_bytes() { return 32 * HD * 2 * 2 * (sizeof(KV) == 4 ? 2 : 1); }
 // grid = (tiles, KV heads); keys from n_keys on are zeros
 template <typename KV, int HD>

@@ -280,9 +280,10 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
 // 256 x 256 tile, eight wavefronts as 2 x 4, each 128 rows x 64 tokens: 24 KB of fragments per wavefront and K step of 64
 // against 32 KB of the same work on 128 x 128 tiles, whose four wavefronts read LDS for as long as they multiply.  One
 // barrier a K step, in its middle: behind it the step's second half is in registers, so its buffer takes the K step after
-// next while that half is multiplied.  What bounds it: LDS (2048 of the 2660 clocks that a K step of a workgroup takes alone)
-// beside the matrix cores (2048), and the clock, which a full chip lowers to 2.2 GHz.  28672 x 4096 times 2048 / 512 tokens:
-// 1100 / 1040 TFLOP/s, 128 x 128 tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
+// next while that half is multiplied.  What bounds it: a K step is 2048 clocks of the matrix cores and 2048 of LDS (192 KB
+// read, 64 KB written at 128 bytes a clock); one workgroup alone takes 2660 for it, a full chip 3440, with the matrix cores busy
+// for 52 % of 28672 x 4096 times 1900 tokens (3.5 rounds).  28672 x 4096 times 2048 / 512 tokens: 1100 / 1040 TFLOP/s, 128 x 128
+// tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
 template <int EPI, int SN>
 __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
     constexpr int B = 256, BK = 64, MI = 8, NI = 4, HALF = B * BK, BUF = 2 * HALF;

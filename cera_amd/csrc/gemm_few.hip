@@ -4,14 +4,15 @@
 // A wavefront owns 16 weight rows and streams their super-blocks straight into registers, two to four of them ahead; the tokens, in
 // tiles of 16, come from LDS, where the workgroup's eight wavefronts put them as f16 (the Q8_0 codes are whole numbers, exact
 // in f16), a chunk of super-blocks ahead.  One v_mfma_f32_16x16x32_f16 is one 32-weight block: Q4_K weights enter as
-// scale * code, at most 945 and exact in f16; Q6_K weights, at most 4064, as two f16 parts whose sum they are.  So a block's
-// result is the exact whole number sum(scale * code * quant), below 2^24, and what the vector ALU adds is one FMA with the
-// token's block scale per output and block, one with the row's d per super-block, and for Q4_K one with dmin on the mins'
-// own product (mins times the tokens' block sums in three bf16 parts).  Sums over K go in order within a slice.
+// scale * code, at most 945 and exact in f16; Q6_K weights, up to 4096 (-128 times -32), as two f16 parts whose sum they are.
+// So a block's result is the exact whole number sum(scale * code * quant): quants are at most 127 (the quantizer's scale is the
+// largest magnitude over 127), and 32 * 4096 * 127 is 1 % below 2^24.  What the vector ALU adds is one FMA with the token's
+// block scale per output and block, one with the row's d per super-block, and for Q4_K one with dmin on the mins' own product
+// (mins times the tokens' block sums in three bf16 parts).  Sums over K go in order within a slice.
 //
-// What bounds it: up to 16 tokens the weights' way from HBM, above that the vector ALU, about 130 (Q4_K) and 225 (Q6_K)
-// instructions per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens (45 tokens: vector ALU 56 % busy, matrix cores
-// 15 %).  Gate | up, 14336 x 4096 Q4_K as a pair: 22 us at 5 tokens, 37 at 45; down, 4096 x 14336 Q6_K: 20 and 25.  The 64-token
+// What bounds it: up to 16 tokens the weights' way from HBM (gate | up at 3.0 TB/s), above that the vector instructions, about
+// 130 (Q4_K) and 225 (Q6_K) per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens (gate | up with 45 tokens: vector
+// ALU busy for half of the time, matrix cores for 15 %).  Gate | up, 14336 x 4096 Q4_K as a pair: 22 us at 5 tokens, 37 at 45; down, 4096 x 14336 Q6_K: 20 and 25.  The 64-token
 // tiles before it took 36 us for a down product and 50 for a pair, with a launch for the tokens' copy before and one for the sums
 // behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 289 us, 45 tokens 466 -> 322.
 #include <algorithm>
@@ -399,8 +400,8 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k);
     auto tiles = [](const cera_hip_dtensor* t) { return static_cast<uint32_t>((t->m + FEW_ROWS - 1) / FEW_ROWS); };
     a.tiles_a = tiles(w);
-    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = 8 / FEW_WAVES * ctx->n_cu;
-    // K is split where the rows leave more than a quarter of two workgroups per CU idle, down to two super-blocks a slice
+    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = ctx->n_cu;
+    // K is split where the rows leave more than a quarter of one workgroup per CU idle, down to two super-blocks a slice
     uint32_t split = wgs * 4 >= want * 3 ? 1 : std::min({(want + wgs - 1) / wgs, std::max(nsb / 2, 1u), 8u});
     a.sb_per = (nsb + split - 1) / split;
     split = (nsb + a.sb_per - 1) / a.sb_per;

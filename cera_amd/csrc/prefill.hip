@@ -289,7 +289,7 @@ extern "C" cera_hip_status cera_hip_gemm(cera_hip_ctx* ctx, const cera_hip_tenso
 }
 
 // The GEMM's integer block dots as the matrix cores deliver them (debug instances of the same
-// kernels): dots [m][n][k/32] int32 -- Q4_0 sum (q-8)a, Q8_0 sum w a, Q4_1 / Q4_K sum q a -- and
+// kernels, for Q6_K of the one for up to 64 tokens): dots [m][n][k/32] int32 -- Q4_0 sum (q-8)a, Q8_0 sum w a, Q4_1 / Q4_K sum q a -- and
 // for Q6_K [m][n][k/16], each the f32 result of the f16 MFMA for one 16-element scale group,
 // sum (q-32)a, returned as f32 so that a test can see it is an exact integer.  out (nullable)
 // receives the float result of the same launch.
@@ -475,7 +475,8 @@ extern "C" cera_hip_status cera_hip_gemm_swiglu_f16(cera_hip_ctx* ctx, const cer
 static constexpr uint32_t PREFILL_CHUNK = CERA_PREFILL_CHUNK;
 // batches up to this many tokens run their projections on the multi-token GEMV instead of the GEMM
 // (measured on the 8B shapes: 2 tokens 2.8 ms against 7.7 ms, 8 tokens 5.4 against 7.9, 16 tokens
-// 10.7 against 9.4 -- the per-token dots grow with the batch while the GEMM's tile fills up)
+// 10.7 against 9.4 -- the per-token dots grow with the batch while the GEMM's tile fills up); Q4_K and Q6_K
+// rows of FEW_MIN_K and more have a kernel of their own from three tokens on (gemm_few.hip)
 static constexpr uint32_t PREFILL_SMALL_BATCH = 8;
 
 cera_hip_status cera_model_ensure_prefill_buffers(cera_hip_model* m, uint32_t n) {
@@ -559,8 +560,8 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     // the f32 activations whose hi / lo split (Q5_K GEMMs) the context's workspace holds now
     const float* split_of = nullptr;
     // split-K partial sums of pf_hidden that the next row norm adds up (n_split = 0: none).  From 128 rows on:
-    // the norm runs one workgroup per row, and a few dozen workgroups adding up partial sums take longer than
-    // the reduction launch they save (12.8 against 4.8 + 5.7 us at 16 rows, 11.3 against 6.3 + 7.4 at 512).
+    // rmsnorm_pending_kernel runs a workgroup of 256 threads per row, and a few dozen of them adding up partial sums take
+    // longer than the reduction launch they save (12.8 against 4.8 + 5.7 us at 16 rows, 11.3 against 6.3 + 7.4 at 512).
     RowsPending pend{};
     // A few rows take a workgroup of 1024 threads each that keeps its row in registers and has all slices on their way at once.
     const bool norm_row = few_tokens && hs <= 16384, norm_adds = n >= 128 || norm_row;

@@ -213,7 +213,7 @@ CERA_HIP_API cera_hip_status cera_hip_gemm(cera_hip_ctx*, const cera_hip_tensor*
                                            float* out);
 
 /* cera_hip_gemm with the integer block dots its matrix-core instructions produced, from debug
- * instances of the same kernels (the integer quantities cera's own test reference defines,
+ * instances of the same kernels -- for Q6_K of the one for up to 64 tokens (the integer quantities cera's own test reference defines,
  * cera/src/backend/simd.rs:6609-6629): dots [m][n][k/32] int32 -- Q4_0 sum (q-8)a, Q8_0 sum w a,
  * Q4_1 / Q4_K sum q a, q in 0..15.  Q6_K forms its dots per 16-element scale group on the f16
  * matrix cores: dots [m][n][k/16], each the f32 bit pattern of that instruction's result,
