@@ -111,7 +111,8 @@ CERA_HIP_API cera_hip_status cera_hip_sync(cera_hip_ctx*);
  * for one kernel, as the reference's x86 path does with repack_q4_k_8x8
  * (cera/src/backend/cpu.rs:1282-1358); it has no switch there. */
 CERA_HIP_API cera_hip_status cera_hip_ctx_set_decode_copies(cera_hip_ctx* ctx, int enabled);
-/* The most bytes one of the context's workspaces may grow to (0, the default: no limit).  A call that
+/* The most bytes one of the context's workspaces may grow to (0, the default: no limit; attention's partial
+ * results, which a context holds apart, are not counted).  A call that
  * cannot do without more fails with CERA_HIP_ERR_OOM, as it does where the device has no more memory; one
  * that is only faster with it (key and value tiles of a large attention batch laid out once, sums over
  * parts of K) runs without it.  Workspaces that are already larger stay. */
