@@ -9,6 +9,7 @@
 #include "gemm_q5k_f16.hip.h"
 #include "gemm_q6k_f16.hip.h"
 #include "gemm_fp8.hip.h"
+#include "gemm_i8.h"
 #include "gemm_kq.h"
 #include "gemm_few.h"
 #include "glue.hip.h"
@@ -72,6 +73,8 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     const bool dense = ((ld_m == 1 && ld_n == a.m) || (ld_n == 1 && ld_m == n)) && (static_cast<uint64_t>(a.m) * n) % 4 == 0;
     // Q6_K with many tokens: gemm_kq.hip, in this many slices of K (0: not there)
     const uint32_t kq = dbg_dots || !dense ? 0 : kq_slices(w->dtype, a.m, pair ? w2->m : 0, n, a.k, ctx->n_cu);
+    // Q8_0 and Q4_0: gemm_i8.hip
+    const bool i8 = !dbg_dots && i8_takes(w, bq) && (!pair || i8_takes(w2, bq));
     // Q6_K runs its block dots on the f16 matrix cores and reads the quants as f16: converted here
     // unless the caller says its workspace (bh_ws) still holds these activations in that form (*staged)
     a.bh = nullptr;
@@ -108,7 +111,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         }
         a.bf8 = static_cast<const uint8_t*>(b8_ws);
     }
-    const uint32_t BM = kq ? KQ_ROWS : fp8 ? G8_BM : GEMM_BM, BN = kq ? KQ_TOKENS : fp8 ? G8_BN : GEMM_BN;
+    const uint32_t BM = kq ? KQ_ROWS : fp8 ? G8_BM : i8 ? I8_ROWS : GEMM_BM, BN = kq ? KQ_TOKENS : fp8 ? G8_BN : i8 ? i8_tokens(n) : GEMM_BN;
     if (q5) {
         // hi | lo f16 halves of x and its f32 block sums, in one scratch allocation
         const uint64_t nk = static_cast<uint64_t>(n) * a.k;
@@ -137,9 +140,9 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     }
     // Few output tiles and a long K (the down projection at a few hundred tokens): split K over
     // grid.z so the chip is filled, partial sums to scratch, then one fixed-order reduction.
-    uint32_t split = kq ? kq : 1;
+    uint32_t split = kq ? kq : i8 && dense ? i8_slices(a.m, pair ? w2->m : 0, n, a.k, ctx->n_cu) : 1;
     const uint32_t wgs = grid.x * grid.y, nsb = a.k / GEMM_KSUPER;
-    if (!kq && !dbg_dots && wgs < 2 * ctx->n_cu && nsb >= 8 && dense) {   // (a CU holds two workgroups)
+    if (!kq && !i8 && !dbg_dots && wgs < 2 * ctx->n_cu && nsb >= 8 && dense) {   // (a CU holds two workgroups)
         // smallest divisor of the super-block count that fills every CU
         const uint32_t want = std::min<uint32_t>(8, (2 * ctx->n_cu + wgs - 1) / wgs);
         // (a slice keeps at least two super-blocks: below that the tile's prologue outweighs its K loop)
@@ -172,7 +175,11 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         HIP_TRY(ctx, hipGetLastError());
         return CERA_HIP_OK;
     }
-    switch (w->dtype) {
+    if (i8) {
+        I8Args b{a.w, a.w2, bq, bs, a.out, a.out2, a.m, a.m2, n, a.k, a.row_bytes, a.tiles1, a.k_chunk, ld_m, ld_n, ld_n2, a.part_stride, a.resid, resid_scale,
+                 nullptr, nullptr, nullptr};
+        CERA_TRY(cera_launch_i8(ctx, w->dtype, b, split));
+    } else switch (w->dtype) {
         case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false>), grid, dim3(256), 0, ctx->stream, a); break;
         case CERA_HIP_Q6_K:
             if (kq)
@@ -230,7 +237,10 @@ cera_hip_status cera_launch_gemm_swiglu(cera_hip_ctx* ctx, const cera_hip_dtenso
         }
         a.bf8 = static_cast<const uint8_t*>(b8_ws);
     }
-    switch (gate->dtype) {
+    if (i8_takes(gate, bq) && i8_takes(up, bq)) {
+        I8Args b{a.w, a.w2, bq, bs, nullptr, nullptr, a.m, a.m, n, a.k, a.row_bytes, 0, a.k, 0, 0, 0, 0, nullptr, 1.0f, hq, hs, hbsum};
+        CERA_TRY(cera_launch_i8_swiglu(ctx, gate->dtype, b));
+    } else switch (gate->dtype) {
         case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false>), grid, dim3(256), 0, ctx->stream, a); break;
         case CERA_HIP_Q4_0: hipLaunchKernelGGL((gemm_kernel<GemmQ4_0, true>), grid, dim3(256), 0, ctx->stream, a); break;
         case CERA_HIP_Q4_1: hipLaunchKernelGGL((gemm_kernel<GemmQ4_1, true>), grid, dim3(256), 0, ctx->stream, a); break;

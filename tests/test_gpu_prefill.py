@@ -158,6 +158,33 @@ def test_gemm_q6k_of_many_tokens(hip, orc, ma, mb, n, k):
         assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
 
 
+@pytest.mark.parametrize("dtype,bytes_", [(Q8_0, 34), (Q4_0, 18)])
+@pytest.mark.parametrize("ma,mb,n,k", [(1, 4, 65, 256), (127, 129, 68, 512), (128, 36, 128, 8192), (260, 17, 132, 2304),
+                                       (1028, 300, 257, 4096), (132, 2052, 1001, 1024), (5, 64, 4, 256), (130, 62, 64, 2304), (36, 4, 33, 8192)])
+def test_gemm_of_32_weight_blocks(hip, orc, dtype, bytes_, ma, mb, n, k):
+    """Q8_0 and Q4_0 against the exact product of the dequantized weights and quantized tokens, alone and as a pair: tiles of
+    64 and of 128 tokens, last tiles of rows and tokens, one row, one to eight slices of K.  Codes are random bytes, -128 and -8
+    among them, scales have both signs; the bound is that of the products of a few tokens above, of an output's rms over
+    random signs."""
+    _say(f"many tokens {util.NAMES[dtype]} ma={ma} mb={mb} n={n} k={k}")
+    r = util.rng(ma + n + k)
+    def weights(m):
+        w = r.integers(0, 256, (m, k // 32, bytes_), dtype=np.uint8)
+        d = r.uniform(0.5, 2.0, (m, k // 32, 1)) * 1e-3 * r.choice([-1.0, 1.0], (m, k // 32, 1))
+        w[:, :, :2] = d.astype(np.float16).view(np.uint8)
+        return w.reshape(-1)
+    wa, wb = weights(ma), weights(mb)
+    x = r.standard_normal((n, k)).astype(np.float32) * np.exp2(r.integers(-6, 7, (n, 1))).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    alone = hip.gemm(dtype, wa, x, ma, n, k)
+    oa, ob = hip.gemm_pair(dtype, wa, ma, dtype, wb, mb, x, n, k)
+    for got, w, m in ((alone.reshape(ma, n).T, wa, ma), (oa, wa, ma), (ob, wb, mb)):
+        wd = util.dequant_np(dtype, w, m, k).astype(np.float64)
+        rms = np.sqrt((xd * xd).sum(1, keepdims=True) * (wd * wd).sum(1) / k)
+        assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
+
+
 @pytest.mark.parametrize("dtype,m,k,n", [(Q4_K, 132, 2304, 5), (Q4_K, 300, 4096, 48), (Q6_K, 132, 2304, 3), (Q6_K, 300, 4096, 33),
                                          (Q6_K, 300, 4096, 160), (Q6_K, 516, 2304, 384)])
 def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
@@ -214,7 +241,7 @@ def test_products_without_room_for_partial_sums(dtype, n, m, k, limit):
 
 
 @pytest.mark.parametrize("dtype", [Q4_K, Q4_0, Q4_1, Q8_0])
-@pytest.mark.parametrize("m,k,n,want_fused", [(2048, 512, 1040, True), (1056, 256, 2000, True), (512, 256, 70, False)])
+@pytest.mark.parametrize("m,k,n,want_fused", [(2048, 512, 1040, True), (1056, 256, 2000, True), (512, 256, 70, False), (32800, 256, 33, True)])
 def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n, want_fused):
     """gate | up | SwiGLU | Q8_0 in one launch: the quants and scales must be, byte for byte, the
     oracle's quantization of the oracle's SwiGLU of the two GEMM outputs the pair launch gives
