@@ -9,7 +9,7 @@
 // Cache of one layer, element type T (bf16 or f32): K [kv_heads][cap][dim_p], V transposed
 // [kv_heads][vdim_p][cap].  dim_p and vdim_p are the head sizes rounded up to 32 (pad columns zero),
 // cap the positions rounded up to 64; every entry is finite from the start.  With V transposed, both
-// matrix products read their cache operand in 16-byte runs and no operand passes through LDS.
+// matrix products read their cache operand in 16-byte runs: from the cache itself, or, with many queries, from blocks in LDS.
 #pragma once
 #include "host_common.h"
 

@@ -13,6 +13,7 @@
 #include <algorithm>
 
 #include "bf16.hip.h"
+#include "lds_dma.hip.h"
 #include "sigmoid_attn.h"
 
 namespace {
@@ -32,6 +33,7 @@ struct AArgs {
     uint64_t out_ld;
     float* part;            // [split][n][heads][vdim_p], splits > 1
     uint32_t splits;
+    uint32_t tiles, round;  // shared rows: column tiles of a kv head, workgroups of a kv head in one round of the chip
     uint32_t attn_blocks;   // fused step: workgroups past these add up the convolution history
     ConvRing ring;
     ConvHist hist;
@@ -252,6 +254,130 @@ __global__ __launch_bounds__(256) void sattn_rows_kernel(AArgs a) {
             for (int vt = 0; vt < t.MV; ++vt)
                 if (VT || vt < static_cast<int>(nv)) finish4<T>(a, col.query[ct], col.head[ct], vt * 16 + (lane >> 4) * 4, t.o[ct][vt]);
         }
+}
+
+// ---- many queries, heads of 64 or 128 in bf16: four wavefronts' columns share the keys and values in LDS -------------
+// A workgroup walks its columns' keys in blocks of 64 that direct loads bring into LDS one block ahead, K rows and V's
+// transposed rows alike in 16-byte chunks: chunk c of key k in a slot of its group of eight that depends on k (key_slot), chunk c
+// of value column v in slot c ^ (v % 8), so that eight lanes always read eight different bank groups.  The products are
+// sattn_rows_kernel's, in its order.  1900 queries, 32 heads of 128 on 8: 185 us with every wavefront reading its own keys and
+// values, V in pieces of half a cache line; 87 with blocks of 32 in LDS, 70 with blocks of 64, which leave a wavefront fewer
+// waits in a row (630 TFLOP/s of matrix instructions).  What bounds it: those waits, and the sigmoids between the products.
+template <int DK> __device__ __forceinline__ uint32_t key_slot(uint32_t key, uint32_t chunk) {
+    return (chunk & ~7u) | ((chunk ^ ((key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2))) & 7);
+}
+template <int DK, int VT, int CT>
+__global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a) {
+    constexpr uint32_t ROW = DK * 64, KB = 64 * ROW, VB = VT * 2048, SEGS = (KB + VB) / 4096;   // 1 KB pieces of a wavefront
+    static_assert(KB % 4096 == 0 && VB % 4096 == 0, "a wavefront's pieces are whole");
+    __shared__ __align__(1024) uint8_t lds[2][KB + VB];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+    // launch index: kv heads (consecutive ones on different XCDs), then tiles: the longest key ranges first, and every second
+    // round of the chip the other way, so that a CU's tiles add up to about the same
+    const uint32_t kvh = blockIdx.x % a.kv_heads, t = blockIdx.x / a.kv_heads, round = t / a.round, at = t - round * a.round;
+    const uint32_t tile = a.tiles - 1 - (round & 1 ? round * a.round + min(a.round, a.tiles - round * a.round) - 1 - at : t);
+    const uint32_t cols = a.n * a.per, wg_c0 = tile * 64 * CT, c0 = wg_c0 + wave * 16 * CT;
+    const bool wave_live = c0 < cols;
+    Columns<__bf16, DK, VT, CT> col;
+    col.set(a, min(c0, cols - 1), kvh, lane);
+    const uint32_t first = first_visible(a.start + wg_c0 / a.per, a.chunk) / 64, last = (a.start + min(wg_c0 + 64 * CT - 1, cols - 1) / a.per) / 64;
+    // this lane's source of each of the wavefront's pieces, from the kv head's K or V
+    const uint8_t* const kbase = lds_dma_base(static_cast<const uint8_t*>(a.kc) + static_cast<uint64_t>(kvh) * a.cap * ROW);
+    const uint8_t* const vbase = lds_dma_base(static_cast<const uint8_t*>(a.vc) + static_cast<uint64_t>(kvh) * (VT * 16) * a.cap * 2);
+    uint32_t off[SEGS];
+#pragma unroll
+    for (uint32_t s = 0; s < SEGS; ++s) {
+        if (s < KB / 4096) {
+            const uint32_t i = (wave * (KB / 4096) + s) * 64 + lane, key = i / (DK * 4);
+            off[s] = key * ROW + key_slot<DK>(key, i % (DK * 4)) * 16;
+        } else {
+            const uint32_t i = (wave * (VB / 4096) + s - KB / 4096) * 64 + lane, v = i >> 3;
+            off[s] = v * a.cap * 2 + ((i ^ v) & 7) * 16;
+        }
+    }
+    const uint32_t dst = lds_addr(&lds[0][0]);
+    auto stage = [&](uint32_t b, uint32_t buf) {
+#pragma unroll
+        for (uint32_t s = 0; s < SEGS; ++s) {
+            if (s < KB / 4096) lds_dma_1k(kbase + static_cast<uint64_t>(b) * KB, off[s], dst + buf * (KB + VB) + (wave * (KB / 4096) + s) * 1024);
+            else lds_dma_1k(vbase + static_cast<uint64_t>(b) * 128, off[s], dst + buf * (KB + VB) + KB + (wave * (VB / 4096) + s - KB / 4096) * 1024);
+        }
+    };
+    stage(first, 0);
+    bf16x8 q[CT][DK];
+    f32x4 o[CT][VT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const __bf16* const row = static_cast<const __bf16*>(a.q) + (static_cast<uint64_t>(col.query[ct]) * a.heads + col.head[ct]) * (DK * 32) + g * 8;
+#pragma unroll
+        for (int kd = 0; kd < DK; ++kd) q[ct][kd] = *reinterpret_cast<const bf16x8*>(row + kd * 32);
+#pragma unroll
+        for (int vt = 0; vt < VT; ++vt) o[ct][vt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // keys 8 (r / 4) + r % 4 and that plus 4 of each half; value columns r of sixteen
+    const uint32_t key = (r >> 2) * 8 + (r & 3), k0 = key * ROW, v0 = KB + r * 128;
+    auto block = [&](const uint8_t* base, uint32_t kb) {
+        f32x4 sc[CT][4];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sc[ct][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kd = 0; kd < DK; ++kd)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {   // half j / 2, keys 4 (j % 2) on
+                const bf16x8 f = *reinterpret_cast<const bf16x8*>(base + k0 + (j >> 1) * (32 * ROW) + (j & 1) * (4 * ROW) + key_slot<DK>(key + 4 * (j & 1), kd * 4 + g) * 16);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) sc[ct][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, q[ct][kd], sc[ct][j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[ct][i >> 2][i & 3] = fmaf(sc[ct][i >> 2][i & 3], a.scale, col.bias[ct]);
+        if (kb < col.lo_max || kb + 63 > col.hi_min)   // a key that some column does not see: a weight of 0
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const uint32_t k = kb + (i >> 3) * 32 + g * 8 + (i & 7);
+                    sc[ct][i >> 2][i & 3] = k >= col.lo[ct] && k <= col.hi[ct] ? sc[ct][i >> 2][i & 3] : -__builtin_inff();
+                }
+        bf16x8 ph[CT][2], pl[CT][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float p = sigmoid_fast(sc[ct][2 * h + (i >> 2)][i & 3]);
+                    const __bf16 w = static_cast<__bf16>(p);
+                    ph[ct][h][i] = w;
+                    pl[ct][h][i] = static_cast<__bf16>(p - static_cast<float>(w));
+                }
+#pragma unroll
+            for (int vt = 0; vt < VT; ++vt) {
+                const bf16x8 v = *reinterpret_cast<const bf16x8*>(base + v0 + vt * 2048 + ((4 * h + g) ^ (r & 7)) * 16);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    o[ct][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, ph[ct][h], o[ct][vt], 0, 0, 0);
+                    o[ct][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pl[ct][h], o[ct][vt], 0, 0, 0);
+                }
+            }
+        }
+    };
+    for (uint32_t b = first; b <= last; ++b) {
+        const uint32_t buf = (b - first) & 1, kb = b * 64;
+        // this block is in, and every wavefront is past its reads of the other buffer
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (b < last) stage(b + 1, buf ^ 1);
+        if (!wave_live || kb > col.hi_max || kb + 63 < col.lo_min) continue;
+        block(lds[buf], kb);
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+        if (wave_live && col.live[ct])
+#pragma unroll
+            for (int vt = 0; vt < VT; ++vt) finish4<__bf16>(a, col.query[ct], col.head[ct], vt * 16 + g * 4, o[ct][vt]);
 }
 
 // ---- few queries: the wavefronts of a workgroup (and `splits` workgroups) share the keys ---------
@@ -559,11 +685,20 @@ cera_hip_status cera_launch_sattn(cera_hip_ctx* ctx, const SAttnShape& s, const 
     const bool wide = static_cast<uint64_t>(cols) / 32 * s.kv_heads >= 4 * ctx->n_cu;
     by_size(a, f32, [&](auto dk, auto vt) {
         constexpr int DK = decltype(dk)::value, VT = decltype(vt)::value;
-        const uint32_t per_wg = 64 * (wide && VT ? 2 : 1);
-        const dim3 grid((cols + per_wg - 1) / per_wg, s.kv_heads);
-        if (f32) hipLaunchKernelGGL((sattn_rows_kernel<float, 0, 0, 1>), grid, dim3(256), 0, ctx->stream, a);
-        else if (VT && wide) hipLaunchKernelGGL((sattn_rows_kernel<__bf16, DK, VT, VT ? 2 : 1>), grid, dim3(256), 0, ctx->stream, a);
-        else hipLaunchKernelGGL((sattn_rows_kernel<__bf16, DK, VT, 1>), grid, dim3(256), 0, ctx->stream, a);
+        if constexpr (DK == 2 || DK == 4) {
+            const uint32_t per_wg = 64 * (wide ? 2 : 1);
+            a.tiles = (cols + per_wg - 1) / per_wg;
+            a.round = std::max(1u, ctx->n_cu / s.kv_heads);
+            const dim3 grid(a.tiles * s.kv_heads);
+            if (wide) hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 2>), grid, dim3(256), 0, ctx->stream, a);
+            else hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 1>), grid, dim3(256), 0, ctx->stream, a);
+        } else {
+            const uint32_t per_wg = 64 * (wide && VT ? 2 : 1);
+            const dim3 grid((cols + per_wg - 1) / per_wg, s.kv_heads);
+            if (f32) hipLaunchKernelGGL((sattn_rows_kernel<float, 0, 0, 1>), grid, dim3(256), 0, ctx->stream, a);
+            else if (VT && wide) hipLaunchKernelGGL((sattn_rows_kernel<__bf16, DK, VT, VT ? 2 : 1>), grid, dim3(256), 0, ctx->stream, a);
+            else hipLaunchKernelGGL((sattn_rows_kernel<__bf16, DK, VT, 1>), grid, dim3(256), 0, ctx->stream, a);
+        }
     });
     HIP_TRY(ctx, hipGetLastError());
     return CERA_HIP_OK;

@@ -289,6 +289,22 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, size, n, cuts", [(6, 2, 64, 33, 1400, [1400]), (5, 1, 128, None, 1650, [1650]), (7, 7, 64, 300, 1180, [1175, 5]),
+                                                                (14, 2, 128, 1000, 2401, [2401]), (16, 8, 64, 31, 2060, [11, 2049])])
+def test_attention_with_keys_and_values_shared_in_lds(tmp_path, heads, kv_heads, dim, size, n, cuts):
+    """One and two tiles of columns a wavefront: ragged last tiles, wavefronts without columns, chunks that are no blocks of 32, groups of
+    one to seven heads, a round of the chip that is not whole, a start inside a chunk.  Tolerance: the operands', as everywhere here."""
+    assert max(cuts) * heads >= 16 * 512   # below, the keys are split over workgroups instead
+    cfg = U.config([U.attention(heads, kv_heads, dim, dim, size, dim, 10000.0)], width=64, vocab=40, taps=2, positions=n)
+    w = R.random_model(cfg, 53)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 7)
+    err = U.rel(_feed(m, toks, cuts), U.reference(cfg, w, toks))
+    print(f"heads={heads}/{kv_heads} dim={dim} chunk={size} n={n}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 @pytest.mark.parametrize("width, ff, n, vocab", [(60, 16384, 300, 64), (130, 2600, 1800, 64), (200, 16300, 290, 64), (260, 2700, 1777, 64),
                                                  (330, 64, 1800, 5203), (5200, 64, 1800, 64), (5201, 200, 1799, 64)])
 def test_products_on_the_widest_tiles(tmp_path, width, ff, n, vocab):
