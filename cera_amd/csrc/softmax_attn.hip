@@ -1,6 +1,8 @@
 // Kernels of softmax_attn.h.
 //
-// A workgroup of four wavefronts walks the keys in blocks of 32 rows that it stages in LDS by direct
+// A workgroup of four wavefronts walks the keys in blocks of 32 rows (64 where a wavefront has two tiles of columns: a wavefront
+// alone on its SIMD waits for each part of a block in turn, and twice the keys a turn take 110 us in place of 139 for 24 heads
+// of 128 with 2048 queries behind 777 keys, 120 in place of 134 with latent keys of 192) that it stages in LDS by direct
 // global-to-LDS loads (16-byte chunk c of row k sits in slot c ^ swz(k) of its group of eight).  Wavefronts are
 // `cg` column groups times `kg` key groups times VG value groups: a column is one (query, query head of the kv head)
 // pair, 16 * CT of them per wavefront; key groups take blocks in turn and add up through LDS at the end; value groups
@@ -37,7 +39,7 @@ struct FArgs {
     uint64_t out_ld;
     uint32_t out_head;
     float *part, *ml;                // [split][n][heads][vp], [split][n][heads][2]; splits > 1 or merged by the consumer
-    uint32_t splits, tiles, cg, kg, stages;
+    uint32_t splits, tiles, round, cg, kg, stages;   // round: workgroups of a kv head in one round of the chip
 };
 
 __device__ __forceinline__ uint32_t swz(uint32_t key) { return (key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2); }
@@ -84,9 +86,10 @@ template <int MV> struct Column {    // one lane's column: running maximum, its 
     }
 };
 
-template <typename T, int MK, int MV, int CT, bool EXACT> struct Block;
+// H: halves of 32 keys that go through the softmax together
+template <typename T, int MK, int MV, int CT, int H, bool EXACT> struct Block;
 
-template <int MK, int MV, int CT, bool EXACT> struct Block<__bf16, MK, MV, CT, EXACT> {
+template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV, CT, H, EXACT> {
     bf16x8 q[CT][MK];
     __device__ __forceinline__ void load_q(int ct, const __bf16* row, bool live, int nk, uint32_t lane) {
         const uint32_t g = lane >> 4;
@@ -104,35 +107,40 @@ template <int MK, int MV, int CT, bool EXACT> struct Block<__bf16, MK, MV, CT, E
         const uint32_t ka = (r >> 2) * 8 + (r & 3), e = (g ^ swz(ka)) * 16;
         const char* const k0 = base + ka * row * 2;
         const char* const k1 = k0 + 8 * row;
-        f32x4 s0[CT], s1[CT];
+        f32x4 sc[CT][2 * H];
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) s0[ct] = s1[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int j = 0; j < 2 * H; ++j) sc[ct][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kd = 0; kd < MK; ++kd)
             if (EXACT || kd < nk) {
                 const uint32_t off = (kd >> 1) * 128, el = kd & 1 ? e ^ 64 : e;
-                const bf16x8 fa = *reinterpret_cast<const bf16x8*>(k0 + off + el), fb = *reinterpret_cast<const bf16x8*>(k1 + off + (el ^ 64));
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    s0[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, q[ct][kd], s0[ct], 0, 0, 0);
-                    s1[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb, q[ct][kd], s1[ct], 0, 0, 0);
+                for (int h = 0; h < H; ++h) {
+                    const bf16x8 fa = *reinterpret_cast<const bf16x8*>(k0 + h * 64 * row + off + el), fb = *reinterpret_cast<const bf16x8*>(k1 + h * 64 * row + off + (el ^ 64));
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        sc[ct][2 * h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, q[ct][kd], sc[ct][2 * h], 0, 0, 0);
+                        sc[ct][2 * h + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb, q[ct][kd], sc[ct][2 * h + 1], 0, 0, 0);
+                    }
                 }
             }
-        bf16x8 ph[CT], pl[CT];
+        bf16x8 ph[CT][H], pl[CT][H];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            float s[8];
+            float s[8 * H];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                s[i] = (i < 4 ? s0[ct][i & 3] : s1[ct][i & 3]) * scale2;
-                if (!inside) s[i] = kb + g * 8 + i <= hi[ct] ? s[i] : -__builtin_inff();
+            for (int i = 0; i < 8 * H; ++i) {
+                s[i] = sc[ct][i >> 2][i & 3] * scale2;
+                if (!inside) s[i] = kb + (i >> 3) * 32 + g * 8 + (i & 7) <= hi[ct] ? s[i] : -__builtin_inff();
             }
             col[ct].weigh(s, nv);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < 8 * H; ++i) {
                 const __bf16 h = static_cast<__bf16>(s[i]);
-                ph[ct][i] = h;
-                pl[ct][i] = static_cast<__bf16>(s[i] - static_cast<float>(h));
+                ph[ct][i >> 3][i & 7] = h;
+                pl[ct][i >> 3][i & 7] = static_cast<__bf16>(s[i] - static_cast<float>(h));
             }
         }
         // values: lane i of a 16-lane group supplies the address of four columns of row i / 4 and receives column i of
@@ -143,24 +151,26 @@ template <int MK, int MV, int CT, bool EXACT> struct Block<__bf16, MK, MV, CT, E
         typedef short s16x4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
 #pragma unroll
-        for (int vt = 0; vt < MV; ++vt)
-            if (EXACT || vt < nv) {
-                const uint32_t off = (vt >> 2) * 128, el = ev ^ ((vt & 3) << 5);
-                const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v0 + off + el)));
-                const bf16x4 up = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v1 + off + (el ^ 64))));
-                const bf16x8 v = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
+        for (int h = 0; h < H; ++h)
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    col[ct].o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, ph[ct], col[ct].o[vt], 0, 0, 0);
-                    col[ct].o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pl[ct], col[ct].o[vt], 0, 0, 0);
+            for (int vt = 0; vt < MV; ++vt)
+                if (EXACT || vt < nv) {
+                    const uint32_t off = (vt >> 2) * 128 + h * 64 * row, el = ev ^ ((vt & 3) << 5);
+                    const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v0 + off + el)));
+                    const bf16x4 up = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v1 + off + (el ^ 64))));
+                    const bf16x8 v = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        col[ct].o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, ph[ct][h], col[ct].o[vt], 0, 0, 0);
+                        col[ct].o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pl[ct][h], col[ct].o[vt], 0, 0, 0);
+                    }
                 }
-            }
     }
 };
 
 // true f32: two runs of 16 keys on v_mfma_f32_16x16x4_f32; a lane's four consecutive entries of a 16-wide run feed
 // four steps of the product
-template <int MK, int MV, int CT, bool EXACT> struct Block<float, MK, MV, CT, EXACT> {
+template <int MK, int MV, int CT, bool EXACT> struct Block<float, MK, MV, CT, 1, EXACT> {
     f32x4 q[CT][2 * MK];
     __device__ __forceinline__ void load_q(int ct, const float* row, bool live, int nk, uint32_t lane) {
         const uint32_t g = lane >> 4;
@@ -226,19 +236,23 @@ template <typename T> __device__ __forceinline__ void finish4(const FArgs& a, ui
     }
 }
 
-template <typename T, int MK, int MV, int CT, int VG, bool EXACT, int WPE>
+template <typename T, int MK, int MV, int CT, int VG, int H, bool EXACT, int WPE>
 __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
     static_assert(VG == 1 || (EXACT && MV / VG % 4 == 0), "value groups start at whole 64 columns");
     constexpr int MW = MV / VG;
+    constexpr uint32_t BLOCK = 32 * H;   // keys of a block
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t cgi = wave % a.cg, kgi = wave / a.cg % a.kg, vgi = VG > 1 ? wave / a.cg / a.kg : 0;
-    // launch index: kv heads (consecutive ones on different XCDs), column tiles with the longest key ranges first, splits
-    const uint32_t kvh = blockIdx.x % a.kv_heads, tile = a.tiles - 1 - blockIdx.x / a.kv_heads % a.tiles, split = blockIdx.x / a.kv_heads / a.tiles;
+    // launch index: kv heads (consecutive ones on different XCDs), column tiles, splits.  The longest key ranges come first, and
+    // every second round of the chip the other way, so that the tiles that share a CU add up to about the same
+    const uint32_t kvh = blockIdx.x % a.kv_heads, ti = blockIdx.x / a.kv_heads % a.tiles, split = blockIdx.x / a.kv_heads / a.tiles;
+    const uint32_t r0 = ti / a.round * a.round, back = r0 + min(a.round, a.tiles - r0) - 1 - (ti - r0);
+    const uint32_t tile = a.tiles - 1 - (ti / a.round & 1 ? back : ti);
     const uint32_t cols = a.n * a.per, wg_c0 = tile * a.cg * 16 * CT, wg_c1 = min(wg_c0 + a.cg * 16 * CT, cols);
     const int nk = EXACT ? MK : static_cast<int>(a.kp / 32), nv = EXACT ? MW : static_cast<int>(a.vp / 16);
     // this workgroup's key blocks
-    const uint32_t nb = (a.start + (wg_c1 - 1) / a.per) / 32 + 1;
+    const uint32_t nb = (a.start + (wg_c1 - 1) / a.per) / BLOCK + 1;
     const uint32_t share = ((nb + a.splits - 1) / a.splits + a.kg - 1) / a.kg * a.kg;
     const uint32_t first = min(nb, split * share), last = min(nb, first + share);
     // this wavefront's columns
@@ -257,12 +271,12 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
     const uint32_t hi_min = a.start + min(c0, cols - 1) / a.per, hi_max = a.start + min(c0 + 16 * CT - 1, cols - 1) / a.per;
     // staging
     constexpr uint32_t E = 16 / sizeof(T);
-    const uint32_t cpr = a.row / E, segs = 32 * cpr / 64;
-    const uint32_t block_bytes = 32 * a.row * sizeof(T);
+    const uint32_t cpr = a.row / E, segs = BLOCK * cpr / 64;
+    const uint32_t block_bytes = BLOCK * a.row * sizeof(T);
     const T* const kv = static_cast<const T*>(a.kv) + kvh * a.head_stride;
     auto stage = [&](uint32_t b, uint32_t buf) {
         unsigned char* const dst = smem + (buf * a.kg + kgi) * block_bytes;
-        const T* const src = kv + static_cast<uint64_t>(b) * 32 * a.row;
+        const T* const src = kv + static_cast<uint64_t>(b) * BLOCK * a.row;
         for (uint32_t s = cgi + vgi * a.cg; s < segs; s += a.cg * VG) {
             const uint32_t i = s * 64 + lane, key = (i * a.row_magic) >> 20, slot = i - key * cpr;
             __builtin_amdgcn_global_load_lds(
@@ -272,7 +286,7 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
     };
     uint32_t b = first + kgi;
     if (b < last) stage(b, 0);
-    Block<T, MK, MW, CT, EXACT> t;
+    Block<T, MK, MW, CT, H, EXACT> t;
     Column<MW> col[CT];
     const uint32_t vc0 = vgi * MW * 16;   // this wavefront's first value column
 #pragma unroll
@@ -289,8 +303,8 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (a.stages == 2 && b + a.kg < last) stage(b + a.kg, buf ^ 1);
-        if (b < last && wave_live && b * 32 <= hi_max)
-            t.run(reinterpret_cast<const T*>(smem + (buf * a.kg + kgi) * block_bytes), a.row, a.v_off + vc0, b * 32, nk, nv, hi, b * 32 + 31 <= hi_min,
+        if (b < last && wave_live && b * BLOCK <= hi_max)
+            t.run(reinterpret_cast<const T*>(smem + (buf * a.kg + kgi) * block_bytes), a.row, a.v_off + vc0, b * BLOCK, nk, nv, hi, b * BLOCK + BLOCK - 1 <= hi_min,
                   a.scale2, col, lane);
         if (a.stages == 2) {
             buf ^= 1;
@@ -500,9 +514,9 @@ template <class F> void by_size(const FArgs& a, bool f32, F&& f) {
 }
 
 constexpr int wavefronts_per_simd(int mk) { return mk <= 6 ? 2 : 1; }   // what the registers leave room for
-template <typename T, int MK, int MV, int CT, int VG, bool EXACT>
+template <typename T, int MK, int MV, int CT, int VG, int H, bool EXACT>
 cera_hip_status launch(cera_hip_ctx* ctx, const FArgs& a, uint32_t grid, uint64_t lds) {
-    auto* const fn = fattn_kernel<T, MK, MV, CT, VG, EXACT, wavefronts_per_simd(MK)>;
+    auto* const fn = fattn_kernel<T, MK, MV, CT, VG, H, EXACT, wavefronts_per_simd(MK)>;
     if (lds > 64 * 1024) {
         static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, FATTN_LDS_MAX);
         HIP_TRY(ctx, allowed);
@@ -537,7 +551,7 @@ cera_hip_status cera_launch_fattn(cera_hip_ctx* ctx, const FAttnShape& s, const 
     a.n = p.n; a.start = p.start; a.heads = s.heads; a.kv_heads = s.kv_heads; a.per = s.heads / s.kv_heads;
     a.kp = s.kp; a.vp = s.vp; a.vdim = s.vdim; a.v_off = s.v_off; a.scale2 = s.scale * LOG2E; a.sink = s.sink;
     a.out = p.out; a.out_ld = p.out_ld; a.out_head = p.out_head;
-    const uint32_t cols = p.n * a.per, col_tiles = (cols + 15) / 16, nb = (p.start + p.n + 31) / 32;
+    const uint32_t cols = p.n * a.per, col_tiles = (cols + 15) / 16, nb = (p.start + p.n + 31) / 32;   // blocks of 32 keys
     cera_hip_status st = CERA_HIP_OK;
     by_size(a, f32, [&](auto mk, auto mv, auto exact) {
         constexpr int MK = decltype(mk)::value, MV = decltype(mv)::value;
@@ -552,16 +566,18 @@ cera_hip_status cera_launch_fattn(cera_hip_ctx* ctx, const FAttnShape& s, const 
         a.cg = share ? 2 : tiles >= 3 ? 4 : tiles;
         a.kg = share ? 1 : FW / a.cg;
         a.tiles = (tiles + a.cg - 1) / a.cg;
-        const uint64_t block = 32ull * s.row * esz, red = a.kg > 1 ? static_cast<uint64_t>(a.cg) * (two ? 2 : 1) * (MV * 256 + 128) * 4 : 0;
+        a.round = std::max(1u, ctx->n_cu / s.kv_heads);
+        const uint32_t halves = two ? 2 : 1;
+        const uint64_t block = 32ull * halves * s.row * esz, red = a.kg > 1 ? static_cast<uint64_t>(a.cg) * (two ? 2 : 1) * (MV * 256 + 128) * 4 : 0;
         while (a.kg > 1 && a.kg * block > FATTN_LDS_MAX) a.kg /= 2;
         if (!share && a.cg * a.kg != FW) {   // wavefronts without a key group take columns that do not exist: they only help staging
             a.cg = FW / a.kg;
             a.tiles = (tiles + a.cg - 1) / a.cg;
         }
-        a.stages = 2 * a.kg * block <= (wavefronts_per_simd(MK) == 1 ? FATTN_LDS_MAX : 64 * 1024) ? 2 : 1;
+        a.stages = 2 * a.kg * block <= (wavefronts_per_simd(MK) == 1 ? FATTN_LDS_MAX : two ? 80 * 1024 : 64 * 1024) ? 2 : 1;
         // share the keys out where the column tiles do not fill the chip: at least two steps of a workgroup each,
         // one for a single token (its launch is all latency)
-        const uint32_t wgs = a.tiles * s.kv_heads, steps = (nb + a.kg - 1) / a.kg, least = p.n == 1 ? 1 : 2;
+        const uint32_t wgs = a.tiles * s.kv_heads, steps = (nb + a.kg * halves - 1) / (a.kg * halves), least = p.n == 1 ? 1 : 2;
         a.splits = std::max(1u, std::min({std::max(1u, 2 * ctx->n_cu / wgs), steps / least, p.n == 1 ? 256u : 16u}));
         if (merge) {
             most = std::min(most, PARTIALS_MAX / s.heads);
@@ -579,12 +595,12 @@ cera_hip_status cera_launch_fattn(cera_hip_ctx* ctx, const FAttnShape& s, const 
         const uint32_t grid = wgs * a.splits;
         const uint64_t lds = std::max(a.stages * a.kg * block, red);
         if constexpr (!EX) {
-            st = f32 ? launch<float, MK, MV, 1, 1, EX>(ctx, a, grid, lds) : launch<__bf16, MK, MV, 1, 1, EX>(ctx, a, grid, lds);
+            st = f32 ? launch<float, MK, MV, 1, 1, 1, EX>(ctx, a, grid, lds) : launch<__bf16, MK, MV, 1, 1, 1, EX>(ctx, a, grid, lds);
         } else {
             st = CERA_HIP_ERR_SHAPE;
-            if constexpr (CAN2) { if (two) st = launch<__bf16, MK, MV, 2, 1, EX>(ctx, a, grid, lds); }
-            if constexpr (CAN_SHARE) { if (share) st = launch<__bf16, MK, MV, 1, 2, EX>(ctx, a, grid, lds); }
-            if (!two && !share) st = launch<__bf16, MK, MV, 1, 1, EX>(ctx, a, grid, lds);
+            if constexpr (CAN2) { if (two) st = launch<__bf16, MK, MV, 2, 1, 2, EX>(ctx, a, grid, lds); }
+            if constexpr (CAN_SHARE) { if (share) st = launch<__bf16, MK, MV, 1, 2, 1, EX>(ctx, a, grid, lds); }
+            if (!two && !share) st = launch<__bf16, MK, MV, 1, 1, 1, EX>(ctx, a, grid, lds);
         }
     });
     CERA_TRY(st);

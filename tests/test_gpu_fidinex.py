@@ -321,6 +321,22 @@ def test_long_prompts_take_the_large_tiles(tmp_path, f32):
     m.close()
 
 
+@pytest.mark.parametrize("layer, n, cuts", [(U.latent(16, 128, 64, 128, 192, 10000.0), 2100, [2100]), (U.latent(17, 128, 64, 128, 64, 500.0), 2017, [31, 1986]),
+                                            (U.attention(15, 3, 128, 128, None, False), 2255, [65, 2190]), (U.attention(32, 32, 64, 64), 1099, [1099])])
+def test_attention_in_blocks_of_64_keys(tmp_path, layer, n, cuts):
+    """Two column tiles a wavefront: a last block that is half or nearly empty, ragged tiles, rounds of the chip that are not whole,
+    rows whose two blocks take more than 64 KB of LDS.  Tolerance: the operands', as everywhere here."""
+    assert max(cuts) * layer["mixer"]["heads"] >= 128 * 256
+    cfg = U.config([layer], width=64, vocab=40, streams=2)
+    w = U.random_model(cfg, 59)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 7)
+    err = U.rel(_feed(m, toks, cuts), U.reference(cfg, w, toks))
+    print(f"{layer['mixer']['heads']} heads n={n} cuts={cuts}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 @pytest.mark.parametrize("width, ff, n, streams", [(70, 32768, 300, 2), (130, 5200, 1800, 2), (200, 5300, 1777, 1), (260, 32700, 287, 2),
                                                    (5200, 64, 1800, 4), (5200, 130, 1800, 3), (5203, 200, 1799, 4), (5200, 330, 1800, 2)])
 def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
