@@ -678,6 +678,21 @@ static int dense_shape(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uin
     if (n > 64 && (large >= n_cu || (kp >= 8192 && large * 4 >= n_cu))) return 0;
     return n > 32 ? 1 : 2;
 }
+// Parts of K in which 256 x 256 tiles take a product whose sums go through the reduction anyway in place of 128 x 128 tiles with
+// `split` parts, or 0: the fewest, up to four of at least eight steps of 64, whose tiles are at least 55 % of their rounds, as
+// above, and fill theirs well enough: they multiply about 1.3 times as fast on a full chip, and 1.2 times has to be left.
+// Products and reductions of one layer's streams, before and now: 3072 x 8192 times 2048 tokens (384 tiles in a round of 512; 96 x 2
+// in 256) 140 + 47 -> 105 + 52 us, 3072 x 3072 62 + 47 -> 50 + 52; 2048 x 8192 and 2048 x 2048 (256 x 2 in 512; 64 x 3 in 256: left
+// alone) take 1.5 % longer over a whole pass on the larger tiles.
+static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_t wgs, uint32_t split, uint32_t n_cu) {
+    const uint64_t per_xcd = std::max<uint64_t>(n_cu / 8, 1), most = ((m + 255) / 256 + 7) / 8 * ((n + 255) / 256);
+    const uint64_t rounds128 = (wgs * split + 2 * n_cu - 1) / (2 * n_cu);
+    for (uint32_t parts = 2; n > 128 && parts <= 4 && steps / parts >= 8; ++parts) {
+        const uint64_t rounds = (most * parts + per_xcd - 1) / per_xcd;
+        if (m * n * parts * 20 >= rounds * per_xcd * 8 * 65536 * 11) return parts * rounds128 * 20 >= split * rounds * 33 ? parts : 0;
+    }
+    return 0;
+}
 extern "C" uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu) {
     return DENSE_BM[dense_shape(rows, (k + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD, n, 1, n_cu)];
 }
@@ -707,11 +722,16 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     const uint32_t want_wgs = 2 * ctx->n_cu;
     if (shape != 3 && wgs * 4 < want_wgs * (shape == 0 ? 3ull : 4ull) && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
     if (split < 1) split = 1;
-    const uint32_t per = (steps + split - 1) / split;
-    split = (steps + per - 1) / per;
     // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
     // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
     const bool apart = o.epi == DENSE_STREAMS && (o.streams->count != 4 || shape == 0 || shape == 3);
+    if (const uint32_t parts = apart && shape == 0 ? dense_wide_parts(a.m, n, steps, wgs, split, ctx->n_cu) : 0) {
+        shape = 3;
+        bm = bn = 256;
+        split = parts;
+    }
+    const uint32_t per = (steps + split - 1) / split;
+    split = (steps + per - 1) / per;
     if (split > 1 || apart) {
         void* part = nullptr;
         CERA_TRY(cera_scratch_if_room(ctx, 9, static_cast<uint64_t>(split) * n * a.m * sizeof(float), &part));

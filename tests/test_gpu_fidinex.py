@@ -353,6 +353,21 @@ def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
     m.close()
 
 
+@pytest.mark.parametrize("width, ff, n, streams", [(3072, 1030, 1800, 4), (3000, 1100, 2047, 3), (3072, 8200, 1010, 4), (4096, 8300, 600, 2)])
+def test_streams_on_the_widest_tiles_in_parts_of_k(tmp_path, width, ff, n, streams):
+    """The residual streams' products whose 256 x 256 tiles fill their rounds in two, three and four parts of K only: uneven parts, ragged
+    last tiles of rows and tokens.  Tolerance: the operands', as everywhere here."""
+    assert hip_api.dense_tile(width, ff, n) == 128
+    cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=ff)], width=width, vocab=64, streams=streams)
+    w = U.random_model(cfg, 61)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 5)
+    err = U.rel(m.forward_prefill_logits_all(toks, 0), U.reference(cfg, w, toks))
+    print(f"width={width} ff={ff} n={n}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 def test_streams_of_large_tiles_without_room_for_partial_sums():
     """Large tiles hand the streams' products to the reduction, which needs room for them; where there is none (here by a
     limit), smaller tiles update the four streams themselves."""
