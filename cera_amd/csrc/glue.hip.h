@@ -333,25 +333,11 @@ static __global__ __launch_bounds__(1024) void rmsnorm_few_kernel(const float* x
 // threads: blocks [0, n_heads) rotate q; the next n_kv_heads rotate k and
 // store it; the last n_kv_heads copy v.
 // KV cache layout: [kv_head][max_seq][head_dim] f32.
-// Split-K partial sums of q, k or v that this kernel adds up itself instead of a reduction launch in front
-// of it: value e = sum_z part[z * stride + e] in that order (n_split = 0: the rows are complete as they are).
-struct RopePending {
-    const float* part;
-    uint32_t n_split;
-    uint64_t stride;
-};
-__device__ __forceinline__ float rope_pending_ld(const float* rows, const RopePending& pd, uint64_t e) {
-    if (pd.n_split == 0) return rows[e];
-    float s = pd.part[e];
-    for (uint32_t z = 1; z < pd.n_split; ++z) s += pd.part[z * pd.stride + e];
-    return s;
-}
 template <typename KV>
 __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __restrict__ k, const float* v,
                                const float* __restrict__ cs_table, const uint32_t* __restrict__ pos_ptr,
                                uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
-                               KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
-                               RopePending pq = RopePending{}, RopePending pk = RopePending{}, RopePending pv = RopePending{}) {
+                               KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq) {
     // grid.y = tokens of a prefill batch: token t sits at position *pos_ptr + t and its
     // q/k/v rows follow each other ([n][n_heads*head_dim], [n][n_kv_heads*head_dim])
     const uint32_t pos = *pos_ptr + blockIdx.y;
@@ -364,8 +350,7 @@ __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __res
         float* head = rows + at;
         float2 cs = reinterpret_cast<const float2*>(cs_table)[static_cast<uint64_t>(pos) * half + i];
         uint32_t i0 = rope_type == 1 ? 2 * i : i, i1 = rope_type == 1 ? 2 * i + 1 : i + half;
-        const RopePending& pd = is_q ? pq : pk;
-        float x0 = rope_pending_ld(rows, pd, at + i0), x1 = rope_pending_ld(rows, pd, at + i1);
+        float x0 = rows[at + i0], x1 = rows[at + i1];
         float r0 = __fsub_rn(__fmul_rn(x0, cs.x), __fmul_rn(x1, cs.y));
         float r1 = __fadd_rn(__fmul_rn(x0, cs.y), __fmul_rn(x1, cs.x));
         head[i0] = r0;
@@ -378,8 +363,8 @@ __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __res
     } else if (v_cache) {
         uint32_t h = b - n_heads - n_kv_heads;
         KV* dst = v_cache + (static_cast<uint64_t>(h) * max_seq + pos) * head_dim;
-        dst[2 * i] = static_cast<KV>(rope_pending_ld(v, pv, kv_row + h * head_dim + 2 * i));
-        dst[2 * i + 1] = static_cast<KV>(rope_pending_ld(v, pv, kv_row + h * head_dim + 2 * i + 1));
+        dst[2 * i] = static_cast<KV>(v[kv_row + h * head_dim + 2 * i]);
+        dst[2 * i + 1] = static_cast<KV>(v[kv_row + h * head_dim + 2 * i + 1]);
     }
 }
 template <typename KV>
@@ -389,14 +374,78 @@ static __global__ void rope_kv_kernel(float* __restrict__ q, float* __restrict__
                                KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq) {
     rope_kv_body<KV>(q, k, v, cs_table, pos_ptr, n_heads, n_kv_heads, head_dim, rope_type, k_cache, v_cache, max_seq);
 }
-// The same over q / k / v rows whose split-K partial sums are still pending.
+// Split-K partial sums of q, k or v that the kernel below adds up itself instead of a reduction launch in front
+// of it: value e = sum_z part[z * stride + e] in that order (n_split = 0: the rows are complete as they are).
+struct RopePending {
+    const float* part;
+    uint32_t n_split;
+    uint64_t stride;
+};
+// The same for a prompt's pass, which adds pending partial sums up: a thread takes a quad of a head's columns and the one head_dim / 2
+// further on, 256 threads the heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by
+// bytes: 512 tokens of 32 + 8 + 8 heads of 128, K in two parts, 13.7 us, where one pair a
+// thread in workgroups of 64 took 23; 1001 tokens of 24 + 8 + 8: 15 and 21.
+__device__ __forceinline__ float4 rope_pending_ld4(const float* rows, const RopePending& pd, uint64_t e) {
+    if (pd.n_split == 0) return *reinterpret_cast<const float4*>(rows + e);
+    float4 s = *reinterpret_cast<const float4*>(pd.part + e);
+#pragma unroll 4
+    for (uint32_t z = 1; z < pd.n_split; ++z) {
+        const float4 t = *reinterpret_cast<const float4*>(pd.part + z * pd.stride + e);
+        s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+    }
+    return s;
+}
+__device__ __forceinline__ void rope_turn(float& x, float& y, float c, float s) {
+    const float a = __fsub_rn(__fmul_rn(x, c), __fmul_rn(y, s));
+    y = __fadd_rn(__fmul_rn(x, s), __fmul_rn(y, c));
+    x = a;
+}
 template <typename KV>
-static __global__ void rope_kv_pending_kernel(float* __restrict__ q, float* __restrict__ k, const float* v,
+static __global__ __launch_bounds__(256) void rope_kv_quads_kernel(float* __restrict__ q, float* __restrict__ k, const float* v,
                                const float* __restrict__ cs_table, const uint32_t* __restrict__ pos_ptr,
                                uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
                                KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
                                RopePending pq, RopePending pk, RopePending pv) {
-    rope_kv_body<KV>(q, k, v, cs_table, pos_ptr, n_heads, n_kv_heads, head_dim, rope_type, k_cache, v_cache, max_seq, pq, pk, pv);
+    const uint32_t quads = head_dim / 8, item = blockIdx.x * 256 + threadIdx.x, b = item / quads, j = item - b * quads;
+    if (b >= n_heads + 2 * n_kv_heads) return;
+    const uint32_t pos = *pos_ptr + blockIdx.y;
+    const uint64_t tok = blockIdx.y;
+    if (b >= n_heads + n_kv_heads) {
+        const uint32_t h = b - n_heads - n_kv_heads;
+        const uint64_t at = (tok * n_kv_heads + h) * head_dim + 4 * j;
+        KV* const dst = v_cache + (static_cast<uint64_t>(h) * max_seq + pos) * head_dim;
+        const float4 x = rope_pending_ld4(v, pv, at), y = rope_pending_ld4(v, pv, at + 4 * quads);
+        KvOps<KV>::st4(dst, j, x);
+        KvOps<KV>::st4(dst, j + quads, y);
+        return;
+    }
+    const bool is_q = b < n_heads;
+    const uint32_t h = is_q ? b : b - n_heads;
+    float* const rows = is_q ? q : k;
+    const RopePending& pd = is_q ? pq : pk;
+    const uint64_t at = (tok * (is_q ? n_heads : n_kv_heads) + h) * head_dim + 4 * j;
+    float4 x = rope_pending_ld4(rows, pd, at), y = rope_pending_ld4(rows, pd, at + 4 * quads);
+    const float4* const cs = reinterpret_cast<const float4*>(cs_table + static_cast<uint64_t>(pos) * head_dim);
+    if (rope_type == 1) {   // pairs (2i, 2i + 1)
+        const float4 c = cs[j], d = cs[j + quads];
+        rope_turn(x.x, x.y, c.x, c.y);
+        rope_turn(x.z, x.w, c.z, c.w);
+        rope_turn(y.x, y.y, d.x, d.y);
+        rope_turn(y.z, y.w, d.z, d.w);
+    } else {                // pairs (i, i + head_dim / 2)
+        const float4 c = cs[2 * j], d = cs[2 * j + 1];
+        rope_turn(x.x, y.x, c.x, c.y);
+        rope_turn(x.y, y.y, c.z, c.w);
+        rope_turn(x.z, y.z, d.x, d.y);
+        rope_turn(x.w, y.w, d.z, d.w);
+    }
+    *reinterpret_cast<float4*>(rows + at) = x;
+    *reinterpret_cast<float4*>(rows + at + 4 * quads) = y;
+    if (!is_q) {
+        KV* const dst = k_cache + (static_cast<uint64_t>(h) * max_seq + pos) * head_dim;
+        KvOps<KV>::st4(dst, j, x);
+        KvOps<KV>::st4(dst, j + quads, y);
+    }
 }
 
 // n_keep context shift (cera/src/kv_cache.rs:1091-1310): rows [src_row, src_row + n_rows) of every

@@ -533,15 +533,27 @@ static __global__ __launch_bounds__(256) void act_fp8_records_kernel(const int8_
     else kq_act_record(blockIdx.x - fp8_records, xq, records, n, k);
 }
 
-// The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.
+// The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.  With
+// many tokens a thread takes four elements (512 tokens of 4096, Q4_K: 12.4 us by one element, 8.2 by four); with a few the launch is
+// a chain of loads, which one element keeps the shortest (45 tokens: 4.8 us, four elements 5.7).
+constexpr uint32_t embed_elems(int ids) { return ids > 64 ? 4 : 1; }
 template <int N>
 static __global__ __launch_bounds__(256) void embed_ids_kernel(uint32_t dtype, const uint8_t* __restrict__ w, uint64_t row_bytes, CeraIds<N> tokens, uint32_t first,
                                                                uint32_t pos, uint32_t* __restrict__ scalars, uint32_t k, float scale, float* __restrict__ out) {
-    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    constexpr uint32_t E = embed_elems(N);
+    const uint32_t e = (blockIdx.x * 256 + threadIdx.x) * E;   // k is a multiple of 32
     if (e == 0 && first + blockIdx.y == 0) scalars[1] = pos;
     if (e >= k) return;
-    const float v = dequant_elem(dtype, w + static_cast<uint64_t>(tokens.id[blockIdx.y]) * row_bytes, e);
-    out[static_cast<uint64_t>(first + blockIdx.y) * k + e] = scale != 1.0f ? __fmul_rn(v, scale) : v;
+    const uint8_t* const row = w + static_cast<uint64_t>(tokens.id[blockIdx.y]) * row_bytes;
+    float v[E];
+#pragma unroll
+    for (uint32_t i = 0; i < E; ++i) {
+        v[i] = dequant_elem(dtype, row, e + i);
+        if (scale != 1.0f) v[i] = __fmul_rn(v[i], scale);
+    }
+    float* const o = out + static_cast<uint64_t>(first + blockIdx.y) * k + e;
+    if constexpr (E == 4) *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+    else *o = v[0];
 }
 
 // all_logits (host, [n][vocab]): when set, every position is projected through the LM head in one
@@ -555,7 +567,8 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     const float scale = c.attn_scale != 0.0f ? c.attn_scale : 1.0f / std::sqrt(static_cast<float>(c.head_dim));
     CERA_TRY(cera_model_ensure_prefill_buffers(m, n));
     cera_by_ids(tokens, n, [&](const auto& ids, uint32_t first, uint32_t count) {
-        hipLaunchKernelGGL(embed_ids_kernel, dim3((hs + 255) / 256, count), dim3(256), 0, s, m->embd->dtype, m->embd->dev, m->embd->row_bytes, ids, first,
+        const uint32_t per = 256 * embed_elems(static_cast<int>(sizeof(ids.id) / sizeof(ids.id[0])));
+        hipLaunchKernelGGL(embed_ids_kernel, dim3((hs + per - 1) / per, count), dim3(256), 0, s, m->embd->dtype, m->embd->dev, m->embd->row_bytes, ids, first,
                            start_pos, m->scalars, hs, c.embed_scale, m->pf_hidden);
     });
     HIP_TRY(ctx, hipGetLastError());
@@ -726,26 +739,20 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             hipLaunchKernelGGL((rmsnorm_kernel<false>), dim3(n * c.n_kv_heads), dim3(256), 0, s, m->pf_k, L.k_norm, c.head_dim,
                                c.rms_eps, m->pf_k, nullptr, nullptr, nullptr);
         }
-        if (pqk.n_split || pvv.n_split) {
+        {
             const RopePending rq{pqk.part, pqk.n_split, pqk.stride};
             const RopePending rk{pqk.n_split ? pqk.part + static_cast<uint64_t>(n) * q_dim : nullptr, pqk.n_split, pqk.stride};
             const RopePending rv{pvv.part, pvv.n_split, pvv.stride};
-            if (m->kv_f16)
-                hipLaunchKernelGGL(rope_kv_pending_kernel<kv_half>, dim3(c.n_heads + 2 * c.n_kv_heads, n), dim3(c.head_dim / 2), 0, s,
+            // (heads come in whole eights of columns, so that rows and slices of partial sums start on whole quads)
+            auto rope = [&](auto tag) {
+                using KV = decltype(tag);
+                hipLaunchKernelGGL(rope_kv_quads_kernel<KV>, dim3(((c.n_heads + 2 * c.n_kv_heads) * (c.head_dim / 8) + 255) / 256, n), dim3(256), 0, s,
                                    m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads, c.head_dim,
-                                   c.rope_type, static_cast<kv_half*>(L.kc), static_cast<kv_half*>(L.vc), c.max_seq_len, rq, rk, rv);
-            else
-                hipLaunchKernelGGL(rope_kv_pending_kernel<float>, dim3(c.n_heads + 2 * c.n_kv_heads, n), dim3(c.head_dim / 2), 0, s,
-                                   m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads, c.head_dim,
-                                   c.rope_type, static_cast<float*>(L.kc), static_cast<float*>(L.vc), c.max_seq_len, rq, rk, rv);
-        } else if (m->kv_f16)
-            hipLaunchKernelGGL(rope_kv_kernel<kv_half>, dim3(c.n_heads + 2 * c.n_kv_heads, n), dim3(c.head_dim / 2), 0, s,
-                               m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads, c.head_dim,
-                               c.rope_type, static_cast<kv_half*>(L.kc), static_cast<kv_half*>(L.vc), c.max_seq_len);
-        else
-            hipLaunchKernelGGL(rope_kv_kernel<float>, dim3(c.n_heads + 2 * c.n_kv_heads, n), dim3(c.head_dim / 2), 0, s,
-                               m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads, c.head_dim,
-                               c.rope_type, static_cast<float*>(L.kc), static_cast<float*>(L.vc), c.max_seq_len);
+                                   c.rope_type, static_cast<KV*>(L.kc), static_cast<KV*>(L.vc), c.max_seq_len, rq, rk, rv);
+            };
+            if (m->kv_f16) rope(kv_half{});
+            else rope(float{});
+        }
         HIP_TRY(ctx, hipGetLastError());
         // causal attention: query t sees positions 0 .. start_pos + t
         CERA_TRY(cera_launch_attn(ctx, m->pf_q, L.kc, L.vc, c.n_heads, c.n_kv_heads, c.head_dim, start_pos + 1ull,

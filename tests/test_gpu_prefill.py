@@ -466,6 +466,28 @@ def test_prefill_where_the_norm_adds_split_k_partial_sums(hip, orc, rope_type, k
     gm.close(); om.close()
 
 
+@pytest.mark.parametrize("head_dim,n_heads,n_kv_heads", [(8, 32, 8), (40, 32, 2), (64, 4, 4), (256, 3, 1)])
+@pytest.mark.parametrize("rope_type,kv_f16", [(1, False), (0, False), (1, True), (0, True)])
+def test_prefill_rotates_heads_of_every_size(hip, orc, head_dim, n_heads, n_kv_heads, rope_type, kv_f16):
+    """Rotation and append over heads that do not fill a workgroup's threads evenly, both pair orders and cache types, from position 0
+    and from inside a sequence.  Layer 0's rows are one product away from the oracle's: its tolerance, as above."""
+    cfg = dict(synth.TINY, n_layers=1, hidden=512, n_heads=n_heads, n_kv_heads=n_kv_heads, head_dim=head_dim, max_seq_len=96, rope_type=rope_type)
+    weights = synth.make_llama(cfg, seed=83, sigma=0.03, norm_jitter=0.1)
+    gm = hip_api.Model(hip, cfg, weights)
+    om = orc.Llama(cfg, weights)
+    if kv_f16:
+        gm.configure_kv(True); om.set_kv_f16(True)
+    toks = [int(t) for t in util.rng(head_dim).integers(0, cfg["vocab"], 81)]
+    _say(f"model: heads of {head_dim}, {n_heads} / {n_kv_heads}, rope {rope_type}, f16 cache {kv_f16}")
+    for first, last in ((0, 10), (10, 81)):
+        gm.forward_prefill(toks[first:last], first)
+        om.forward_prefill_batched(toks[first:last], first)
+    (kg, vg), (ko, vo) = gm.read_kv(0), om.kv(0)
+    assert np.abs(kg - ko).max() <= 2e-3 * util.rms(ko)
+    assert np.abs(vg - vo).max() <= 2e-3 * util.rms(vo)
+    gm.close(); om.close()
+
+
 # a pass of a few tokens: (config, make_llama's arguments, biases, QK norm, f16 cache)
 FEW_MODELS = {
     "q4_k_m": (dict(), dict(), False, False, False),                                        # Q | K and a Q6_K V in one launch
