@@ -23,7 +23,7 @@ struct GemmDArgs {
     const void* x;
     uint64_t ldx;
     uint32_t m, n, kp, k_chunk;
-    uint32_t tiles_m, tiles_n;
+    uint32_t tiles_m, tiles_n, whole;   // whole: of an XCD, 256 x 256 tiles that are not cut in halves
     int epi;
     void* out;
     uint64_t ldo;
@@ -284,35 +284,42 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
 // read, 64 KB written at 128 bytes a clock); one workgroup alone takes 2660 for it, a full chip 3440, with the matrix cores busy
 // for 52 % of 28672 x 4096 times 1900 tokens (3.5 rounds).  28672 x 4096 times 2048 / 512 tokens: 1100 / 1040 TFLOP/s, 128 x 128
 // tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
-template <int EPI, int SN>
-__global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
-    constexpr int B = 256, BK = 64, MI = 8, NI = 4, HALF = B * BK, BUF = 2 * HALF;
-    __shared__ __align__(1024) __bf16 lds[2][BUF];
-    uint32_t tm, tn, group;
-    if (!dense_tile(a, tm, tn, group)) return;
+// MI: 16-row tiles of a wavefront: 8, or 4 for 128 x 256 (row0: the workgroup's first weight row)
+constexpr int WIDE_BK = 64, WIDE_HALF = 256 * WIDE_BK, WIDE_BUF = 2 * WIDE_HALF;
+template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_body(GemmDArgs& a, __bf16 (*lds)[WIDE_BUF], uint32_t row0, uint32_t tn, uint32_t group) {
+    constexpr int B = 256, BK = WIDE_BK, NI = 4, HALF = WIDE_HALF, BUF = WIDE_BUF, WP = MI / 2, LOADS = WP + 4;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t k0 = blockIdx.y * a.k_chunk, k1 = min(a.kp, k0 + a.k_chunk), steps = (k1 - k0) / BK;
-    // wavefronts 0 - 3 bring the weight rows in, 4 - 7 the tokens, 64 rows each; rows past the end re-read the last one
+    // MI = 8: wavefronts 0 - 3 bring the weight rows in, 4 - 7 the tokens, eight pieces of eight rows each; 4: each two pieces of
+    // weight rows and four of tokens (which at 8 takes 4 % longer).  Rows past the end re-read the last one
+    const uint32_t last_w = a.m - 1 - row0, first_x = tn * B, last_x = a.n - 1 - first_x, ldw = a.kp * 2, ldx = static_cast<uint32_t>(a.ldx) * 2;
+    const uint8_t* const base_w = reinterpret_cast<const uint8_t*>(a.w + group * a.gw) + static_cast<uint64_t>(row0) * ldw + k0 * 2;
+    const uint8_t* const base_x = static_cast<const uint8_t*>(a.x) + group * a.gx * 2 + first_x * a.ldx * 2 + k0 * 2;
     const bool toks = wave >= 4;
-    const uint32_t first = toks ? tn * B : tm * B, last = (toks ? a.n : a.m) - 1 - first;
-    const uint64_t ld = (toks ? a.ldx : a.kp) * 2;
-    const uint8_t* const base = toks ? static_cast<const uint8_t*>(a.x) + group * a.gx * 2 : reinterpret_cast<const uint8_t*>(a.w + group * a.gw);
-    const uint8_t* src = lds_dma_base(base + first * ld + k0 * 2);
+    const uint8_t *src = lds_dma_base(MI == 8 && toks ? base_x : base_w), *src_x = lds_dma_base(base_x);
     const uint32_t sub = lane >> 3, slot = lane & 7;
-    uint32_t off[8];
+    uint32_t off[LOADS];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) off[s] = min((wave & 3) * 64 + s * 8 + sub, last) * static_cast<uint32_t>(ld) + (slot ^ sub) * 16;
-    const uint32_t dst = lds_addr(&lds[0][0]) + wave * 8192;
+    for (int s = 0; s < LOADS; ++s) {
+        const bool x = MI == 8 ? toks : s >= WP;
+        const uint32_t r = (MI == 8 ? (wave & 3) * 8 + s : x ? wave * 4 + s - WP : wave * WP + s) * 8 + sub;
+        off[s] = min(r, x ? last_x : last_w) * (x ? ldx : ldw) + (slot ^ sub) * 16;
+    }
+    const uint32_t dst = lds_addr(&lds[0][0]) + wave * (MI == 8 ? 8192 : WP * 1024), dst_x = lds_addr(&lds[0][0]) + HALF * 2 + wave * 4096;
     auto stage = [&](int buf) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) lds_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
+        for (int s = 0; s < LOADS; ++s) {
+            if (MI == 8 || s < WP) lds_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
+            else lds_dma_1k(src_x, off[s], dst_x + buf * BUF * 2 + (s - WP) * 1024);
+        }
         src = lds_dma_base(src + BK * 2);
+        if (MI != 8) src_x = lds_dma_base(src_x + BK * 2);
     };
     const uint32_t wm = wave >> 2, wn = wave & 3, fr = lane & 15, fg = lane >> 4;
     bf16x8 fa[2][MI], fb[2][NI];
     auto frags = [&](int buf, int kk) {
         const uint32_t o = ((kk * 4 + fg) ^ (fr & 7)) * 8;
-        const __bf16* const aw = &lds[buf][(wm * 128 + fr) * BK + o];
+        const __bf16* const aw = &lds[buf][(wm * (MI * 16) + fr) * BK + o];
         const __bf16* const bx = &lds[buf][HALF + (wn * 64 + fr) * BK + o];
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) fa[kk][mi] = *reinterpret_cast<const bf16x8*>(aw + mi * 16 * BK);
@@ -333,9 +340,9 @@ __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
         // the reads of the next fragments between the matrix instructions
         __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
 #pragma unroll
-        for (int i = 0; i < 12; ++i) {
+        for (int i = 0; i < MI + NI; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, (MI * NI - 8) / (MI + NI), 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
     };
@@ -352,7 +359,7 @@ __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
     stage(0);
     if (steps > 1) {
         stage(1);
-        asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
     } else {
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -362,7 +369,29 @@ __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
         if (s + 1 < steps) step(s + 1, 1);
     }
     a.out = static_cast<char*>(a.out) + group * a.go;
-    dense_epilogue<__bf16, EPI, SN, MI, NI>(a, tm * B + wm * 128, tn * B + wn * 64, lane, blockIdx.y, acc);
+    dense_epilogue<__bf16, EPI, SN, MI, NI>(a, row0 + wm * (MI * 16), tn * B + wn * 64, lane, blockIdx.y, acc);
+}
+// HALVES: the last round's tiles, at most half of one, go to twice as many workgroups of half their rows (of an XCD, those from
+// `whole` on; an instance of its own, since the others take 2 % longer with both bodies in one).  28672 x 4096 times 1900 tokens, 3.5
+// rounds: 389 us, 404 in four.
+template <int EPI, int SN, bool HALVES>
+__global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
+    __shared__ __align__(1024) __bf16 lds[2][WIDE_BUF];
+    uint32_t tm, tn, group;
+    if constexpr (HALVES) {
+        const uint32_t xcd = blockIdx.x & 7, at = blockIdx.x >> 3, half = at < a.whole ? 0 : at - a.whole, t = at < a.whole ? at : a.whole + half / 2;
+        const uint32_t i = t / a.tiles_n * 8 + xcd;   // dense_tile's order
+        tn = t % a.tiles_n;
+        if (i >= a.tiles_m * a.groups) return;
+        group = a.groups > 1 ? i / a.tiles_m : 0;
+        tm = i - group * a.tiles_m;
+        if (at >= a.whole) {
+            const uint32_t row0 = tm * 256 + (half & 1) * 128;
+            if (row0 < a.m) dense_wide_body<EPI, SN, 4>(a, lds, row0, tn, group);
+            return;
+        }
+    } else if (!dense_tile(a, tm, tn, group)) return;
+    dense_wide_body<EPI, SN, 8>(a, lds, tm * 256, tn, group);
 }
 
 // 64 x 64 tile in true f32: weights widened on their way into LDS, K in steps of 32.  A lane's four
@@ -746,14 +775,19 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     a.k_chunk = (steps + split - 1) / split * DENSE_PAD;
     a.tiles_m = (a.m + bm - 1) / bm;
     a.tiles_n = (n + bn - 1) / bn;
-    const dim3 grid((a.tiles_m * groups.count + 7) / 8 * 8 * a.tiles_n, split);
+    const uint32_t per_xcd = std::max(1u, ctx->n_cu / 8), units = (a.tiles_m * groups.count + 7) / 8 * a.tiles_n;   // of an XCD
+    // the last units of 256 x 256 tiles by halves: where they are no more than half a round behind whole ones
+    const uint32_t rest = units % per_xcd, halves = shape == 3 && split == 1 && units > per_xcd && rest * 2 <= per_xcd ? rest : 0;
+    a.whole = units - halves;
+    const dim3 grid((units + halves) * 8, split);
     const uint64_t quads = (a.epi == DENSE_SWIGLU ? (a.m / 2 + 3) / 4 : (a.m + 3) / 4) * static_cast<uint64_t>(n);
     const dim3 rg(static_cast<uint32_t>((quads + 255) / 256)), block(256);
     auto go = [&](auto epi, auto streams) {
         constexpr int E = decltype(epi)::value, SN = decltype(streams)::value;
         constexpr int EG = E == DENSE_STREAMS && SN == 0 ? DENSE_STORE : E, EL = E == DENSE_STREAMS ? DENSE_STORE : E;   // leave partial sums, whatever it is
         if (f32) hipLaunchKernelGGL((dense_gemm_f32_kernel<EG, SN>), grid, block, 0, ctx->stream, a);
-        else if (shape == 3) hipLaunchKernelGGL((dense_gemm_wide_kernel<EL, 0>), grid, dim3(512), 0, ctx->stream, a);
+        else if (shape == 3 && halves) hipLaunchKernelGGL((dense_gemm_wide_kernel<EL, 0, true>), grid, dim3(512), 0, ctx->stream, a);
+        else if (shape == 3) hipLaunchKernelGGL((dense_gemm_wide_kernel<EL, 0, false>), grid, dim3(512), 0, ctx->stream, a);
         else if (shape == 0) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EL, 0, 128, 128, 2, 2>), grid, block, 0, ctx->stream, a);
         else if (shape == 1) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 64, 2, 2>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 32, 2, 2>), grid, block, 0, ctx->stream, a);

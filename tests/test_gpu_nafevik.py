@@ -322,6 +322,23 @@ def test_products_on_the_widest_tiles(tmp_path, width, ff, n, vocab):
     m.close()
 
 
+@pytest.mark.parametrize("width, ff, n, vocab", [(60, 5000, 1999, 64), (130, 5120, 2048, 64), (200, 64, 1990, 9899), (260, 4928, 2001, 64)])
+def test_products_whose_last_tiles_go_by_halves(tmp_path, width, ff, n, vocab):
+    """40 tiles of 256 x 256 an XCD, 32 of them at a time: the last eight by halves of their rows.  One to five K steps, ragged last rows
+    that end in a first half and in a second one, ragged tokens; gate | up and the head of all positions."""
+    wide, k = max((2 * ff, width), (vocab, width))
+    units = -(-(-(-wide // 256)) // 8) * -(-n // 256)
+    assert hip_api.dense_tile(wide, k, n) == 256 and units > 32 and 0 < units % 32 <= 16
+    cfg = U.config([U.attention(2, 1, 32, 32, 700, 32, 10000.0, ff=ff)], width=width, vocab=vocab, taps=2, positions=n)
+    w = R.random_model(cfg, 67)
+    m = _open(U.save(tmp_path / "m", cfg, w), False, n)
+    toks = U.tokens(cfg, n, 5)
+    err = U.rel(m.forward_prefill_logits_all(toks, 0), U.reference(cfg, w, toks))
+    print(f"width={width} ff={ff} n={n}: {err:.2e}", flush=True)
+    assert err < TOL[False]
+    m.close()
+
+
 @DTYPES
 def test_steps_behind_a_very_long_context(tmp_path, f32):
     """Thousands of visible keys: decode steps and short portions split them over many workgroups."""
