@@ -247,8 +247,11 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
     // launch index: kv heads (consecutive ones on different XCDs), column tiles, splits.  The longest key ranges come first, and
     // every second round of the chip the other way, so that the tiles that share a CU add up to about the same
     const uint32_t kvh = blockIdx.x % a.kv_heads, ti = blockIdx.x / a.kv_heads % a.tiles, split = blockIdx.x / a.kv_heads / a.tiles;
-    const uint32_t r0 = ti / a.round * a.round, back = r0 + min(a.round, a.tiles - r0) - 1 - (ti - r0);
-    const uint32_t tile = a.tiles - 1 - (ti / a.round & 1 ? back : ti);
+    uint32_t tile = a.tiles - 1 - ti;
+    if (a.tiles > a.round) {
+        const uint32_t round = ti / a.round, r0 = round * a.round;
+        if (round & 1) tile = a.tiles - 1 - (r0 + min(a.round, a.tiles - r0) - 1 - (ti - r0));
+    }
     const uint32_t cols = a.n * a.per, wg_c0 = tile * a.cg * 16 * CT, wg_c1 = min(wg_c0 + a.cg * 16 * CT, cols);
     const int nk = EXACT ? MK : static_cast<int>(a.kp / 32), nv = EXACT ? MW : static_cast<int>(a.vp / 16);
     // this workgroup's key blocks
