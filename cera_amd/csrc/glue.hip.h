@@ -382,7 +382,7 @@ struct RopePending {
     uint64_t stride;
 };
 // The same for a prompt's pass, which adds pending partial sums up: a thread takes a quad of a head's columns and the one head_dim / 2
-// further on, 256 threads the heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by
+// further on, a few workgroups the heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by
 // bytes: 512 tokens of 32 + 8 + 8 heads of 128, K in two parts, 13.7 us, where one pair a
 // thread in workgroups of 64 took 23; 1001 tokens of 24 + 8 + 8: 15 and 21.
 __device__ __forceinline__ float4 rope_pending_ld4(const float* rows, const RopePending& pd, uint64_t e) {
@@ -406,7 +406,7 @@ static __global__ __launch_bounds__(256) void rope_kv_quads_kernel(float* __rest
                                uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
                                KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
                                RopePending pq, RopePending pk, RopePending pv) {
-    const uint32_t quads = head_dim / 8, item = blockIdx.x * 256 + threadIdx.x, b = item / quads, j = item - b * quads;
+    const uint32_t quads = head_dim / 8, item = blockIdx.x * blockDim.x + threadIdx.x, b = item / quads, j = item - b * quads;
     if (b >= n_heads + 2 * n_kv_heads) return;
     const uint32_t pos = *pos_ptr + blockIdx.y;
     const uint64_t tok = blockIdx.y;
