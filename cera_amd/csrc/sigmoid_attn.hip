@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void sattn_rows_kernel(AArgs a) {
 // sattn_rows_kernel's, in its order.  1900 queries, 32 heads of 128 on 8: 185 us with every wavefront reading its own keys and
 // values, V in pieces of half a cache line; 87 with blocks of 32 in LDS, 70 with blocks of 64, which leave a wavefront fewer
 // waits in a row (630 TFLOP/s of matrix instructions).  What bounds it: those waits, and the sigmoids between the products.
-template <int DK> __device__ __forceinline__ uint32_t key_slot(uint32_t key, uint32_t chunk) {
+__device__ __forceinline__ uint32_t key_slot(uint32_t key, uint32_t chunk) {
     return (chunk & ~7u) | ((chunk ^ ((key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2))) & 7);
 }
 template <int DK, int VT, int CT>
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a) {
     for (uint32_t s = 0; s < SEGS; ++s) {
         if (s < KB / 4096) {
             const uint32_t i = (wave * (KB / 4096) + s) * 64 + lane, key = i / (DK * 4);
-            off[s] = key * ROW + key_slot<DK>(key, i % (DK * 4)) * 16;
+            off[s] = key * ROW + key_slot(key, i % (DK * 4)) * 16;
         } else {
             const uint32_t i = (wave * (VB / 4096) + s - KB / 4096) * 64 + lane, v = i >> 3;
             off[s] = v * a.cap * 2 + ((i ^ v) & 7) * 16;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a) {
         for (int kd = 0; kd < DK; ++kd)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {   // half j / 2, keys 4 (j % 2) on
-                const bf16x8 f = *reinterpret_cast<const bf16x8*>(base + k0 + (j >> 1) * (32 * ROW) + (j & 1) * (4 * ROW) + key_slot<DK>(key + 4 * (j & 1), kd * 4 + g) * 16);
+                const bf16x8 f = *reinterpret_cast<const bf16x8*>(base + k0 + (j >> 1) * (32 * ROW) + (j & 1) * (4 * ROW) + key_slot(key + 4 * (j & 1), kd * 4 + g) * 16);
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct) sc[ct][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, q[ct][kd], sc[ct][j], 0, 0, 0);
             }
