@@ -33,7 +33,6 @@ struct AArgs {
     uint64_t out_ld;
     float* part;            // [split][n][heads][vdim_p], splits > 1
     uint32_t splits;
-    uint32_t tiles, round;  // shared rows: column tiles of a kv head, workgroups of a kv head in one round of the chip
     uint32_t attn_blocks;   // fused step: workgroups past these add up the convolution history
     ConvRing ring;
     ConvHist hist;
@@ -266,16 +265,17 @@ __global__ __launch_bounds__(256) void sattn_rows_kernel(AArgs a) {
 __device__ __forceinline__ uint32_t key_slot(uint32_t key, uint32_t chunk) {
     return (chunk & ~7u) | ((chunk ^ ((key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2))) & 7);
 }
+// tiles: column tiles of a kv head; per_round: workgroups of a kv head in one round of the chip
 template <int DK, int VT, int CT>
-__global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a) {
+__global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a, uint32_t tiles, uint32_t per_round) {
     constexpr uint32_t ROW = DK * 64, KB = 64 * ROW, VB = VT * 2048, SEGS = (KB + VB) / 4096;   // 1 KB pieces of a wavefront
     static_assert(KB % 4096 == 0 && VB % 4096 == 0, "a wavefront's pieces are whole");
     __shared__ __align__(1024) uint8_t lds[2][KB + VB];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
     // launch index: kv heads (consecutive ones on different XCDs), then tiles: the longest key ranges first, and every second
     // round of the chip the other way, so that a CU's tiles add up to about the same
-    const uint32_t kvh = blockIdx.x % a.kv_heads, t = blockIdx.x / a.kv_heads, round = t / a.round, at = t - round * a.round;
-    const uint32_t tile = a.tiles - 1 - (round & 1 ? round * a.round + min(a.round, a.tiles - round * a.round) - 1 - at : t);
+    const uint32_t kvh = blockIdx.x % a.kv_heads, t = blockIdx.x / a.kv_heads, round = t / per_round, at = t - round * per_round;
+    const uint32_t tile = tiles - 1 - (round & 1 ? round * per_round + min(per_round, tiles - round * per_round) - 1 - at : t);
     const uint32_t cols = a.n * a.per, wg_c0 = tile * 64 * CT, c0 = wg_c0 + wave * 16 * CT;
     const bool wave_live = c0 < cols;
     Columns<__bf16, DK, VT, CT> col;
@@ -687,11 +687,10 @@ cera_hip_status cera_launch_sattn(cera_hip_ctx* ctx, const SAttnShape& s, const 
         constexpr int DK = decltype(dk)::value, VT = decltype(vt)::value;
         if constexpr (DK == 2 || DK == 4) {
             const uint32_t per_wg = 64 * (wide ? 2 : 1);
-            a.tiles = (cols + per_wg - 1) / per_wg;
-            a.round = std::max(1u, ctx->n_cu / s.kv_heads);
-            const dim3 grid(a.tiles * s.kv_heads);
-            if (wide) hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 2>), grid, dim3(256), 0, ctx->stream, a);
-            else hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 1>), grid, dim3(256), 0, ctx->stream, a);
+            const uint32_t tiles = (cols + per_wg - 1) / per_wg, per_round = std::max(1u, ctx->n_cu / s.kv_heads);
+            const dim3 grid(tiles * s.kv_heads);
+            if (wide) hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 2>), grid, dim3(256), 0, ctx->stream, a, tiles, per_round);
+            else hipLaunchKernelGGL((sattn_shared_kernel<DK, VT, 1>), grid, dim3(256), 0, ctx->stream, a, tiles, per_round);
         } else {
             const uint32_t per_wg = 64 * (wide && VT ? 2 : 1);
             const dim3 grid((cols + per_wg - 1) / per_wg, s.kv_heads);

@@ -39,7 +39,8 @@ struct FArgs {
     uint64_t out_ld;
     uint32_t out_head;
     float *part, *ml;                // [split][n][heads][vp], [split][n][heads][2]; splits > 1 or merged by the consumer
-    uint32_t splits, tiles, round, cg, kg, stages;   // round: workgroups of a kv head in one round of the chip
+    uint32_t splits, tiles, cg, kg, stages;
+    uint32_t round;                  // blocks of 64 keys: workgroups of a kv head in one round of the chip
 };
 
 __device__ __forceinline__ uint32_t swz(uint32_t key) { return (key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2); }
@@ -107,11 +108,11 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
         const uint32_t ka = (r >> 2) * 8 + (r & 3), e = (g ^ swz(ka)) * 16;
         const char* const k0 = base + ka * row * 2;
         const char* const k1 = k0 + 8 * row;
-        f32x4 sc[CT][2 * H];
+        f32x4 s0[CT][H], s1[CT][H];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-            for (int j = 0; j < 2 * H; ++j) sc[ct][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int h = 0; h < H; ++h) s0[ct][h] = s1[ct][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kd = 0; kd < MK; ++kd)
             if (EXACT || kd < nk) {
@@ -121,8 +122,8 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
                     const bf16x8 fa = *reinterpret_cast<const bf16x8*>(k0 + h * 64 * row + off + el), fb = *reinterpret_cast<const bf16x8*>(k1 + h * 64 * row + off + (el ^ 64));
 #pragma unroll
                     for (int ct = 0; ct < CT; ++ct) {
-                        sc[ct][2 * h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, q[ct][kd], sc[ct][2 * h], 0, 0, 0);
-                        sc[ct][2 * h + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb, q[ct][kd], sc[ct][2 * h + 1], 0, 0, 0);
+                        s0[ct][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, q[ct][kd], s0[ct][h], 0, 0, 0);
+                        s1[ct][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb, q[ct][kd], s1[ct][h], 0, 0, 0);
                     }
                 }
             }
@@ -132,7 +133,7 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
             float s[8 * H];
 #pragma unroll
             for (int i = 0; i < 8 * H; ++i) {
-                s[i] = sc[ct][i >> 2][i & 3] * scale2;
+                s[i] = (i & 4 ? s1[ct][i >> 3][i & 3] : s0[ct][i >> 3][i & 3]) * scale2;
                 if (!inside) s[i] = kb + (i >> 3) * 32 + g * 8 + (i & 7) <= hi[ct] ? s[i] : -__builtin_inff();
             }
             col[ct].weigh(s, nv);
@@ -244,11 +245,10 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t cgi = wave % a.cg, kgi = wave / a.cg % a.kg, vgi = VG > 1 ? wave / a.cg / a.kg : 0;
-    // launch index: kv heads (consecutive ones on different XCDs), column tiles, splits.  The longest key ranges come first, and
-    // every second round of the chip the other way, so that the tiles that share a CU add up to about the same
+    // launch index: kv heads (consecutive ones on different XCDs), column tiles with the longest key ranges first, splits
     const uint32_t kvh = blockIdx.x % a.kv_heads, ti = blockIdx.x / a.kv_heads % a.tiles, split = blockIdx.x / a.kv_heads / a.tiles;
     uint32_t tile = a.tiles - 1 - ti;
-    if (a.tiles > a.round) {
+    if constexpr (H == 2) {   // many tiles: every second round of the chip the other way, so that a CU's tiles add up to about the same
         const uint32_t round = ti / a.round, r0 = round * a.round;
         if (round & 1) tile = a.tiles - 1 - (r0 + min(a.round, a.tiles - r0) - 1 - (ti - r0));
     }
