@@ -79,6 +79,10 @@ cera_hip_status cera_scratch(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void*
 
 cera_hip_status cera_scratch_if_room(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out) {
     *out = nullptr;
+    // a workspace that cannot grow stays as it is: a caller whose second choice it still holds would free it and take it anew every time
+    size_t free_b = 0, total_b = 0;
+    if (ctx->scratch[slot] && ctx->scratch_bytes[slot] < nbytes && hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b + ctx->scratch_bytes[slot] < nbytes)
+        return CERA_HIP_OK;
     const cera_hip_status st = cera_scratch(ctx, slot, nbytes, out);
     if (st != CERA_HIP_ERR_OOM) return st;
     (void)hipGetLastError();   // or the next launch would report it

@@ -722,8 +722,54 @@ static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_
     }
     return 0;
 }
-extern "C" uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu) {
-    return DENSE_BM[dense_shape(rows, (k + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD, n, 1, n_cu)];
+// How a product is cut: its tile, the parts of K, and whether its sums go through the reduction.
+struct DensePlan {
+    int shape;
+    uint32_t split;
+    bool apart;   // even if K is whole
+    bool wide;    // 256 x 256 tiles by dense_wide_parts
+    uint64_t sums(uint64_t m, uint64_t n) const { return split > 1 || apart ? split * n * m * sizeof(float) : 0; }   // bytes of partial sums
+};
+// streams: of DENSE_STREAMS, else 0.  wide: 256 x 256 tiles may take streams in parts of K
+static DensePlan dense_plan(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uint32_t streams, bool f32, bool wide, uint32_t n_cu) {
+    DensePlan p{f32 ? 2 : dense_shape(m, kp, n, groups, n_cu), 1, false, false};
+    const uint64_t bm = f32 ? 64 : DENSE_BM[p.shape], bn = f32 ? 64 : DENSE_BN[p.shape], wgs = (m + bm - 1) / bm * ((n + bn - 1) / bn) * groups;
+    const uint32_t steps = static_cast<uint32_t>(kp / DENSE_PAD);
+    // two workgroups per CU; three quarters of that are left alone on large tiles, whose partial sums cost more than the idle
+    // quarter: 3072 x 3072 times 2048 tokens (384) 51 us whole, 50 + 24 in two parts
+    const uint32_t want_wgs = 2 * n_cu;
+    if (p.shape != 3 && wgs * 4 < want_wgs * (p.shape == 0 ? 3ull : 4ull) && groups == 1) p.split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
+    if (p.split < 1) p.split = 1;
+    // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
+    // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
+    p.apart = streams && (streams != 4 || p.shape == 0 || p.shape == 3);
+    if (const uint32_t parts = wide && p.apart && p.shape == 0 ? dense_wide_parts(m, n, steps, wgs, p.split, n_cu) : 0) {
+        p.shape = 3;
+        p.split = parts;
+        p.wide = true;
+    }
+    const uint32_t per = (steps + p.split - 1) / p.split;
+    p.split = (steps + per - 1) / per;
+    return p;
+}
+// The same for what there is room for, room(bytes) saying so.  Where the larger tiles' parts do not fit, the smaller tiles', which may
+// be fewer; without room for those either, the whole of K in one workgroup, four streams by small tiles' own lanes.
+template <class Room> static DensePlan dense_plan_in(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uint32_t streams, bool f32, uint32_t n_cu, Room&& room) {
+    DensePlan p = dense_plan(m, kp, n, groups, streams, f32, true, n_cu);
+    if (!p.sums(m, n) || room(p.sums(m, n))) return p;
+    if (p.wide) {
+        p = dense_plan(m, kp, n, groups, streams, f32, false, n_cu);
+        if (room(p.sums(m, n))) return p;
+    }
+    p.split = 1;
+    if (p.apart && streams == 4) { p.shape = 1; p.apart = false; }
+    return p;
+}
+extern "C" uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu) { return DENSE_BM[dense_shape(rows, dense_pad(k), n, 1, n_cu)]; }
+extern "C" uint32_t cera_hip_dense_streams_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t streams, uint64_t room, uint32_t n_cu, uint32_t* parts) {
+    const DensePlan p = dense_plan_in(rows, dense_pad(k), n, 1, streams, false, n_cu, [&](uint64_t bytes) { return bytes <= room; });
+    if (parts) *parts = p.split;
+    return DENSE_BM[p.shape];
 }
 
 cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, const void* x, uint64_t ldx, uint32_t n,
@@ -741,37 +787,17 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     if (o.streams) a.st = *o.streams;
     a.epi = o.epi; a.out = o.out; a.ldo = o.ld; a.bias = o.bias; a.mult = o.mult; a.out_rows = o.rows;
     // tile: large where it fills the chip, else smaller, else K is split
-    int shape = f32 ? 2 : dense_shape(a.m, a.kp, n, groups.count, ctx->n_cu);
-    uint32_t bm = f32 ? 64 : DENSE_BM[shape], bn = f32 ? 64 : DENSE_BN[shape];
-    const uint64_t wgs = static_cast<uint64_t>((a.m + bm - 1) / bm) * ((n + bn - 1) / bn) * groups.count;
-    const uint32_t steps = a.kp / DENSE_PAD;
-    uint32_t split = 1;
-    // two workgroups per CU; three quarters of that are left alone on large tiles, whose partial sums cost more than the idle
-    // quarter: 3072 x 3072 times 2048 tokens (384) 51 us whole, 50 + 24 in two parts
-    const uint32_t want_wgs = 2 * ctx->n_cu;
-    if (shape != 3 && wgs * 4 < want_wgs * (shape == 0 ? 3ull : 4ull) && groups.count == 1) split = static_cast<uint32_t>(std::min<uint64_t>({(want_wgs + wgs - 1) / wgs, steps / 4, 16}));
-    if (split < 1) split = 1;
-    // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
-    // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
-    const bool apart = o.epi == DENSE_STREAMS && (o.streams->count != 4 || shape == 0 || shape == 3);
-    if (const uint32_t parts = apart && shape == 0 ? dense_wide_parts(a.m, n, steps, wgs, split, ctx->n_cu) : 0) {
-        shape = 3;
-        bm = bn = 256;
-        split = parts;
-    }
-    const uint32_t per = (steps + split - 1) / split;
-    split = (steps + per - 1) / per;
-    if (split > 1 || apart) {
-        void* part = nullptr;
-        CERA_TRY(cera_scratch_if_room(ctx, 9, static_cast<uint64_t>(split) * n * a.m * sizeof(float), &part));
-        // without room: the whole of K in one workgroup, four streams by small tiles' own lanes
-        if (!part) {
-            split = 1;
-            if (apart && o.streams->count != 4) CERA_TRY(cera_scratch(ctx, 9, static_cast<uint64_t>(n) * a.m * sizeof(float), &part));
-            else if (apart) { shape = 1; bm = bn = 64; }
-        }
-        a.part = static_cast<float*>(part);
-    }
+    void* part = nullptr;
+    cera_hip_status st = CERA_HIP_OK;
+    const DensePlan plan = dense_plan_in(a.m, a.kp, n, groups.count, o.epi == DENSE_STREAMS ? o.streams->count : 0, f32, ctx->n_cu, [&](uint64_t bytes) {
+        st = cera_scratch_if_room(ctx, 9, bytes, &part);
+        return st != CERA_HIP_OK || part;
+    });
+    CERA_TRY(st);
+    if (!part && plan.apart) CERA_TRY(cera_scratch(ctx, 9, plan.sums(a.m, n), &part));
+    a.part = static_cast<float*>(part);
+    const int shape = plan.shape;
+    const uint32_t split = plan.split, steps = a.kp / DENSE_PAD, bm = f32 ? 64 : DENSE_BM[shape], bn = f32 ? 64 : DENSE_BN[shape];
     a.k_chunk = (steps + split - 1) / split * DENSE_PAD;
     a.tiles_m = (a.m + bm - 1) / bm;
     a.tiles_n = (n + bn - 1) / bn;

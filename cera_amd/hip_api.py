@@ -35,7 +35,7 @@ SYMBOLS = [
     "cera_hip_set_reference_order", "cera_hip_reference_order",
     "cera_hip_rmsnorm_q8_0", "cera_hip_attn_decode_step", "cera_hip_attn_decode_dev_noalloc", "cera_hip_gemm_block_dots",
     "cera_hip_ffn_gate_up_fused", "cera_hip_qkv_fused",
-    "cera_hip_layered_create", "cera_hip_dense_tile", "cera_hip_read_conv", "cera_hip_write_conv",
+    "cera_hip_layered_create", "cera_hip_dense_tile", "cera_hip_dense_streams_tile", "cera_hip_read_conv", "cera_hip_write_conv",
 ]
 
 
@@ -188,6 +188,7 @@ def load_library() -> C.CDLL:
         "cera_hip_gemm_block_dots": (i32, [vp, C.POINTER(Tensor), vp, u64, vp, vp]),
         "cera_hip_layered_create": (i32, [vp, C.POINTER(LayeredConfig), C.POINTER(LayeredLayer), pp]),
         "cera_hip_dense_tile": (u32, [u64, u64, u32, u32]),
+        "cera_hip_dense_streams_tile": (u32, [u64, u64, u32, u32, u64, u32, C.POINTER(u32)]),
         "cera_hip_read_conv": (i32, [vp, u32, vp]), "cera_hip_write_conv": (i32, [vp, u32, vp, u32]),
         "cera_hip_rmsnorm_q8_0": (i32, [vp, vp, vp, u64, f32, vp, vp, vp]),
         "cera_hip_attn_decode_step": (i32, [vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, f32, u32, vp, f32, u32,
@@ -237,6 +238,12 @@ def decode_copy_plan(copy_bytes, free_bytes: int, reserve_bytes: int):
 def dense_tile(rows: int, k: int, n: int, n_cu: int = 256) -> int:
     """Weight rows of the tile that a bf16 product [rows][k] times n tokens takes (plain arithmetic, no GPU)."""
     return int(load_library().cera_hip_dense_tile(rows, k, n, n_cu))
+
+
+def dense_streams_tile(rows: int, k: int, n: int, streams: int, room: int = 1 << 62, n_cu: int = 256):
+    """(weight rows of the tile, parts of K) of a product that updates residual streams, with room for that many bytes of partial sums."""
+    parts = C.c_uint32()
+    return int(load_library().cera_hip_dense_streams_tile(rows, k, n, streams, room, n_cu, C.byref(parts))), parts.value
 
 
 def make_tensor(ggml_type: int, m: int, k: int, blocks: np.ndarray) -> Tensor:

@@ -115,7 +115,7 @@ CERA_HIP_API cera_hip_status cera_hip_ctx_set_decode_copies(cera_hip_ctx* ctx, i
  * results, which a context holds apart, are not counted).  A call that
  * cannot do without more fails with CERA_HIP_ERR_OOM, as it does where the device has no more memory; one
  * that is only faster with it (key and value tiles of a large attention batch laid out once, sums over
- * parts of K) runs without it.  Workspaces that are already larger stay. */
+ * parts of K) runs without it, or with fewer parts; its sums then have another order.  Workspaces that are already larger stay. */
 CERA_HIP_API cera_hip_status cera_hip_ctx_set_workspace_limit(cera_hip_ctx* ctx, uint64_t bytes);
 /* The rule by which cera_hip_model_create hands out decode copies, as plain arithmetic (no device
  * is touched; callable without a GPU).  A model's copies are built last -- after every native
@@ -550,6 +550,9 @@ CERA_HIP_API cera_hip_status cera_hip_layered_create(cera_hip_ctx*, const cera_h
 /* The rule by which a bf16 product [rows][k] times n tokens of such a model takes its tile, as plain arithmetic (no device
  * is touched): weight rows of the tile -- 256 (times 256 tokens), 128 (128) or 64 (64 or 32) -- on a device of n_cu CUs. */
 CERA_HIP_API uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu);
+/* The same for a product that updates `streams` residual streams, which may take larger tiles in parts of K: with room for
+ * `room` bytes of partial sums; *parts (nullable): the parts of K. */
+CERA_HIP_API uint32_t cera_hip_dense_streams_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t streams, uint64_t room, uint32_t n_cu, uint32_t* parts);
 CERA_HIP_API void cera_hip_model_destroy(cera_hip_model*);
 /* Model::forward (cera/src/model/mod.rs:200-606; LlamaModel::forward,
  * cera/src/model/llama.rs:1585-1605): one token at `pos` -> vocab logits.

@@ -738,6 +738,7 @@ pub fn cera_hip_ctx_create(
         out: *mut *mut cera_hip_model,
     ) -> cera_hip_status;
     pub fn cera_hip_dense_tile(rows: u64, k: u64, n: u32, n_cu: u32) -> u32;
+    pub fn cera_hip_dense_streams_tile(rows: u64, k: u64, n: u32, streams: u32, room: u64, n_cu: u32, parts: *mut u32) -> u32;
     pub fn cera_hip_set_seq_len(model: *mut cera_hip_model, len: u32) -> cera_hip_status;
     pub fn cera_hip_read_hidden(
         model: *mut cera_hip_model,

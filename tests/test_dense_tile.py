@@ -1,4 +1,4 @@
-"""The rule by which a bf16 product takes its tile (cera_hip_dense_tile): plain arithmetic, checked without a GPU."""
+"""The rules by which a bf16 product takes its tile (cera_hip_dense_tile, cera_hip_dense_streams_tile): plain arithmetic, checked without a GPU."""
 import pytest
 
 from cera_amd import hip_api
@@ -30,3 +30,20 @@ def test_the_largest_tiles_fill_their_rounds():
             assert got == (fills >= 0.55), (rows, n, fills)
             seen.add(got)
     assert seen == {True, False}
+
+
+@pytest.mark.parametrize("rows,k,n,streams,want", [(3072, 1030, 2040, 4, (256, 2)), (3000, 1100, 2047, 3, (256, 2)), (3072, 8200, 1010, 4, (256, 3)),
+                                                   (4096, 8300, 600, 2, (256, 4)), (3072, 64, 2048, 4, (128, 1)), (2048, 8192, 2048, 4, (128, 2)),
+                                                   (5200, 200, 1800, 4, (256, 1)), (2048, 2048, 40, 4, (64, 8)), (2048, 2048, 40, 3, (64, 8))])
+def test_tiles_of_streams(rows, k, n, streams, want):
+    assert hip_api.dense_streams_tile(rows, k, n, streams) == want
+
+
+@pytest.mark.parametrize("streams", [1, 3, 4])
+def test_streams_with_less_room_take_the_next_smaller_plan(streams):
+    """Two parts on 256 x 256 tiles; with room for one part's sums the 128 x 128 tiles, as if there were no larger ones; without, K whole,
+    four streams by small tiles."""
+    rows, k, n = 3072, 1030, 2048
+    one = rows * n * 4
+    for room, want in ((2 * one, (256, 2)), (2 * one - 1, (128, 1)), (one, (128, 1)), (one - 1, (64 if streams == 4 else 128, 1)), (0, (64 if streams == 4 else 128, 1))):
+        assert hip_api.dense_streams_tile(rows, k, n, streams, room) == want

@@ -353,11 +353,11 @@ def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):
     m.close()
 
 
-@pytest.mark.parametrize("width, ff, n, streams", [(3072, 1030, 1800, 4), (3000, 1100, 2047, 3), (3072, 8200, 1010, 4), (4096, 8300, 600, 2)])
-def test_streams_on_the_widest_tiles_in_parts_of_k(tmp_path, width, ff, n, streams):
+@pytest.mark.parametrize("width, ff, n, streams, parts", [(3072, 1030, 1800, 4, 2), (3000, 1100, 2047, 3, 2), (3072, 8200, 1010, 4, 3), (4096, 8300, 600, 2, 4)])
+def test_streams_on_the_widest_tiles_in_parts_of_k(tmp_path, width, ff, n, streams, parts):
     """The residual streams' products whose 256 x 256 tiles fill their rounds in two, three and four parts of K only: uneven parts, ragged
     last tiles of rows and tokens.  Tolerance: the operands', as everywhere here."""
-    assert hip_api.dense_tile(width, ff, n) == 128
+    assert hip_api.dense_streams_tile(width, ff, n, streams) == (256, parts)
     cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=ff)], width=width, vocab=64, streams=streams)
     w = U.random_model(cfg, 61)
     m = _open(U.save(tmp_path / "m", cfg, w), False, n)
@@ -386,6 +386,33 @@ def test_streams_of_large_tiles_without_room_for_partial_sums():
         ctx.close()
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
     assert U.rel(out[1], U.reference(cfg, w, toks)) < TOL[False]
+
+
+@pytest.mark.parametrize("streams", [3, 4])
+def test_streams_with_room_for_fewer_partial_sums(streams):
+    """Two parts on 256 x 256 tiles, then (here by limits) room for the sums of one, and for none: the smaller tiles with K whole, whose
+    sums have one order whoever stores them."""
+    width, ff, n = 3072, 1030, 2040
+    cfg = U.config([U.attention(2, 1, 32, 32, (0.1, 200), True, ff=ff)], width=width, vocab=64, streams=streams)
+    w = U.random_model(cfg, 71)
+    bits = {name: U.bf16_bits(a) if a.ndim == 2 and ".hc" not in name else a for name, a in w.items()}
+    toks = U.tokens(cfg, n, 5)
+    want, out = U.reference(cfg, w, toks), []
+    for limit, tile in ((0, (256, 2)), (40 << 20, (128, 1)), (16 << 20, (64, 1))):   # the sums of one part are 25 MB
+        if streams == 3 and tile[0] == 64:
+            continue    # three streams cannot do without the sums of one
+        assert hip_api.dense_streams_tile(width, ff, n, streams, limit or 1 << 62) == tile
+        ctx = hip_api.Context(0)
+        ctx.set_workspace_limit(limit)
+        m = hip_api.LayeredModel(ctx, cfg, bits, n)
+        out.append(m.forward_prefill_logits_all(np.asarray(toks, np.uint32), 0))
+        err = U.rel(out[-1], want)
+        print(f"streams={streams} limit {limit}: {err:.2e}", flush=True)
+        assert err < TOL[False]
+        m.close()
+        ctx.close()
+    for a in out[2:]:
+        assert np.array_equal(out[1].view(np.uint32), a.view(np.uint32))
 
 
 @DTYPES
