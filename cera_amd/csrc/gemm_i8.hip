@@ -103,10 +103,10 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
         for (int j = 0; j < T / 2; ++j) lds_dma_1k(xq + part * 64, xoff[j], act_lds + buf * (T * 2048) + j * 1024);
         lds_dma_256(xs + part * 2, xs_off, acs_lds + buf * (T * 256));
     };
-    auto weights = [&](uint32_t h, int s) {   // half super-block h
+    auto weights = [&](uint32_t h, uint32_t to, int s) {   // half super-block h
         const uint8_t* const b = (s ? base1 : base0) + (h >> 1) * W::SB + (h & 1) * (W::SB / 2 - W::START);
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j) lds_dma_1k(b, woff[s][j], wts_lds + (h & 1) * BUF + s * HALF16 + j * 1024);
+        for (int j = 0; j < LOADS; ++j) lds_dma_1k(b, woff[s][j], wts_lds + to * BUF + s * HALF16 + j * 1024);
     };
     float acc[T][16];
 #pragma unroll
@@ -121,15 +121,16 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
     f32x zero;
 #pragma unroll
     for (int e = 0; e < 32; ++e) zero[e] = 0.0f;
-    weights(2 * sb0, 0);
-    weights(2 * sb0, 1);
+    weights(2 * sb0, 0, 0);
+    weights(2 * sb0, 0, 1);
     tokens(4 * sb0, 0);
     uint32_t buf = 0;
     auto part = [&](uint32_t sb, auto q_) {   // a quarter of a super-block: two blocks
         constexpr uint32_t q = decltype(q_)::value, odd = q >> 1, z = 2 * (q & 1);
         // this part's tokens and rows are in, and no wavefront reads the other buffers any more
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const uint32_t next = min(sb * 4 + q + 1, sb1 * 4 - 1), next_half = min(sb * 2 + odd + 1, sb1 * 2 - 1);   // the last ones once more: no branch
+        // into the buffers that nobody reads now.  Behind the last ones these are the last ones once more: no branch
+        const uint32_t next = min(sb * 4 + q + 1, sb1 * 4 - 1), next_half = min(sb * 2 + odd + 1, sb1 * 2 - 1);
         const uint8_t *const xl = act[buf] + col * 64, *const sl = acs[buf] + lane * 4, *const wr = my_row + odd * (BUF + W::START);
         i4x a[2], x[2][2];
         float ts[2];
@@ -158,8 +159,8 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
             __builtin_amdgcn_sched_barrier(0);
             if (!(i & 1) && t + 1 < T) read(t + 1);
             if (i == 1) tokens(next, buf ^ 1);
-            if ((q & 1) == 0 && i == 2) weights(next_half, 0);
-            if ((q & 1) == 0 && i == 3) weights(next_half, 1);
+            if ((q & 1) == 0 && i == 2) weights(next_half, odd ^ 1, 0);
+            if ((q & 1) == 0 && i == 3) weights(next_half, odd ^ 1, 1);
             __builtin_amdgcn_sched_barrier(0);
             const f16x f = __builtin_bit_cast(f16x, r[i & 1]);
 #pragma unroll
