@@ -342,6 +342,9 @@ __global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a, uint32_t 
                     const uint32_t k = kb + (i >> 3) * 32 + g * 8 + (i & 7);
                     sc[ct][i >> 2][i & 3] = k >= col.lo[ct] && k <= col.hi[ct] ? sc[ct][i >> 2][i & 3] : -__builtin_inff();
                 }
+        // a half that no column sees has weights of 0 only: they take the other half's values, since its own rows may be what a longer
+        // sequence has left, infinities among them
+        const uint32_t from[2] = {kb + 31 < col.lo_min ? 4u : 0u, kb + 32 > col.hi_max ? 0u : 4u};
         bf16x8 ph[CT][2], pl[CT][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -356,7 +359,7 @@ __global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a, uint32_t 
                 }
 #pragma unroll
             for (int vt = 0; vt < VT; ++vt) {
-                const bf16x8 v = *reinterpret_cast<const bf16x8*>(base + v0 + vt * 2048 + ((4 * h + g) ^ (r & 7)) * 16);
+                const bf16x8 v = *reinterpret_cast<const bf16x8*>(base + v0 + vt * 2048 + ((from[h] + g) ^ (r & 7)) * 16);
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct) {
                     o[ct][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, ph[ct][h], o[ct][vt], 0, 0, 0);

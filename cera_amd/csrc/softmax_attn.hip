@@ -100,9 +100,9 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
             if ((EXACT || kd < nk) && live) q[ct][kd] = *reinterpret_cast<const bf16x8*>(row + kd * 32 + g * 8);
         }
     }
-    // lds: the block's rows; hi: last visible key of the lane's column; inside: every key is visible to every column
+    // lds: the block's rows; hi: last visible key of the lane's column, hi_max: of any; inside: every key is visible to every column
     __device__ __forceinline__ void run(const __bf16* lds, uint32_t row, uint32_t v_off, uint32_t kb, int nk, int nv, const uint32_t (&hi)[CT],
-                                        bool inside, float scale2, Column<MV> (&col)[CT], uint32_t lane) {
+                                        uint32_t hi_max, bool inside, float scale2, Column<MV> (&col)[CT], uint32_t lane) {
         const uint32_t r = lane & 15, g = lane >> 4;
         const char* const base = reinterpret_cast<const char*>(lds);
         const uint32_t ka = (r >> 2) * 8 + (r & 3), e = (g ^ swz(ka)) * 16;
@@ -152,11 +152,14 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
         typedef short s16x4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
 #pragma unroll
-        for (int h = 0; h < H; ++h)
+        for (int h = 0; h < H; ++h) {
+            // a half that no column sees has weights of 0 only: they take the first half's values, since its own rows may be what a
+            // longer sequence has left, infinities among them
+            const uint32_t rows = h == 0 || kb + 32 > hi_max ? 0 : 64 * row;
 #pragma unroll
             for (int vt = 0; vt < MV; ++vt)
                 if (EXACT || vt < nv) {
-                    const uint32_t off = (vt >> 2) * 128 + h * 64 * row, el = ev ^ ((vt & 3) << 5);
+                    const uint32_t off = (vt >> 2) * 128 + rows, el = ev ^ ((vt & 3) << 5);
                     const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v0 + off + el)));
                     const bf16x4 up = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(v1 + off + (el ^ 64))));
                     const bf16x8 v = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -166,6 +169,7 @@ template <int MK, int MV, int CT, int H, bool EXACT> struct Block<__bf16, MK, MV
                         col[ct].o[vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pl[ct][h], col[ct].o[vt], 0, 0, 0);
                     }
                 }
+        }
     }
 };
 
@@ -182,7 +186,7 @@ template <int MK, int MV, int CT, bool EXACT> struct Block<float, MK, MV, CT, 1,
         }
     }
     __device__ __forceinline__ void run(const float* lds, uint32_t row, uint32_t v_off, uint32_t kb, int nk, int nv, const uint32_t (&hi)[CT],
-                                        bool inside, float scale2, Column<MV> (&col)[CT], uint32_t lane) {
+                                        uint32_t, bool inside, float scale2, Column<MV> (&col)[CT], uint32_t lane) {
         const uint32_t r = lane & 15, g = lane >> 4;
         for (uint32_t h = 0; h < 32; h += 16) {
             const float* const k0 = lds + (h + r) * row;
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(FW * 64, WPE) void fattn_kernel(FArgs a) {
         __syncthreads();
         if (a.stages == 2 && b + a.kg < last) stage(b + a.kg, buf ^ 1);
         if (b < last && wave_live && b * BLOCK <= hi_max)
-            t.run(reinterpret_cast<const T*>(smem + (buf * a.kg + kgi) * block_bytes), a.row, a.v_off + vc0, b * BLOCK, nk, nv, hi, b * BLOCK + BLOCK - 1 <= hi_min,
+            t.run(reinterpret_cast<const T*>(smem + (buf * a.kg + kgi) * block_bytes), a.row, a.v_off + vc0, b * BLOCK, nk, nv, hi, hi_max, b * BLOCK + BLOCK - 1 <= hi_min,
                   a.scale2, col, lane);
         if (a.stages == 2) {
             buf ^= 1;

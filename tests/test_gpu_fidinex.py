@@ -337,6 +337,28 @@ def test_attention_in_blocks_of_64_keys(tmp_path, layer, n, cuts):
     m.close()
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim", [(32, 8, 64), (30, 10, 128)])
+def test_rows_that_no_query_of_a_half_block_sees_are_not_read(hip, heads, kv_heads, dim):
+    """Values that are not finite, left 32 rows and more behind the last position by a longer sequence: outputs do not depend on them."""
+    start, n = 40, 1124                                         # positions 40 .. 1163: the last block's rows 1152 .. 1215, halves at 1184
+    assert n * heads >= 128 * 256
+    cfg = U.config([U.attention(heads, kv_heads, dim, dim)], width=64, vocab=40, streams=2)
+    w = U.random_model(cfg, 57)
+    toks = np.asarray(U.tokens(cfg, start + n, 3), np.uint32)
+    r, out = np.random.default_rng(1), []
+    k, v = r.standard_normal((2, start + n + 64, kv_heads * dim)).astype(np.float32)
+    for bad in (0.0, np.nan, np.inf):
+        m = hip_api.LayeredModel(hip, cfg, U.as_arrays(w), start + n + 64)
+        m.forward_prefill(toks[:start], 0)
+        v[1184:] = bad
+        hip.check(hip.lib.cera_hip_write_kv(m.h, 0, k.ctypes.data, v.ctypes.data, len(k)))
+        out.append(m.forward_prefill_logits_all(toks[start:], start))
+        m.close()
+    assert np.isfinite(out[0]).all()
+    for a in out[1:]:
+        assert np.array_equal(out[0].view(np.uint32), a.view(np.uint32))
+
+
 @pytest.mark.parametrize("width, ff, n, streams", [(70, 32768, 300, 2), (130, 5200, 1800, 2), (200, 5300, 1777, 1), (260, 32700, 287, 2),
                                                    (5200, 64, 1800, 4), (5200, 130, 1800, 3), (5203, 200, 1799, 4), (5200, 330, 1800, 2)])
 def test_products_on_the_widest_tiles(tmp_path, width, ff, n, streams):

@@ -305,6 +305,30 @@ def test_attention_with_keys_and_values_shared_in_lds(tmp_path, heads, kv_heads,
     m.close()
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim", [(8, 4, 128), (32, 8, 64), (32, 32, 128)])
+def test_rows_that_no_query_of_a_half_block_sees_are_not_read(hip, heads, kv_heads, dim):
+    """Values that are not finite, left 32 rows and more behind the last position by a longer sequence, and in front of the first chunk's
+    end by an earlier one: outputs do not depend on them, with one and with two tiles of columns a wavefront."""
+    chunk, start, n = 96, 100, 1080                             # positions 100 .. 1179: the last block's rows 1152 .. 1215, halves at 1184
+    assert (start + n) % 64 <= 28 and n * heads >= 16 * 512
+    cfg = U.config([U.attention(heads, kv_heads, dim, dim, chunk, dim, 10000.0)], width=64, vocab=40, taps=2, positions=start + n + 64)
+    w = R.random_model(cfg, 57)
+    raw = {k: (v if k.endswith(R_VECTORS) else U.bf16_bits(v)) for k, v in w.items()}
+    toks = np.asarray(U.tokens(cfg, start + n, 3), np.uint32)
+    r, out = np.random.default_rng(1), []
+    k, v = r.standard_normal((2, start + n + 64, kv_heads * dim)).astype(np.float32)
+    for bad in (0.0, np.nan, np.inf):
+        m = hip_api.LayeredModel(hip, cfg, raw, start + n + 64)
+        m.forward_prefill(toks[:start], 0)
+        v[:chunk], v[1184:] = bad, bad
+        hip.check(hip.lib.cera_hip_write_kv(m.h, 0, k.ctypes.data, v.ctypes.data, len(k)))
+        out.append(m.forward_prefill_logits_all(toks[start:], start))
+        m.close()
+    assert np.isfinite(out[0]).all()
+    for a in out[1:]:
+        assert np.array_equal(out[0].view(np.uint32), a.view(np.uint32))
+
+
 @pytest.mark.parametrize("width, ff, n, vocab", [(60, 16384, 300, 64), (130, 2600, 1800, 64), (200, 16300, 290, 64), (260, 2700, 1777, 64),
                                                  (330, 64, 1800, 5203), (5200, 64, 1800, 64), (5201, 200, 1799, 64)])
 def test_products_on_the_widest_tiles(tmp_path, width, ff, n, vocab):
