@@ -164,7 +164,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
         grid.z = split;
     }
     if (dbg_dots) {
-        // the same kernels, compiled to also store every block's integer tile (no K split, no pair)
+        // compiled to also store every block's integer tile (no K split, no pair)
         switch (w->dtype) {
             case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, true>), grid, dim3(256), 0, ctx->stream, a); break;
             case CERA_HIP_Q6_K: hipLaunchKernelGGL(gemm_q6k_f16_kernel<true>, grid, dim3(256), 0, ctx->stream, a); break;
@@ -298,8 +298,8 @@ extern "C" cera_hip_status cera_hip_gemm(cera_hip_ctx* ctx, const cera_hip_tenso
     return st;
 }
 
-// The GEMM's integer block dots as the matrix cores deliver them (debug instances of the same
-// kernels, for Q6_K of the one for up to 64 tokens): dots [m][n][k/32] int32 -- Q4_0 sum (q-8)a, Q8_0 sum w a, Q4_1 / Q4_K sum q a -- and
+// The GEMM's integer block dots as the matrix cores deliver them (debug instances of the kernels that products run; for Q6_K of
+// the one for up to 64 tokens, for Q4_0 and Q8_0 of the one that gemm_i8.hip leaves the longest rows): dots [m][n][k/32] int32 -- Q4_0 sum (q-8)a, Q8_0 sum w a, Q4_1 / Q4_K sum q a -- and
 // for Q6_K [m][n][k/16], each the f32 result of the f16 MFMA for one 16-element scale group,
 // sum (q-32)a, returned as f32 so that a test can see it is an exact integer.  out (nullable)
 // receives the float result of the same launch.

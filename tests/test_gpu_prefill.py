@@ -186,23 +186,24 @@ def test_gemm_of_32_weight_blocks(hip, orc, dtype, bytes_, ma, mb, n, k):
 
 
 @pytest.mark.parametrize("dtype,m,k,n", [(Q4_K, 132, 2304, 5), (Q4_K, 300, 4096, 48), (Q6_K, 132, 2304, 3), (Q6_K, 300, 4096, 33),
-                                         (Q6_K, 300, 4096, 160), (Q6_K, 516, 2304, 384)])
+                                         (Q6_K, 300, 4096, 160), (Q6_K, 516, 2304, 384), (Q8_0, 132, 2304, 9), (Q8_0, 300, 4096, 64), (Q8_0, 516, 2304, 200),
+                                         (Q4_0, 132, 2304, 9), (Q4_0, 300, 4096, 64), (Q4_0, 516, 2304, 200)])
 def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
     """The products of a few and of many tokens in the kernels that passes run: tokens of a single block each and scales
     that are powers of two leave one block's whole number in every output, so any rounding on the way would show.  Weights
     of random bytes take the whole range; the last row's scales and codes and the first token's quants are the largest, 32
-    of -128 * -32 * 127 for Q6_K, 1 % below 2^24."""
+    of -128 * -32 * 127 for Q6_K, 1 % below 2^24, and of -128 * 127 for Q8_0, whose sums leave the matrix cores as floats."""
     _say(f"whole numbers {util.NAMES[dtype]} m={m} k={k} n={n}")
     r = util.rng(m + n)
-    bytes_ = 144 if dtype == Q4_K else 210
+    bytes_ = {Q4_K: 144, Q6_K: 210, Q8_0: 8 * 34, Q4_0: 8 * 18}[dtype]
     w = r.integers(0, 256, (m, k // 256, bytes_), dtype=np.uint8)
-    w[-1] = 255 if dtype == Q4_K else 0     # the largest scales, mins and codes; for Q6_K code 0 is -32
+    w[-1] = {Q4_K: 255, Q6_K: 0, Q8_0: 128, Q4_0: 0}[dtype]     # the largest scales, mins and codes; for Q6_K code 0 is -32, for Q4_0 -8
     if dtype == Q6_K:
         w[-1, :, 192:208] = 128
     d = np.exp2(r.integers(-12, -5, (m, k // 256, 1))).astype(np.float16).view(np.uint8)
     if dtype == Q4_K:
         w[:, :, 0:2], w[:, :, 2:4] = d, d
-    else:
+    elif dtype == Q6_K:
         w[:, :, 208:210] = d
     x = np.zeros((n, k // 32, 32), np.float32)
     for t in range(n):
@@ -222,6 +223,8 @@ def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
         assert np.array_equal(hip.gemm(dtype, w.reshape(-1), x, m, n, k).reshape(m, n).T, want)
 
 
+    else:
+        w.reshape(m, k // 32, -1)[:, :, :2] = np.exp2(r.integers(-12, -5, (m, k // 32, 1))).astype(np.float16).view(np.uint8)
 @pytest.mark.parametrize("dtype,n,m,k,limit", [(Q4_K, 48, 4096, 2048, 2 << 20), (Q6_K, 5, 4096, 2048, 1 << 18), (Q6_K, 128, 4096, 2048, 4 << 20)])
 def test_products_without_room_for_partial_sums(dtype, n, m, k, limit):
     """Sums over parts of K are a workspace that a product can do without: where it cannot be had (here by a limit that the
@@ -845,7 +848,8 @@ def test_gemm_integer_block_dots_bit_exact(hip, orc, dtype, m, n, k):
     """Every (row, token, block) integer dot the matrix cores produce inside the prefill GEMM equals
     the brute-force integer reference (the quantities of simd.rs:6609-6629): int32 tiles of the
     int8 MFMA for Q4_0 / Q8_0 / Q4_1 / Q4_K, and for Q6_K the f32 results of the f16 MFMA, one per
-    16-element scale group, which must be exact integers sum (q - 32) a."""
+    16-element scale group, which must be exact integers sum (q - 32) a.  Products of Q4_0, Q8_0 and, with many
+    tokens, Q6_K run other kernels: test_block_results_are_whole_numbers reads theirs from the outputs."""
     _say(f"gemm block dots {util.NAMES[dtype]} m={m} n={n} k={k}")
     w, _ = util.make_weights(dtype, m, k, seed=dtype + m)
     x = util.rng(n + k).standard_normal((n, k)).astype(np.float32) * np.float32(3.0)
