@@ -20,7 +20,8 @@ struct I8Args {
     float *hs, *hbsum;
 };
 
-// What the kernel takes: rows in whole 16-byte pieces at a base aligned to them.
+// What the kernel takes: rows that 128 of a lane's 32-bit offsets reach, in whole 16-byte pieces at a base aligned to them (as every
+// matrix here has them).
 static inline bool i8_takes(const cera_hip_dtensor* w, const int8_t* xq) {
     return (w->dtype == CERA_HIP_Q8_0 || w->dtype == CERA_HIP_Q4_0) && w->k % 256 == 0 && w->row_bytes % 16 == 0 && w->row_bytes < (1u << 24) &&
            w->k < (1u << 24) && ((reinterpret_cast<uintptr_t>(w->dev) | reinterpret_cast<uintptr_t>(xq)) & 15) == 0;

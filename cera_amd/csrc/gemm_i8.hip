@@ -11,7 +11,7 @@
 //
 // What bounds it: one subtraction and one FMA per output and block, at the clocks that the power limit leaves (2.0 GHz); at
 // 28672 x 4096 Q8_0 with 2048 tokens 716 us, 672 TOP/s, of which the FMAs and matrix instructions alone take 615.  The kernel
-// before it (gemm.hip.h, which keeps Q4_1, rows that are not 16-byte aligned, the block dots and the code object's export)
+// before it (gemm.hip.h, which keeps Q4_1, rows of about 2^24 columns and more, the block dots and the code object's export)
 // unpacks into LDS, converts, and reads both operands through LDS.  Passes of two layers, before and now:
 //   hidden 3072, Q8_0:  9 tokens 272 -> 242 us, 64: 354 -> 307, 128: 456 -> 376, 512: 867 -> 639, 1001: 1321 -> 1049
 //   hidden 4096, Q4_0:  9 tokens 335 -> 302 us, 64: 451 -> 379, 128: 592 -> 477, 512: 1205 -> 973, 1001: 2046 -> 1671

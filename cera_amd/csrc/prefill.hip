@@ -73,7 +73,7 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
     const bool dense = ((ld_m == 1 && ld_n == a.m) || (ld_n == 1 && ld_m == n)) && (static_cast<uint64_t>(a.m) * n) % 4 == 0;
     // Q6_K with many tokens: gemm_kq.hip, in this many slices of K (0: not there)
     const uint32_t kq = dbg_dots || !dense ? 0 : kq_slices(w->dtype, a.m, pair ? w2->m : 0, n, a.k, ctx->n_cu);
-    // Q8_0 and Q4_0: gemm_i8.hip
+    // Q8_0 and Q4_0: gemm_i8.hip, but for rows of about 2^24 columns and more, whose offsets only gemm.hip.h holds
     const bool i8 = !dbg_dots && i8_takes(w, bq) && (!pair || i8_takes(w2, bq));
     // Q6_K runs its block dots on the f16 matrix cores and reads the quants as f16: converted here
     // unless the caller says its workspace (bh_ws) still holds these activations in that form (*staged)
@@ -203,8 +203,8 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
 
 // First half of the FFN in one launch: hq/hs/hbsum [n][m] = Q8_0(silu(gate.B) * (up.B)), the
 // activation of the down projection, quantized in the GEMM's epilogue.  *fused = false (nothing
-// launched) when the pair is not two int8-GEMM matrices of one shape or when the launch would
-// need a K split to fill the chip; the caller then takes the GEMM pair and the SwiGLU kernel.
+// launched) when the pair is not two int8-GEMM matrices of one shape or when it is better off with K in
+// parts; the caller then takes the GEMM pair and the SwiGLU kernel.
 cera_hip_status cera_launch_gemm_swiglu(cera_hip_ctx* ctx, const cera_hip_dtensor* gate, const cera_hip_dtensor* up,
                                         const float* bs, const int8_t* bq, const float* bsum, uint32_t n, int8_t* hq,
                                         float* hs, float* hbsum, bool* fused, void* b8_ws = nullptr, bool* staged8 = nullptr,
@@ -224,7 +224,14 @@ cera_hip_status cera_launch_gemm_swiglu(cera_hip_ctx* ctx, const cera_hip_dtenso
     a.hh = fp8 ? static_cast<uint16_t*>(hh_ws) : nullptr;
     const uint32_t BM = fp8 ? G8_BM : GEMM_BM, BN = fp8 ? G8_BN : GEMM_BN;
     const dim3 grid((n + BN - 1) / BN, (a.m + BM / 2 - 1) / (BM / 2));
+    // Two workgroups of 64 tokens a CU.  Q8_0 and Q4_0 then launch half as many, of 128 tokens, and are still better off whole, since a
+    // pair in parts pays for its sums and for the SwiGLU launch.  Passes of two layers, fused and as a pair: Q8_0, hidden 4096, ffn
+    // 14336, 192 tokens (448 workgroups on 256 CUs) 613 / 628 us; hidden 3072, ffn 8192, 384 tokens (384) 569 / 587; hidden 2048,
+    // ffn 4096, 449 tokens (256) 387 / 399; only where 256 of them walk a long K is the pair as good or better: hidden 3072, ffn 8192,
+    // 225 tokens 458 / 457, Q4_0, hidden 4096, ffn 8192, 200 tokens 495 / 481.
     if (grid.x * grid.y < 2 * ctx->n_cu) return CERA_HIP_OK;
+    const bool i8 = gate->dtype == CERA_HIP_Q8_0 || gate->dtype == CERA_HIP_Q4_0;
+    if (i8 && !(i8_takes(gate, bq) && i8_takes(up, bq))) return CERA_HIP_OK;
     if (fp8) {
         if (!b8_ws) {
             CERA_TRY(cera_scratch(ctx, 12, cera_gemm_fp8_ws_bytes(n, a.k), &b8_ws));
@@ -237,15 +244,11 @@ cera_hip_status cera_launch_gemm_swiglu(cera_hip_ctx* ctx, const cera_hip_dtenso
         }
         a.bf8 = static_cast<const uint8_t*>(b8_ws);
     }
-    if (i8_takes(gate, bq) && i8_takes(up, bq)) {
+    if (i8) {
         I8Args b{a.w, a.w2, bq, bs, nullptr, nullptr, a.m, a.m, n, a.k, a.row_bytes, 0, a.k, 0, 0, 0, 0, nullptr, 1.0f, hq, hs, hbsum};
         CERA_TRY(cera_launch_i8_swiglu(ctx, gate->dtype, b));
-    } else switch (gate->dtype) {
-        case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false>), grid, dim3(256), 0, ctx->stream, a); break;
-        case CERA_HIP_Q4_0: hipLaunchKernelGGL((gemm_kernel<GemmQ4_0, true>), grid, dim3(256), 0, ctx->stream, a); break;
-        case CERA_HIP_Q4_1: hipLaunchKernelGGL((gemm_kernel<GemmQ4_1, true>), grid, dim3(256), 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL((gemm_kernel<GemmQ8_0, true>), grid, dim3(256), 0, ctx->stream, a); break;
-    }
+    } else if (fp8) hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false>), grid, dim3(256), 0, ctx->stream, a);
+    else hipLaunchKernelGGL((gemm_kernel<GemmQ4_1, true>), grid, dim3(256), 0, ctx->stream, a);
     HIP_TRY(ctx, hipGetLastError());
     *fused = true;
     return CERA_HIP_OK;

@@ -185,6 +185,24 @@ def test_gemm_of_32_weight_blocks(hip, orc, dtype, bytes_, ma, mb, n, k):
         assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
 
 
+@pytest.mark.parametrize("dtype,bytes_", [(Q8_0, 34), (Q4_0, 18)])
+def test_gemm_of_rows_of_16_million_columns(hip, orc, dtype, bytes_):
+    """Rows that the kernel of the other Q8_0 and Q4_0 products has no offsets for.  A slice of K adds 2^16 blocks one after the other:
+    roundings of at most 2^-24 of sums that grow as a random walk come to 2^-24 * sqrt(2^16 / 6) of the output's rms; 2.5 times that."""
+    m, n, k = 4, 2, 1 << 24
+    _say(f"{util.NAMES[dtype]} m={m} k={k} n={n}")
+    r = util.rng(bytes_)
+    w = r.integers(0, 256, (m, k // 32, bytes_), dtype=np.uint8)
+    d = r.uniform(0.5, 2.0, (m, k // 32, 1)).astype(np.float32) * r.choice(np.float32([-1e-3, 1e-3]), (m, k // 32, 1))
+    w[:, :, :2] = d.astype(np.float16).view(np.uint8)
+    x = r.standard_normal((n, k), dtype=np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    wd = util.dequant_np(dtype, w.reshape(-1), m, k).astype(np.float64)
+    rms = np.sqrt((wd * wd).sum(1, keepdims=True) * (xd * xd).sum(1) / k)
+    assert (np.abs(hip.gemm(dtype, w.reshape(-1), x, m, n, k) - wd @ xd.T) / rms).max() <= 2.0 ** -16
+
+
 @pytest.mark.parametrize("dtype,m,k,n", [(Q4_K, 132, 2304, 5), (Q4_K, 300, 4096, 48), (Q6_K, 132, 2304, 3), (Q6_K, 300, 4096, 33),
                                          (Q6_K, 300, 4096, 160), (Q6_K, 516, 2304, 384), (Q8_0, 132, 2304, 9), (Q8_0, 300, 4096, 64), (Q8_0, 516, 2304, 200),
                                          (Q4_0, 132, 2304, 9), (Q4_0, 300, 4096, 64), (Q4_0, 516, 2304, 200)])
@@ -205,6 +223,8 @@ def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
         w[:, :, 0:2], w[:, :, 2:4] = d, d
     elif dtype == Q6_K:
         w[:, :, 208:210] = d
+    else:
+        w.reshape(m, k // 32, -1)[:, :, :2] = np.exp2(r.integers(-12, -5, (m, k // 32, 1))).astype(np.float16).view(np.uint8)
     x = np.zeros((n, k // 32, 32), np.float32)
     for t in range(n):
         q = r.integers(-127, 128, 32) if t else np.full(32, 127)
@@ -223,8 +243,6 @@ def test_block_results_are_whole_numbers(hip, dtype, m, k, n):
         assert np.array_equal(hip.gemm(dtype, w.reshape(-1), x, m, n, k).reshape(m, n).T, want)
 
 
-    else:
-        w.reshape(m, k // 32, -1)[:, :, :2] = np.exp2(r.integers(-12, -5, (m, k // 32, 1))).astype(np.float16).view(np.uint8)
 @pytest.mark.parametrize("dtype,n,m,k,limit", [(Q4_K, 48, 4096, 2048, 2 << 20), (Q6_K, 5, 4096, 2048, 1 << 18), (Q6_K, 128, 4096, 2048, 4 << 20)])
 def test_products_without_room_for_partial_sums(dtype, n, m, k, limit):
     """Sums over parts of K are a workspace that a product can do without: where it cannot be had (here by a limit that the
