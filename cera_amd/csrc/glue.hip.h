@@ -333,11 +333,25 @@ static __global__ __launch_bounds__(1024) void rmsnorm_few_kernel(const float* x
 // threads: blocks [0, n_heads) rotate q; the next n_kv_heads rotate k and
 // store it; the last n_kv_heads copy v.
 // KV cache layout: [kv_head][max_seq][head_dim] f32.
+// Split-K partial sums of q, k or v that this kernel adds up itself instead of a reduction launch in front
+// of it: value e = sum_z part[z * stride + e] in that order (n_split = 0: the rows are complete as they are).
+struct RopePending {
+    const float* part;
+    uint32_t n_split;
+    uint64_t stride;
+};
+__device__ __forceinline__ float rope_pending_ld(const float* rows, const RopePending& pd, uint64_t e) {
+    if (pd.n_split == 0) return rows[e];
+    float s = pd.part[e];
+    for (uint32_t z = 1; z < pd.n_split; ++z) s += pd.part[z * pd.stride + e];
+    return s;
+}
 template <typename KV>
 __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __restrict__ k, const float* v,
                                const float* __restrict__ cs_table, const uint32_t* __restrict__ pos_ptr,
                                uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
-                               KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq) {
+                               KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
+                               RopePending pq = RopePending{}, RopePending pk = RopePending{}, RopePending pv = RopePending{}) {
     // grid.y = tokens of a prefill batch: token t sits at position *pos_ptr + t and its
     // q/k/v rows follow each other ([n][n_heads*head_dim], [n][n_kv_heads*head_dim])
     const uint32_t pos = *pos_ptr + blockIdx.y;
@@ -350,7 +364,8 @@ __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __res
         float* head = rows + at;
         float2 cs = reinterpret_cast<const float2*>(cs_table)[static_cast<uint64_t>(pos) * half + i];
         uint32_t i0 = rope_type == 1 ? 2 * i : i, i1 = rope_type == 1 ? 2 * i + 1 : i + half;
-        float x0 = rows[at + i0], x1 = rows[at + i1];
+        const RopePending& pd = is_q ? pq : pk;
+        float x0 = rope_pending_ld(rows, pd, at + i0), x1 = rope_pending_ld(rows, pd, at + i1);
         float r0 = __fsub_rn(__fmul_rn(x0, cs.x), __fmul_rn(x1, cs.y));
         float r1 = __fadd_rn(__fmul_rn(x0, cs.y), __fmul_rn(x1, cs.x));
         head[i0] = r0;
@@ -363,8 +378,8 @@ __device__ __forceinline__ void rope_kv_body(float* __restrict__ q, float* __res
     } else if (v_cache) {
         uint32_t h = b - n_heads - n_kv_heads;
         KV* dst = v_cache + (static_cast<uint64_t>(h) * max_seq + pos) * head_dim;
-        dst[2 * i] = static_cast<KV>(v[kv_row + h * head_dim + 2 * i]);
-        dst[2 * i + 1] = static_cast<KV>(v[kv_row + h * head_dim + 2 * i + 1]);
+        dst[2 * i] = static_cast<KV>(rope_pending_ld(v, pv, kv_row + h * head_dim + 2 * i));
+        dst[2 * i + 1] = static_cast<KV>(rope_pending_ld(v, pv, kv_row + h * head_dim + 2 * i + 1));
     }
 }
 template <typename KV>
@@ -374,17 +389,22 @@ static __global__ void rope_kv_kernel(float* __restrict__ q, float* __restrict__
                                KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq) {
     rope_kv_body<KV>(q, k, v, cs_table, pos_ptr, n_heads, n_kv_heads, head_dim, rope_type, k_cache, v_cache, max_seq);
 }
-// Split-K partial sums of q, k or v that the kernel below adds up itself instead of a reduction launch in front
-// of it: value e = sum_z part[z * stride + e] in that order (n_split = 0: the rows are complete as they are).
-struct RopePending {
-    const float* part;
-    uint32_t n_split;
-    uint64_t stride;
-};
-// The same for a prompt's pass, which adds pending partial sums up: a thread takes a quad of a head's columns and the one head_dim / 2
-// further on, a few workgroups the heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by
-// bytes: 512 tokens of 32 + 8 + 8 heads of 128, K in two parts, 13.7 us, where one pair a
-// thread in workgroups of 64 took 23; 1001 tokens of 24 + 8 + 8: 15 and 21.
+// The same over q / k / v rows whose split-K partial sums are still pending.
+template <typename KV>
+static __global__ void rope_kv_pending_kernel(float* __restrict__ q, float* __restrict__ k, const float* v,
+                               const float* __restrict__ cs_table, const uint32_t* __restrict__ pos_ptr,
+                               uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
+                               KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
+                               RopePending pq, RopePending pk, RopePending pv) {
+    rope_kv_body<KV>(q, k, v, cs_table, pos_ptr, n_heads, n_kv_heads, head_dim, rope_type, k_cache, v_cache, max_seq, pq, pk, pv);
+}
+
+// The same for more than 64 tokens: a thread takes a quad of a head's columns and the one head_dim / 2 further on, 256 threads the
+// heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by bytes: 512 tokens of
+// 32 + 8 + 8 heads of 128, K in two parts, 13.7 us, where one pair a thread in workgroups of 64 takes 23; 1001 tokens of
+// 24 + 8 + 8: 15 and 21.  With fewer tokens the launch is a chain of loads, which one pair keeps shorter.  Passes of two layers by
+// pairs and by quads: 32 + 8 + 8 heads of 128: 45 tokens 318 / 320 us, 64: 433 / 438, 128: 539 / 538, 192: 653 / 645; 64 + 32 + 32 heads
+// of 64: 10 tokens 239 / 241, 65: 486 / 481.
 __device__ __forceinline__ float4 rope_pending_ld4(const float* rows, const RopePending& pd, uint64_t e) {
     if (pd.n_split == 0) return *reinterpret_cast<const float4*>(rows + e);
     float4 s = *reinterpret_cast<const float4*>(pd.part + e);
@@ -406,7 +426,7 @@ static __global__ __launch_bounds__(256) void rope_kv_quads_kernel(float* __rest
                                uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t rope_type,
                                KV* __restrict__ k_cache, KV* __restrict__ v_cache, uint32_t max_seq,
                                RopePending pq, RopePending pk, RopePending pv) {
-    const uint32_t quads = head_dim / 8, item = blockIdx.x * blockDim.x + threadIdx.x, b = item / quads, j = item - b * quads;
+    const uint32_t quads = head_dim / 8, item = blockIdx.x * 256 + threadIdx.x, b = item / quads, j = item - b * quads;
     if (b >= n_heads + 2 * n_kv_heads) return;
     const uint32_t pos = *pos_ptr + blockIdx.y;
     const uint64_t tok = blockIdx.y;

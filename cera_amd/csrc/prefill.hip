@@ -746,14 +746,17 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             const RopePending rq{pqk.part, pqk.n_split, pqk.stride};
             const RopePending rk{pqk.n_split ? pqk.part + static_cast<uint64_t>(n) * q_dim : nullptr, pqk.n_split, pqk.stride};
             const RopePending rv{pvv.part, pvv.n_split, pvv.stride};
-            // (heads come in whole eights of columns, so that rows and slices of partial sums start on whole quads.  A few tokens' chains
-            // of loads are spread over more CUs by workgroups of one wavefront.)
-            const uint32_t wg = n <= 64 ? 64 : 256;
             auto rope = [&](auto tag) {
                 using KV = decltype(tag);
-                hipLaunchKernelGGL(rope_kv_quads_kernel<KV>, dim3(((c.n_heads + 2 * c.n_kv_heads) * (c.head_dim / 8) + wg - 1) / wg, n), dim3(wg), 0, s,
-                                   m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads, c.head_dim,
-                                   c.rope_type, static_cast<KV*>(L.kc), static_cast<KV*>(L.vc), c.max_seq_len, rq, rk, rv);
+                auto go = [&](auto* fn, dim3 grid, uint32_t threads, auto... pending) {
+                    hipLaunchKernelGGL(fn, grid, dim3(threads), 0, s, m->pf_q, m->pf_k, m->pf_v, m->rope_table, m->scalars + 1, c.n_heads, c.n_kv_heads,
+                                       c.head_dim, c.rope_type, static_cast<KV*>(L.kc), static_cast<KV*>(L.vc), c.max_seq_len, pending...);
+                };
+                const uint32_t heads = c.n_heads + 2 * c.n_kv_heads;
+                // (heads come in whole eights of columns, so that rows and slices of partial sums start on whole quads)
+                if (n > 64) go(&rope_kv_quads_kernel<KV>, dim3((heads * (c.head_dim / 8) + 255) / 256, n), 256, rq, rk, rv);
+                else if (pqk.n_split || pvv.n_split) go(&rope_kv_pending_kernel<KV>, dim3(heads, n), c.head_dim / 2, rq, rk, rv);
+                else go(&rope_kv_kernel<KV>, dim3(heads, n), c.head_dim / 2);
             };
             if (m->kv_f16) rope(kv_half{});
             else rope(float{});
