@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
 // barrier a K step, in its middle: behind it the step's second half is in registers, so its buffer takes the K step after
 // next while that half is multiplied.  What bounds it: a K step is 2048 clocks of the matrix cores and 2048 of LDS (192 KB
 // read, 64 KB written at 128 bytes a clock); one workgroup alone takes 2660 for it, a full chip 3440, with the matrix cores busy
-// for 52 % of 28672 x 4096 times 1900 tokens (3.5 rounds).  28672 x 4096 times 2048 / 512 tokens: 1100 / 1040 TFLOP/s, 128 x 128
+// for 52 % of 28672 x 4096 times 1900 tokens in four rounds, and for 56 % with the last one by halves (below).  28672 x 4096 times 2048 / 512 tokens: 1100 / 1040 TFLOP/s, 128 x 128
 // tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
 // MI: 16-row tiles of a wavefront: 8, or 4 for 128 x 256 (row0: the workgroup's first weight row)
 constexpr int WIDE_BK = 64, WIDE_HALF = 256 * WIDE_BK, WIDE_BUF = 2 * WIDE_HALF;
@@ -373,7 +373,7 @@ template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_bo
 }
 // HALVES: the last round's tiles, at most half of one, go to twice as many workgroups of half their rows (of an XCD, those from
 // `whole` on; an instance of its own, since the others take 2 % longer with both bodies in one).  28672 x 4096 times 1900 tokens, 3.5
-// rounds: 389 us, 404 in four.
+// rounds: 382 us, 399 in four.
 template <int EPI, int SN, bool HALVES>
 __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
     __shared__ __align__(1024) __bf16 lds[2][WIDE_BUF];
@@ -708,11 +708,15 @@ static int dense_shape(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uin
     return n > 32 ? 1 : 2;
 }
 // Parts of K in which 256 x 256 tiles take a product whose sums go through the reduction anyway in place of 128 x 128 tiles with
-// `split` parts, or 0: the fewest, up to four of at least eight steps of 64, whose tiles are at least 55 % of their rounds, as
-// above, and fill theirs well enough: they multiply about 1.3 times as fast on a full chip, and 1.2 times has to be left.
-// Products and reductions of one layer's streams, before and now: 3072 x 8192 times 2048 tokens (384 tiles in a round of 512; 96 x 2
-// in 256) 140 + 47 -> 105 + 52 us, 3072 x 3072 62 + 47 -> 50 + 52; 2048 x 8192 and 2048 x 2048 (256 x 2 in 512; 64 x 3 in 256: left
-// alone) take 1.5 % longer over a whole pass on the larger tiles.
+// `split` parts, or 0: the fewest, up to four of at least eight steps of 64, whose tiles are at least 55 % of their rounds on the
+// fullest XCD, as above, if those rounds cost less.  A round of the larger tiles, one a CU, is twice the work of one of the smaller, two
+// a CU and counted over the chip, at about 1.3 times the rate: by that, they are 1.3 / 2 * parts * rounds128 / (split * rounds) times as
+// fast, and have to be 1.07 times so.  At 1792 to 4096 rows and 200 to 2048 tokens that comes to 1.3, 1.7 or 1.95, or to 0.98, which
+// stays.  Passes of two layers on the smaller tiles and by the rule: 1.3, 4096 wide, 1409 tokens (384 workgroups whole; 96 x 2) 1492 /
+// 1448 us, 3328 wide, 1459 (312 x 2; 78 x 2) 1276 / 1174, 4096 wide, 617 (160 x 4; 48 x 4) 909 / 872; 1.7, 3584 wide, 796 (196 x 3; 56 x 4)
+// 982 / 890; 1.95, 3584 wide, 1224 (280 x 2; 70 x 3) 1293 / 1100; 24 sizes in all, 2.3 to 15 % faster each.  2048 wide times 2048 tokens
+// (256 x 2; 64 x 3: 0.98) takes 1.5 % longer on the larger tiles.  Product and reduction alone: 3072 x 8192 times 2048 tokens
+// 140 + 47 -> 105 + 52 us, 3072 x 3072 62 + 47 -> 50 + 52.
 static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_t wgs, uint32_t split, uint32_t n_cu) {
     const uint64_t per_xcd = std::max<uint64_t>(n_cu / 8, 1), most = ((m + 255) / 256 + 7) / 8 * ((n + 255) / 256);
     const uint64_t rounds128 = (wgs * split + 2 * n_cu - 1) / (2 * n_cu);

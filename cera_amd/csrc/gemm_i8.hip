@@ -6,15 +6,15 @@
 // ahead; the tokens, 64 of k at a time, straight from their quants, row by row, with one barrier.  Nothing is staged through
 // registers and a Q8_0 code needs no unpacking.  The sums start from 1.5 * 2^23 as an integer, so that the matrix core's result,
 // read as a float, is that number plus the dot: a subtraction in place of the conversion, which the vector ALU issues at half
-// the rate (1.0 against 1.95 ns an instruction with two wavefronts a SIMD).  The product of the two scales is an outer product
-// on the matrix core, two blocks an instruction.
+// the rate.  The product of the two scales is an outer product on the matrix core, two blocks an instruction.  A slice of K adds its
+// blocks in the order of the kernel before it; the number of slices is i8_slices' own, so that sums in parts have another order.
 //
-// What bounds it: one subtraction and one FMA per output and block, at the clocks that the power limit leaves (2.0 GHz); at
-// 28672 x 4096 Q8_0 with 2048 tokens 716 us, 672 TOP/s, of which the FMAs and matrix instructions alone take 615.  The kernel
+// What bounds it: one subtraction and one FMA per output and block.  In 16384 x 3072 Q8_0 (gate | up) times 1001 tokens the vector
+// ALU is busy for 0.66 of the time and the matrix cores for 0.27, in turns; 28672 x 4096 times 2048 tokens 671 us, 717 TOP/s.  The kernel
 // before it (gemm.hip.h, which keeps Q4_1, rows of about 2^24 columns and more, the block dots and the code object's export)
 // unpacks into LDS, converts, and reads both operands through LDS.  Passes of two layers, before and now:
-//   hidden 3072, Q8_0:  9 tokens 272 -> 242 us, 64: 354 -> 307, 128: 456 -> 376, 512: 867 -> 639, 1001: 1321 -> 1049
-//   hidden 4096, Q4_0:  9 tokens 335 -> 302 us, 64: 451 -> 379, 128: 592 -> 477, 512: 1205 -> 973, 1001: 2046 -> 1671
+//   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039
+//   hidden 4096, Q4_0:  9 tokens 331 -> 300 us, 64: 440 -> 374, 128: 591 -> 477, 512: 1181 -> 947, 1001: 2055 -> 1673
 #include "f16_codes.hip.h"
 #include "gemm_i8.h"
 #include "lds_dma.hip.h"

@@ -399,12 +399,12 @@ static __global__ void rope_kv_pending_kernel(float* __restrict__ q, float* __re
     rope_kv_body<KV>(q, k, v, cs_table, pos_ptr, n_heads, n_kv_heads, head_dim, rope_type, k_cache, v_cache, max_seq, pq, pk, pv);
 }
 
-// The same for more than 64 tokens: a thread takes a quad of a head's columns and the one head_dim / 2 further on, 256 threads the
+// The same for many tokens: a thread takes a quad of a head's columns and the one head_dim / 2 further on, 256 threads the
 // heads of a token; head_dim a multiple of 8, rows and partial sums 16-byte aligned.  It is bound by bytes: 512 tokens of
 // 32 + 8 + 8 heads of 128, K in two parts, 13.7 us, where one pair a thread in workgroups of 64 takes 23; 1001 tokens of
-// 24 + 8 + 8: 15 and 21.  With fewer tokens the launch is a chain of loads, which one pair keeps shorter.  Passes of two layers by
-// pairs and by quads: 32 + 8 + 8 heads of 128: 45 tokens 318 / 320 us, 64: 433 / 438, 128: 539 / 538, 192: 653 / 645; 64 + 32 + 32 heads
-// of 64: 10 tokens 239 / 241, 65: 486 / 481.
+// 24 + 8 + 8: 15 and 21.  While the pairs' wavefronts are less than one round of the chip (8192 on 256 CUs) they are a chain of loads,
+// the shorter for one pair a thread.  By pairs and by quads: 18 + 9 + 9 heads of 128: 97 tokens (3492 wavefronts) 4.8 / 5.4 us, 192
+// (6912) 4.9 / 5.9; 32 + 16 + 16 heads of 64: 128 tokens (8192) 4.8 / 4.8, 192 7.4 / 5.3; 64 + 32 + 32: 65 tokens (8320) 8.6 / 6.4.
 __device__ __forceinline__ float4 rope_pending_ld4(const float* rows, const RopePending& pd, uint64_t e) {
     if (pd.n_split == 0) return *reinterpret_cast<const float4*>(rows + e);
     float4 s = *reinterpret_cast<const float4*>(pd.part + e);

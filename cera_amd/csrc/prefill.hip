@@ -537,13 +537,11 @@ static __global__ __launch_bounds__(256) void act_fp8_records_kernel(const int8_
 }
 
 // The pass's first launch: embedding rows of the tokens it brings along, and the first position for the kernels behind it.  With
-// many tokens a thread takes four elements (512 tokens of 4096, Q4_K: 12.4 us by one element, 8.2 by four); with a few the launch is
-// a chain of loads, which one element keeps the shortest (45 tokens: 4.8 us, four elements 5.7).
-constexpr uint32_t embed_elems(int ids) { return ids > 64 ? 4 : 1; }
-template <int N>
+// many tokens a thread takes E = four elements (512 tokens of 4096, Q4_K: 12.4 us by one element, 8.2 by four); with a few the launch
+// is a chain of loads, which one element keeps the shortest (45 tokens: 4.8 us, four elements 5.7).
+template <uint32_t E, int N>
 static __global__ __launch_bounds__(256) void embed_ids_kernel(uint32_t dtype, const uint8_t* __restrict__ w, uint64_t row_bytes, CeraIds<N> tokens, uint32_t first,
                                                                uint32_t pos, uint32_t* __restrict__ scalars, uint32_t k, float scale, float* __restrict__ out) {
-    constexpr uint32_t E = embed_elems(N);
     const uint32_t e = (blockIdx.x * 256 + threadIdx.x) * E;   // k is a multiple of 32
     if (e == 0 && first + blockIdx.y == 0) scalars[1] = pos;
     if (e >= k) return;
@@ -569,10 +567,19 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     const uint32_t hs = c.hidden, q_dim = c.n_heads * c.head_dim, kv_dim = c.n_kv_heads * c.head_dim;
     const float scale = c.attn_scale != 0.0f ? c.attn_scale : 1.0f / std::sqrt(static_cast<float>(c.head_dim));
     CERA_TRY(cera_model_ensure_prefill_buffers(m, n));
+    // Wavefronts that the chip holds at a time.  Launches that handle one element or pair a thread are as long as their longest chain
+    // of loads while they are one round of it, and the shorter the fewer loads a chain has; beyond, those that handle four are
+    // faster.  Passes of two layers, embedding by one element and by four: hidden 4096, 128 tokens (8192 wavefronts) 532 / 533 us, 512:
+    // 1115 / 1111; hidden 2304, 192 tokens (6912) 421 / 422, 256 (9216) 453 / 451.
+    const uint64_t round = 32ull * ctx->n_cu;
     cera_by_ids(tokens, n, [&](const auto& ids, uint32_t first, uint32_t count) {
-        const uint32_t per = 256 * embed_elems(static_cast<int>(sizeof(ids.id) / sizeof(ids.id[0])));
-        hipLaunchKernelGGL(embed_ids_kernel, dim3((hs + per - 1) / per, count), dim3(256), 0, s, m->embd->dtype, m->embd->dev, m->embd->row_bytes, ids, first,
-                           start_pos, m->scalars, hs, c.embed_scale, m->pf_hidden);
+        auto embed = [&](auto elems) {
+            constexpr uint32_t E = decltype(elems)::value;
+            hipLaunchKernelGGL((embed_ids_kernel<E>), dim3((hs + 256 * E - 1) / (256 * E), count), dim3(256), 0, s, m->embd->dtype, m->embd->dev, m->embd->row_bytes, ids,
+                               first, start_pos, m->scalars, hs, c.embed_scale, m->pf_hidden);
+        };
+        if ((hs + 255) / 256 * 4ull * n > round) embed(std::integral_constant<uint32_t, 4>{});
+        else embed(std::integral_constant<uint32_t, 1>{});
     });
     HIP_TRY(ctx, hipGetLastError());
 
@@ -754,7 +761,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
                 };
                 const uint32_t heads = c.n_heads + 2 * c.n_kv_heads;
                 // (heads come in whole eights of columns, so that rows and slices of partial sums start on whole quads)
-                if (n > 64) go(&rope_kv_quads_kernel<KV>, dim3((heads * (c.head_dim / 8) + 255) / 256, n), 256, rq, rk, rv);
+                if (static_cast<uint64_t>(n) * heads * ((c.head_dim + 127) / 128) >= round) go(&rope_kv_quads_kernel<KV>, dim3((heads * (c.head_dim / 8) + 255) / 256, n), 256, rq, rk, rv);
                 else if (pqk.n_split || pvv.n_split) go(&rope_kv_pending_kernel<KV>, dim3(heads, n), c.head_dim / 2, rq, rk, rv);
                 else go(&rope_kv_kernel<KV>, dim3(heads, n), c.head_dim / 2);
             };

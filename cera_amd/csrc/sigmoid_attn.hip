@@ -258,10 +258,11 @@ __global__ __launch_bounds__(256) void sattn_rows_kernel(AArgs a) {
 // ---- many queries, heads of 64 or 128 in bf16: four wavefronts' columns share the keys and values in LDS -------------
 // A workgroup walks its columns' keys in blocks of 64 that direct loads bring into LDS one block ahead, K rows and V's
 // transposed rows alike in 16-byte chunks: chunk c of key k in a slot of its group of eight that depends on k (key_slot), chunk c
-// of value column v in slot c ^ (v % 8), so that eight lanes always read eight different bank groups.  The products are
-// sattn_rows_kernel's, in its order.  1900 queries, 32 heads of 128 on 8: 185 us with every wavefront reading its own keys and
-// values, V in pieces of half a cache line; 87 with blocks of 32 in LDS, 70 with blocks of 64, which leave a wavefront fewer
-// waits in a row (630 TFLOP/s of matrix instructions).  What bounds it: those waits, and the sigmoids between the products.
+// of value column v in slot c ^ (v % 8), so that eight lanes in a row read eight different bank groups (two clocks of conflicts a
+// read are left).  The products are sattn_rows_kernel's, in its order.  1900 queries, 32 heads of 128 on 8: 182 us with every
+// wavefront reading its own keys and values, V in pieces of half a cache line; 87 with blocks of 32 in LDS, 70 with blocks of 64,
+// which leave a wavefront fewer waits in a row.  What bounds it: those waits, with the matrix cores busy for 0.25 of the time and the
+// vector ALU, the sigmoids, for 0.30.
 __device__ __forceinline__ uint32_t key_slot(uint32_t key, uint32_t chunk) {
     return (chunk & ~7u) | ((chunk ^ ((key & 3) | ((((key >> 3) ^ (key >> 2)) & 1) << 2))) & 7);
 }

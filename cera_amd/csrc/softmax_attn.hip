@@ -1,8 +1,9 @@
 // Kernels of softmax_attn.h.
 //
 // A workgroup of four wavefronts walks the keys in blocks of 32 rows (64 where a wavefront has two tiles of columns: a wavefront
-// alone on its SIMD waits for each part of a block in turn, and twice the keys a turn take 110 us in place of 139 for 24 heads
-// of 128 with 2048 queries behind 777 keys, 120 in place of 134 with latent keys of 192) that it stages in LDS by direct
+// alone on its SIMD waits for each part of a block in turn, and twice the keys a turn take 108 us in place of 138 for 24 heads
+// of 128 with 2048 queries behind 777 keys, 119 in place of 132 with latent keys of 192; heads of 64, whose wavefronts go from four
+// a SIMD to three: five layers of 32 of them with 2048 queries 1753 -> 1726 us, behind 2000 keys 2239 -> 2185) that it stages in LDS by direct
 // global-to-LDS loads (16-byte chunk c of row k sits in slot c ^ swz(k) of its group of eight).  Wavefronts are
 // `cg` column groups times `kg` key groups times VG value groups: a column is one (query, query head of the kv head)
 // pair, 16 * CT of them per wavefront; key groups take blocks in turn and add up through LDS at the end; value groups

@@ -509,6 +509,31 @@ def test_prefill_rotates_heads_of_every_size(hip, orc, head_dim, n_heads, n_kv_h
     gm.close(); om.close()
 
 
+@pytest.mark.parametrize("head_dim,n_heads,n_kv_heads,hidden,cuts", [(8, 64, 64, 512, (42, 43)), (40, 32, 32, 512, (85, 86)), (64, 32, 32, 512, (1, 97)),
+                                                                     (256, 16, 16, 512, (86, 85)), (64, 4, 1, 2048, (256, 257)), (64, 4, 1, 16384, (32, 33))])
+@pytest.mark.parametrize("rope_type,kv_f16", [(1, False), (0, True)])
+def test_prefill_on_both_sides_of_a_round_of_the_chip(hip, orc, head_dim, n_heads, n_kv_heads, hidden, cuts, rope_type, kv_f16):
+    """Rotation by pairs and by quads, embedding by one element and by four: the launches in passes of up to, and of more than, the
+    8192 wavefronts that 256 CUs hold.  Tolerance: as above, and in an f16 cache a step of the value on top, 2^-10 of it at most: both
+    sides round to f16, and a difference of any size may put them on neighbours."""
+    n = sum(cuts)
+    cfg = dict(synth.TINY, n_layers=1, hidden=hidden, ffn=256, n_heads=n_heads, n_kv_heads=n_kv_heads, head_dim=head_dim, max_seq_len=n, rope_type=rope_type)
+    weights = synth.make_llama(cfg, seed=89, sigma=0.03, norm_jitter=0.1)
+    gm = hip_api.Model(hip, cfg, weights)
+    om = orc.Llama(cfg, weights)
+    if kv_f16:
+        gm.configure_kv(True); om.set_kv_f16(True)
+    toks = [int(t) for t in util.rng(head_dim).integers(0, cfg["vocab"], n)]
+    _say(f"model: heads of {head_dim}, {n_heads} / {n_kv_heads}, hidden {hidden}, rope {rope_type}, f16 cache {kv_f16}, passes of {cuts}")
+    for first, last in ((0, cuts[0]), (cuts[0], n)):
+        gm.forward_prefill(toks[first:last], first)
+        om.forward_prefill_batched(toks[first:last], first)
+    (kg, vg), (ko, vo) = gm.read_kv(0), om.kv(0)
+    for got, want in ((kg, ko), (vg, vo)):
+        assert (np.abs(got - want) <= 2e-3 * util.rms(want) + (np.abs(want) * 2.0 ** -10 if kv_f16 else 0)).all()
+    gm.close(); om.close()
+
+
 # a pass of a few tokens: (config, make_llama's arguments, biases, QK norm, f16 cache)
 FEW_MODELS = {
     "q4_k_m": (dict(), dict(), False, False, False),                                        # Q | K and a Q6_K V in one launch
