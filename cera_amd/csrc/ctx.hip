@@ -432,3 +432,26 @@ cera_hip_status cera_tensor_upload_concat(cera_hip_ctx* ctx, const cera_hip_tens
     *fused = f;
     return CERA_HIP_OK;
 }
+
+// A pass's logits (whole 16-byte pieces of an allocation of this library's own) to pageable host memory.  Up to one pinned chunk, a
+// kernel writes them into it and the stream is waited for: the runtime's copy has a start of its own, and so has an event.
+// Launch, copy, wait and memcpy, by the runtime's copy and an event / by the kernel: 128 000 bytes 33.5 / 20.7 us, 256 000
+// 40.3 / 25.7, 640 000 56.7 / 41.8, a whole chunk 83 / 69; up to 4 KB the same.  Beyond it the copies of chunks overlap with the
+// memcpy.  One token of a four-layer llama 240 -> 230 us.
+static __global__ __launch_bounds__(256) void to_host_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, uint32_t n16) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n16) dst[i] = src[i];
+}
+cera_hip_status cera_logits_to_host(cera_hip_ctx* ctx, float* dst, const float* src, uint64_t n) {
+    if (n == 0 || n > PIN_CHUNK || n % 16 || reinterpret_cast<uintptr_t>(src) % 16) return cera_hip_download(ctx, dst, src, n);
+    std::lock_guard<std::mutex> lk(ctx->pin_mu);
+    if (!ctx->pin[0]) HIP_TRY(ctx, hipHostMalloc(&ctx->pin[0], PIN_CHUNK, hipHostMallocDefault));
+    void* out = nullptr;
+    HIP_TRY(ctx, hipHostGetDevicePointer(&out, ctx->pin[0], 0));
+    const uint32_t n16 = static_cast<uint32_t>(n / 16);
+    hipLaunchKernelGGL(to_host_kernel, dim3((n16 + 255) / 256), dim3(256), 0, ctx->stream, static_cast<uint4*>(out), reinterpret_cast<const uint4*>(src), n16);
+    HIP_TRY(ctx, hipGetLastError());
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(dst, ctx->pin[0], n);
+    return CERA_HIP_OK;
+}

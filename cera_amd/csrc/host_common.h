@@ -81,6 +81,8 @@ cera_hip_status cera_check_tensor(cera_hip_ctx* ctx, const cera_hip_tensor* t, u
 cera_hip_status cera_scratch(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out);
 // a workspace that a call is faster with but can do without: *out = nullptr where there is no room for it
 cera_hip_status cera_scratch_if_room(cera_hip_ctx* ctx, int slot, uint64_t nbytes, void** out);
+// bytes of a pass's logits to host memory; waits for the stream
+cera_hip_status cera_logits_to_host(cera_hip_ctx* ctx, float* dst, const float* src, uint64_t n);
 // kernel `name` of the context's loaded code object, nullptr when there is no module or no such kernel
 hipFunction_t cera_module_fn(cera_hip_ctx* ctx, const std::string& name);
 // launch a one-struct-argument kernel of the loaded code object

@@ -90,14 +90,14 @@ cera_hip_status layered_portions(cera_hip_model* m, LayeredPass pass, const uint
     if (n == 1) {
         CERA_TRY(m->ops->decode(m, tokens[0], start, true));
         m->seq_len = start + 1;
-        return cera_hip_download(m->ctx, all ? all : last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+        return cera_logits_to_host(m->ctx, all ? all : last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
     }
     for (uint32_t off = 0; off < n; off += CERA_PREFILL_CHUNK) {
         const uint32_t len = std::min(CERA_PREFILL_CHUNK, n - off);
         CERA_TRY(pass(m, tokens + off, len, start + off, !all && off + len == n, all ? all + static_cast<uint64_t>(off) * m->cfg.vocab : nullptr));
         m->seq_len = start + off + len;
     }
-    return all ? CERA_HIP_OK : cera_hip_download(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return all ? CERA_HIP_OK : cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
 }
 
 namespace {
@@ -307,7 +307,7 @@ cera_hip_status batch_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n
     DenseOut out;
     out.out = all ? g.blogits : m->logits; out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
     CERA_TRY(cera_launch_dense_gemm(ctx, g.head, g.ba, g.ld, nc.n, out, g.f32));
-    return all ? cera_hip_download(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
+    return all ? cera_logits_to_host(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
 }
 
 cera_hip_status prefill(cera_hip_model* m, const uint32_t* tokens, uint32_t n, uint32_t start, float* last_logits) {

@@ -219,7 +219,7 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
     DenseOut out;
     out.out = all ? g.blogits : m->logits; out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
     CERA_TRY(cera_launch_dense_gemm(ctx, g.head, g.ba, g.ld, rows, out, g.f32));
-    return all ? cera_hip_download(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
+    return all ? cera_logits_to_host(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
 }
 
 cera_hip_status prefill(cera_hip_model* m, const uint32_t* tokens, uint32_t n, uint32_t start, float* last_logits) {

@@ -671,7 +671,7 @@ static cera_hip_status set_token_pos(cera_hip_model* m, uint32_t token, uint32_t
 cera_hip_status cera_model_decode_logits(cera_hip_model* m, uint32_t token, uint32_t pos, float* logits) {
     CERA_TRY(decode_step(m, token, pos, true));
     m->seq_len = pos + 1;
-    return cera_hip_download(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return cera_logits_to_host(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
 }
 
 // Token-at-a-time prefill (LlamaModel::forward_prefill's per-token route,
@@ -683,7 +683,7 @@ cera_hip_status cera_model_prefill_per_token(cera_hip_model* m, const uint32_t* 
         CERA_TRY(decode_step(m, tokens[i], start_pos + i, i + 1 == n));
         m->seq_len = start_pos + i + 1;
     }
-    return cera_hip_download(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
 }
 
 static cera_hip_status write_kv(cera_hip_model* m, uint32_t layer, const float* k, const float* v, uint32_t n_pos) {

@@ -119,7 +119,7 @@ extern "C" cera_hip_status cera_hip_forward(cera_hip_model* m, uint32_t token, u
     ModelLock lk(m);
     CERA_TRY(check_step(m, token, pos));
     CERA_TRY(m->ops->decode(m, token, pos, true));
-    CERA_TRY(cera_hip_download(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4));
+    CERA_TRY(cera_logits_to_host(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4));
     m->seq_len = pos + 1;
     return CERA_HIP_OK;
 }

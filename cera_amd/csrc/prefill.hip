@@ -845,7 +845,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
                                1.0f / c.logit_scale, static_cast<uint32_t>(tot));
             HIP_TRY(ctx, hipGetLastError());
         }
-        return cera_hip_download(ctx, all_logits, m->pf_logits, static_cast<uint64_t>(n) * rows * 4);
+        return cera_logits_to_host(ctx, all_logits, m->pf_logits, static_cast<uint64_t>(n) * rows * 4);
     }
     if (want_logits) {
         // last token: final norm then the decode-style GEMV (project_logits)
@@ -926,12 +926,12 @@ cera_hip_status cera_model_prefill(cera_hip_model* m, const uint32_t* tokens, ui
             uint32_t len = std::min(PREFILL_CHUNK, n - off);
             CERA_TRY(cera_model_prefill_ref_batched(m, tokens + off, len, start_pos + off, off + len == n));
         }
-        return cera_hip_download(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+        return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
     }
     if (n == 1 || !prefill_batchable(m)) return cera_model_prefill_per_token(m, tokens, n, start_pos, last_logits);
     for (uint32_t off = 0; off < n; off += PREFILL_CHUNK) {
         uint32_t len = std::min(PREFILL_CHUNK, n - off);
         CERA_TRY(prefill_chunk(m, tokens + off, len, start_pos + off, off + len == n));
     }
-    return cera_hip_download(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
 }
