@@ -297,6 +297,32 @@ cera_hip_status cera_launch_row_gemv_store(cera_hip_ctx* ctx, const cera_hip_dte
     return CERA_HIP_OK;
 }
 
+// The vocabulary head from its decode copy with the final norm in front (head_gemv_kernel): y = W . Q8_0(rmsnorm(x, norm_w)), the
+// normalized vector to norm_out.  *launched = false: no decode copy, or a row length without an instance.
+cera_hip_status cera_launch_head_fused(cera_hip_ctx* ctx, const cera_hip_dtensor* w, const float* x, const float* norm_w, float eps,
+                                       float* y, float* norm_out, bool* launched) {
+    *launched = false;
+    const uint32_t tiles = short_tiles(w->dtype, w->k);
+    if (tiles == 0 || !w->dev_stream || w->m > (1u << 24) || x == norm_out) return CERA_HIP_OK;
+    constexpr int NW = 8;
+    HeadGemvArgs a{w->dev_stream, x, norm_w, eps, static_cast<uint32_t>(w->m), static_cast<uint32_t>(w->k), static_cast<uint32_t>(w->stream_row_bytes), y, norm_out};
+    const dim3 grid(std::min<uint32_t>(2 * ctx->n_cu, (a.m + NW - 1) / NW)), block(64 * NW);
+#define HEAD_LAUNCH(TT)                                                                                       \
+    do {                                                                                                      \
+        if (tiles == 1) hipLaunchKernelGGL((head_gemv_kernel<TT, NW, 1>), grid, block, 0, ctx->stream, a);    \
+        else hipLaunchKernelGGL((head_gemv_kernel<TT, NW, 2>), grid, block, 0, ctx->stream, a);               \
+    } while (0)
+    if (w->dtype == CERA_HIP_Q4_K) HEAD_LAUNCH(Q4K);
+    else if (w->dtype == CERA_HIP_Q6_K) HEAD_LAUNCH(Q6K);
+    else if (w->dtype == CERA_HIP_Q4_0) HEAD_LAUNCH(Q4_0);
+    else if (w->dtype == CERA_HIP_Q4_1) HEAD_LAUNCH(Q4_1);
+    else HEAD_LAUNCH(Q8_0);
+#undef HEAD_LAUNCH
+    HIP_TRY(ctx, hipGetLastError());
+    *launched = true;
+    return CERA_HIP_OK;
+}
+
 // y = resid + W . (xs, xq) for long rows (see row_gemv_long_kernel); *launched = false when the
 // shape has no instance.
 cera_hip_status cera_launch_row_gemv_long_add(cera_hip_ctx* ctx, const cera_hip_dtensor* w, const float* xs, const int8_t* xq,

@@ -63,7 +63,8 @@ struct NormQuant {
             }
         }
     }
-    __device__ __forceinline__ void finish(uint32_t k, float eps, uint32_t* s_xq, float* s_xs, double* s_part) {
+    // y (nullable): the normalized vector also goes there
+    __device__ __forceinline__ void finish(uint32_t k, float eps, uint32_t* s_xq, float* s_xs, double* s_part, float* y = nullptr) {
         double s = 0.0;
 #pragma unroll
         for (int it = 0; it < MAXIT; ++it) {   // elements past k are zero
@@ -88,6 +89,7 @@ struct NormQuant {
                 o.y = __fmul_rn(__fmul_rn(v[it].y, inv), g[it].y);
                 o.z = __fmul_rn(__fmul_rn(v[it].z, inv), g[it].z);
                 o.w = __fmul_rn(__fmul_rn(v[it].w, inv), g[it].w);
+                if (y) *reinterpret_cast<float4*>(y + i) = o;
                 float sc;
                 const uint32_t packed = q8_quantize_quad(o, sc);
                 s_xq[i >> 2] = packed;
@@ -247,6 +249,71 @@ static __global__ __launch_bounds__(64 * NW, 2) void row_gemv_pair_kernel(RowGem
     __shared__ double s_part[NW];
     if (blockIdx.x < p.n_blocks_a) row_gemv_body<TA, NW, ROWS, NORM, FEPI_STORE, STREAM, TILES, MAXK>(p.a, blockIdx.x, s_xq, s_xs, s_part, nullptr);
     else row_gemv_body<TB, NW, ROWS, NORM, FEPI_STORE, STREAM, TILES, MAXK>(p.b, blockIdx.x - p.n_blocks_a, s_xq, s_xs, s_part, nullptr);
+}
+
+// The vocabulary head with the final norm in front: wavefront g of the launch owns rows [g * m / G, (g + 1) * m / G), walks them two
+// at a time and stores a lane's row per lane, up to 64 at once.  One launch of two workgroups a CU, so that the norm (a memory round
+// trip, an f64 reduction, two barriers) is done once per workgroup behind its first two rows' loads.  The first workgroup leaves the
+// normalized vector in norm_out, which must not be x.  Same T::dot and wave_sum in the same order as row_gemv_kernel: same bits.
+// Bound by the bytes and its start.  Q6_K alone, against row_gemv_kernel without the norm's launch of 3.3 us: 32000 x 4096 20.7 / 19.4 us,
+// x 3072 16.1 / 16.3, x 2048 13.2 / 14.5, 128256 x 4096 66.8 / 63.1; three or four workgroups a CU or rows in flight are slower.
+struct HeadGemvArgs {
+    const uint8_t* w;   // decode copy
+    const float *x, *norm_w;
+    float eps;
+    uint32_t m, k, row_bytes;
+    float *y, *norm_out;
+};
+template <class T, int NW, int TILES>
+static __global__ __launch_bounds__(64 * NW, 2) void head_gemv_kernel(HeadGemvArgs p) {
+    constexpr int MAXK = 4096 * TILES;
+    __shared__ uint32_t s_xq[MAXK / 4];
+    __shared__ float s_xs[MAXK / 32];
+    __shared__ double s_part[NW];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_units = p.k / T::ELEMS_PER_UNIT;
+    bool live[TILES];
+    uint32_t unit[TILES];
+#pragma unroll
+    for (int tt = 0; tt < TILES; ++tt) {
+        live[tt] = 64 * tt + lane < n_units;
+        unit[tt] = live[tt] ? 64 * tt + lane : 0;   // dead lanes re-read unit 0 with zeroed activations
+    }
+    const uint64_t g = static_cast<uint64_t>(blockIdx.x) * NW + wave, G = static_cast<uint64_t>(gridDim.x) * NW;
+    const uint32_t r0 = static_cast<uint32_t>(g * p.m / G), r1 = static_cast<uint32_t>((g + 1) * p.m / G);
+    NormQuant<NW, MAXK> nq;
+    nq.load(p.x, p.norm_w, p.k);
+    __builtin_amdgcn_sched_barrier(0);
+    RowGemvArgs q{};
+    q.w = p.w; q.m = p.m; q.k = p.k; q.row_bytes = p.row_bytes;
+    RowTile<T, 1, true, TILES> t[2];
+    t[0].load(q, unit, min(r0, p.m - 1));   // rows past the end re-read the last row
+    t[1].load(q, unit, min(r0 + 1, p.m - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    nq.finish(p.k, p.eps, s_xq, s_xs, s_part, blockIdx.x == 0 ? p.norm_out : nullptr);
+    typename T::Act act[TILES];
+#pragma unroll
+    for (int tt = 0; tt < TILES; ++tt) T::load_act(act[tt], reinterpret_cast<const int8_t*>(s_xq), s_xs, unit[tt], live[tt]);
+    float mine = 0.0f;   // of row first + lane
+    uint32_t first = r0;
+    auto row = [&](uint32_t r, RowTile<T, 1, true, TILES>& b) {
+        float part[TILES], tot = 0.0f;
+#pragma unroll
+        for (int tt = 0; tt < TILES; ++tt) part[tt] = T::dot(b.w[0][tt], act[tt], unit[tt], nullptr);
+        __builtin_amdgcn_sched_barrier(0);
+        if (r + 2 < r1) b.load(q, unit, r + 2);   // (one row more than it has would be an eighth of 32000 rows' bytes again)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tt = 0; tt < TILES; ++tt) tot = TILES == 1 ? wave_sum(part[tt]) : tot + wave_sum(part[tt]);
+        if (lane == r - first) mine = tot;
+        if (r - first == 63 || r + 1 == r1) {
+            if (first + lane <= r) p.y[first + lane] = mine;
+            first = r + 1;
+        }
+    };
+    for (uint32_t r = r0; r < r1; r += 2) {
+        row(r, t[0]);
+        if (r + 1 < r1) row(r + 1, t[1]);
+    }
 }
 
 // Long rows (beyond the short kernels, k <= 32768 for the K-quants: the down projection): still one wavefront per row, walking the

@@ -139,6 +139,8 @@ cera_hip_status cera_launch_ffn_gate_up_fused(cera_hip_ctx* ctx, const cera_hip_
                                               bool* launched);
 cera_hip_status cera_launch_qkv_fused(cera_hip_ctx* ctx, const cera_hip_dtensor* wa, const cera_hip_dtensor* wb, const float* x,
                                       const float* norm_w, float eps, float* ya, float* yb, bool* launched);
+cera_hip_status cera_launch_head_fused(cera_hip_ctx* ctx, const cera_hip_dtensor* w, const float* x, const float* norm_w, float eps,
+                                       float* y, float* norm_out, bool* launched);
 // one query, any head_dim % 8 == 0 up to 256, any heads per kv head (reforder.hip); scores: [n_heads][max_seq] floats
 cera_hip_status cera_launch_attn_generic(cera_hip_ctx* ctx, const float* q, const void* kc, const void* vc, uint32_t n_heads,
                                          uint32_t n_kv_heads, uint32_t head_dim, uint32_t seq_len, uint32_t max_seq, float scale,

@@ -639,13 +639,17 @@ static cera_hip_status decode_step(cera_hip_model* m, uint32_t token, uint32_t p
                                static_cast<uint64_t>(c.ffn), m->act, m->xs, m->xq, static_cast<float*>(nullptr));
             HIP_TRY(ctx, hipGetLastError());
         }
-        CERA_TRY(project(m, L.down, m->act, m->hidden, m->hidden));
+        // the last layer's sums where the head reads them while it leaves the normalized vector in m->hidden
+        CERA_TRY(project(m, L.down, m->act, i + 1 == c.n_layers && want_logits ? m->normed : m->hidden, m->hidden));
     }
-    // final norm in place (run_layers ends with rmsnorm(hidden, output_norm))
-    CERA_TRY(norm_quant(m, m->hidden, m->output_norm, c.hidden, 1, m->hidden));
+    // final norm (run_layers ends with rmsnorm(hidden, output_norm))
+    const float* const last = want_logits ? m->normed : m->hidden;
+    const cera_hip_dtensor* o = m->output ? m->output : m->embd;
+    bool head_done = false;
+    if (want_logits) CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, m->logits, m->hidden, &head_done));
+    if (!head_done) CERA_TRY(norm_quant(m, last, m->output_norm, c.hidden, 1, m->hidden));
     if (want_logits) {
-        const cera_hip_dtensor* o = m->output ? m->output : m->embd;
-        CERA_TRY(project(m, o, m->hidden, m->logits, nullptr));
+        if (!head_done) CERA_TRY(project(m, o, m->hidden, m->logits, nullptr));
         if (c.logit_scale != 1.0f) {
             hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, m->logits,
                                1.0f / c.logit_scale, c.vocab);

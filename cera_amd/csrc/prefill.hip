@@ -850,16 +850,19 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     if (want_logits) {
         // last token: final norm then the decode-style GEMV (project_logits)
         const float* last = m->pf_hidden + static_cast<uint64_t>(n - 1) * hs;
-        hipLaunchKernelGGL((rmsnorm_kernel<true>), dim3(1), dim3(256), 0, s, last, m->output_norm, hs, c.rms_eps, m->hidden,
-                           m->xs, m->xq, static_cast<float*>(nullptr));
-        HIP_TRY(ctx, hipGetLastError());
         const cera_hip_dtensor* o = m->output ? m->output : m->embd;
-        if (o->dtype == CERA_HIP_Q5_K) {
-            CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, m->logits));
-        } else {   // from the decode copy where the head has one, as the decode step
-            bool done = false;
-            CERA_TRY(cera_launch_row_gemv_store(ctx, o, m->xs, m->xq, m->logits, &done));
-            if (!done) CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, m->logits, nullptr, CERA_EPI_STORE));
+        bool done = false;   // from the decode copy where the head has one, as the decode step
+        CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, m->logits, m->hidden, &done));
+        if (!done) {
+            hipLaunchKernelGGL((rmsnorm_kernel<true>), dim3(1), dim3(256), 0, s, last, m->output_norm, hs, c.rms_eps, m->hidden,
+                               m->xs, m->xq, static_cast<float*>(nullptr));
+            HIP_TRY(ctx, hipGetLastError());
+            if (o->dtype == CERA_HIP_Q5_K) {
+                CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, m->logits));
+            } else {
+                CERA_TRY(cera_launch_row_gemv_store(ctx, o, m->xs, m->xq, m->logits, &done));
+                if (!done) CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, m->logits, nullptr, CERA_EPI_STORE));
+            }
         }
         if (c.logit_scale != 1.0f) {
             hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, m->logits, 1.0f / c.logit_scale, c.vocab);
