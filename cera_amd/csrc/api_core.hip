@@ -342,6 +342,20 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
     const bool batch = n_queries >= 16;
     if (batch && (reinterpret_cast<uintptr_t>(q) & 15)) return cera_fail(ctx, CERA_HIP_ERR_ARGUMENT, "attention: a query batch must be 16-byte aligned");
     const AttnNewKV nk = new_kv ? *new_kv : AttnNewKV{};
+    if (new_kv && out_quants && !out_bsum && n_splits == 0 && last_len <= attn_short_max_keys(head_dim)) {
+        const uint32_t len = static_cast<uint32_t>(last_len), chunks = (len + 16 * ATTN_SHORT_NW - 1) / (16 * ATTN_SHORT_NW);
+        auto launch = [&](auto tag, auto dim) {
+            using KV = decltype(tag);
+            hipLaunchKernelGGL((attn_decode_short_kernel<KV, decltype(dim)::value>), dim3(n_heads), dim3(64 * ATTN_SHORT_NW), 0, ctx->stream, q, static_cast<const KV*>(kc),
+                               static_cast<const KV*>(vc), len, static_cast<uint32_t>(max_seq), scale, chunks, n_kv_heads, G, nk, out, out_scales, out_quants);
+        };
+        const std::integral_constant<int, 128> d128{};
+        const std::integral_constant<int, 64> d64{};
+        if (head_dim == 128) { if (kv_f16) launch(kv_half{}, d128); else launch(0.0f, d128); }
+        else { if (kv_f16) launch(kv_half{}, d64); else launch(0.0f, d64); }
+        HIP_TRY(ctx, hipGetLastError());
+        return CERA_HIP_OK;
+    }
     uint32_t n_parts, part_keys = 0, chunks_per_part = 0;
     uint32_t S = 1;
     uint32_t Gw = G;   // decode: heads per wavefront

@@ -435,6 +435,57 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
     attn_decode_partial_body<G, S, NEWKV, KV, HD, NT>(q, kc, vc, seq_len, max_seq, scale, chunks_per_part, n_parts, q_stride, g_total, n_kv, n_queries, part_acc, part_ml, nk);
 }
 
+// The decode step of a short context in one launch: a workgroup of ATTN_SHORT_NW wavefronts serves one query head over all keys, each
+// wavefront `chunks` chunks of 16 positions; the states meet in LDS, where they are added up as attn_decode_merge_body does (weights
+// against the largest maximum; parts are fewer and longer) and the head's outputs quantized.  grid = heads; those of a kv head take
+// indices n_kv apart, so with eight kv heads one XCD's L2 reads its rows.  What bounds it is a wavefront's chain: one memory round trip
+// and the scores, softmax and sums of its chunks.  Against the partial and merge launches, f32 cache, 32 / 8 heads of 128: 38 keys
+// 7.98 -> 4.91 us, 128 8.25 -> 6.53, 192 8.40 -> 7.01, 256 8.35 -> 7.54, 384 8.69 -> 9.08; heads of 64: 7.47 -> 4.46 at 38, 7.74 -> 7.00
+// at 320.  Two or four heads a wavefront, chunks of 8, sixteen wavefronts: slower (38 keys: 6.16, 10.8; 5.11; 6.26).
+constexpr int ATTN_SHORT_NW = 8;
+template <typename KV, int HD>
+__global__ __launch_bounds__(64 * ATTN_SHORT_NW) void attn_decode_short_kernel(const float* __restrict__ q, const KV* __restrict__ kc, const KV* __restrict__ vc,
+                                                                               uint32_t seq_len, uint32_t max_seq, float scale, uint32_t chunks, uint32_t n_kv,
+                                                                               uint32_t group, AttnNewKV nk, float* __restrict__ out,
+                                                                               float* __restrict__ scales, int8_t* __restrict__ quants) {
+    using Lay = AttnLay<KV, HD>;
+    constexpr int NQ = Lay::NQ, S = 2, NW = ATTN_SHORT_NW;
+    constexpr uint32_t C4 = HD / 4;
+    __shared__ __align__(16) float s_acc[NW][HD];
+    __shared__ float s_ml[NW][2];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t kvh = blockIdx.x % n_kv, sub = blockIdx.x / n_kv, head = kvh * group + sub;
+    const uint32_t keys = chunks * 8 * S, t_begin = wave * keys, parts = (seq_len + keys - 1) / keys;   // parts <= NW
+    if (wave < parts) {
+        float o[1][NQ / 2], m[1], l[1];
+        attn_decode_range<1, S, true, KV, HD, false>(q + static_cast<uint64_t>(head) * HD, kc + static_cast<uint64_t>(kvh) * max_seq * HD,
+                                                     vc + static_cast<uint64_t>(kvh) * max_seq * HD, kvh, max_seq, seq_len, t_begin,
+                                                     min(seq_len, t_begin + keys), 8 * S, scale, nk, sub == 0, lane, o, m, l);
+        const uint32_t col = attn_fold_column<Lay>(lane);
+#pragma unroll
+        for (int i = 0; i < NQ / 2; ++i) s_acc[wave][col + i] = o[0][i];
+        if (lane == 0) { s_ml[wave][0] = m[0]; s_ml[wave][1] = l[0]; }
+    }
+    __syncthreads();
+    if (threadIdx.x >= C4) return;   // whole groups of eight lanes stay
+    float M = -__builtin_inff(), L = 0.0f;
+    for (uint32_t p = 0; p < parts; ++p) M = fmaxf(M, s_ml[p][0]);
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t p = 0; p < parts; ++p) {
+        const float w = cera_expf(s_ml[p][0] - M);
+        L = fmaf(w, s_ml[p][1], L);
+        const float4 a = reinterpret_cast<const float4*>(s_acc[p])[threadIdx.x];
+        acc.x = fmaf(w, a.x, acc.x); acc.y = fmaf(w, a.y, acc.y); acc.z = fmaf(w, a.z, acc.z); acc.w = fmaf(w, a.w, acc.w);
+    }
+    const float inv = 1.0f / L;
+    const float4 o = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    reinterpret_cast<float4*>(out + static_cast<uint64_t>(head) * HD)[threadIdx.x] = o;
+    float sc;
+    const uint32_t packed = q8_quantize_quad(o, sc);
+    reinterpret_cast<uint32_t*>(quants)[head * C4 + threadIdx.x] = packed;
+    if ((threadIdx.x & 7) == 0) scales[head * (HD / 32) + (threadIdx.x >> 3)] = sc;
+}
+
 // ---------------------------------------------------------------------------
 // Causal attention for a batch of queries (prefill) on the f16 matrix cores, at f32
 // accuracy.

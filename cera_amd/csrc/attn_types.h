@@ -14,6 +14,11 @@
 // the same point.
 #define ATTN_FUSED_NEW_KV_MAX_KEYS 1024u
 
+// Up to this many keys the fused step runs in one launch, a workgroup per query head (attn_decode_short_kernel); behind them the two
+// launches, whose wavefronts hold fewer keys each.  Level at 256 keys with heads of 128 (24 / 8 heads: 7.45 against 7.41 us;
+// 32 / 8: 7.54, 8.35) and at 400 with heads of 64.
+static inline uint32_t attn_short_max_keys(uint32_t head_dim) { return head_dim == 64 ? 320u : 192u; }
+
 struct AttnNewKV {
     const float* rope_row;   // [64] (cos, sin) pairs of the token's position
     uint32_t rope_type;      // 0 NEOX, 1 NORM
