@@ -492,80 +492,188 @@ constexpr int GEMV_WAVES = 8;
 template <int R> constexpr int GEMV_U = 8 / R;
 template <int R> constexpr uint32_t GEMV_STEP = 64 * 8 * GEMV_U<R>;
 
-// Fills the workgroup's activation vector xs[0, stage_len).
-template <typename T, int KIND>
-__device__ __forceinline__ void gemv_stage(const GemvDArgs& a, bool second, bool store_h, T* xs, float* red, float* wz) {
-    const DenseIn& in = a.in;
-    if (KIND == DenseIn::RAW) {
-        const T* x = static_cast<const T*>(in.x);
-        constexpr uint32_t V = 16 / sizeof(T);
-#pragma unroll 4
-        for (uint32_t i = threadIdx.x * V; i < a.stage_len; i += GEMV_WAVES * 64 * V)
-            *reinterpret_cast<uint4*>(xs + i) = i < a.kp ? *reinterpret_cast<const uint4*>(x + i) : make_uint4(0, 0, 0, 0);
-    } else if (KIND == DenseIn::MERGE) {
-        const T* x = static_cast<const T*>(in.x);
-        const SAttnPartials& m = in.merge;
-        const uint32_t cols = m.heads * m.vdim, cols_p = (cols + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD;
-        partials_weights(m, 0, m.heads, threadIdx.x, GEMV_WAVES * 64, wz);
-        constexpr uint32_t V = 16 / sizeof(T);
-#pragma unroll 4
-        for (uint32_t i = cols_p + threadIdx.x * V; i < a.stage_len; i += GEMV_WAVES * 64 * V)
-            *reinterpret_cast<uint4*>(xs + i) = i < a.kp ? *reinterpret_cast<const uint4*>(x + i) : make_uint4(0, 0, 0, 0);
-        lds_barrier();
-#pragma unroll 2
-        for (uint32_t i = threadIdx.x * 4; i < cols_p; i += GEMV_WAVES * 256) {
-            if (i + 4 <= cols && m.vdim % 4 == 0) {
-                const uint32_t h = i / m.vdim;
-                const f32x4 s = partials_sum4(m, wz + h * m.splits, h, i - h * m.vdim);
-                ElemOps<T>::store4(xs + i, s.x, s.y, s.z, s.w);
-            } else {
+// Fills the workgroup's activation vector xs[0, stage_len), in two parts with the first weights' loads in between: the hardware counts
+// loads in order, so a wait for an input loaded behind weights is a wait for the weights.  load() takes what the first EARLY steps of
+// the workgroup read into registers, finish() the rest from memory.  With the weights in front of the inputs, before, and now, over
+// rotating weights: 3072 x 2048 behind a norm 5.9 -> 5.5 us, 8192 x 2048 8.8 -> 8.1, 32000 x 2048 24.3 -> 22.9, 2048 x 8192 of a finished
+// input 8.6 -> 7.9, 2048 x 2048 behind eight parts of attention 6.1 -> 5.6, 3072 x 11264 behind eight the same, 16.8.
+template <typename T, int KIND> struct GemvStage {
+    static constexpr uint32_t V = KIND == DenseIn::RAW || KIND == DenseIn::MERGE ? 16 / sizeof(T) : 4, STEP = GEMV_WAVES * 64 * V;
+    static constexpr int EARLY = KIND == DenseIn::RAW ? 3 : 2, PARTS = 8;
+    uint4 x[EARLY];
+    float4 s[KIND == DenseIn::NORM ? EARLY : 1], ad[KIND == DenseIn::NORM ? EARLY : 1], pl[KIND == DenseIn::NORM ? EARLY : 1];
+    PartialsAhead ahead;
+    f32x4 part[KIND == DenseIn::MERGE ? EARLY : 1][KIND == DenseIn::MERGE ? PARTS : 1];
+
+    // columns of attention's result, and where the finished part behind them begins
+    static __device__ __forceinline__ uint32_t merged(const GemvDArgs& a) { return a.in.merge.heads * a.in.merge.vdim; }
+    static __device__ __forceinline__ uint32_t merged_pad(const GemvDArgs& a) { return (merged(a) + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD; }
+    // four merged columns from i on: whole, and of one head
+    static __device__ __forceinline__ bool quad(const GemvDArgs& a, uint32_t i) { return i + 4 <= merged(a) && a.in.merge.vdim % 4 == 0; }
+
+    __device__ __forceinline__ void load(const GemvDArgs& a, bool second, bool store_h) {
+        const DenseIn& in = a.in;
+        if constexpr (KIND == DenseIn::RAW || KIND == DenseIn::MERGE) {
+            uint32_t first = 0;
+            if constexpr (KIND == DenseIn::MERGE) {
+                first = merged_pad(a);
+                const SAttnPartials& m = in.merge;
+                ahead.load(m, threadIdx.x);
+                const uint64_t slice = static_cast<uint64_t>(m.heads) * m.vdim_p;
 #pragma unroll
-                for (uint32_t e = i; e < i + 4; ++e) {
-                    const float s = e < cols ? partials_sum(m, wz + e / m.vdim * m.splits, e / m.vdim, e % m.vdim) : 0.0f;
-                    xs[e] = ElemOps<T>::from(s);
+                for (int e = 0; e < EARLY; ++e) {
+                    if (e * (GEMV_WAVES * 256) >= merged(a)) break;
+                    const uint32_t i = threadIdx.x * 4 + e * (GEMV_WAVES * 256);
+                    const uint32_t h = quad(a, i) ? i / m.vdim : 0, c = quad(a, i) ? i - h * m.vdim : 0;
+                    const float* const src = m.part + static_cast<uint64_t>(h) * m.vdim_p + c;   // 16-byte aligned: vdim_p is a multiple of four
+#pragma unroll
+                    for (int z = 0; z < PARTS; ++z) {
+                        if (z >= static_cast<int>(m.splits)) break;
+                        part[e][z] = *reinterpret_cast<const f32x4*>(src + z * slice);
+                    }
                 }
             }
-        }
-    } else if (KIND == DenseIn::CONCAT) {
-        const float* x = static_cast<const float*>(in.x);
-        const uint32_t half = a.kp / 2;
-        for (uint32_t i = threadIdx.x * 4; i < a.stage_len; i += GEMV_WAVES * 256) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (i < a.kp) v = *reinterpret_cast<const float4*>(i < half ? x + i : in.x2 + (i - half));
-            ElemOps<T>::store4(xs + i, v.x, v.y, v.z, v.w);
-        }
-    } else {
-        const float* x = static_cast<const float*>(in.x);
-        const float *sc = second ? in.scale_b : in.scale_a, *ad = second ? in.add_b : in.add_a;
-        float ss = 0.0f;
-        for (uint32_t i = threadIdx.x * 4; i < a.kp; i += GEMV_WAVES * 256) {
-            const float4 v = *reinterpret_cast<const float4*>(x + i);
-            ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
-        }
-        ss = wave_sum(ss);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-        lds_barrier();
-        float tot = 0.0f;
 #pragma unroll
-        for (int i = 0; i < GEMV_WAVES; ++i) tot += red[i];
-        const float inv = 1.0f / sqrtf(tot / static_cast<float>(in.n_mean) + in.eps);
-        for (uint32_t i = threadIdx.x * 4; i < a.stage_len; i += GEMV_WAVES * 256) {
-            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (i < a.kp) {
-                const float4 v = *reinterpret_cast<const float4*>(x + i), s = *reinterpret_cast<const float4*>(sc + i);
-                if (ad) o = *reinterpret_cast<const float4*>(ad + i);
-                o.x = fmaf(v.x * inv, s.x, o.x); o.y = fmaf(v.y * inv, s.y, o.y);
-                o.z = fmaf(v.z * inv, s.z, o.z); o.w = fmaf(v.w * inv, s.w, o.w);
-                if (store_h) {
-                    const float4 p = *reinterpret_cast<const float4*>(in.plain + i);
-                    *reinterpret_cast<float4*>(in.h_out + i) = make_float4(v.x * inv * p.x, v.y * inv * p.y, v.z * inv * p.z, v.w * inv * p.w);
+            for (int e = 0; e < EARLY; ++e) {
+                if (first + e * STEP >= a.kp) break;
+                const uint32_t i = first + threadIdx.x * V + e * STEP;
+                x[e] = *reinterpret_cast<const uint4*>(static_cast<const T*>(in.x) + min(i, a.kp - V));
+            }
+        } else {
+            const float* const v = static_cast<const float*>(in.x);
+            const float *sc = second ? in.scale_b : in.scale_a, *add = second ? in.add_b : in.add_a;
+            const uint32_t half = a.kp / 2;
+#pragma unroll
+            for (int e = 0; e < EARLY; ++e) {
+                if (e * STEP >= a.kp) break;
+                const uint32_t i = min(threadIdx.x * V + e * STEP, a.kp - V);
+                x[e] = *reinterpret_cast<const uint4*>(KIND == DenseIn::CONCAT && i >= half ? in.x2 + (i - half) : v + i);
+                if constexpr (KIND == DenseIn::NORM) {
+                    s[e] = *reinterpret_cast<const float4*>(sc + i);
+                    if (add) ad[e] = *reinterpret_cast<const float4*>(add + i);
+                    if (store_h) pl[e] = *reinterpret_cast<const float4*>(in.plain + i);
                 }
             }
-            ElemOps<T>::store4(xs + i, o.x, o.y, o.z, o.w);
         }
     }
-    lds_barrier();
-}
+
+    __device__ __forceinline__ void finish(const GemvDArgs& a, bool second, bool store_h, T* xs, float* red, float* wz) {
+        const DenseIn& in = a.in;
+        if constexpr (KIND == DenseIn::RAW || KIND == DenseIn::MERGE) {
+            uint32_t first = 0;
+            if constexpr (KIND == DenseIn::MERGE) {
+                first = merged_pad(a);
+                ahead.weights(in.merge, threadIdx.x, GEMV_WAVES * 64, wz);
+            }
+#pragma unroll
+            for (int e = 0; e < EARLY; ++e) {
+                const uint32_t i = first + threadIdx.x * V + e * STEP;
+                if (i < a.stage_len) *reinterpret_cast<uint4*>(xs + i) = i < a.kp ? x[e] : make_uint4(0, 0, 0, 0);
+            }
+            for (uint32_t i = first + threadIdx.x * V + EARLY * STEP; i < a.stage_len; i += STEP)
+                *reinterpret_cast<uint4*>(xs + i) = i < a.kp ? *reinterpret_cast<const uint4*>(static_cast<const T*>(in.x) + i) : make_uint4(0, 0, 0, 0);
+            if constexpr (KIND == DenseIn::MERGE) {
+                const SAttnPartials& m = in.merge;
+                const uint32_t cols = merged(a);
+                const uint64_t slice = static_cast<uint64_t>(m.heads) * m.vdim_p;
+                lds_barrier();
+                auto single = [&](uint32_t i) {
+#pragma unroll
+                    for (uint32_t e = i; e < i + 4; ++e) {
+                        const float v = e < cols ? partials_sum(m, wz + e / m.vdim * m.splits, e / m.vdim, e % m.vdim) : 0.0f;
+                        xs[e] = ElemOps<T>::from(v);
+                    }
+                };
+#pragma unroll
+                for (int e = 0; e < EARLY; ++e) {
+                    const uint32_t i = threadIdx.x * 4 + e * (GEMV_WAVES * 256);
+                    if (i >= first) continue;
+                    if (!quad(a, i)) {
+                        single(i);
+                        continue;
+                    }
+                    const uint32_t h = i / m.vdim;
+                    const float *const w = wz + h * m.splits, *const src = m.part + static_cast<uint64_t>(h) * m.vdim_p + (i - h * m.vdim);
+                    f32x4 v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int z = 0; z < PARTS; ++z)
+                        if (z < static_cast<int>(m.splits)) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) v[k] = fmaf(part[e][z][k], w[z], v[k]);
+                        }
+                    for (uint32_t z = PARTS; z < m.splits; ++z) {
+                        const f32x4 q = *reinterpret_cast<const f32x4*>(src + z * slice);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) v[k] = fmaf(q[k], w[z], v[k]);
+                    }
+                    ElemOps<T>::store4(xs + i, v.x, v.y, v.z, v.w);
+                }
+                for (uint32_t i = threadIdx.x * 4 + EARLY * (GEMV_WAVES * 256); i < first; i += GEMV_WAVES * 256) {
+                    if (!quad(a, i)) {
+                        single(i);
+                        continue;
+                    }
+                    const uint32_t h = i / m.vdim;
+                    const f32x4 v = partials_sum4(m, wz + h * m.splits, h, i - h * m.vdim);
+                    ElemOps<T>::store4(xs + i, v.x, v.y, v.z, v.w);
+                }
+            }
+        } else if constexpr (KIND == DenseIn::CONCAT) {
+            const uint32_t half = a.kp / 2;
+#pragma unroll
+            for (int e = 0; e < EARLY; ++e) {
+                const uint32_t i = threadIdx.x * V + e * STEP;
+                const f32x4 v = i < a.kp ? __builtin_bit_cast(f32x4, x[e]) : f32x4{0.f, 0.f, 0.f, 0.f};
+                if (i < a.stage_len) ElemOps<T>::store4(xs + i, v.x, v.y, v.z, v.w);
+            }
+            for (uint32_t i = threadIdx.x * V + EARLY * STEP; i < a.stage_len; i += STEP) {
+                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (i < a.kp) v = *reinterpret_cast<const float4*>(i < half ? static_cast<const float*>(in.x) + i : in.x2 + (i - half));
+                ElemOps<T>::store4(xs + i, v.x, v.y, v.z, v.w);
+            }
+        } else {
+            const float* const xv = static_cast<const float*>(in.x);
+            const float *sc = second ? in.scale_b : in.scale_a, *add = second ? in.add_b : in.add_a;
+            float sum = 0.0f;
+            auto square = [&](f32x4 v) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sum = fmaf(v[k], v[k], sum);
+            };
+#pragma unroll
+            for (int e = 0; e < EARLY; ++e)
+                if (threadIdx.x * V + e * STEP < a.kp) square(__builtin_bit_cast(f32x4, x[e]));
+            for (uint32_t i = threadIdx.x * V + EARLY * STEP; i < a.kp; i += STEP) square(*reinterpret_cast<const f32x4*>(xv + i));
+            sum = wave_sum(sum);
+            if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+            lds_barrier();
+            float tot = 0.0f;
+#pragma unroll
+            for (int i = 0; i < GEMV_WAVES; ++i) tot += red[i];
+            const float inv = 1.0f / sqrtf(tot / static_cast<float>(in.n_mean) + in.eps);
+            auto put = [&](uint32_t i, f32x4 v, float4 sv, float4 o, float4 p) {
+                if (i < a.kp) {
+                    o.x = fmaf(v.x * inv, sv.x, o.x); o.y = fmaf(v.y * inv, sv.y, o.y);
+                    o.z = fmaf(v.z * inv, sv.z, o.z); o.w = fmaf(v.w * inv, sv.w, o.w);
+                    if (store_h) *reinterpret_cast<float4*>(in.h_out + i) = make_float4(v.x * inv * p.x, v.y * inv * p.y, v.z * inv * p.z, v.w * inv * p.w);
+                }
+                ElemOps<T>::store4(xs + i, o.x, o.y, o.z, o.w);
+            };
+#pragma unroll
+            for (int e = 0; e < EARLY; ++e) {
+                const uint32_t i = threadIdx.x * V + e * STEP;
+                const bool more = add && i < a.kp;
+                if (i < a.stage_len) put(i, __builtin_bit_cast(f32x4, x[e]), s[e], more ? ad[e] : make_float4(0.f, 0.f, 0.f, 0.f), pl[e]);
+            }
+            for (uint32_t i = threadIdx.x * V + EARLY * STEP; i < a.stage_len; i += STEP) {
+                const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+                const bool in_row = i < a.kp;
+                put(i, in_row ? *reinterpret_cast<const f32x4*>(xv + i) : f32x4{0.f, 0.f, 0.f, 0.f}, in_row ? *reinterpret_cast<const float4*>(sc + i) : zero,
+                    in_row && add ? *reinterpret_cast<const float4*>(add + i) : zero, in_row && store_h ? *reinterpret_cast<const float4*>(in.plain + i) : zero);
+            }
+        }
+        lds_barrier();
+    }
+};
 
 // One wavefront's walk over its groups of R rows (g, g + GEMV_WAVES, ... below g1) of one matrix, a step of
 // U * 64 16-byte chunks at a time; SWIGLU: a group is R / 2 gate rows and their up rows.  Two step buffers
@@ -575,7 +683,7 @@ template <typename T, int R, int SN> struct GemvWalk {
     static constexpr int U = GEMV_U<R>, H = R > 1 ? R / 2 : 1;
     typedef uint4 Buf[U][R];
     const __bf16* w;
-    uint32_t rows, kp, stage_len, g1, lane, last;
+    uint32_t rows, kp, stage_len, lane, at, last, left;   // at: the chunk that a lane loads; left: steps whose weights are still to be loaded
     bool swiglu;
     uint32_t lg, lk;            // group and step the next load takes
     const __bf16* p[R];
@@ -592,28 +700,33 @@ template <typename T, int R, int SN> struct GemvWalk {
             p[r] = w + static_cast<uint64_t>(min(row, rows - 1)) * kp;
         }
     }
-    __device__ __forceinline__ void begin(const __bf16* w_, uint32_t rows_, uint32_t kp_, uint32_t stage_len_, bool swiglu_, uint32_t g, uint32_t g1_) {
-        w = w_; rows = rows_; kp = kp_; stage_len = stage_len_; swiglu = R > 1 && swiglu_; g1 = g1_;
-        lane = threadIdx.x & 63; last = kp / 8 - 1;
+    __device__ __forceinline__ void begin(const __bf16* w_, uint32_t rows_, uint32_t kp_, uint32_t stage_len_, bool swiglu_, uint32_t g, uint32_t steps) {
+        w = w_; rows = rows_; kp = kp_; stage_len = stage_len_; swiglu = R > 1 && swiglu_; left = steps;
+        lane = at = threadIdx.x & 63; last = kp / 8 - 1;
         lg = g; lk = 0;
-        if (lg < g1) set_rows();
+        set_rows();
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
     }
-    __device__ __forceinline__ bool load(Buf& b) {
-        if (lg >= g1) return false;
+    // Stands outside every condition, behind the last step with all lanes at one chunk of a row: where paths with and without a
+    // load meet, the compiler's wait for an older one is a wait for all.
+    __device__ __forceinline__ void load(Buf& b) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int r = 0; r < R; ++r)   // past the row's end: its last chunk again, against zeros
-                b[u][r] = ld_u128_nt(p[r] + min(lk / 8 + u * 64 + lane, last) * 8);
+                b[u][r] = ld_u128_nt(p[r] + min(lk / 8 + u * 64 + at, last) * 8);
+        if (left <= 1) {
+            at = lk = 0;
+            return;
+        }
+        --left;
         lk += GEMV_STEP<R>;
         if (lk >= stage_len) {
             lk = 0;
             lg += GEMV_WAVES;
-            if (lg < g1) set_rows();
+            set_rows();
         }
-        return true;
     }
     // multiplies a step of group g at k; at the group's last step reduces and stores, and moves on
     __device__ __forceinline__ void use(const Buf& b, uint32_t& g, uint32_t& k, const T* xs, const DenseOut& o, const DenseStreams& st) {
@@ -655,8 +768,9 @@ template <typename T, int R, int SN> struct GemvWalk {
     }
 };
 
-template <typename T, int KIND, int R, int SN>
-__global__ __launch_bounds__(GEMV_WAVES * 64) void dense_gemv_kernel(GemvDArgs a) {
+// ONE: no wavefront has more than one step.  (A second buffer's load for nothing, or a wait that counts it, costs 0.4 to 1.3 us.)
+template <typename T, int KIND, int R, int SN, bool ONE = false>
+__global__ __launch_bounds__(GEMV_WAVES * 64, 4) void dense_gemv_kernel(GemvDArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[GEMV_WAVES], wz[KIND == DenseIn::MERGE ? PARTIALS_MAX : 1];
     T* const xs = reinterpret_cast<T*>(smem);
@@ -670,17 +784,39 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void dense_gemv_kernel(GemvDArgs a
     GemvWalk<T, R, SN> walk;
     typename GemvWalk<T, R, SN>::Buf w0, w1;
     uint32_t g = g0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), k = 0;
-    walk.begin(second ? a.wb : a.wa, second ? a.rows_b : a.rows_a, a.kp, a.stage_len, o.epi == DENSE_SWIGLU, g, g1);
+    const uint32_t steps = g < g1 ? (g1 - g + GEMV_WAVES - 1) / GEMV_WAVES * (a.stage_len / GEMV_STEP<R>) : 0;
+    walk.begin(second ? a.wb : a.wa, second ? a.rows_b : a.rows_a, a.kp, a.stage_len, o.epi == DENSE_SWIGLU, g, steps);
+    const bool store_h = KIND == DenseIn::NORM && a.in.h_out && blockIdx.x == 0;
+    GemvStage<T, KIND> stage;
+    stage.load(a, second, store_h);
+    __builtin_amdgcn_sched_barrier(0);   // the inputs' loads first: they are waited for first
     // the first weights are on their way while the activation vector is prepared
-    bool more0 = walk.load(w0);
-    gemv_stage<T, KIND>(a, second, KIND == DenseIn::NORM && a.in.h_out && blockIdx.x == 0, xs, red, wz);
-    while (more0) {
-        const bool more1 = walk.load(w1);
-        walk.use(w0, g, k, xs, o, a.st);
-        if (!more1) break;
-        more0 = walk.load(w0);
-        walk.use(w1, g, k, xs, o, a.st);
+    walk.load(w0);
+    if constexpr (!ONE && KIND != DenseIn::MERGE) walk.load(w1);
+    __builtin_amdgcn_sched_barrier(0);
+    stage.finish(a, second, store_h, xs, red, wz);
+    if constexpr (!ONE && KIND == DenseIn::MERGE) walk.load(w1);   // attention's parts take its registers until here
+    if constexpr (ONE) {
+        if (steps) walk.use(w0, g, k, xs, o, a.st);
+        return;
     }
+    uint32_t s = 0;
+    for (; s + 3 < steps; s += 2) {
+        walk.use(w0, g, k, xs, o, a.st);
+        walk.load(w0);
+        walk.use(w1, g, k, xs, o, a.st);
+        walk.load(w1);
+    }
+    // one to three steps are left
+    if (s + 3 == steps) {
+        walk.use(w0, g, k, xs, o, a.st);
+        walk.load(w0);
+        walk.use(w1, g, k, xs, o, a.st);
+        walk.use(w0, g, k, xs, o, a.st);
+        return;
+    }
+    if (s < steps) walk.use(w0, g, k, xs, o, a.st);
+    if (s + 1 < steps) walk.use(w1, g, k, xs, o, a.st);
 }
 
 constexpr uint64_t GEMV_LDS_MAX = 60 * 1024;
@@ -873,15 +1009,19 @@ cera_hip_status cera_launch_dense_gemv(cera_hip_ctx* ctx, const DenseIn& in, con
     a.blocks_a = std::max(1u, std::min(a.groups_a, wb ? static_cast<uint32_t>(static_cast<uint64_t>(want) * a.groups_a / total) : want));
     a.blocks_b = wb ? std::max(1u, std::min(a.groups_b, want > a.blocks_a ? want - a.blocks_a : 1u)) : 0;
     const dim3 grid(a.blocks_a + a.blocks_b), block(GEMV_WAVES * 64);
+    const bool one = a.stage_len == 512u * (8 / r) && a.groups_a <= a.blocks_a * GEMV_WAVES && a.groups_b <= a.blocks_b * GEMV_WAVES;
     auto go = [&](auto tag, auto rows) {
         using T = decltype(tag);
         constexpr int R = decltype(rows)::value;
         auto kind = [&](auto streams) {
             constexpr int SN = decltype(streams)::value;
-            if (in.kind == DenseIn::RAW) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::RAW, R, SN>), grid, block, lds, ctx->stream, a);
+            if (in.kind == DenseIn::RAW && one) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::RAW, R, SN, true>), grid, block, lds, ctx->stream, a);
+            else if (in.kind == DenseIn::RAW) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::RAW, R, SN>), grid, block, lds, ctx->stream, a);
+            else if (in.kind == DenseIn::MERGE && one) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::MERGE, R, SN, true>), grid, block, lds, ctx->stream, a);
             else if (in.kind == DenseIn::MERGE) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::MERGE, R, SN>), grid, block, lds, ctx->stream, a);
             else if constexpr (SN < 0) {
-                if (in.kind == DenseIn::NORM) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::NORM, R, SN>), grid, block, lds, ctx->stream, a);
+                if (in.kind == DenseIn::NORM && one) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::NORM, R, SN, true>), grid, block, lds, ctx->stream, a);
+                else if (in.kind == DenseIn::NORM) hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::NORM, R, SN>), grid, block, lds, ctx->stream, a);
                 else hipLaunchKernelGGL((dense_gemv_kernel<T, DenseIn::CONCAT, R, SN>), grid, block, lds, ctx->stream, a);
             }
         };

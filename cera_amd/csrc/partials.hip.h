@@ -12,10 +12,10 @@ __device__ __forceinline__ float wave_row_max(float v) {
 }
 // Weights of the parts of heads h0 .. h0 + n - 1 into wz [n][splits], sixteen threads per head (`threads` a multiple of
 // 64, all of them call): softmax parts carry their own maximum and sum, sigmoid parts just add and are gated.  The
-// caller puts a barrier behind it.
-__device__ __forceinline__ void partials_weights(const SAttnPartials& p, uint32_t h0, uint32_t n, uint32_t thread, uint32_t threads, float* wz) {
+// caller puts a barrier behind it.  The heads before `first` are left out.
+__device__ __forceinline__ void partials_weights(const SAttnPartials& p, uint32_t h0, uint32_t n, uint32_t thread, uint32_t threads, float* wz, uint32_t first = 0) {
     const uint32_t l16 = thread & 15;
-    for (uint32_t i = thread >> 4; i < n; i += threads >> 4) {
+    for (uint32_t i = first + (thread >> 4); i < n; i += threads >> 4) {
         const uint32_t h = h0 + i;
         float* const w = wz + i * p.splits;
         if (!p.ml) {
@@ -37,6 +37,33 @@ __device__ __forceinline__ void partials_weights(const SAttnPartials& p, uint32_
         for (uint32_t z = l16; z < p.splits; z += 16) w[z] *= inv;
     }
 }
+// The same for h0 = 0 with what a thread of the first threads / 16 heads reads taken ahead, up to 16 parts.
+struct PartialsAhead {
+    float gate;   // or the sink
+    float2 e;
+    __device__ __forceinline__ void load(const SAttnPartials& p, uint32_t thread) {
+        const uint32_t h = min(thread >> 4, p.heads - 1), z = thread & 15;
+        gate = p.ml ? p.sink[h] : p.gate[h];
+        e = make_float2(-__builtin_inff(), 0.0f);
+        if (p.ml && z < p.splits) e = reinterpret_cast<const float2*>(p.ml)[z * p.heads + h];
+    }
+    __device__ __forceinline__ void weights(const SAttnPartials& p, uint32_t thread, uint32_t threads, float* wz) const {
+        if (p.splits > 16) return partials_weights(p, 0, p.heads, thread, threads, wz);
+        const uint32_t h = thread >> 4, z = thread & 15;
+        if (h < p.heads) {
+            float w = 0.0f;
+            if (!p.ml) {
+                w = sigmoid_f32(gate);
+            } else {
+                const float sink2 = gate * 1.44269504088896340736f, m = wave_row_max(fmaxf(sink2, e.x));
+                w = __builtin_amdgcn_exp2f(e.x - m);
+                w *= 1.0f / (wave_row_sum(fmaf(e.y, w, 0.0f)) + __builtin_amdgcn_exp2f(sink2 - m));
+            }
+            if (z < p.splits) wz[h * p.splits + z] = w;
+        }
+        partials_weights(p, 0, p.heads, thread, threads, wz, threads >> 4);
+    }
+};
 // columns c .. c + 3 (c a multiple of 4, below vdim_p) of head h; wz: the head's weights
 __device__ __forceinline__ f32x4 partials_sum4(const SAttnPartials& p, const float* wz, uint32_t h, uint32_t c) {
     const uint64_t slice = static_cast<uint64_t>(p.heads) * p.vdim_p;
