@@ -40,6 +40,10 @@ struct DenseOut {
     uint32_t rows = 0;            // output elements per token
     const DenseStreams* streams = nullptr;   // DENSE_STREAMS, host
     float* u = nullptr;                      // DENSE_STREAMS: the next reader's input, rows as x's
+    // DENSE_STREAMS of many tokens: that input's RMS norm with the weights `norm` [ld] into `normed` [n][ld], pads zero (nullable; u is then scratch)
+    const float* norm = nullptr;
+    void* normed = nullptr;
+    float eps = 0;
 };
 // Several products of the same shape in one launch, as the heads of a layer have them: number g reads rows
 // [g * w.rows / count, ...) of the matrix and its own columns of x, and writes its own columns of out.

@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "bf16.hip.h"
+#include "conv_norm.h"
 #include "dense.h"
 #include "lds_dma.hip.h"
 #include "partials.hip.h"
@@ -38,8 +39,8 @@ struct GemmDArgs {
     DenseStreams st;
 };
 
-// four consecutive channels of every stream (n < 4: the first n of them).  S: the number of streams, 0: any, at run time
-template <int SN> __device__ __forceinline__ void dense_streams4(const DenseStreams& st, float* x, float* u, bool vec, int n, const float (&y)[4]) {
+// four consecutive channels of every stream (n < 4: the first n of them); sum: the next reader's.  S: the number of streams, 0: any, at run time
+template <int SN> __device__ __forceinline__ void dense_streams4(const DenseStreams& st, float* x, bool vec, int n, const float (&y)[4], float (&sum)[4]) {
     constexpr int S = SN ? SN : static_cast<int>(DENSE_MAX_STREAMS);
     float o[S][4];
 #pragma unroll
@@ -54,7 +55,8 @@ template <int SN> __device__ __forceinline__ void dense_streams4(const DenseStre
                 for (int i = 0; i < 4; ++i) o[s][i] = i < n ? p[i] : 0.0f;
             }
         }
-    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = 0.0f;
 #pragma unroll
     for (int t = 0; t < S; ++t)
         if (SN || t < static_cast<int>(st.count)) {
@@ -74,11 +76,6 @@ template <int SN> __device__ __forceinline__ void dense_streams4(const DenseStre
                 for (int i = 0; i < 4; ++i)
                     if (i < n) p[i] = v[i];
         }
-    if (vec) *reinterpret_cast<float4*>(u) = make_float4(sum[0], sum[1], sum[2], sum[3]);
-    else
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i < n) u[i] = sum[i];
 }
 // one channel of every stream
 template <int SN> __device__ __forceinline__ void dense_streams1(const DenseStreams& st, float* x, float* u, float y) {
@@ -135,7 +132,15 @@ template <typename T, int EPI, int SN> __device__ __forceinline__ void dense_sto
         const float y[4] = {v.x, v.y, v.z, v.w};
         float* const x = static_cast<float*>(a.out) + at;
         const int n = static_cast<int>(min(4u, a.m - row));
-        dense_streams4<SN>(a.st, x, a.u + at, n == 4 && a.vec, n, y);
+        const bool vec = n == 4 && a.vec;
+        float* const u = a.u + at;
+        float sum[4];
+        dense_streams4<SN>(a.st, x, vec, n, y, sum);
+        if (vec) *reinterpret_cast<float4*>(u) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+        else
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i < n) u[i] = sum[i];
     } else {
         float* o = static_cast<float*>(a.out) + at;
         if (row + 4 <= a.m && a.vec) {
@@ -444,6 +449,25 @@ template <int EPI, int SN> __global__ __launch_bounds__(256) void dense_gemm_f32
     dense_epilogue<float, EPI, SN, 2, 2>(a, tm * BM + wm * 32, tn * BN + wn * 32, lane, blockIdx.y, acc);
 }
 
+// four rows of a token's partial sums, added in split order
+__device__ __forceinline__ f32x4 dense_parts4(const GemmDArgs& a, uint32_t split, uint32_t tok, uint32_t row) {
+    const uint64_t slice = static_cast<uint64_t>(a.n) * a.m;
+    const float* p = a.part + static_cast<uint64_t>(tok) * a.m + row;
+    f32x4 v{0.f, 0.f, 0.f, 0.f};
+    if ((a.m & 3) == 0) {
+#pragma unroll 4
+        for (uint32_t z = 0; z < split; ++z) v += *reinterpret_cast<const f32x4*>(p + z * slice);
+        return v;
+    }
+    for (uint32_t z = 0; z < split; ++z) {
+        const float* s = p + z * slice;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (row + i < a.m) v[i] += s[i];
+    }
+    return v;
+}
+
 // split K: adds the partial sums in split order, then the epilogue.  One thread per four rows of a token
 // (SWIGLU: per four outputs).
 template <typename T, int EPI, int SN>
@@ -452,28 +476,48 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(GemmDArgs a, uint32_t
     const uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (t >= static_cast<uint64_t>(quads) * a.n) return;
     const uint32_t tok = static_cast<uint32_t>(t / quads), q = static_cast<uint32_t>(t % quads) * 4;
-    const uint64_t slice = static_cast<uint64_t>(a.n) * a.m;
-    const float* p = a.part + static_cast<uint64_t>(tok) * a.m;
-    auto sum4 = [&](uint32_t row) {
-        f32x4 v{0.f, 0.f, 0.f, 0.f};
-        if ((a.m & 3) == 0) {
-#pragma unroll 4
-            for (uint32_t z = 0; z < split; ++z) v += *reinterpret_cast<const f32x4*>(p + z * slice + row);
-            return v;
-        }
-        for (uint32_t z = 0; z < split; ++z) {
-            const float* s = p + z * slice + row;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (row + i < a.m) v[i] += s[i];
-        }
-        return v;
-    };
+    auto sum4 = [&](uint32_t row) { return dense_parts4(a, split, tok, row); };
     if constexpr (EPI == DENSE_SWIGLU) {
         const uint32_t row = (q >> 4) * 32 + (q & 15);
         dense_swiglu4<T>(a, q, tok, sum4(row), sum4(row + 16));
     } else {
         dense_store4<T, EPI, SN>(a, q, tok, sum4(q));
+    }
+}
+
+// The same for streams, with the next reader's RMS norm behind it: a workgroup takes a token, keeps the next reader's input in LDS and
+// writes that input's norm alone.  Bound by bytes, of which the input's way out and back is a fifth with four streams and two parts.
+// Every wavefront takes the whole row's sum of squares, in norm_conv_kernel's order: the same bits, and no second barrier.
+// Threads: four channels each, up to 1024 while there are no more workgroups than CUs, 512 beyond (256 / 512 / 1024: 40 tokens of 4096
+// channels 11.2 / 8.3 / 7.8 us, 2048 tokens 68 / 63 / 77).  3072 channels, 2048 tokens, four streams in two parts: 50 us and 12.5 of the
+// norm before, 47 now (5.6 TB/s).
+template <typename T, int SN>
+__global__ __launch_bounds__(1024) void dense_reduce_norm_kernel(GemmDArgs a, uint32_t split, const float* w, float eps, T* out) {
+    extern __shared__ __align__(16) float next_row[];   // [ldo]
+    const uint32_t tok = blockIdx.x, ld = static_cast<uint32_t>(a.ldo), step = blockDim.x * 4;
+    const uint64_t at = static_cast<uint64_t>(tok) * ld;
+    for (uint32_t c = threadIdx.x * 4; c < ld; c += step) {
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        if (c < a.m) {
+            const f32x4 v = dense_parts4(a, split, tok, c);
+            const float y[4] = {v.x, v.y, v.z, v.w};
+            const int n = static_cast<int>(min(4u, a.m - c));
+            dense_streams4<SN>(a.st, static_cast<float*>(a.out) + at + c, n == 4 && a.vec, n, y, sum);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] = i < n ? sum[i] : 0.0f;
+        }
+        *reinterpret_cast<float4*>(next_row + c) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    }
+    __syncthreads();
+    float ss = 0.0f;
+    for (uint32_t c = (threadIdx.x & 63) * 4; c < ld; c += 256) {
+        const float4 v = *reinterpret_cast<const float4*>(next_row + c);
+        ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
+    }
+    const float s = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(a.m) + eps);
+    for (uint32_t c = threadIdx.x * 4; c < ld; c += step) {
+        const float4 v = *reinterpret_cast<const float4*>(next_row + c), g = *reinterpret_cast<const float4*>(w + c);
+        ElemOps<T>::store4(out + at + c, v.x * s * g.x, v.y * s * g.y, v.z * s * g.z, v.w * s * g.w);
     }
 }
 
@@ -918,6 +962,7 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
         return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "dense_gemm: bad shape");
     if (o.epi == DENSE_SWIGLU && w.rows % 32) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "dense_gemm: gate | up rows come in groups of 32");
     if (o.epi == DENSE_STREAMS && (!streams_ok(o) || groups.count != 1)) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "dense_gemm: streams");
+    if (o.norm && (o.epi != DENSE_STREAMS || !o.normed || o.ld % 4 || o.rows != w.rows)) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "dense_gemm: norm");
     GemmDArgs a{};
     a.w = static_cast<const __bf16*>(w.w); a.x = x; a.ldx = ldx; a.m = w.rows / groups.count; a.n = n; a.kp = w.kp;
     a.gw = static_cast<uint64_t>(a.m) * w.kp; a.groups = groups.count; a.gx = groups.x_stride;
@@ -948,6 +993,10 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
     const dim3 grid((units + halves) * 8, split);
     const uint64_t quads = (a.epi == DENSE_SWIGLU ? (a.m / 2 + 3) / 4 : (a.m + 3) / 4) * static_cast<uint64_t>(n);
     const dim3 rg(static_cast<uint32_t>((quads + 255) / 256)), block(256);
+    // the norm behind streams, in the reduction where there is one and its LDS holds a row
+    const uint64_t row_bytes = o.ld * sizeof(float);
+    const bool norm_here = o.norm && a.part && row_bytes <= 65536;
+    const uint32_t norm_threads = static_cast<uint32_t>(std::min<uint64_t>(n > ctx->n_cu ? 512 : 1024, (o.ld / 4 + 63) / 64 * 64));
     auto go = [&](auto epi, auto streams) {
         constexpr int E = decltype(epi)::value, SN = decltype(streams)::value;
         constexpr int EG = E == DENSE_STREAMS && SN == 0 ? DENSE_STORE : E, EL = E == DENSE_STREAMS ? DENSE_STORE : E;   // leave partial sums, whatever it is
@@ -958,6 +1007,13 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
         else if (shape == 1) hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 64, 2, 2>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((dense_gemm_bf16_kernel<EG, SN, 64, 32, 2, 2>), grid, block, 0, ctx->stream, a);
         if (!a.part) return;
+        if constexpr (E == DENSE_STREAMS) {
+            if (norm_here) {
+                if (f32) hipLaunchKernelGGL((dense_reduce_norm_kernel<float, SN>), dim3(n), dim3(norm_threads), row_bytes, ctx->stream, a, split, o.norm, o.eps, static_cast<float*>(o.normed));
+                else hipLaunchKernelGGL((dense_reduce_norm_kernel<__bf16, SN>), dim3(n), dim3(norm_threads), row_bytes, ctx->stream, a, split, o.norm, o.eps, static_cast<__bf16*>(o.normed));
+                return;
+            }
+        }
         if (f32) hipLaunchKernelGGL((dense_reduce_kernel<float, E, SN>), rg, block, 0, ctx->stream, a, split);
         else hipLaunchKernelGGL((dense_reduce_kernel<__bf16, E, SN>), rg, block, 0, ctx->stream, a, split);
     };
@@ -973,7 +1029,10 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
             else go(std::integral_constant<int, DENSE_STREAMS>{}, any);
     }
     HIP_TRY(ctx, hipGetLastError());
-    return CERA_HIP_OK;
+    if (!o.norm || norm_here) return CERA_HIP_OK;
+    NormConv nc;
+    nc.x = o.u; nc.ld = o.ld; nc.n = n; nc.width = o.rows; nc.eps = o.eps; nc.w = o.norm; nc.out_a = o.normed;
+    return cera_launch_norm_conv(ctx, nc, f32);
 }
 
 cera_hip_status cera_launch_dense_gemv(cera_hip_ctx* ctx, const DenseIn& in, const DenseMat& wa, const DenseOut& oa,

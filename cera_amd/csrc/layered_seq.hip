@@ -183,12 +183,17 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
         nc.x = x; nc.ld = g.ld; nc.n = rows; nc.width = width; nc.eps = g.cfg.eps; nc.w = w; nc.out_a = g.ba;
         return cera_launch_norm_conv(ctx, nc, g.f32);
     };
-    auto streams = [&](DenseStreams& st) {
+    // next: the norm in front of the next sublayer, none behind the last one, whose u is the result
+    auto streams = [&](DenseStreams& st, const float* next) {
         st.stride = stride;
-        return to_streams(st, g.bx, g.bu, g.ld, width);
+        DenseOut o = to_streams(st, g.bx, g.bu, g.ld, width);
+        o.norm = next; o.normed = g.ba; o.eps = g.cfg.eps;
+        return o;
     };
-    for (SeqLayer& W : g.seq) {
-        CERA_TRY(norm(g.bu, n, W.norm));
+    CERA_TRY(norm(g.bu, n, g.seq[0].norm));
+    for (size_t i = 0; i < g.seq.size(); ++i) {
+        SeqLayer& W = g.seq[i];
+        const float* const next = i + 1 < g.seq.size() ? g.seq[i + 1].norm : nullptr;
         DenseOut proj;
         proj.out = g.bqkvg; proj.ld = dense_pad(W.in.rows); proj.rows = W.in.rows;
         CERA_TRY(cera_launch_dense_gemm(ctx, W.in, g.ba, g.ld, n, proj, g.f32));
@@ -203,13 +208,12 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
             CERA_TRY(cera_launch_fattn_prep(ctx, W.attn, p, prep, g.f32));
             CERA_TRY(cera_launch_fattn(ctx, W.attn, p, nullptr, 0, g.f32));
         }
-        CERA_TRY(cera_launch_dense_gemm(ctx, W.o, g.bcat, W.o.kp, n, streams(W.st_mixer), g.f32));
+        CERA_TRY(cera_launch_dense_gemm(ctx, W.o, g.bcat, W.o.kp, n, streams(W.st_mixer, W.ff ? W.norm_ffn : next), g.f32));
         if (!W.ff) continue;
-        CERA_TRY(norm(g.bu, n, W.norm_ffn));
         DenseOut act;
         act.epi = DENSE_RELU2; act.out = g.bb; act.ld = W.down.kp; act.rows = W.ff;
         CERA_TRY(cera_launch_dense_gemm(ctx, W.up, g.ba, g.ld, n, act, g.f32));
-        CERA_TRY(cera_launch_dense_gemm(ctx, W.down, g.bb, W.down.kp, n, streams(W.st_ffn), g.f32));
+        CERA_TRY(cera_launch_dense_gemm(ctx, W.down, g.bb, W.down.kp, n, streams(W.st_ffn, next), g.f32));
     }
     m->hidden = g.bu + static_cast<uint64_t>(n - 1) * g.ld;
     if (!last && !all) return CERA_HIP_OK;
