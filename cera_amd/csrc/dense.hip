@@ -285,13 +285,19 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(GemmDArgs a) {
 // 256 x 256 tile, eight wavefronts as 2 x 4, each 128 rows x 64 tokens: 24 KB of fragments per wavefront and K step of 64
 // against 32 KB of the same work on 128 x 128 tiles, whose four wavefronts read LDS for as long as they multiply.  One
 // barrier a K step, in its middle: behind it the step's second half is in registers, so its buffer takes the K step after
-// next while that half is multiplied.  What bounds it: a K step is 2048 clocks of the matrix cores and 2048 of LDS (192 KB
-// read, 64 KB written at 128 bytes a clock); one workgroup alone takes 2660 for it, a full chip 3440, with the matrix cores busy
-// for 52 % of 28672 x 4096 times 1900 tokens in four rounds, and for 56 % with the last one by halves (below).  28672 x 4096 times 2048 / 512 tokens: 1100 / 1040 TFLOP/s, 128 x 128
-// tiles 900 / 750; 8192 x 3072 times 2048 tokens 1070, 990.  The sums have the same order.
+// next while that half is multiplied.  The order is written out: before each twelfth of the products a fragment of the next half and,
+// in the second half, a piece of the step after next; the compiler's own had all pieces in one burst and takes 2 % longer.  A step's
+// weights come from HBM to the first workgroup of an XCD that asks, and the others, in step with it, wait as well, for longer than two
+// steps last: so each, of the rows that all share, reads its part of the lines into the L2 WIDE_AHEAD steps before they are staged.
+// What bounds it: the chip's power.  A K step is 2048 clocks of the matrix cores and 2048 of LDS (192 KB read, 64 KB written at 128
+// bytes a clock); it takes 2600 on a full chip, at 1.5 to 1.85 GHz (3050 at up to 2.0 with neither).  Before and now, over rotating
+// weights: 28672 x 4096 times 2048 / 1024 / 512 tokens 475 -> 448, 253 -> 248, 143 -> 140 us, 8192 x 8192 times 2048 268 -> 245 (1120
+// TFLOP/s), 8192 x 3072 119 -> 112, 3072 x 8192 in two parts 124 -> 118.  128 x 128 tiles are at 750 to 900 TFLOP/s.  The sums have the
+// same order.
 // MI: 16-row tiles of a wavefront: 8, or 4 for 128 x 256 (row0: the workgroup's first weight row)
+constexpr int WIDE_AHEAD = 3;   // 2 and 5: the same within 1 %
 constexpr int WIDE_BK = 64, WIDE_HALF = 256 * WIDE_BK, WIDE_BUF = 2 * WIDE_HALF;
-template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_body(GemmDArgs& a, __bf16 (*lds)[WIDE_BUF], uint32_t row0, uint32_t tn, uint32_t group) {
+template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_body(GemmDArgs& a, __bf16 (*lds)[WIDE_BUF], const uint32_t* sink, uint32_t row0, uint32_t tn, uint32_t group) {
     constexpr int B = 256, BK = WIDE_BK, NI = 4, HALF = WIDE_HALF, BUF = WIDE_BUF, WP = MI / 2, LOADS = WP + 4;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t k0 = blockIdx.y * a.k_chunk, k1 = min(a.kp, k0 + a.k_chunk), steps = (k1 - k0) / BK;
@@ -311,68 +317,77 @@ template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_bo
         off[s] = min(r, x ? last_x : last_w) * (x ? ldx : ldw) + (slot ^ sub) * 16;
     }
     const uint32_t dst = lds_addr(&lds[0][0]) + wave * (MI == 8 ? 8192 : WP * 1024), dst_x = lds_addr(&lds[0][0]) + HALF * 2 + wave * 4096;
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int s = 0; s < LOADS; ++s) {
-            if (MI == 8 || s < WP) lds_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
-            else lds_dma_1k(src_x, off[s], dst_x + buf * BUF * 2 + (s - WP) * 1024);
-        }
+    auto stage1 = [&](int buf, int s) {
+        if (MI == 8 || s < WP) lds_dma_1k(src, off[s], dst + buf * BUF * 2 + s * 1024);
+        else lds_dma_1k(src_x, off[s], dst_x + buf * BUF * 2 + (s - WP) * 1024);
+    };
+    // `s`: the step staged last.  Behind the end of K the last step comes again, into a buffer that is not read
+    auto next_step = [&](uint32_t s) {
+        if (s + 1 >= steps) return;
         src = lds_dma_base(src + BK * 2);
         if (MI != 8) src_x = lds_dma_base(src_x + BK * 2);
     };
+    // this workgroup's share of the weight rows that its neighbours on the XCD read too: a line of them each step, ahead of its use
+    const uint32_t share = (MI * 32 + a.tiles_n - 1) / a.tiles_n;
+    const uint32_t ahead_row = min(min(tn * share + (threadIdx.x * share >> 9), MI * 32u - 1), last_w) * ldw;
+    auto ahead = [&](uint32_t s) { lds_dma_256(lds_dma_base(base_w + min(s, steps - 1) * (BK * 2)), ahead_row, lds_addr(sink)); };
     const uint32_t wm = wave >> 2, wn = wave & 3, fr = lane & 15, fg = lane >> 4;
+    constexpr int FR = MI + NI;
+    static_assert(LOADS <= FR);
     bf16x8 fa[2][MI], fb[2][NI];
-    auto frags = [&](int buf, int kk) {
+    // fragment f of half a step, in the order of their use
+    auto frag = [&](int buf, int kk, int f) {
         const uint32_t o = ((kk * 4 + fg) ^ (fr & 7)) * 8;
         const __bf16* const aw = &lds[buf][(wm * (MI * 16) + fr) * BK + o];
         const __bf16* const bx = &lds[buf][HALF + (wn * 64 + fr) * BK + o];
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) fa[kk][mi] = *reinterpret_cast<const bf16x8*>(aw + mi * 16 * BK);
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) fb[kk][ni] = *reinterpret_cast<const bf16x8*>(bx + ni * 16 * BK);
+        if (f == 0) fb[kk][0] = *reinterpret_cast<const bf16x8*>(bx);
+        else if (f <= MI) fa[kk][f - 1] = *reinterpret_cast<const bf16x8*>(aw + (f - 1) * 16 * BK);
+        else fb[kk][f - MI] = *reinterpret_cast<const bf16x8*>(bx + (f - MI) * 16 * BK);
     };
     f32x4 acc[MI][NI];
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int kk) {
+    // the products of half a step, and before each FR-th of them what `before` does: left in this order
+    auto multiply = [&](int kk, auto&& before) {
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
+        for (int f = 0; f < FR; ++f) {
+            before(f);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[kk][mi], fb[kk][ni], acc[mi][ni], 0, 0, 0);
-        // the reads of the next fragments between the matrix instructions
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-#pragma unroll
-        for (int i = 0; i < MI + NI; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, (MI * NI - 8) / (MI + NI), 0);
+            for (int j = f * MI * NI / FR; j < (f + 1) * MI * NI / FR; ++j)
+                acc[j % MI][j / MI] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[kk][j % MI], fb[kk][j / MI], acc[j % MI][j / MI], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
     };
     auto step = [&](uint32_t s, int buf) {
-        frags(buf, 1);
-        multiply(0);
-        // the next step's pieces are in, and no wavefront reads this buffer any more
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (s + 2 < steps) stage(buf);
-        if (s + 1 < steps) frags(buf ^ 1, 0);
-        multiply(1);
-        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, [&](int f) { frag(buf, 1, f); });
+        // the next step's pieces are in, if not what is read ahead, and no wavefront reads this buffer any more
+        asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        multiply(1, [&](int f) {
+            frag(buf ^ 1, 0, f);   // behind the last step what is there, for nothing
+            if (f < LOADS) stage1(buf, f);
+        });
+        next_step(s + 2);
+        ahead(s + 2 + WIDE_AHEAD);
     };
-    stage(0);
-    if (steps > 1) {
-        stage(1);
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS) : "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int f = 0; f < LOADS; ++f) stage1(i, f);
+        next_step(i);
     }
-    frags(0, 0);
+#pragma unroll
+    for (int i = 0; i < WIDE_AHEAD; ++i) ahead(2 + i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LOADS + WIDE_AHEAD) : "memory");
+#pragma unroll
+    for (int f = 0; f < FR; ++f) frag(0, 0, f);
     for (uint32_t s = 0; s < steps; s += 2) {
         step(s, 0);
         if (s + 1 < steps) step(s + 1, 1);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     a.out = static_cast<char*>(a.out) + group * a.go;
     dense_epilogue<__bf16, EPI, SN, MI, NI>(a, row0 + wm * (MI * 16), tn * B + wn * 64, lane, blockIdx.y, acc);
 }
@@ -382,6 +397,7 @@ template <int EPI, int SN, int MI> __device__ __forceinline__ void dense_wide_bo
 template <int EPI, int SN, bool HALVES>
 __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
     __shared__ __align__(1024) __bf16 lds[2][WIDE_BUF];
+    __shared__ uint32_t sink[64];   // what is read ahead
     uint32_t tm, tn, group;
     if constexpr (HALVES) {
         const uint32_t xcd = blockIdx.x & 7, at = blockIdx.x >> 3, half = at < a.whole ? 0 : at - a.whole, t = at < a.whole ? at : a.whole + half / 2;
@@ -392,11 +408,11 @@ __global__ __launch_bounds__(512, 2) void dense_gemm_wide_kernel(GemmDArgs a) {
         tm = i - group * a.tiles_m;
         if (at >= a.whole) {
             const uint32_t row0 = tm * 256 + (half & 1) * 128;
-            if (row0 < a.m) dense_wide_body<EPI, SN, 4>(a, lds, row0, tn, group);
+            if (row0 < a.m) dense_wide_body<EPI, SN, 4>(a, lds, sink, row0, tn, group);
             return;
         }
     } else if (!dense_tile(a, tm, tn, group)) return;
-    dense_wide_body<EPI, SN, 8>(a, lds, tm * 256, tn, group);
+    dense_wide_body<EPI, SN, 8>(a, lds, sink, tm * 256, tn, group);
 }
 
 // 64 x 64 tile in true f32: weights widened on their way into LDS, K in steps of 32.  A lane's four
