@@ -922,15 +922,39 @@ static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_
     }
     return 0;
 }
+// The same for a product whose sums need no reduction, or 0: the number of parts, up to eight of at least eight steps, for which
+// the estimates below are least, if that is less than 0.92 of the one of 128 x 128 tiles with `split` parts; from 2048 columns on, the
+// shortest measured.  In us, from 48 products of 1024 to 6144 rows, 2048 to 18432 columns and 200 to 2048 tokens, reductions included,
+// most within 15 %: 256 x 256 tiles 1.1 a step and round and, as power is what they run out of, up to 1.65 with how full the rounds are;
+// 128 x 128 ones 1.0, in rounds of two a CU; partial sums 3.5 TB/s and a launch.  On 128 x 128 tiles and by the rule: 4096 x 18432
+// times 1900 / 2048 tokens (2 parts) 342 -> 259 and 344 -> 265 us, 3072 x 11264 times 1900 / 1024 / 700 (2, 4, 5) 196 -> 152, 135 -> 89
+// and 98 -> 74, 6144 x 8192 times 700 (3) 139 -> 85, 6144 x 4096 times 1400 (1) 104 -> 89; of 80 sizes the worst 1 % behind.  Refused: 5120 x
+// 8192 times 1400 130 (153 in 3), 4096 x 4096 times 1900 68 (77 in 2), 3072 x 2048 times 1568 46.5 (49 in 2).  64 x 64 tiles, where they
+// are taken, are ahead at all of 36 sizes.
+static uint32_t dense_wide_split(uint64_t m, uint64_t n, uint32_t steps, uint64_t wgs, uint32_t split, uint32_t n_cu) {
+    const uint64_t per_xcd = std::max<uint64_t>(n_cu / 8, 1), most = ((m + 255) / 256 + 7) / 8 * ((n + 255) / 256), tiles = (m + 255) / 256 * ((n + 255) / 256);
+    auto sums = [&](uint32_t parts) { return parts > 1 ? 2.0 + parts * m * n * 4 / 3.5e6 : 0.0; };
+    const uint64_t rounds128 = (wgs * split + 2 * n_cu - 1) / (2 * n_cu);
+    double best = 0.92 * (4.0 + rounds128 * ((steps + split - 1) / split) * 1.0 + sums(split));
+    uint32_t take = 0;
+    for (uint32_t parts = 1; n > 128 && steps >= 32 && parts <= 8; ++parts) {
+        const uint32_t per = (steps + parts - 1) / parts;
+        if (per < 8 || (steps + per - 1) / per != parts) continue;
+        const uint64_t rounds = (most * parts + per_xcd - 1) / per_xcd;
+        const double fill = static_cast<double>(tiles * parts) / (rounds * per_xcd * 8), t = 8.0 + rounds * per * (1.1 + 0.55 * fill) + (parts > 1 ? 2.0 + sums(parts) : 0.0);
+        if (t < best) { best = t; take = parts; }
+    }
+    return take;
+}
 // How a product is cut: its tile, the parts of K, and whether its sums go through the reduction.
 struct DensePlan {
     int shape;
     uint32_t split;
     bool apart;   // even if K is whole
-    bool wide;    // 256 x 256 tiles by dense_wide_parts
+    bool wide;    // 256 x 256 tiles by dense_wide_parts or dense_wide_split
     uint64_t sums(uint64_t m, uint64_t n) const { return split > 1 || apart ? split * n * m * sizeof(float) : 0; }   // bytes of partial sums
 };
-// streams: of DENSE_STREAMS, else 0.  wide: 256 x 256 tiles may take streams in parts of K
+// streams: of DENSE_STREAMS, else 0.  wide: 256 x 256 tiles may take in parts of K what 128 x 128 ones would
 static DensePlan dense_plan(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uint32_t streams, bool f32, bool wide, uint32_t n_cu) {
     DensePlan p{f32 ? 2 : dense_shape(m, kp, n, groups, n_cu), 1, false, false};
     const uint64_t bm = f32 ? 64 : DENSE_BM[p.shape], bn = f32 ? 64 : DENSE_BN[p.shape], wgs = (m + bm - 1) / bm * ((n + bn - 1) / bn) * groups;
@@ -943,7 +967,9 @@ static DensePlan dense_plan(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups
     // streams on large tiles, and any number of them but four: through the reduction, whose threads hold little else and walk
     // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
     p.apart = streams && (streams != 4 || p.shape == 0 || p.shape == 3);
-    if (const uint32_t parts = wide && p.apart && p.shape == 0 ? dense_wide_parts(m, n, steps, wgs, p.split, n_cu) : 0) {
+    uint32_t parts = 0;
+    if (wide && p.shape == 0 && groups == 1) parts = p.apart ? dense_wide_parts(m, n, steps, wgs, p.split, n_cu) : dense_wide_split(m, n, steps, wgs, p.split, n_cu);
+    if (parts) {
         p.shape = 3;
         p.split = parts;
         p.wide = true;

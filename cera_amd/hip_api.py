@@ -241,7 +241,7 @@ def dense_tile(rows: int, k: int, n: int, n_cu: int = 256) -> int:
 
 
 def dense_streams_tile(rows: int, k: int, n: int, streams: int, room: int = 1 << 62, n_cu: int = 256):
-    """(weight rows of the tile, parts of K) of a product that updates residual streams, with room for that many bytes of partial sums."""
+    """(weight rows of the tile, parts of K) of a product that updates that many residual streams (0: none), with room for that many bytes of partial sums."""
     parts = C.c_uint32()
     return int(load_library().cera_hip_dense_streams_tile(rows, k, n, streams, room, n_cu, C.byref(parts))), parts.value
 

@@ -548,10 +548,11 @@ typedef struct {
 CERA_HIP_API cera_hip_status cera_hip_layered_create(cera_hip_ctx*, const cera_hip_layered_config*,
                                                      const cera_hip_layered_layer* layers, cera_hip_model** out);
 /* The rule by which a bf16 product [rows][k] times n tokens of such a model takes its tile, as plain arithmetic (no device
- * is touched): weight rows of the tile -- 256 (times 256 tokens), 128 (128) or 64 (64 or 32) -- on a device of n_cu CUs. */
+ * is touched), from K taken whole: weight rows of the tile -- 256 (times 256 tokens), 128 (128) or 64 (64 or 32) -- on a device of n_cu
+ * CUs.  Where that is 128, 256 x 256 tiles in parts of K may still be faster, and are taken: cera_hip_dense_streams_tile. */
 CERA_HIP_API uint32_t cera_hip_dense_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t n_cu);
-/* The same for a product that updates `streams` residual streams, which may take larger tiles in parts of K: with room for
- * `room` bytes of partial sums; *parts (nullable): the parts of K. */
+/* The tile in the end, of a product that updates `streams` residual streams (0: none), which may take larger tiles in parts of K: with
+ * room for `room` bytes of partial sums; *parts (nullable): the parts of K. */
 CERA_HIP_API uint32_t cera_hip_dense_streams_tile(uint64_t rows, uint64_t k, uint32_t n, uint32_t streams, uint64_t room, uint32_t n_cu, uint32_t* parts);
 CERA_HIP_API void cera_hip_model_destroy(cera_hip_model*);
 /* Model::forward (cera/src/model/mod.rs:200-606; LlamaModel::forward,

@@ -47,3 +47,18 @@ def test_streams_with_less_room_take_the_next_smaller_plan(streams):
     one = rows * n * 4
     for room, want in ((2 * one, (256, 2)), (2 * one - 1, (128, 1)), (one, (128, 1)), (one - 1, (64 if streams == 4 else 128, 1)), (0, (64 if streams == 4 else 128, 1))):
         assert hip_api.dense_streams_tile(rows, k, n, streams, room) == want
+
+
+@pytest.mark.parametrize("rows,k,n,want", [(4096, 18400, 1900, (256, 2)), (3072, 11264, 700, (256, 5)), (6144, 4090, 1400, (256, 1)), (5120, 8192, 1400, (128, 1)),
+                                           (4096, 4096, 1900, (128, 1)), (3072, 2048, 1568, (128, 2)), (4096, 18432, 130, (128, 8)), (8192, 1984, 1000, (128, 1))])
+def test_larger_tiles_in_parts_of_k(rows, k, n, want):
+    """Products that with K whole would take 128 x 128 tiles: 256 x 256 ones in the parts that are estimated fastest, where they are by far;
+    from 2048 columns and 129 tokens on."""
+    assert hip_api.dense_tile(rows, k, n) == 128
+    assert hip_api.dense_streams_tile(rows, k, n, 0) == want
+
+
+def test_less_room_takes_the_smaller_tiles():
+    rows, k, n = 4096, 18432, 2000
+    assert hip_api.dense_streams_tile(rows, k, n, 0, 2 * rows * n * 4) == (256, 2)
+    assert hip_api.dense_streams_tile(rows, k, n, 0, 2 * rows * n * 4 - 1) == (128, 1)
