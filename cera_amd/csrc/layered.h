@@ -112,6 +112,7 @@ const CeraModelOps* layered_seq_ops();
 cera_hip_status layered_seq_check(cera_hip_ctx* ctx, const cera_hip_layered_config& c, const cera_hip_layered_layer* layers);
 cera_hip_status layered_seq_build(cera_hip_model* m, const cera_hip_layered_config& c, const cera_hip_layered_layer* layers);
 void layered_destroy(cera_hip_model* m);
+bool layered_head_direct(const cera_hip_model* m);
 // logits of one residual row through the final norm and the GEMV (the caller has seen that it fits)
 cera_hip_status layered_row_logits(cera_hip_model* m, const float* x);
 // n tokens from start_pos on through `pass`, in portions of one pass

@@ -87,17 +87,18 @@ cera_hip_status layered_batch_logits(cera_hip_model* m, uint32_t n) {
     return CERA_HIP_OK;
 }
 cera_hip_status layered_portions(cera_hip_model* m, LayeredPass pass, const uint32_t* tokens, uint32_t n, uint32_t start, float* last_logits, float* all) {
+    HeadOut head(m);
     if (n == 1) {
         CERA_TRY(m->ops->decode(m, tokens[0], start, true));
         m->seq_len = start + 1;
-        return cera_logits_to_host(m->ctx, all ? all : last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+        return head.fetch(all ? all : last_logits);
     }
     for (uint32_t off = 0; off < n; off += CERA_PREFILL_CHUNK) {
         const uint32_t len = std::min(CERA_PREFILL_CHUNK, n - off);
         CERA_TRY(pass(m, tokens + off, len, start + off, !all && off + len == n, all ? all + static_cast<uint64_t>(off) * m->cfg.vocab : nullptr));
         m->seq_len = start + off + len;
     }
-    return all ? CERA_HIP_OK : cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return all ? CERA_HIP_OK : head.fetch(last_logits);
 }
 
 namespace {
@@ -145,12 +146,13 @@ cera_hip_status layered_rotation(cera_hip_model* m, const cera_hip_attn_spec& s,
     return CERA_HIP_OK;
 }
 
+bool layered_head_direct(const cera_hip_model* m) { return m->layered->step_fits; }
 cera_hip_status layered_row_logits(cera_hip_model* m, const float* x) {
     CeraLayered& g = *m->layered;
     DenseIn in;
     in.kind = DenseIn::NORM; in.x = x; in.n_mean = g.cfg.width; in.eps = g.cfg.eps; in.scale_a = g.final_norm;
     DenseOut out;
-    out.out = m->logits; out.rows = g.cfg.vocab;
+    out.out = cera_head_out(m); out.rows = g.cfg.vocab;
     bool ok = false;
     CERA_TRY(cera_launch_dense_gemv(m->ctx, in, g.head, out, nullptr, nullptr, g.f32, &ok));
     return ok ? CERA_HIP_OK : cera_fail(m->ctx, CERA_HIP_ERR_SHAPE, "logits: the row does not fit the GEMV");
@@ -257,7 +259,7 @@ cera_hip_status ensure_batch(cera_hip_model* m, uint32_t n, bool logits) {
     return CERA_HIP_OK;
 }
 
-// n tokens (at most CERA_PREFILL_CHUNK) from `start`; `last`: the last position's logits into m->logits;
+// n tokens (at most CERA_PREFILL_CHUNK) from `start`; `last`: the last position's logits into cera_head_out(m);
 // all (nullable): every position's logits, host
 cera_hip_status batch_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, uint32_t start, bool last, float* all) {
     L& g = *m->layered;
@@ -305,7 +307,7 @@ cera_hip_status batch_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n
     nc.x = all ? g.bx : m->hidden; nc.ld = g.ld; nc.n = all ? n : 1; nc.width = width; nc.eps = g.cfg.eps; nc.w = g.final_norm; nc.out_a = g.ba;
     CERA_TRY(cera_launch_norm_conv(ctx, nc, g.f32));
     DenseOut out;
-    out.out = all ? g.blogits : m->logits; out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
+    out.out = all ? g.blogits : cera_head_out(m); out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
     CERA_TRY(cera_launch_dense_gemm(ctx, g.head, g.ba, g.ld, nc.n, out, g.f32));
     return all ? cera_logits_to_host(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
 }
@@ -388,7 +390,7 @@ cera_hip_status write_conv(cera_hip_model* m, uint32_t run, const float* rows, u
     return CERA_HIP_OK;
 }
 
-const CeraModelOps OPS = {decode, prefill, prefill_all, truncate, read_kv, write_kv, read_conv, write_conv, layered_destroy};
+const CeraModelOps OPS = {decode, prefill, prefill_all, truncate, read_kv, write_kv, read_conv, write_conv, layered_destroy, layered_head_direct};
 
 }  // namespace
 
@@ -402,6 +404,7 @@ void layered_destroy(cera_hip_model* m) {
     }
     for (void* p : m->owned)
         if (p) (void)hipFree(p);
+    if (m->logits_host) (void)hipHostFree(m->logits_host);
     delete m;
 }
 cera_hip_status layered_bad(cera_hip_ctx* ctx, const std::string& what) { return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "layered_create: " + what); }
@@ -477,6 +480,7 @@ cera_hip_status build(cera_hip_model* m, const cera_hip_layered_config& c, const
     }
     CERA_TRY(layered_put_vec(m, c.final_norm, c.width, ld, &g.final_norm));
     CERA_TRY(layered_alloc_t(m, dense_pad(c.vocab), &m->logits));
+    HeadOut::create(m, c.vocab);
     CERA_TRY(layered_alloc_t(m, 4, &m->scalars));
     if (c.block == CERA_HIP_BLOCK_SEQUENTIAL) return layered_seq_build(m, c, layers);
     CERA_TRY(table(c.pos, &g.pos));

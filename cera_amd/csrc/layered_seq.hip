@@ -221,7 +221,7 @@ cera_hip_status seq_pass(cera_hip_model* m, const uint32_t* tokens, uint32_t n, 
     const uint32_t rows = all ? n : 1;
     CERA_TRY(norm(all ? g.bu : m->hidden, rows, g.final_norm));
     DenseOut out;
-    out.out = all ? g.blogits : m->logits; out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
+    out.out = all ? g.blogits : cera_head_out(m); out.ld = g.cfg.vocab; out.rows = g.cfg.vocab;
     CERA_TRY(cera_launch_dense_gemm(ctx, g.head, g.ba, g.ld, rows, out, g.f32));
     return all ? cera_logits_to_host(ctx, all, g.blogits, static_cast<uint64_t>(n) * g.cfg.vocab * 4) : CERA_HIP_OK;
 }
@@ -282,7 +282,7 @@ DenseStreams streams_of(const float* p, uint32_t n) {   // in | out | mix
     return s;
 }
 
-const CeraModelOps OPS = {seq_decode, prefill, prefill_all, nullptr, read_kv, write_kv, nullptr, nullptr, layered_destroy};
+const CeraModelOps OPS = {seq_decode, prefill, prefill_all, nullptr, read_kv, write_kv, nullptr, nullptr, layered_destroy, layered_head_direct};
 
 }  // namespace
 

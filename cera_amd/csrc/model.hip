@@ -147,6 +147,7 @@ static void free_model(cera_hip_model* m) {
     for (void* p : m->pf_owned)
         if (p) (void)hipFree(p);
     if (m->pf_logits) (void)hipFree(m->pf_logits);
+    if (m->logits_host) (void)hipHostFree(m->logits_host);
     delete m;
 }
 
@@ -298,6 +299,7 @@ extern "C" cera_hip_status cera_hip_model_create(cera_hip_ctx* ctx, const cera_h
         CERA_TRY(af(c.ffn, &m->up));
         CERA_TRY(af(maxk / 32, &m->xs));
         CERA_TRY(af(c.vocab, &m->logits));
+        HeadOut::create(m, c.vocab);
         CERA_TRY(dev_alloc_t(ctx, maxk, &m->xq, tot));
         m->owned.push_back(m->xq);
         CERA_TRY(dev_alloc_t(ctx, 4, &m->scalars, tot));  // [token, pos, argmax, spare]
@@ -646,12 +648,12 @@ static cera_hip_status decode_step(cera_hip_model* m, uint32_t token, uint32_t p
     const float* const last = want_logits ? m->normed : m->hidden;
     const cera_hip_dtensor* o = m->output ? m->output : m->embd;
     bool head_done = false;
-    if (want_logits) CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, m->logits, m->hidden, &head_done));
+    if (want_logits) CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, cera_head_out(m), m->hidden, &head_done));
     if (!head_done) CERA_TRY(norm_quant(m, last, m->output_norm, c.hidden, 1, m->hidden));
     if (want_logits) {
-        if (!head_done) CERA_TRY(project(m, o, m->hidden, m->logits, nullptr));
+        if (!head_done) CERA_TRY(project(m, o, m->hidden, cera_head_out(m), nullptr));
         if (c.logit_scale != 1.0f) {
-            hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, m->logits,
+            hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, cera_head_out(m),
                                1.0f / c.logit_scale, c.vocab);
             HIP_TRY(ctx, hipGetLastError());
         }
@@ -671,11 +673,17 @@ static cera_hip_status set_token_pos(cera_hip_model* m, uint32_t token, uint32_t
     return CERA_HIP_OK;
 }
 
+static bool head_direct(const cera_hip_model* m) {
+    const cera_hip_dtensor* o = m->output ? m->output : m->embd;
+    return !m->ref_order && m->cfg.logit_scale == 1.0f && o->dev_stream;
+}
+
 // one decode step with the logits copied out (the per-token route of the all-logits call)
 cera_hip_status cera_model_decode_logits(cera_hip_model* m, uint32_t token, uint32_t pos, float* logits) {
+    HeadOut head(m);
     CERA_TRY(decode_step(m, token, pos, true));
     m->seq_len = pos + 1;
-    return cera_logits_to_host(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return head.fetch(logits);
 }
 
 // Token-at-a-time prefill (LlamaModel::forward_prefill's per-token route,
@@ -683,11 +691,12 @@ cera_hip_status cera_model_decode_logits(cera_hip_model* m, uint32_t token, uint
 // weight types support the int8 GEMM.
 cera_hip_status cera_model_prefill_per_token(cera_hip_model* m, const uint32_t* tokens, uint32_t n,
                                              uint32_t start_pos, float* last_logits) {
+    HeadOut head(m);
     for (uint32_t i = 0; i < n; ++i) {
         CERA_TRY(decode_step(m, tokens[i], start_pos + i, i + 1 == n));
         m->seq_len = start_pos + i + 1;
     }
-    return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return head.fetch(last_logits);
 }
 
 static cera_hip_status write_kv(cera_hip_model* m, uint32_t layer, const float* k, const float* v, uint32_t n_pos) {
@@ -745,7 +754,7 @@ static cera_hip_status read_kv(cera_hip_model* m, uint32_t layer, float* k_out, 
 // what the model-level entry points (model_api.hip) call for a llama
 static const CeraModelOps* llama_ops() {
     static const CeraModelOps ops = {decode_step, cera_model_prefill, cera_model_prefill_logits_all, nullptr, read_kv, write_kv,
-                                     nullptr, nullptr, free_model};
+                                     nullptr, nullptr, free_model, head_direct};
     return &ops;
 }
 

@@ -103,6 +103,24 @@ static cera_hip_status begin_at(cera_hip_model* m, uint32_t pos) {
     return CERA_HIP_OK;
 }
 
+// The row is read behind a wait for the stream, as the pinned chunks are.
+void HeadOut::create(cera_hip_model* m, uint32_t vocab) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, static_cast<uint64_t>(vocab) * 4, hipHostMallocDefault) == hipSuccess) m->logits_host = static_cast<float*>(p);
+    else (void)hipGetLastError();   // without one the logits go through the context's pinned chunk
+}
+HeadOut::HeadOut(cera_hip_model* model) : m(model) {
+    void* p = nullptr;
+    if (m->logits_host && m->ops->head_direct(m) && hipHostGetDevicePointer(&p, m->logits_host, 0) == hipSuccess) m->head_out = static_cast<float*>(p);
+}
+cera_hip_status HeadOut::fetch(float* logits) {
+    const uint64_t n = static_cast<uint64_t>(m->cfg.vocab) * 4;
+    if (!m->head_out) return cera_logits_to_host(m->ctx, logits, m->logits, n);
+    HIP_TRY(m->ctx, hipStreamSynchronize(m->ctx->stream));
+    std::memcpy(logits, m->logits_host, n);
+    return CERA_HIP_OK;
+}
+
 static cera_hip_status check_step(cera_hip_model* m, uint32_t token, uint32_t pos) {
     CERA_TRY(begin_at(m, pos));
     if (token >= m->cfg.vocab)
@@ -118,8 +136,9 @@ extern "C" cera_hip_status cera_hip_forward(cera_hip_model* m, uint32_t token, u
     if (!m || !logits) return CERA_HIP_ERR_ARGUMENT;
     ModelLock lk(m);
     CERA_TRY(check_step(m, token, pos));
+    HeadOut head(m);
     CERA_TRY(m->ops->decode(m, token, pos, true));
-    CERA_TRY(cera_logits_to_host(m->ctx, logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4));
+    CERA_TRY(head.fetch(logits));
     m->seq_len = pos + 1;
     return CERA_HIP_OK;
 }

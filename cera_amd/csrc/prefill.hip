@@ -852,20 +852,20 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         const float* last = m->pf_hidden + static_cast<uint64_t>(n - 1) * hs;
         const cera_hip_dtensor* o = m->output ? m->output : m->embd;
         bool done = false;   // from the decode copy where the head has one, as the decode step
-        CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, m->logits, m->hidden, &done));
+        CERA_TRY(cera_launch_head_fused(ctx, o, last, m->output_norm, c.rms_eps, cera_head_out(m), m->hidden, &done));
         if (!done) {
             hipLaunchKernelGGL((rmsnorm_kernel<true>), dim3(1), dim3(256), 0, s, last, m->output_norm, hs, c.rms_eps, m->hidden,
                                m->xs, m->xq, static_cast<float*>(nullptr));
             HIP_TRY(ctx, hipGetLastError());
             if (o->dtype == CERA_HIP_Q5_K) {
-                CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, m->logits));
+                CERA_TRY(cera_launch_gemv_q5k_f32(ctx, o, m->hidden, cera_head_out(m)));
             } else {
-                CERA_TRY(cera_launch_row_gemv_store(ctx, o, m->xs, m->xq, m->logits, &done));
-                if (!done) CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, m->logits, nullptr, CERA_EPI_STORE));
+                CERA_TRY(cera_launch_row_gemv_store(ctx, o, m->xs, m->xq, cera_head_out(m), &done));
+                if (!done) CERA_TRY(cera_launch_gemv(ctx, o, nullptr, m->xs, m->xq, cera_head_out(m), nullptr, CERA_EPI_STORE));
             }
         }
         if (c.logit_scale != 1.0f) {
-            hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, m->logits, 1.0f / c.logit_scale, c.vocab);
+            hipLaunchKernelGGL(scale_kernel, dim3((c.vocab + 255) / 256), dim3(256), 0, s, cera_head_out(m), 1.0f / c.logit_scale, c.vocab);
             HIP_TRY(ctx, hipGetLastError());
         }
     }
@@ -932,9 +932,10 @@ cera_hip_status cera_model_prefill(cera_hip_model* m, const uint32_t* tokens, ui
         return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
     }
     if (n == 1 || !prefill_batchable(m)) return cera_model_prefill_per_token(m, tokens, n, start_pos, last_logits);
+    HeadOut head(m);
     for (uint32_t off = 0; off < n; off += PREFILL_CHUNK) {
         uint32_t len = std::min(PREFILL_CHUNK, n - off);
         CERA_TRY(prefill_chunk(m, tokens + off, len, start_pos + off, off + len == n));
     }
-    return cera_logits_to_host(m->ctx, last_logits, m->logits, static_cast<uint64_t>(m->cfg.vocab) * 4);
+    return head.fetch(last_logits);
 }
