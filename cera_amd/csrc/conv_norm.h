@@ -8,6 +8,11 @@
 cera_hip_status cera_launch_embed_pos(cera_hip_ctx* ctx, const void* embed, const void* pos, const uint32_t* tokens, uint32_t n, uint32_t start, uint32_t width,
                                       uint64_t ld, float* x, float* x0);
 
+// The same for one token, and in the launch the convolutions' history sums of all layers for the token at `start`; jobs: device, all
+// of rows of `ld`.
+cera_hip_status cera_launch_embed_hist(cera_hip_ctx* ctx, const void* embed, const void* pos, uint32_t token, uint32_t start, uint32_t width, uint64_t ld,
+                                       float* x, float* x0, const ConvJob* jobs, uint32_t n_jobs);
+
 // x_s[t] = embed[token[t]] for every one of `streams` streams, `stride` floats apart, and u[t] = u_scale * embed[token[t]]
 cera_hip_status cera_launch_embed_streams(cera_hip_ctx* ctx, const void* embed, const uint32_t* tokens, uint32_t n, uint32_t width, uint64_t ld, float* x,
                                           uint32_t streams, uint64_t stride, float u_scale, float* u);

@@ -64,6 +64,7 @@ struct CeraLayered {
     float *x = nullptr, *xb = nullptr, *x0 = nullptr, *qkvg = nullptr;
     void *cat = nullptr, *q = nullptr;
     // state of the sequence
+    ConvJob* conv_jobs = nullptr;      // device: of every pass over a layer, in order; none without convolutions
     uint32_t hist_pos = UINT32_MAX;    // position the convolution history sums are for
     uint32_t ring_lo = 0;              // oldest position the rings still hold
     // batched pass, token-major, `cap_n` rows

@@ -187,7 +187,10 @@ cera_hip_status decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool wan
         if (st == CERA_HIP_OK && !ok) st = cera_fail(ctx, CERA_HIP_ERR_SHAPE, "decode: a product's input does not fit the GEMV");
         return st;
     };
-    CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, &token, 1, pos, width, g.ld, g.x, g.x0));
+    if (g.conv_jobs && g.hist_pos != pos)
+        CERA_TRY(cera_launch_embed_hist(ctx, g.embed, g.pos, token, pos, width, g.ld, g.x, g.x0, g.conv_jobs, static_cast<uint32_t>(g.runs.size())));
+    else
+        CERA_TRY(cera_launch_embed_pos(ctx, g.embed, g.pos, &token, 1, pos, width, g.ld, g.x, g.x0));
     for (Run& R : g.runs) {
         const LayerW& W = g.layers[R.layer];
         if (R.step >= 0) {
@@ -198,7 +201,6 @@ cera_hip_status decode(cera_hip_model* m, uint32_t token, uint32_t pos, bool wan
             CERA_TRY(gemv(in, g.loop_in, out));
             std::swap(g.x, g.xb);
         }
-        if (R.ring.rows && g.hist_pos != pos) CERA_TRY(cera_launch_conv_hist(ctx, R.ring, R.hist, pos));
         DenseIn in;
         in.kind = DenseIn::NORM; in.x = g.x; in.n_mean = width; in.eps = g.cfg.eps;
         in.scale_a = W.scale_a; in.scale_b = W.scale_b;
@@ -570,6 +572,12 @@ cera_hip_status build(cera_hip_model* m, const cera_hip_layered_config& c, const
             CERA_TRY(layered_alloc_t(m, ld, &R.hist.a));
             CERA_TRY(layered_alloc_t(m, ld, &R.hist.b));
         }
+    }
+    if (c.conv_taps > 1) {
+        std::vector<ConvJob> jobs;
+        for (const Run& R : g.runs) jobs.push_back({R.ring, R.hist});
+        CERA_TRY(layered_alloc_t(m, jobs.size(), &g.conv_jobs));
+        CERA_TRY(cera_hip_upload(m->ctx, g.conv_jobs, jobs.data(), jobs.size() * sizeof(ConvJob)));
     }
     CERA_TRY(layered_alloc_t(m, ld, &g.x));
     CERA_TRY(layered_alloc_t(m, ld, &g.xb));

@@ -69,5 +69,10 @@ struct SAttnPartials {
 };
 cera_hip_status cera_launch_sattn_step(cera_hip_ctx* ctx, const SAttnShape& s, const SAttnPass& p, const ConvRing& ring,
                                        const ConvHist& hist, SAttnPartials* merge, bool f32);
+// a layer's, as kernels that add up several layers' read them from memory
+struct ConvJob {
+    ConvRing ring;
+    ConvHist hist;
+};
 // the history sums alone, for the token at `pos`
 cera_hip_status cera_launch_conv_hist(cera_hip_ctx* ctx, const ConvRing& ring, const ConvHist& hist, uint32_t pos);

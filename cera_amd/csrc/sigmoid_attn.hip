@@ -13,6 +13,7 @@
 #include <algorithm>
 
 #include "bf16.hip.h"
+#include "conv_hist.hip.h"
 #include "lds_dma.hip.h"
 #include "sigmoid_attn.h"
 
@@ -386,19 +387,6 @@ __global__ __launch_bounds__(256, 2) void sattn_shared_kernel(AArgs a, uint32_t 
 
 // ---- few queries: the wavefronts of a workgroup (and `splits` workgroups) share the keys ---------
 constexpr int SPLIT_WAVES = 8;
-
-__device__ __forceinline__ void conv_hist_body(const ConvRing& ring, const ConvHist& h, uint32_t pos, uint32_t i) {
-    // history of the token at `pos`: taps 0 .. taps-2 against rows pos - taps + 1 .. pos - 1
-    const float* const w = i < ring.width ? h.wa : h.wb;
-    const uint32_t c = i < ring.width ? i : i - ring.width;
-    if (!w || c >= ring.width) return;
-    float s = 0.0f;
-    for (uint32_t j = 0; j + 1 < h.taps; ++j) {
-        const uint32_t back = h.taps - 1 - j;
-        if (back <= pos) s = fmaf(w[static_cast<uint64_t>(j) * ring.width + c], ring.rows[static_cast<uint64_t>((pos - back) & (ring.depth - 1)) * ring.ld + c], s);
-    }
-    (i < ring.width ? h.a : h.b)[c] = s;
-}
 
 // FUSED: the decode step (n == 1, per <= 16): q, k, v come straight from the projections.  Every workgroup
 // rotates the queries of its kv head; all of a kv head's workgroups but one read a cache that the new
