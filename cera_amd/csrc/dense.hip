@@ -922,7 +922,7 @@ static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_
     }
     return 0;
 }
-// The same for a product whose sums need no reduction, or 0: the number of parts, up to eight of at least eight steps, for which
+// The same for a product whose sums need no reduction, or (`apart`) do and that has no parts by the rule above, or 0: the number of parts, up to eight of at least eight steps, for which
 // the estimates below are least, if that is less than 0.92 of the one of 128 x 128 tiles with `split` parts; from 2048 columns on, the
 // shortest measured.  In us, from 48 products of 1024 to 6144 rows, 2048 to 18432 columns and 200 to 2048 tokens, reductions included,
 // most within 15 %: 256 x 256 tiles 1.1 a step and round and, as power is what they run out of, up to 1.65 with how full the rounds are;
@@ -930,10 +930,11 @@ static uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_
 // times 1900 / 2048 tokens (2 parts) 342 -> 259 and 344 -> 265 us, 3072 x 11264 times 1900 / 1024 / 700 (2, 4, 5) 196 -> 152, 135 -> 89
 // and 98 -> 74, 6144 x 8192 times 700 (3) 139 -> 85, 6144 x 4096 times 1400 (1) 104 -> 89; of 80 sizes the worst 1 % behind.  Refused: 5120 x
 // 8192 times 1400 130 (153 in 3), 4096 x 4096 times 1900 68 (77 in 2), 3072 x 2048 times 1568 46.5 (49 in 2).  64 x 64 tiles, where they
-// are taken, are ahead at all of 36 sizes.
-static uint32_t dense_wide_split(uint64_t m, uint64_t n, uint32_t steps, uint64_t wgs, uint32_t split, uint32_t n_cu) {
+// are taken, are ahead at all of 36 sizes.  With streams, two-layer passes of 14 sizes, before and by the rule: 3072 wide, 8192 inside, 690
+// tokens (5 parts) 676 -> 636 us, 1450 (2) 993 -> 924; 4096 / 14336, 520 (5) 895 -> 822, 380 (8) 691 -> 639; 2048 / 8192, 850 (8) 502 -> 490.
+static uint32_t dense_wide_split(uint64_t m, uint64_t n, uint32_t steps, uint64_t wgs, uint32_t split, bool apart, uint32_t n_cu) {
     const uint64_t per_xcd = std::max<uint64_t>(n_cu / 8, 1), most = ((m + 255) / 256 + 7) / 8 * ((n + 255) / 256), tiles = (m + 255) / 256 * ((n + 255) / 256);
-    auto sums = [&](uint32_t parts) { return parts > 1 ? 2.0 + parts * m * n * 4 / 3.5e6 : 0.0; };
+    auto sums = [&](uint32_t parts) { return parts > 1 || apart ? 2.0 + parts * m * n * 4 / 3.5e6 : 0.0; };
     const uint64_t rounds128 = (wgs * split + 2 * n_cu - 1) / (2 * n_cu);
     double best = 0.92 * (4.0 + rounds128 * ((steps + split - 1) / split) * 1.0 + sums(split));
     uint32_t take = 0;
@@ -968,7 +969,10 @@ static DensePlan dense_plan(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups
     // along the rows.  3072 x 8192 times 2048 tokens, four streams: 118 + 45 us, as the tiles' own epilogue 230
     p.apart = streams && (streams != 4 || p.shape == 0 || p.shape == 3);
     uint32_t parts = 0;
-    if (wide && p.shape == 0 && groups == 1) parts = p.apart ? dense_wide_parts(m, n, steps, wgs, p.split, n_cu) : dense_wide_split(m, n, steps, wgs, p.split, n_cu);
+    if (wide && p.shape == 0 && groups == 1) {
+        if (p.apart) parts = dense_wide_parts(m, n, steps, wgs, p.split, n_cu);
+        if (!parts) parts = dense_wide_split(m, n, steps, wgs, p.split, p.apart, n_cu);
+    }
     if (parts) {
         p.shape = 3;
         p.split = parts;

@@ -62,3 +62,10 @@ def test_less_room_takes_the_smaller_tiles():
     rows, k, n = 4096, 18432, 2000
     assert hip_api.dense_streams_tile(rows, k, n, 0, 2 * rows * n * 4) == (256, 2)
     assert hip_api.dense_streams_tile(rows, k, n, 0, 2 * rows * n * 4 - 1) == (128, 1)
+
+
+@pytest.mark.parametrize("rows,k,n,want", [(3072, 8192, 690, (256, 5)), (4096, 14336, 520, (256, 5)), (2048, 8192, 850, (256, 8)), (3072, 8192, 1450, (256, 2)),
+                                           (3072, 1984, 1450, (128, 2)), (2048, 8192, 400, (128, 8))])
+def test_streams_in_more_parts_of_k(rows, k, n, want):
+    """Where two to four parts do not fill their rounds, as without streams."""
+    assert hip_api.dense_streams_tile(rows, k, n, 4) == want

@@ -12,8 +12,8 @@ from cera_amd import hip_api
 pytestmark = pytest.mark.gpu
 
 
-def _in_parts(rows, k, n):
-    tile, parts = hip_api.dense_streams_tile(rows, k, n, 0)
+def _in_parts(rows, k, n, streams=0):
+    tile, parts = hip_api.dense_streams_tile(rows, k, n, streams)
     return hip_api.dense_tile(rows, k, n) == 128 and tile == 256 and parts > 1
 
 
@@ -32,14 +32,14 @@ def test_residual_swiglu_and_plain_sums(tmp_path, width, ff, n, vocab, products)
     assert err < TN.TOL[False]
 
 
-def test_squared_relu_sums(tmp_path):
-    width, ff, n = 2060, 3001, 1290
-    assert _in_parts(ff, width, n)
-    cfg = F.config([F.attention(2, 1, 32, 32, (0.3, 8), True, ff=ff)], width=width, vocab=40, streams=4)
+@pytest.mark.parametrize("width, ff, n, streams, product", [(2060, 3001, 1290, 4, (3001, 2060, 1290, 0)), (1500, 8200, 700, 3, (1500, 8200, 700, 3)), (1500, 8200, 700, 4, (1500, 8200, 700, 4))])
+def test_squared_relu_and_streams(tmp_path, width, ff, n, streams, product):
+    assert _in_parts(*product)
+    cfg = F.config([F.attention(2, 1, 32, 32, (0.3, 8), True, ff=ff)], width=width, vocab=40, streams=streams)
     w = F.random_model(cfg, 73)
     m = TF._open(F.save(tmp_path / "m", cfg, w), False, n)
     toks = F.tokens(cfg, n, 7)
     err = F.rel(m.forward_prefill_logits_all(toks, 0), F.reference(cfg, w, toks))
     m.close()
-    print(f"parts: squared relu: {err:.2e}", flush=True)
+    print(f"parts: width={width} ff={ff} streams={streams}: {err:.2e}", flush=True)
     assert err < TF.TOL[False]
