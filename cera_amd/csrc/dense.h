@@ -1,11 +1,9 @@
 // Launchers of the float-weight (bfloat16) matrix products: a matrix-core GEMM for many rows of
 // activations and a streaming GEMV for one, with the small operations around them folded in.
 #pragma once
+#include "dense_plan.h"   // DENSE_PAD
 #include "host_common.h"
 #include "sigmoid_attn.h"   // SAttnPartials
-
-constexpr uint32_t DENSE_PAD = 64;   // K is padded with zeros to whole 128-byte lines of bf16
-static inline uint64_t dense_pad(uint64_t k) { return (k + DENSE_PAD - 1) / DENSE_PAD * DENSE_PAD; }
 
 // bf16 weights [rows][kp] in HBM.  kp: a multiple of DENSE_PAD, the pad columns zero.
 struct DenseMat {
