@@ -920,8 +920,9 @@ cera_hip_status cera_launch_dense_gemm(cera_hip_ctx* ctx, const DenseMat& w, con
         return st != CERA_HIP_OK || part;
     });
     CERA_TRY(st);
-    if (!part && plan.apart) CERA_TRY(cera_scratch(ctx, 9, plan.sums(a.m, n), &part));
-    a.part = static_cast<float*>(part);
+    const uint64_t sums = plan.sums(a.m, n);
+    if (sums && !part) CERA_TRY(cera_scratch(ctx, 9, sums, &part));   // cannot do without
+    a.part = sums ? static_cast<float*>(part) : nullptr;              // the kernels take it for partial sums wherever it is set
     const int shape = plan.shape;
     const uint32_t split = plan.split, steps = a.kp / DENSE_PAD, bm = f32 ? 64 : DENSE_BM[shape], bn = f32 ? 64 : DENSE_BN[shape];
     a.k_chunk = (steps + split - 1) / split * DENSE_PAD;

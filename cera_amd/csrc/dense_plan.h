@@ -99,14 +99,15 @@ inline DensePlan dense_plan(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups
     p.split = (steps + per - 1) / per;
     return p;
 }
-// The same for what there is room for, room(bytes) saying so.  Where the larger tiles' parts do not fit, the smaller tiles', which may
-// be fewer; without room for those either, the whole of K in one workgroup, four streams by small tiles' own lanes.
+// The same for what there is room for, room(bytes) saying so; a plan without sums does not ask.  Where the larger tiles' parts do not fit,
+// the smaller tiles', which may be fewer; without room for those either, the whole of K in one workgroup, four streams by small tiles'
+// own lanes.
 template <class Room> inline DensePlan dense_plan_in(uint64_t m, uint64_t kp, uint64_t n, uint64_t groups, uint32_t streams, bool f32, uint32_t n_cu, Room&& room) {
     DensePlan p = dense_plan(m, kp, n, groups, streams, f32, true, n_cu);
     if (!p.sums(m, n) || room(p.sums(m, n))) return p;
     if (p.wide) {
         p = dense_plan(m, kp, n, groups, streams, f32, false, n_cu);
-        if (room(p.sums(m, n))) return p;
+        if (!p.sums(m, n) || room(p.sums(m, n))) return p;
     }
     p.split = 1;
     if (p.apart && streams == 4) { p.shape = 1; p.apart = false; }

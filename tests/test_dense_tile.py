@@ -1,4 +1,7 @@
 """The rules by which a bf16 product takes its tile (cera_hip_dense_tile, cera_hip_dense_streams_tile): plain arithmetic, checked without a GPU."""
+import subprocess
+from pathlib import Path
+
 import pytest
 
 from cera_amd import hip_api
@@ -69,3 +72,15 @@ def test_less_room_takes_the_smaller_tiles():
 def test_streams_in_more_parts_of_k(rows, k, n, want):
     """Where two to four parts do not fill their rounds, as without streams."""
     assert hip_api.dense_streams_tile(rows, k, n, 4) == want
+
+
+def test_the_plan_and_its_workspace_agree(tmp_path):
+    """No product asks for a workspace that its plan does not use, and none has a plan whose sums it was refused."""
+    root = Path(__file__).resolve().parent.parent
+    exe = tmp_path / "dense_plan_room"
+    b = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{root / 'cera_amd' / 'csrc'}", str(root / "tests" / "native" / "dense_plan_room.cpp"), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert b.returncode == 0, b.stderr[-2000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+    assert " 0 of them" not in r.stdout
