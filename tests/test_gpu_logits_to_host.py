@@ -24,7 +24,10 @@ def base(hip):
     return cfg, weights, one, many
 
 
-@pytest.mark.parametrize("vocab", [6, 8, 513, 1000, CHUNK // 12, CHUNK // 12 + 1, CHUNK // 4, CHUNK // 4 + 4])
+ROWS = [6, 8, 513, 1000, CHUNK // 12, CHUNK // 12 + 1, CHUNK // 4, CHUNK // 4 + 4]
+
+
+@pytest.mark.parametrize("vocab", ROWS)
 def test_logits_of_any_number_of_rows(hip, base, vocab):
     cfg, weights, one, many = base
     print(f"logits to host: {vocab} rows", flush=True)
@@ -35,3 +38,22 @@ def test_logits_of_any_number_of_rows(hip, base, vocab):
     m.close()
     assert np.array_equal(got_one.view(np.uint32), np.resize(one, vocab).view(np.uint32))
     assert np.abs(got_many - np.stack([np.resize(r, vocab) for r in many])).max() <= 1e-5 * np.abs(many).max()   # splits of K may follow the row count
+
+
+@pytest.mark.parametrize("vocab", ROWS)
+@pytest.mark.parametrize("route", ["logit scale", "no decode copies"])
+def test_one_row_by_the_copy(hip, base, route, vocab):
+    """One position's logits where the head's launch does not write them into host memory itself."""
+    cfg, weights, one, _ = base
+    print(f"logits to host: {vocab} rows, {route}", flush=True)
+    w = {**weights, **{name: _rows(weights[name], vocab) for name in ("token_embd.weight", "output.weight")}}
+    scale = 4.0 if route == "logit scale" else 1.0
+    m = hip_api.Model(hip, {**cfg, "vocab": vocab, "logit_scale": scale}, w)
+    if route != "logit scale":
+        m.drop_decode_copies()
+    got = [m.forward(3, 0), m.forward_prefill([5, 1, 4], 1)]
+    m.truncate_kv(0)
+    again = [m.forward(3, 0), m.forward_prefill([5, 1, 4], 1)]
+    m.close()
+    assert np.array_equal(got[0].view(np.uint32), np.resize(one * np.float32(1 / scale), vocab).view(np.uint32))   # a power of two: exact
+    assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(got, again))
