@@ -828,7 +828,9 @@ template <typename T, int R, int SN> struct GemvWalk {
     }
 };
 
-// ONE: no wavefront has more than one step.  (A second buffer's load for nothing, or a wait that counts it, costs 0.4 to 1.3 us.)
+// ONE: no wavefront has more than one step, and none loads a second buffer for nothing or waits for it.  Without and with it, 1792 and
+// 2048 wide: behind a norm 5.3 -> 4.6, 6.4 -> 5.6 and 8.9 -> 8.3 us (f32 6.6 -> 5.6, 9.0 -> 8.4), of a finished input 5.7 -> 5.2 and
+// 4.9 -> 4.5 (f32 4.84 -> 4.76), of attention's parts 6.1 -> 5.9 and 6.0 -> 5.7 (f32 6.20 -> 6.12).
 template <typename T, int KIND, int R, int SN, bool ONE = false>
 __global__ __launch_bounds__(GEMV_WAVES * 64, 4) void dense_gemv_kernel(GemvDArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];

@@ -39,11 +39,15 @@ inline uint32_t dense_wide_parts(uint64_t m, uint64_t n, uint32_t steps, uint64_
     }
     return 0;
 }
-// The same for a product whose sums need no reduction, or (`apart`) do and that has no parts by the rule above, or 0: the number of parts, up to eight of at least eight steps, for which
-// the estimates below are least, if that is less than 0.92 of the one of 128 x 128 tiles with `split` parts; from 2048 columns on, the
-// shortest measured.  In us, from 48 products of 1024 to 6144 rows, 2048 to 18432 columns and 200 to 2048 tokens, reductions included,
-// most within 15 %: 256 x 256 tiles 1.1 a step and round and, as power is what they run out of, up to 1.65 with how full the rounds are;
-// 128 x 128 ones 1.0, in rounds of two a CU; partial sums 3.5 TB/s and a launch.  On 128 x 128 tiles and by the rule: 4096 x 18432
+// The same by an estimate, from 2048 columns on, the shortest measured: for products whose sums need no reduction, and for those whose
+// sums go through it anyway (`apart`) where the rule above has no parts.  The number of parts, from K whole to eight of at least eight
+// steps, whose estimate is least, if that is below 0.92 of the one of 128 x 128 tiles with `split` parts, else 0.  In us, from 48 products
+// of 1024 to 6144 rows, 2048 to 18432 columns and 200 to 2048 tokens, most within 15 %: 256 x 256 tiles 1.1 a step and round and, as power
+// is what they run out of, up to 1.65 with how full the rounds are; 128 x 128 ones 1.0, in rounds of two a CU; partial sums 3.5 TB/s and 2
+// for their launch, and 2 more for parts of the larger tiles, which have to earn their workspace.  K whole on the larger tiles counts no
+// sums, also where they go through the reduction: with them the choice would be another at 96 of 1.5 million sizes, five parts in place of
+// one at 8224 to 8800 rows, 14912 columns and 1029 to 1110 tokens, and two-layer passes there 0 to 1.6 % slower (8256 wide, 1040 tokens
+// 2058 -> 2086 us, 8704, 1050 2155 -> 2165, 8448, 1090 2154 -> 2147).  On 128 x 128 tiles and by the rule: 4096 x 18432
 // times 1900 / 2048 tokens (2 parts) 342 -> 259 and 344 -> 265 us, 3072 x 11264 times 1900 / 1024 / 700 (2, 4, 5) 196 -> 152, 135 -> 89
 // and 98 -> 74, 6144 x 8192 times 700 (3) 139 -> 85, 6144 x 4096 times 1400 (1) 104 -> 89; of 80 sizes the worst 1 % behind.  Refused: 5120 x
 // 8192 times 1400 130 (153 in 3), 4096 x 4096 times 1900 68 (77 in 2), 3072 x 2048 times 1568 46.5 (49 in 2).  64 x 64 tiles, where they

@@ -74,5 +74,3 @@ struct ConvJob {
     ConvRing ring;
     ConvHist hist;
 };
-// the history sums alone, for the token at `pos`
-cera_hip_status cera_launch_conv_hist(cera_hip_ctx* ctx, const ConvRing& ring, const ConvHist& hist, uint32_t pos);

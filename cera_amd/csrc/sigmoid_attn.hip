@@ -695,6 +695,12 @@ cera_hip_status cera_launch_sattn(cera_hip_ctx* ctx, const SAttnShape& s, const 
     return CERA_HIP_OK;
 }
 
+// the convolution history alone, for the token at `pos`
+static cera_hip_status launch_conv_hist(cera_hip_ctx* ctx, const ConvRing& ring, const ConvHist& hist, uint32_t pos) {
+    hipLaunchKernelGGL(conv_hist_kernel, dim3((2 * ring.width + 255) / 256), dim3(256), 0, ctx->stream, ring, hist, pos);
+    HIP_TRY(ctx, hipGetLastError());
+    return CERA_HIP_OK;
+}
 cera_hip_status cera_launch_sattn_step(cera_hip_ctx* ctx, const SAttnShape& s, const SAttnPass& p, const ConvRing& ring,
                                        const ConvHist& hist, SAttnPartials* merge, bool f32) {
     if (merge) *merge = SAttnPartials{};
@@ -703,16 +709,10 @@ cera_hip_status cera_launch_sattn_step(cera_hip_ctx* ctx, const SAttnShape& s, c
     if (p.n != 1) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "sigmoid attention step: one token");
     if (a.per > 16) {   // more query heads per kv head than one tile of columns: separate append
         CERA_TRY(cera_launch_sattn_append(ctx, s, p, ConvRing{}, nullptr, 0, nullptr, nullptr, f32));
-        if (ring.rows) CERA_TRY(cera_launch_conv_hist(ctx, ring, hist, p.start + 1));
+        if (ring.rows) CERA_TRY(launch_conv_hist(ctx, ring, hist, p.start + 1));
         return run_split(ctx, a, f32, false, nullptr);
     }
     a.ring = ring;
     a.hist = hist;
     return run_split(ctx, a, f32, true, merge);
-}
-
-cera_hip_status cera_launch_conv_hist(cera_hip_ctx* ctx, const ConvRing& ring, const ConvHist& hist, uint32_t pos) {
-    hipLaunchKernelGGL(conv_hist_kernel, dim3((2 * ring.width + 255) / 256), dim3(256), 0, ctx->stream, ring, hist, pos);
-    HIP_TRY(ctx, hipGetLastError());
-    return CERA_HIP_OK;
 }
