@@ -10,10 +10,10 @@
 // blocks in the order of the kernel before it; the number of slices is i8_slices' own, so that sums in parts have another order.
 //
 // What bounds it: one subtraction and one FMA per output and block.  In 16384 x 3072 Q8_0 (gate | up) times 1001 tokens the vector
-// ALU is busy for 0.66 of the time and the matrix cores for 0.27, in turns; 28672 x 4096 times 2048 tokens 671 us, 717 TOP/s.  The kernel
+// ALU is busy for 0.66 of the time and the matrix cores for 0.27, in turns; 28672 x 4096 times 2048 tokens 671 us, 717 TOP/s, before the order of the folds.  The kernel
 // before it (gemm.hip.h, which keeps Q4_1, rows of about 2^24 columns and more, the block dots and the code object's export)
 // unpacks into LDS, converts, and reads both operands through LDS.  Passes of two layers, before and now:
-//   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039
+//   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039 (986 with the folds in order)
 //   hidden 4096, Q4_0:  9 tokens 331 -> 300 us, 64: 440 -> 374, 128: 591 -> 477, 512: 1181 -> 947, 1001: 2055 -> 1673
 #include "f16_codes.hip.h"
 #include "gemm_i8.h"
@@ -162,9 +162,14 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
             if ((q & 1) == 0 && i == 2) weights(next_half, odd ^ 1, 0);
             if ((q & 1) == 0 && i == 3) weights(next_half, odd ^ 1, 1);
             __builtin_amdgcn_sched_barrier(0);
-            const f16x f = __builtin_bit_cast(f16x, r[i & 1]);
+            f16x f = __builtin_bit_cast(f16x, r[i & 1]);
+            // Sixteen subtractions, then sixteen FMAs: an instruction that waits for the one before it costs its wavefront eight clocks, one that does
+            // not five.  Q8_0, hidden 3072, two layers, 1001 tokens 1023 -> 986 us; 16384 x 3072 times 2048 tokens by itself 336 -> 310.
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[t][e] = fmaf(f[e] - start_f, scale[t & 1][16 * (i & 1) + e], acc[t][e]);
+            for (int e = 0; e < 16; ++e) f[e] -= start_f;
+            asm volatile("" : "+v"(f));
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[t][e] = fmaf(f[e], scale[t & 1][16 * (i & 1) + e], acc[t][e]);
             __builtin_amdgcn_sched_barrier(0);
         }
         buf ^= 1;
