@@ -1,20 +1,22 @@
 // Products of Q4_K and Q6_K matrices with a few tokens at once (2 to 48: drafted tokens to verify, a chat turn), read from
 // their decode copies or, with the same bits, from the native blocks.
 //
-// A wavefront owns 16 weight rows and streams their super-blocks straight into registers, two to four of them ahead; the tokens, in
+// A wavefront owns 16 weight rows and streams their super-blocks straight into registers, two of them ahead; the tokens, in
 // tiles of 16, come from LDS, where the workgroup's eight wavefronts put them as f16 (the Q8_0 codes are whole numbers, exact
 // in f16), a chunk of super-blocks ahead.  One v_mfma_f32_16x16x32_f16 is one 32-weight block: Q4_K weights enter as
-// scale * code, at most 945 and exact in f16; Q6_K weights, up to 4096 (-128 times -32), as two f16 parts whose sum they are.
+// scale * code, at most 945 and exact in f16; Q6_K weights, up to 4096 (-128 times -32), as scale * lower four bits and scale * (16 * upper two - 32), exact both.
 // So a block's result is the exact whole number sum(scale * code * quant): quants are at most 127 (the quantizer's scale is the
 // largest magnitude over 127), and 32 * 4096 * 127 is 1 % below 2^24.  What the vector ALU adds is one FMA with the token's
 // block scale per output and block, one with the row's d per super-block, and for Q4_K one with dmin on the mins' own product
 // (mins times the tokens' block sums in three bf16 parts).  Sums over K go in order within a slice.
 //
-// What bounds it: up to 16 tokens the weights' way from HBM (gate | up at 3.0 TB/s), above that the vector instructions, about
-// 130 (Q4_K) and 225 (Q6_K) per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens (gate | up with 45 tokens: vector
-// ALU busy for half of the time, matrix cores for 15 %).  Gate | up, 14336 x 4096 Q4_K as a pair: 22 us at 5 tokens, 37 at 45; down, 4096 x 14336 Q6_K: 20 and 25.  The 64-token
+// What bounds it: the instructions, about 140 (Q4_K) and 200 (Q6_K) per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens.
+// A SIMD that has matrix instructions among them issues one in four clocks, whichever it is and however many wavefronts it
+// has: gate | up with 5 tokens takes 17 us without its loads, the loads alone 12, both 21.5 (3.1 TB/s).  Gate | up, 14336 x 4096 Q4_K
+// as a pair: 21.5 us at 5 tokens, 36.6 at 45; down, 4096 x 14336 Q6_K: 17.8 and 25.6 (22.3, 37.1, 19.8 and 25.8 with codes in the mantissa of
+// 1024, code and scale of a Q6_K weight put together and then rounded and split, and up to four super-blocks ahead).  The 64-token
 // tiles before it took 36 us for a down product and 50 for a pair, with a launch for the tokens' copy before and one for the sums
-// behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 289 us, 45 tokens 466 -> 322.
+// behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 268 us, 45 tokens 466 -> 301.
 #include <algorithm>
 
 #include "f16_codes.hip.h"
@@ -51,19 +53,17 @@ __device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {   // a's odd 
     a = r[0]; b = r[1];
 }
 
-// Masks and biases in registers of their own: an instruction of this kind takes no literal, and two steps otherwise.
-struct Consts { uint32_t lo, hi, bias; };
-__device__ __forceinline__ Consts consts() {
-    Consts c{0x000F000Fu, 0x00F000F0u, 0x64006400u};
-    asm("" : "+s"(c.lo)); asm("" : "+s"(c.hi)); asm("" : "+v"(c.bias));
-    return c;
-}
+// Bits of a code where they are, cut out with their neighbours' cleared, are a subnormal f16, code * 2^-24 times a power of two: what a
+// product by its scale leaves is exact, a whole number times 2^-19 (Q4_K) or 2^-20, and the tokens' scales make up for it.  Byte j of v,
+// twice, as 2^e + byte * 2^(e - 10) with the upper byte TOP of 2^e (0x64: e = 10, 0x68: 11, 0x74: 14, 0x78: 15).
+template <uint32_t TOP, int J> __device__ __forceinline__ h2v byte_above(uint32_t v) { return as_h2(__builtin_amdgcn_perm(TOP * 0x01010101u, v, 0x04000400u | J | J << 16)); }
 
 // ---- Q4_K -----------------------------------------------------------------------------------------
 // Lane group g (of 16 lanes, one per row) loads unit g of the super-block, the blocks 2g and 2g + 1, in two 16-byte halves,
 // and after the exchange holds dword g of both halves of every unit: codes 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3 of a block.
 struct FewQ4 {
     static constexpr bool MINS = true;
+    static constexpr float XS = 524288.0f;   // 2^19
     struct W { uint4 h, f, s; };
     static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * e + g; }   // e-th dword of a block's quants in lane group g
     // a lane's offsets from the matrix's first byte, and the super-block's three loads at them: the base that moves is scalar
@@ -97,7 +97,6 @@ struct FewQ4 {
         uint32_t dd[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) dd[i] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((lane >> 4) * 4 + i) * 4, static_cast<int>(w.h.x)));
-        const Consts k = consts();
         uint32_t f[4] = {w.f.x, w.f.y, w.f.z, w.f.w}, s[4] = {w.s.x, w.s.y, w.s.z, w.s.w};
         swap32(f[0], f[2]); swap32(f[1], f[3]); swap32(s[0], s[2]); swap32(s[1], s[3]);
         swap16(f[0], f[1]); swap16(f[2], f[3]); swap16(s[0], s[1]); swap16(s[2], s[3]);   // now by unit
@@ -118,15 +117,13 @@ struct FewQ4 {
         // a unit's weights are unpacked while the matrix cores are at the unit before
         auto unit = [&](auto u_) {
             constexpr int u = decltype(u_)::value;
-            // 1024 + code, and for the upper nibbles 1024 + 16 code in place; the FMA leaves scale * code
-            const h2v s0 = byte_twice<2 * (u & 1)>(sc[u >> 1]) - both(1024.f), s1 = fma2(byte_twice<2 * (u & 1) + 1>(sc[u >> 1]), both(0.0625f), both(-64.f));
-            const h2v o0 = s0 * both(-1024.f), o1 = s1 * both(-1024.f);
+            // 32 times the scale, and for the upper nibbles, whose codes stand sixteen times as high, twice the scale
+            const h2v s0 = byte_above<0x78, 2 * (u & 1)>(sc[u >> 1]) - both(32768.f), s1 = byte_above<0x68, 2 * (u & 1) + 1>(sc[u >> 1]) - both(2048.f);
             h8v wt[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const uint32_t q = e ? s[u] : f[u], q8 = q >> 8;
-                const h2v a = fma2(as_h2((q & k.lo) | k.bias), s0, o0), b = fma2(as_h2((q8 & k.lo) | k.bias), s0, o0);
-                const h2v c = fma2(as_h2((q & k.hi) | k.bias), s1, o1), d = fma2(as_h2((q8 & k.hi) | k.bias), s1, o1);
+                const h2v a = as_h2(q & 0x000F000Fu) * s0, b = as_h2(q8 & 0x000F000Fu) * s0, c = as_h2(q & 0x00F000F0u) * s1, d = as_h2(q8 & 0x00F000F0u) * s1;
                 wt[0][4 * e] = a[0]; wt[0][4 * e + 1] = a[1]; wt[0][4 * e + 2] = b[0]; wt[0][4 * e + 3] = b[1];
                 wt[1][4 * e] = c[0]; wt[1][4 * e + 1] = c[1]; wt[1][4 * e + 2] = d[0]; wt[1][4 * e + 3] = d[1];
             }
@@ -162,6 +159,7 @@ struct FewQ4 {
 // group 2a + j, dwords 2a and 2a + 1 of the runs j of both halves: codes 16j + 8a .. 16j + 8a + 7 of a block.
 struct FewQ6 {
     static constexpr bool MINS = false;
+    static constexpr float XS = 1048576.0f;   // 2^20
     struct W { uint4 a, b, q, sc; uint32_t d; };
     static __device__ __forceinline__ uint32_t dword(int g, int e) { return 4 * (g & 1) + 2 * (g >> 1) + e; }
     struct At { uint32_t a, b, q, sc, d; };
@@ -204,8 +202,6 @@ struct FewQ6 {
         uint32_t a[4] = {w.a.x, w.a.y, w.a.z, w.a.w}, b[4] = {w.b.x, w.b.y, w.b.z, w.b.w}, q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
         swap32(a[0], a[2]); swap32(a[1], a[3]); swap32(b[0], b[2]); swap32(b[1], b[3]); swap32(q[0], q[2]); swap32(q[1], q[3]);   // now [half][dword]
         const uint32_t sh = 8 * ((lane >> 4) & 1);
-        uint32_t lo4 = 0x0F0F0F0Fu, hi2 = 0x30303030u;
-        asm("" : "+s"(lo4)); asm("" : "+s"(hi2));
         const f4v zero{0.f, 0.f, 0.f, 0.f};
         f4v sum[T];
         f4v r[T];
@@ -218,16 +214,15 @@ struct FewQ6 {
         auto block = [&](auto b_) {
             constexpr int blk = decltype(b_)::value, h = blk >> 2, z = blk & 3;
             const uint32_t sv = ((z < 2 ? (h ? w.sc.z : w.sc.x) : (h ? w.sc.w : w.sc.y)) ^ 0x80808080u) >> sh;
-            const h2v sc = byte_twice<2 * (z & 1)>(sv) - both(1152.f);
+            // sixteen times the scale for the lower nibbles; what makes the two upper bits, where they stand, 16 * scale * bits; 32 * scale
+            const h2v sl = z < 2 ? byte_above<0x74, 2 * (z & 1)>(sv) - both(18432.f) : byte_above<0x64, 2 * (z & 1)>(sv) - both(1152.f);
+            const h2v su = sl * both(z & 1 ? 4.f : 16.f), off = sl * both(z < 2 ? -0x1p-19f : -0x1p-15f);
+            constexpr uint32_t lower = z < 2 ? 0x000F000Fu : 0x00F000F0u, upper = 0x00030003u << (2 * z);
             h8v hi, lo;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const uint32_t ql = z & 1 ? b[2 * h + e] : a[2 * h + e], qh = q[2 * h + e];
-                const uint32_t top = (z == 0 ? qh << 4 : z == 1 ? qh << 2 : z == 2 ? qh : qh >> 2) & hi2;
-                const uint32_t c = ((z < 2 ? ql : ql >> 4) & lo4) | top;
-                // code - 32, times the scale: rounded to f16, and the remainder
-                const h2v u = bytes02(c) - both(1056.f), v = bytes13(c) - both(1056.f);
-                const h2v uh = u * sc, vh = v * sc, ul = fma2(u, sc, -uh), vl = fma2(v, sc, -vh);
+                const h2v ul = as_h2(ql & lower) * sl, vl = as_h2((ql >> 8) & lower) * sl, uh = fma2(as_h2(qh & upper), su, off), vh = fma2(as_h2((qh >> 8) & upper), su, off);
                 hi[4 * e] = uh[0]; hi[4 * e + 1] = uh[1]; hi[4 * e + 2] = vh[0]; hi[4 * e + 3] = vh[1];
                 lo[4 * e] = ul[0]; lo[4 * e + 1] = ul[1]; lo[4 * e + 2] = vl[0]; lo[4 * e + 3] = vl[1];
             }
@@ -252,12 +247,15 @@ struct FewQ6 {
     }
 };
 
-// T tiles of 16 tokens; S super-blocks a chunk, so that a chunk is four tiles (three for T = 3) and two of them fill half the
-// LDS.  Four tiles of tokens would spill registers.
-template <int T> constexpr int FEW_CHUNK = T == 1 ? 4 : T == 2 ? 2 : 1;
+// T tiles of 16 tokens; S super-blocks a chunk, so that a chunk is up to four tiles and two of them fill at most half the LDS (Q6_K with one
+// tile two: 32000 x 4096 with 5 tokens 35.7 -> 34.6 us).  Four tiles of tokens would spill registers.
+template <typename W, int T> constexpr int FEW_CHUNK = T == 1 ? (W::MINS ? 4 : 2) : T == 2 ? 2 : 1;
+// Two super-blocks are on their way.  With four a slice of a few loads its last one up to four times again: 6144 x 4096 Q4_K in six
+// slices with 5 tokens 10.8 -> 8.6 us, 4096 x 14336 Q6_K in eight 19.6 -> 17.8, 28672 x 4096 in one 21.4 -> 21.6.
+constexpr int FEW_AHEAD = 2;
 template <typename W, int T, bool COPY>
-__device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned char (*lds)[FEW_CHUNK<T> * T * FEW_TILE]) {
-    constexpr int S = FEW_CHUNK<T>, AHEAD = T > 1 ? 2 : 4, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+__device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned char* lds) {
+    constexpr int S = FEW_CHUNK<W, T>, AHEAD = FEW_AHEAD, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
     const FewMat& M = second ? a.b : a.a;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nsb = a.k / 256;
     const uint32_t row0 = (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
@@ -293,7 +291,7 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
             const uint32_t p = pair(i), tok = (p >> 3) & 15, b = p & 7;
-            unsigned char* const t = &lds[buf][(p >> 7) * FEW_TILE];
+            unsigned char* const t = lds + (buf * S * T + (p >> 7)) * FEW_TILE;
             const uint32_t q[8] = {q0[i].x, q0[i].y, q0[i].z, q0[i].w, q1[i].x, q1[i].y, q1[i].z, q1[i].w};
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -306,7 +304,7 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
                 }
                 *reinterpret_cast<h8v*>(t + b * FEW_BLOCK + (g * 16 + tok) * 16) = h8v{v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
             }
-            *reinterpret_cast<float*>(t + FEW_XS + b * 64 + tok * 4) = xs[i];
+            *reinterpret_cast<float*>(t + FEW_XS + b * 64 + tok * 4) = xs[i] * W::XS;
             if (W::MINS) {   // three bf16 parts that add up to the block sum, and a zero
                 float rest = bs[i];
 #pragma unroll
@@ -336,9 +334,9 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
             lds_barrier();
             act_load(min(sb + S, sb1 - 1));
         }
-        W::template multiply<T>(w[i], &lds[buf][(i % S) * T * FEW_TILE], lane, acc);
+        W::template multiply<T>(w[i % AHEAD], lds + (buf * S + i % S) * T * FEW_TILE, lane, acc);
         __builtin_amdgcn_sched_barrier(0);   // the next load into the registers it has left, not into others and then copied, with a wait
-        W::template load<COPY>(w[i], m0, min(sb + AHEAD, sb1 - 1), at);
+        W::template load<COPY>(w[i % AHEAD], m0, min(sb + AHEAD, sb1 - 1), at);
         if (++sb == sb1) return true;
         if (i % S == S - 1) {
             buf ^= 1;
@@ -349,7 +347,7 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
     while (true) {
         if (step(std::integral_constant<int, 0>{})) break;
         if (step(std::integral_constant<int, 1>{})) break;
-        if constexpr (AHEAD > 2) {
+        if constexpr (S > 2) {
             if (step(std::integral_constant<int, 2>{})) break;
             if (step(std::integral_constant<int, 3>{})) break;
         }
@@ -376,7 +374,7 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
 // WA, WB: the types of the two matrices
 template <typename WA, typename WB, int T, bool COPY>
 __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) {
-    __shared__ __align__(16) unsigned char lds[2][FEW_CHUNK<T> * T * FEW_TILE];
+    __shared__ __align__(16) unsigned char lds[2 * std::max(FEW_CHUNK<WA, T>, FEW_CHUNK<WB, T>) * T * FEW_TILE];
     const bool second = blockIdx.x >= a.tiles_a;
     if (std::is_same<WA, WB>::value || !second) few_body<WA, T, COPY>(a, second, lds);
     else few_body<WB, T, COPY>(a, second, lds);
