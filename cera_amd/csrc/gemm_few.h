@@ -33,3 +33,7 @@ bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n);
 // (nullable): a second matrix of the same k in the same launch, of the same type or Q6_K beside Q4_K.
 cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const FewOut* ob, const float* xs, const int8_t* xq, const float* bsum, uint32_t n,
                                      const float* resid, float resid_scale, int part_slot, FewParts* parts);
+// hq / hs / hbsum [n][m] = Q8_0(silu(gate . x) * (up . x)) in one launch.  *fused = false (nothing launched) where the two are not of one type and
+// shape in whole blocks of rows, or where a pair with K in slices is faster.
+cera_hip_status cera_launch_gemm_few_swiglu(cera_hip_ctx* ctx, const cera_hip_dtensor* gate, const cera_hip_dtensor* up, const float* xs, const int8_t* xq, const float* bsum,
+                                            uint32_t n, int8_t* hq, float* hs, float* hbsum, bool* fused);

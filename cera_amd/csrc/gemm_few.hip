@@ -16,12 +16,13 @@
 // as a pair: 21.5 us at 5 tokens, 36.6 at 45; down, 4096 x 14336 Q6_K: 17.8 and 25.6 (22.3, 37.1, 19.8 and 25.8 with codes in the mantissa of
 // 1024, code and scale of a Q6_K weight put together and then rounded and split, and up to four super-blocks ahead).  The 64-token
 // tiles before it took 36 us for a down product and 50 for a pair, with a launch for the tokens' copy before and one for the sums
-// behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 268 us, 45 tokens 466 -> 301.
+// behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 262 us, 45 tokens 466 -> 294 (267 and 299 with SwiGLU in a launch of its own).
 #include <algorithm>
 
 #include "f16_codes.hip.h"
 #include "gemv.hip.h"
 #include "gemm_few.h"
+#include "quantize.hip.h"
 
 namespace {
 
@@ -36,6 +37,8 @@ struct FewArgs {
     uint64_t part_stride;      // floats between the slices of a split K; 0: no split
     const float* resid;        // added to segment 0 of a (unsplit)
     float resid_scale;
+    int8_t* hq;                // SwiGLU: the product's Q8_0 quants [n][m], scales and scale * sum of quants [n][m / 32]
+    float *hs, *hbsum;
 };
 
 constexpr int FEW_WAVES = 8, FEW_ROWS = 16 * FEW_WAVES;
@@ -253,12 +256,81 @@ template <typename W, int T> constexpr int FEW_CHUNK = T == 1 ? (W::MINS ? 4 : 2
 // Two super-blocks are on their way.  With four a slice of a few loads its last one up to four times again: 6144 x 4096 Q4_K in six
 // slices with 5 tokens 10.8 -> 8.6 us, 4096 x 14336 Q6_K in eight 19.6 -> 17.8, 28672 x 4096 in one 21.4 -> 21.6.
 constexpr int FEW_AHEAD = 2;
-template <typename W, int T, bool COPY>
+// The end of a SwiGLU launch.  A gate wavefront has from its up wavefront, in the same lanes, what goes with its sixteen rows; a Q8_0
+// block of a token is its rows and its neighbour's (cera/src/backend/cpu.rs:2570-2575, 942-958).
+template <int T>
+__device__ __forceinline__ void few_swiglu(const FewArgs& a, const f4v (&acc)[T], bool second, uint32_t row0, unsigned char* lds) {
+    constexpr uint32_t HALF = FEW_WAVES / 2, TOKENS = T * 16;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % HALF, col = lane & 15, g = lane >> 4, m = a.a.m;
+    f4v* const ups = reinterpret_cast<f4v*>(lds);                                      // [wave][tile][lane]
+    float* const largest = reinterpret_cast<float*>(lds + HALF * T * 1024);            // [wave][token] largest magnitude of its sixteen rows
+    int* const sums = reinterpret_cast<int*>(largest + HALF * TOKENS);                 // [wave][token] sum of its quants
+    lds_barrier();   // nobody reads the tokens any more
+    if (second)
+#pragma unroll
+        for (int t = 0; t < T; ++t) ups[(wave * T + t) * 64 + lane] = acc[t];
+    lds_barrier();
+    f4v h[T];
+    float amax[T];
+    if (!second)
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const f4v up = ups[(wave * T + t) * 64 + lane];
+            amax[t] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gate = acc[t][i];
+                h[t][i] = __fmul_rn(__fdiv_rn(gate, __fadd_rn(1.0f, cera_expf(-gate))), up[i]);
+                amax[t] = fmaxf(amax[t], fabsf(h[t][i]));   // fmaxf drops a NaN operand, as f32::max does
+            }
+            amax[t] = fmaxf(amax[t], __shfl_xor(amax[t], 16, 64));
+            amax[t] = fmaxf(amax[t], __shfl_xor(amax[t], 32, 64));
+            if (g == 0) largest[wave * TOKENS + t * 16 + col] = amax[t];
+        }
+    lds_barrier();
+    float scale[T];
+    int sum[T];
+    if (!second)
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const uint32_t tok = t * 16 + col;
+            const float d = __fdiv_rn(fmaxf(amax[t], largest[(wave ^ 1) * TOKENS + tok]), 127.0f), r = __fdiv_rn(1.0f, d);
+            const float id = (d != 0.0f && fabsf(r) != __builtin_inff() && r == r) ? r : 0.0f;
+            scale[t] = h2f(f2h(d));
+            uint32_t packed = 0;
+            sum[t] = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int v = q8_round(h[t][i], id);
+                sum[t] += v;
+                packed |= (static_cast<uint32_t>(v) & 0xFF) << (8 * i);
+            }
+            sum[t] += __shfl_xor(sum[t], 16, 64);
+            sum[t] += __shfl_xor(sum[t], 32, 64);
+            if (g == 0) sums[wave * TOKENS + tok] = sum[t];
+            if (tok < a.n && row0 < m) *reinterpret_cast<uint32_t*>(a.hq + static_cast<uint64_t>(tok) * m + row0 + 4 * g) = packed;   // m % 32 == 0
+        }
+    lds_barrier();
+    if (second || g || wave % 2 || row0 >= m) return;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const uint32_t tok = t * 16 + col;
+        if (tok >= a.n) continue;
+        const uint64_t at = static_cast<uint64_t>(tok) * (m / 32) + row0 / 32;
+        a.hs[at] = scale[t];
+        a.hbsum[at] = scale[t] * static_cast<float>(sum[t] + sums[(wave + 1) * TOKENS + tok]);
+    }
+}
+
+// SWIGLU: the lower half of the wavefronts has rows of matrix a, the gate's, the upper half the same rows of b, the up matrix, and
+// the workgroup leaves silu(gate) * up as quants
+template <typename W, int T, bool COPY, bool SWIGLU = false>
 __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned char* lds) {
     constexpr int S = FEW_CHUNK<W, T>, AHEAD = FEW_AHEAD, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
-    const FewMat& M = second ? a.b : a.a;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nsb = a.k / 256;
-    const uint32_t row0 = (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
+    if (SWIGLU) second = wave >= FEW_WAVES / 2;
+    const FewMat& M = second ? a.b : a.a;
+    const uint32_t row0 = SWIGLU ? blockIdx.x * (FEW_ROWS / 2) + wave % (FEW_WAVES / 2) * 16 : (blockIdx.x - (second ? a.tiles_a : 0)) * FEW_ROWS + wave * 16;
     const uint32_t sb0 = blockIdx.y * a.sb_per, sb1 = min(nsb, sb0 + a.sb_per);
     const uint8_t* const m0 = M.w;
     const typename W::At at = W::template at<COPY>(min(row0 + (lane & 15), M.m - 1) * M.row_bytes, lane >> 4, nsb);   // rows past the end: the last one again
@@ -352,6 +424,10 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
             if (step(std::integral_constant<int, 3>{})) break;
         }
     }
+    if constexpr (SWIGLU) {
+        few_swiglu<T>(a, acc, second, row0, lds);
+        return;
+    }
     // four consecutive rows of one token per lane and tile
     const uint32_t r0 = row0 + (lane >> 4) * 4;
     if (r0 >= M.m) return;
@@ -380,7 +456,20 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_kernel(FewArgs a) 
     else few_body<WB, T, COPY>(a, second, lds);
 }
 
+template <typename W, int T, bool COPY>
+__global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_swiglu_kernel(FewArgs a) {
+    __shared__ __align__(16) unsigned char lds[2 * FEW_CHUNK<W, T> * T * FEW_TILE];
+    few_body<W, T, COPY, true>(a, false, lds);
+}
+
 }  // namespace
+
+// Super-blocks of a slice of K.  It is split where the rows leave more than a quarter of one workgroup per CU idle, down to two
+// super-blocks a slice.
+static uint32_t few_slice(uint32_t wgs, uint32_t nsb, uint32_t n_cu) {
+    const uint32_t split = wgs * 4 >= n_cu * 3 ? 1 : std::min({(n_cu + wgs - 1) / wgs, std::max(nsb / 2, 1u), 8u});
+    return (nsb + split - 1) / split;
+}
 
 bool cera_gemm_few_supports(const cera_hip_dtensor* w, uint32_t n) {
     return w && (w->dtype == CERA_HIP_Q6_K || (reinterpret_cast<uintptr_t>(w->dev) & 15) == 0) && (w->dtype == CERA_HIP_Q4_K || w->dtype == CERA_HIP_Q6_K) && w->k >= FEW_MIN_K && w->k % 256 == 0 && w->m % 4 == 0 &&
@@ -398,11 +487,9 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(w->k);
     auto tiles = [](const cera_hip_dtensor* t) { return static_cast<uint32_t>((t->m + FEW_ROWS - 1) / FEW_ROWS); };
     a.tiles_a = tiles(w);
-    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256, want = ctx->n_cu;
-    // K is split where the rows leave more than a quarter of one workgroup per CU idle, down to two super-blocks a slice
-    uint32_t split = wgs * 4 >= want * 3 ? 1 : std::min({(want + wgs - 1) / wgs, std::max(nsb / 2, 1u), 8u});
-    a.sb_per = (nsb + split - 1) / split;
-    split = (nsb + a.sb_per - 1) / a.sb_per;
+    const uint32_t wgs = a.tiles_a + (ob ? tiles(ob->w) : 0), nsb = a.k / 256;
+    a.sb_per = few_slice(wgs, nsb, ctx->n_cu);
+    uint32_t split = (nsb + a.sb_per - 1) / a.sb_per;
     uint64_t rows = 0;
     void* part_room = nullptr;
     if (split > 1) CERA_TRY(cera_scratch_if_room(ctx, part_slot, split * (w->m + (ob ? ob->w->m : 0)) * static_cast<uint64_t>(n) * 4, &part_room));
@@ -449,5 +536,42 @@ cera_hip_status cera_launch_gemm_few(cera_hip_ctx* ctx, const FewOut& oa, const 
     if (copy) of_type(std::true_type{});
     else of_type(std::false_type{});
     HIP_TRY(ctx, hipGetLastError());
+    return CERA_HIP_OK;
+}
+
+cera_hip_status cera_launch_gemm_few_swiglu(cera_hip_ctx* ctx, const cera_hip_dtensor* gate, const cera_hip_dtensor* up, const float* xs, const int8_t* xq, const float* bsum,
+                                            uint32_t n, int8_t* hq, float* hs, float* hbsum, bool* fused) {
+    *fused = false;
+    if (!cera_gemm_few_supports(gate, n) || !cera_gemm_few_supports(up, n) || up->dtype != gate->dtype || up->k != gate->k || up->m != gate->m || gate->m % 32) return CERA_HIP_OK;
+    const uint32_t wgs = static_cast<uint32_t>((gate->m + FEW_ROWS / 2 - 1) / (FEW_ROWS / 2)), nsb = static_cast<uint32_t>(gate->k / 256);
+    // One launch with the whole of K, or a pair that may have it in slices, with their sums and SwiGLU in launches of their own, which
+    // take as long as 8, 5 or 4 super-blocks of one, two or three tiles.  Passes of two layers of hidden x ffn, one launch against a pair, in us:
+    // 4096 x 14336 (whole either way) 5 tokens 262 / 267, 45 tokens 294 / 299; 4096 x 10240 (two slices, 320 workgroups on 256 CUs) 182 / 193 and 263 / 282;
+    // 3072 x 8192 (two slices, 256) 156 / 157 and 223 / 218; 2304 x 6144 (three, 288) 150 / 154 and 204 / 213; 2048 x 4096 (four, 256) 136 / 137 and 188 / 180
+    const uint32_t pair = 2 * static_cast<uint32_t>((gate->m + FEW_ROWS - 1) / FEW_ROWS), slice = few_slice(pair, nsb, ctx->n_cu), slices = (nsb + slice - 1) / slice, cus = ctx->n_cu;
+    if ((wgs + cus - 1) / cus * nsb > (pair * slices + cus - 1) / cus * slice + (n <= 16 ? 8u : n <= 32 ? 5u : 4u)) return CERA_HIP_OK;
+    FewArgs a{};
+    const bool copy = gate->dev_stream && up->dev_stream;
+    a.xq = xq; a.xs = xs; a.bsum = bsum; a.n = n; a.k = static_cast<uint32_t>(gate->k); a.sb_per = a.k / 256;
+    a.hq = hq; a.hs = hs; a.hbsum = hbsum;
+    auto set = [&](FewMat& m, const cera_hip_dtensor* w) {
+        m.w = copy ? w->dev_stream : w->dev;
+        m.row_bytes = static_cast<uint32_t>(copy ? w->stream_row_bytes : w->row_bytes);
+        m.m = static_cast<uint32_t>(w->m);
+    };
+    set(a.a, gate);
+    set(a.b, up);
+    auto go = [&](auto type, auto from_copy) {
+        using W = decltype(type);
+        constexpr bool COPY = decltype(from_copy)::value;
+        const dim3 grid(wgs), block(FEW_WAVES * 64);
+        if (n <= 16) hipLaunchKernelGGL((gemm_few_swiglu_kernel<W, 1, COPY>), grid, block, 0, ctx->stream, a);
+        else if (n <= 32) hipLaunchKernelGGL((gemm_few_swiglu_kernel<W, 2, COPY>), grid, block, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((gemm_few_swiglu_kernel<W, 3, COPY>), grid, block, 0, ctx->stream, a);
+    };
+    if (gate->dtype == CERA_HIP_Q6_K) copy ? go(FewQ6{}, std::true_type{}) : go(FewQ6{}, std::false_type{});
+    else copy ? go(FewQ4{}, std::true_type{}) : go(FewQ4{}, std::false_type{});
+    HIP_TRY(ctx, hipGetLastError());
+    *fused = true;
     return CERA_HIP_OK;
 }

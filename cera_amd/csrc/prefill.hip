@@ -432,8 +432,16 @@ static cera_hip_status gemm_swiglu_host(cera_hip_ctx* ctx, const cera_hip_tensor
         void* hh = nullptr;
         if (halves) CERA_TRY(cera_scratch(ctx, 10, n * mm * 2, &hh));
         // (a Q4_K pair's epilogue writes the f16 words itself; every other route converts the quants afterwards)
-        const bool hh_in_epilogue = halves && wg->dtype == CERA_HIP_Q4_K;
-        CERA_TRY(cera_launch_gemm_swiglu(ctx, wg, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
+        bool hh_in_epilogue = halves && wg->dtype == CERA_HIP_Q4_K;
+        if (n <= FEW_MAX_TOKENS && cera_gemm_few_supports(wg, static_cast<uint32_t>(n)) && cera_gemm_few_supports(wu, static_cast<uint32_t>(n))) {
+            // as the forward pass does, whose matrices have decode copies
+            CERA_TRY(cera_tensor_prepare_stream(ctx, wg));
+            CERA_TRY(cera_tensor_prepare_stream(ctx, wu));
+            CERA_TRY(cera_launch_gemm_few_swiglu(ctx, wg, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db), static_cast<uint32_t>(n),
+                                                 static_cast<int8_t*>(hq), static_cast<float*>(hs), static_cast<float*>(hb), &fused));
+            hh_in_epilogue = hh_in_epilogue && !fused;
+        }
+        if (!fused) CERA_TRY(cera_launch_gemm_swiglu(ctx, wg, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
                                          static_cast<uint32_t>(n), static_cast<int8_t*>(hq), static_cast<float*>(hs),
                                          static_cast<float*>(hb), &fused, nullptr, nullptr, hh_in_epilogue ? hh : nullptr));
         if (!fused) {   // the forward pass's other route: the two GEMMs, then the SwiGLU + quantize kernel
@@ -617,9 +625,10 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
     };
     // the kernel for a few tokens: o (and o2) of the quantized activations; sums over a split K are added up here unless
     // `pending` takes them
-    auto few = [&](const FewOut& o, const FewOut* o2, const float* resid, RowsPending* pending, int part_slot) -> cera_hip_status {
+    struct Quants { const float* xs; const int8_t* xq; const float* bsum; };
+    auto few = [&](const FewOut& o, const FewOut* o2, const float* resid, RowsPending* pending, int part_slot, const Quants& x) -> cera_hip_status {
         FewParts p;
-        CERA_TRY(cera_launch_gemm_few(ctx, o, o2, m->pf_xs, m->pf_xq, m->pf_bsum, n, resid, c.residual_scale, part_slot, &p));
+        CERA_TRY(cera_launch_gemm_few(ctx, o, o2, x.xs, x.xq, x.bsum, n, resid, c.residual_scale, part_slot, &p));
         if (p.n_split == 1) return CERA_HIP_OK;
         if (pending) {
             *pending = RowsPending{p.part, p.n_split, p.stride, resid, c.residual_scale, o.out[0]};
@@ -631,6 +640,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         HIP_TRY(ctx, hipGetLastError());
         return CERA_HIP_OK;
     };
+    const Quants in_pf{m->pf_xs, m->pf_xq, m->pf_bsum};
     // out[n][w->m] (token-major rows) = B . W^T, optionally added onto resid
     // xf: the f32 activations the quantized ones in pf_xs / pf_xq were made from (what a Q5_K matrix reads)
     auto gemm = [&](const cera_hip_dtensor* w, float* out, const float* resid, const float* xf,
@@ -638,7 +648,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         if (few_tokens && cera_gemm_few_supports(w, n)) {
             FewOut o;
             o.w = w; o.out[0] = out;
-            return few(o, nullptr, resid, pending, part_slot);
+            return few(o, nullptr, resid, pending, part_slot, in_pf);
         }
         // a short batch streams the weights once per 8 tokens through the multi-token GEMV (an
         // int8-MFMA tile would be mostly empty); its residual add is unscaled
@@ -666,7 +676,7 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             FewOut oa, ob;
             oa.w = wa; oa.out[0] = outa;
             ob.w = wb; ob.out[0] = outb;
-            return few(oa, &ob, nullptr, pending, 9);
+            return few(oa, &ob, nullptr, pending, 9, in_pf);
         }
         if (n > PREFILL_SMALL_BATCH && gemm_batched(wa->dtype, wa->k) && gemm_batched(wb->dtype, wb->k)) {
             bool paired = false;
@@ -725,10 +735,10 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
             if (whole || (cera_gemm_few_supports(L.v, n) && (L.v->dtype == L.qkv->dtype || L.qkv->dtype == CERA_HIP_Q4_K))) {
                 FewOut ov;
                 ov.w = L.v; ov.out[0] = m->pf_v;
-                CERA_TRY(few(o, whole ? nullptr : &ov, nullptr, &pqk, 9));
+                CERA_TRY(few(o, whole ? nullptr : &ov, nullptr, &pqk, 9, in_pf));
                 if (pqk.n_split) pvv = RowsPending{pqk.part + static_cast<uint64_t>(n) * (q_dim + kv_dim), pqk.n_split, pqk.stride, nullptr, 1.0f, m->pf_v};
             } else {
-                CERA_TRY(few(o, nullptr, nullptr, &pqk, 9));
+                CERA_TRY(few(o, nullptr, nullptr, &pqk, 9, in_pf));
                 CERA_TRY(gemm(L.v, m->pf_v, nullptr, m->pf_normed, &pvv, 14));
             }
         } else {
@@ -792,6 +802,18 @@ static cera_hip_status prefill_chunk(cera_hip_model* m, const uint32_t* tokens, 
         if (n > PREFILL_SMALL_BATCH && !few_gate_up && L.down->dtype != CERA_HIP_Q5_K)   // a Q5_K down projection reads the f32 SwiGLU output
             CERA_TRY(cera_launch_gemm_swiglu(ctx, L.gate, L.up, m->pf_xs, m->pf_xq, m->pf_bsum, n, hq, hs, hb, &fused, m->pf_x8, &staged8,
                                              hh ? m->pf_xh : nullptr));
+        // a few tokens: the same from the kernel for them, to the down projection's
+        if (few_gate_up && L.down->dtype != CERA_HIP_Q5_K && cera_gemm_few_supports(L.down, n)) {
+            CERA_TRY(cera_launch_gemm_few_swiglu(ctx, L.gate, L.up, m->pf_xs, m->pf_xq, m->pf_bsum, n, hq, hs, hb, &fused));
+            if (fused) {
+                FewOut o;
+                o.w = L.down; o.out[0] = m->pf_hidden;
+                CERA_TRY(few(o, nullptr, m->pf_hidden, norm_adds && i + 1 < c.n_layers ? &pend : nullptr, 9, Quants{hs, hq, hb}));
+                staged = ActForm::none;
+                staged8 = false;
+                continue;
+            }
+        }
         staged = fused && hh ? ActForm::rows : ActForm::none;   // pf_xh: the down projection's activations, or stale
         if (fused) staged8 = false;
         if (fused && cera_gemm_supports(L.down->dtype, L.down->k)) {

@@ -282,6 +282,24 @@ def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n,
     assert np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("m,k,n,want_fused", [(12288, 2048, 2, True), (12320, 2304, 5, True), (12288, 2048, 16, True), (12320, 2048, 17, True), (12288, 2048, 48, True), (96, 2048, 5, True), (4096, 2048, 48, False)])
+def test_gemm_swiglu_of_a_few_tokens(hip, orc, dtype, m, k, n, want_fused):
+    """As test_gemm_swiglu_epilogue_matches_separate_kernels for the kernel of 2 to 48 tokens: a last workgroup of 32 rows, one to
+    three tiles of tokens, whole and not; the quants and scales are the oracle's of the two products of the pair launch."""
+    _say(f"few gemm_swiglu {util.NAMES[dtype]} m={m} k={k} n={n}")
+    wg, _ = util.make_weights(dtype, m, k, seed=41)
+    wu, _ = util.make_weights(dtype, m, k, seed=42)
+    x = util.rng(m + 3 * n).standard_normal((n, k)).astype(np.float32)
+    q, sc, fused = hip.gemm_swiglu(dtype, wg, wu, m, x, n, k)
+    assert fused == want_fused
+    if not fused:
+        return
+    g, u = hip.gemm_pair(dtype, wg, m, dtype, wu, m, x, n, k)
+    ref_s, ref_q = orc.quantize_q8_0(orc.silu_mul(g.reshape(-1), u.reshape(-1)))
+    assert np.array_equal(q.reshape(-1), ref_q) and np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
+
+
 @pytest.mark.parametrize("dtype,m,k,n,want_fused", [(Q4_K, 2048, 512, 1040, True), (Q4_K, 1056, 256, 2000, True),
                                                       (Q4_K, 512, 256, 80, False), (Q4_0, 2048, 512, 1040, True)])
 def test_gemm_swiglu_f16_words_for_a_q6k_down_projection(hip, dtype, m, k, n, want_fused):
