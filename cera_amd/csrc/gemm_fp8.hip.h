@@ -27,10 +27,12 @@
 //     six products above 2^-24 of the term take six K slots per block, 48 per super-block, three
 //     v_mfma_f32_32x32x16_bf16 accumulating (negated) into the same tile as the dots.
 //
-// Workgroup: 256 threads = 4 wavefronts stacked along M; tile 128 rows x 64 tokens; a wavefront
-// owns 32 rows x 64 tokens (two MFMA tiles, 32 accumulator registers); two workgroups share a CU.
-// K advances in stages of 128 elements, double-buffered in LDS with one barrier per stage, and the
-// K loop is software-pipelined inside the wavefront (see the kernel).
+// Workgroup: 256 threads = 4 wavefronts stacked along M; tile 128 rows x 64 or 128 tokens; a wavefront
+// owns 32 rows x all of them (two or four MFMA tiles, 16 accumulator registers each); two workgroups share a CU.
+// K advances in stages of 128 or 64 elements, double-buffered in LDS with one barrier per stage, and the
+// K loop is software-pipelined inside the wavefront (see the kernel).  With 128 tokens a row is decoded and
+// unpacked for twice as many products: 28672 x 4096 (gate | up) times 1001 tokens 401 us by 64, 360 by 128; two layers, 2048 tokens 3394 -> 3237; the
+// sums are the same.  g8_four_tiles says which a launch takes.
 //
 // What bounds it: on this chip the matrix core and the vector ALU of a SIMD do not run at the same
 // time in a kernel of this kind (matrix-core busy + vector-ALU busy = 100 % of the dispatch, here as
@@ -159,23 +161,25 @@ __device__ __forceinline__ uint32_t g8_lds_addr(const void* p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)(p)));
 }
 
-struct G8Stage {
-    uint8_t bf[2][4][2048];   // [token tile][block of the stage][piece][lane][16]
-    float xs[2][4][32];       // [token tile][block][token]
+// TT: token tiles of 32 of a workgroup, 2 or 4.  A stage is 8 / TT blocks of all its tokens.
+template <int TT> struct G8Stage {
+    uint8_t bf[TT][8 / TT][2048];     // [token tile][block of the stage][piece][lane][16]
+    float xs[TT][8 / TT][32];         // [token tile][block][token]
 };
-struct G8Mins {
-    uint8_t b[2][4096];       // [token tile][j][lane][16], the last KB unused
+template <int TT> struct G8Mins {
+    uint8_t b[TT][3072];              // [token tile][j][lane][16]
 };
 
-template <bool SWIGLU = false, bool DBG = false, int NW = G8_NW>
+template <bool SWIGLU, bool DBG, int TT>
 __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
-    constexpr uint32_t BM = 32 * NW;   // rows per workgroup
+    constexpr int NW = G8_NW, T = 8 * TT;   // steps of a super-block
+    constexpr uint32_t BM = 32 * NW;        // rows per workgroup
     // the two stage buffers are separate variables so that the compiler can tell the DMA into one
     // from the fragment reads of the other (a shared array would make every LDS read wait for
     // the DMA in flight)
-    __shared__ __attribute__((aligned(16))) G8Stage st0;
-    __shared__ __attribute__((aligned(16))) G8Stage st1;
-    __shared__ __attribute__((aligned(16))) G8Mins mnb_lds;   // min operands of the super-block in progress
+    __shared__ __attribute__((aligned(16))) G8Stage<TT> st0;
+    __shared__ __attribute__((aligned(16))) G8Stage<TT> st1;
+    __shared__ __attribute__((aligned(16))) G8Mins<TT> mnb_lds;   // min operands of the super-block in progress
     // each wavefront's own rows of the next super-block, 32 x 144 bytes as 16-byte pieces in row order
     // (+ 32 unused pieces: the fifth copy instruction runs with all lanes)
     __shared__ __attribute__((aligned(16))) uint8_t wts[NW][320 * 16];
@@ -188,7 +192,7 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     const uint32_t mrows = second ? p.m2 : p.m;
     const uint64_t ldn = second ? p.ld_n2 : p.ld_n;
     const uint32_t m0 = (second ? blockIdx.y - p.tiles1 : blockIdx.y) * (SWIGLU ? BM / 2 : BM);
-    const uint32_t n0 = blockIdx.x * G8_BN;
+    const uint32_t n0 = blockIdx.x * (32 * TT);
     const uint32_t nsb_all = p.k / 256;
     // this wavefront's 32 rows.  SwiGLU: the first half of the wavefronts take rows of the gate
     // matrix and the second half the same rows of the up matrix.
@@ -211,48 +215,45 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     const uint32_t wts_lds = g8_lds_addr(&wts[0][0]) + wave * (320 * 16);
     const uint8_t* const wts_row = &wts[0][0] + wave * (320 * 16) + col * 144;   // this lane's row in the staged copy
     const uint32_t sb_begin = blockIdx.z * (p.k_chunk / 256), sb_end = sb_begin + p.k_chunk / 256;
-    const uint8_t* const rec0 = p.bf8 + static_cast<uint64_t>(blockIdx.x * 2) * nsb_all * G8_REC;   // token tile 2*blockIdx.x
-    const uint64_t rec_tile = static_cast<uint64_t>(nsb_all) * G8_REC;
+    // records of token tile tn of this workgroup; tiles behind the last one read that (their outputs are not stored)
+    const uint32_t last_tile = (p.n + 63) / 64 * 2 - 1;
+    auto records = [&](uint32_t tn) { return p.bf8 + static_cast<uint64_t>(min(blockIdx.x * TT + tn, last_tile)) * nsb_all * G8_REC; };
     const uint32_t lane16 = lane * 16, lane4 = lane * 4;
 
     // stage (sb, s) -> LDS buffer, every wavefront the same share of the 16 KB of fragments; 1 KB of
-    // scales in four quarters; with_mins: also the 8 KB of min operands of super-block sb_mins
-    auto stage_in = [&](uint32_t sb, uint32_t s, G8Stage& dst, bool with_mins, uint32_t sb_mins) {
-        constexpr int CW = 16 / NW;   // fragment chunks of 1 KB per wavefront
-        const uint32_t c0 = wave * CW, tn = c0 >> 3;
-        const uint8_t* const r = rec0 + tn * rec_tile + static_cast<uint64_t>(sb) * G8_REC + s * 8192 + (c0 & 7) * 1024;
-        const uint32_t l = g8_lds_addr(&dst.bf[tn][0][0]) + (c0 & 7) * 1024;
+    // scales in four quarters; with_mins: also the 3 KB a tile of min operands of super-block sb_mins
+    const uint32_t my_tile = wave * TT / NW;
+    const uint8_t* const my_records = records(my_tile);
+    auto stage_in = [&](uint32_t sb, uint32_t s, G8Stage<TT>& dst, bool with_mins, uint32_t sb_mins) {
+        constexpr uint32_t CW = 16 / NW;             // fragment chunks of 1 KB per wavefront
+        const uint32_t part = wave % (NW / TT);      // of the tile's share
+        const uint8_t* const r = my_records + static_cast<uint64_t>(sb) * G8_REC;
+        const uint32_t l = g8_lds_addr(&dst.bf[my_tile][0][0]) + part * (CW * 1024);
 #pragma unroll
-        for (int i = 0; i < CW; ++i) g8_dma_1k(r + i * 1024, lane16, l + i * 1024);
-        if (wave < 4) {
-            const uint8_t* const rx = rec0 + (wave >> 1) * rec_tile + static_cast<uint64_t>(sb) * G8_REC + G8_REC_XS + s * 512 + (wave & 1) * 256;
-            g8_dma_256(rx, lane4, g8_lds_addr(&dst.xs[wave >> 1][0][0]) + (wave & 1) * 256);
-        }
+        for (uint32_t i = 0; i < CW; ++i) g8_dma_1k(r + s * (16384 / TT) + part * (CW * 1024) + i * 1024, lane16, l + i * 1024);
+        g8_dma_256(r + G8_REC_XS + s * (1024 / TT) + part * 256, lane4, g8_lds_addr(&dst.xs[my_tile][0][0]) + part * 256);
         if (with_mins) {
-            constexpr int MW = 8 / NW;   // min-operand chunks per wavefront
-            const uint32_t q0 = wave * MW, tm = q0 >> 2;
-            const uint8_t* const rm = rec0 + tm * rec_tile + static_cast<uint64_t>(sb_mins) * G8_REC + G8_REC_MIN + (q0 & 3) * 1024;
-            const uint32_t lm = g8_lds_addr(mnb_lds.b[tm]) + (q0 & 3) * 1024;
-#pragma unroll
-            for (int j = 0; j < MW; ++j) g8_dma_1k(rm + j * 1024, lane16, lm + j * 1024);
+            const uint8_t* const rm = my_records + static_cast<uint64_t>(sb_mins) * G8_REC + G8_REC_MIN;
+            const uint32_t lm = g8_lds_addr(mnb_lds.b[my_tile]);
+            for (uint32_t j = part; j < 3; j += NW / TT) g8_dma_1k(rm + j * 1024, lane16, lm + j * 1024);
         }
     };
 
     // acc takes the scaled block dots (vector ALU) and, negated, the min terms (matrix core)
-    v16f acc[2];
+    v16f acc[TT];
 #pragma unroll
-    for (int tn = 0; tn < 2; ++tn)
+    for (int tn = 0; tn < TT; ++tn)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[tn][e] = 0.0f;
 
     // The K loop is software-pipelined inside the wavefront.  A step is one (pair g, token tile tn,
-    // block jb of the pair): 16 per super-block.  Tick t issues the matrix-core work of step t+1, reads
+    // block jb of the pair): 8 TT per super-block.  Tick t issues the matrix-core work of step t+1, reads
     // the fragments of step t+3 from LDS and then runs the 16 FMAs of step t while that work
     // executes: on this hardware a SIMD overlaps matrix-core and vector instructions of the SAME
     // wavefront, not those of two different wavefronts.
     //
     // Weight prefetch: a super-block's rows are copied to LDS one super-block ahead (behind the barrier
-    // of tick 13) and read into registers at tick 13 of the super-block before theirs.
+    // of tick T - 3) and read into registers at that tick of the super-block before theirs.
     uint4 hdr, raw[4];
     // global -> this wavefront's LDS rows, super-block sb
     auto weights_in = [&](uint32_t sb) {
@@ -289,10 +290,10 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     v32f sct[2];        // scale tiles of a (pair, token tile), by (step / 2) parity
     v16f dot[2];        // block dots, by step parity
 
-    // LDS reads of step t (0..15) of a super-block: stage t / 8, pair (t / 4) % 2, token tile (t / 2) % 2, block t % 2
+    // LDS reads of step t of a super-block: stage t / 8, pair t / (2 TT), token tile t / 2 % TT, block t % 2
     auto lds_read = [&](int t) {
-        const G8Stage& st = (t & 8) ? st1 : st0;
-        const int pr = (t >> 2) & 1, tn = (t >> 1) & 1, jb = t & 1;
+        const G8Stage<TT>& st = (t & 8) ? st1 : st0;
+        const int pr = t / (2 * TT) % (4 / TT), tn = (t >> 1) % TT, jb = t & 1;
         const uint8_t* f = &st.bf[tn][2 * pr + jb][0] + lane * 16;
         const v4i lo = *reinterpret_cast<const v4i*>(f), hi = *reinterpret_cast<const v4i*>(f + 1024);
         bfr[t & 3] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -302,8 +303,8 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     // scale-tile MFMA, whose 64 clocks are otherwise spent waiting to issue the dot): at a (pair,
     // token tile)'s first step the scale tile ...
     auto issue_s = [&](int t) {
-        const int g = t >> 2;
-        if ((t & 3) == 0) rsl = d18 * static_cast<float>((scb >> (8 * g)) & 0xFF);
+        const int g = t / (2 * TT);
+        if (t % (2 * TT) == 0) rsl = d18 * static_cast<float>((scb >> (8 * g)) & 0xFF);
         if ((t & 1) == 0) {
             v32f z32;
 #pragma unroll
@@ -313,8 +314,8 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     };
     // ... and, after the A operands at a pair's first step, the block dot
     auto issue_d = [&](int t) {
-        const int g = t >> 2, jb = t & 1;
-        if ((t & 3) == 0) {
+        const int g = t / (2 * TT), jb = t & 1;
+        if (t % (2 * TT) == 0) {
             const uint4 q = raw[g];
             const int l0 = q.x & 0x0F0F0F0F, l1 = q.y & 0x0F0F0F0F, l2 = q.z & 0x0F0F0F0F, l3 = q.w & 0x0F0F0F0F;
             const int h0 = (q.x >> 4) & 0x0F0F0F0F, h1 = (q.y >> 4) & 0x0F0F0F0F, h2 = (q.z >> 4) & 0x0F0F0F0F,
@@ -328,9 +329,9 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
         dot[t & 1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[jb], bfr[t & 3], z16, 0, 0, 0, 0, 0, 0);
     };
     auto fma_step = [&](int t, uint32_t sb) {
-        const int tn = (t >> 1) & 1, jb = t & 1;
+        const int tn = (t >> 1) % TT, jb = t & 1;
         if (DBG) {
-            const uint32_t dtok = n0 + tn * 32 + col, dblk = sb * 8 + 2 * (t >> 2) + jb;
+            const uint32_t dtok = n0 + tn * 32 + col, dblk = sb * 8 + 2 * (t / (2 * TT)) + jb;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const uint32_t drow = row0 + (e >> 2) * 8 + half * 4 + (e & 3);
@@ -345,10 +346,10 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
         asm volatile("" : "+v"(acc[tn]));
     };
     // min terms of the super-block in progress: acc -= sum_b (dmin*mn)[row][b] * (xs*sum a)[tok][b]
-    auto mins = [&]() {
-        uint32_t aw[12];
+    uint32_t aw[12];
+    auto mins = [&](int first) {   // of token tiles first and first + 1
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4 && first == 0; ++i) {
             const float rm = ndmin * static_cast<float>((mnb >> (8 * i)) & 0xFF);
             const uint32_t r0 = __builtin_bit_cast(uint32_t, rm) & 0xFFFF0000u;
             const float e1 = rm - __builtin_bit_cast(float, r0);
@@ -361,7 +362,7 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
             aw[3 * i + 2] = (r1 >> 16) | r2;
         }
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+        for (int tn = first; tn < first + 2; ++tn)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const uint4 b = *reinterpret_cast<const uint4*>(mnb_lds.b[tn] + j * 1024 + lane * 16);
@@ -388,30 +389,29 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     issue_d(0);
 
     for (uint32_t sb = sb_begin; sb < sb_end; ++sb) {
-        const uint32_t sb_next = min(sb + 1, sb_end - 1);   // the last super-block re-requests itself: no branch around the loads
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
+        for (int t = 0; t < T; ++t) {
             // matrix-core work of step t+1 first, everything else behind it.  (While a DMA into LDS is
             // in flight the compiler makes every wait for an LDS read a wait for ALL LDS reads, so the
             // reads of step t+3 are requested behind these instructions, not in front of them.)
-            if (t == 15) decode_hdr();   // step 0 of the next super-block: its header
+            if (t == T - 1) decode_hdr();   // step 0 of the next super-block: its header
             __builtin_amdgcn_sched_barrier(0);
-            issue_s((t + 1) & 15);
+            issue_s((t + 1) % T);
             __builtin_amdgcn_sched_barrier(0);
-            if (t == 11) {
-                // the min terms go here: their operands are read before the barrier of tick 13 lets the
-                // next super-block's overwrite them
-                mins();
+            if (t >= 4 * TT + 3 && t < 6 * TT + 3 && t % 4 == 3) {
+                // the min terms of two tiles go into the third pair's steps: their operands are read before the barrier of
+                // tick T - 3 lets the next super-block's overwrite them, and a sum's order is the same in all tiles
+                mins((t - (4 * TT + 3)) / 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
             // ---- the barrier that publishes the stage step t+3 starts, and the DMA of the stage after it
-            if (t == 5 || t == 13) {
+            if (t % 8 == 5) {
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // this wavefront's DMA of that stage has landed
                 __syncthreads();
-                if (t == 5) {
-                    if (sb + 1 < sb_end) stage_in(sb + 1, 0, st0, false, 0);
-                } else {
-                    if (sb + 1 < sb_end) stage_in(sb + 1, 1, st1, true, sb + 1);
+                const int s = t / 8;   // the stage that is read no more: its buffer takes stage s + 2
+                if (s + 2 < TT) stage_in(sb, s + 2, s & 1 ? st1 : st0, false, 0);
+                else if (sb + 1 < sb_end) stage_in(sb + 1, s + 2 - TT, s & 1 ? st1 : st0, s + 1 == TT, sb + 1);
+                if (s + 1 == TT) {
                     // the next super-block's rows into registers (landed: waited for above; every pair of this
                     // one is unpacked), then their LDS copy is free for the super-block after it
                     weights_read();
@@ -420,42 +420,43 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            issue_d((t + 1) & 15);
+            issue_d((t + 1) % T);
             __builtin_amdgcn_sched_barrier(0);
-            lds_read((t + 3) & 15);
+            lds_read((t + 3) % T);
             __builtin_amdgcn_sched_barrier(0);
             fma_step(t, sb);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // the last rows were requested once more: nothing may land behind the kernel's end
 
     // ---- store: a lane holds token n0 + 32 tn + col and rows row0 + 8 blk + 4 half + r
     if (SWIGLU) {
         // The up wavefronts hand their tiles to the gate wavefronts through LDS (the stage buffers are
         // free after the last barrier): same lane, same register positions.
-        float* const xch = reinterpret_cast<float*>(&st0);   // [wave % (NW/2)][tn][e][lane], 8 KB per wavefront
-        static_assert(sizeof(G8Stage) >= (NW / 2) * 8192 || NW == 8, "exchange area");
-        float* const xch2 = NW == 8 ? reinterpret_cast<float*>(&st1) : xch;   // waves 2, 3 of four pairs use the second buffer
-        const uint32_t xw = wave % (NW / 2);
-        float* const myx = (xw >= 2 ? xch2 : xch) + (xw & 1) * 2048;
-        if (wave >= NW / 2) {
-#pragma unroll
-            for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) myx[(tn * 16 + e) * 64 + lane] = acc[tn][e];
-        }
-        __syncthreads();
-        if (wave >= NW / 2) return;
+        static_assert(NW == 4 && sizeof(G8Stage<TT>) >= 8192, "exchange area");
+        float* const myx = reinterpret_cast<float*>(wave & 1 ? &st1 : &st0);   // [tn % 2][e][lane], 8 KB for a pair of wavefronts
         // h = silu(gate) * up (cera/src/backend/cpu.rs:2570-2575), then the Q8_0 block of this token's
         // rows row0 .. row0+31 (cpu.rs:942-958): this lane holds 16 of them, lane ^ 32 the others
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
+        for (int tn = 0; tn < TT; ++tn) {
+            if (tn % 2 == 0) {
+                if (tn) __syncthreads();   // the tiles before are read
+                if (wave >= NW / 2) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) myx[(u * 16 + e) * 64 + lane] = acc[tn + u][e];
+                }
+                __syncthreads();
+            }
+            if (wave >= NW / 2) continue;
             const uint32_t tok = n0 + tn * 32 + col;
             float hv[16];
             float amax = 0.0f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const float g = acc[tn][e], u = myx[(tn * 16 + e) * 64 + lane];
+                const float g = acc[tn][e], u = myx[(tn % 2 * 16 + e) * 64 + lane];
                 hv[e] = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, cera_expf(-g))), u);
                 amax = fmaxf(amax, fabsf(hv[e]));   // fmaxf drops a NaN operand, as f32::max does
             }
@@ -499,7 +500,7 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
         return;
     }
 #pragma unroll
-    for (int tn = 0; tn < 2; ++tn) {
+    for (int tn = 0; tn < TT; ++tn) {
         const uint32_t tok = n0 + tn * 32 + col;
         if (tok >= p.n) continue;
 #pragma unroll
@@ -529,7 +530,19 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
         }
     }
 }
-template <bool SWIGLU = false, bool DBG = false, int NW = G8_NW>
-static __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_q4k_fp8_kernel(GemmArgs p) {
-    gemm_q4k_fp8_body<SWIGLU, DBG, NW>(p);
+template <bool SWIGLU = false, bool DBG = false, int TT = 2>
+static __global__ __launch_bounds__(64 * G8_NW, 2) void gemm_q4k_fp8_kernel(GemmArgs p) {
+    gemm_q4k_fp8_body<SWIGLU, DBG, TT>(p);
+}
+
+// Whether a launch of row_tiles tiles of 128 rows (all slices of K counted) takes 128 tokens a workgroup.  The chip holds two
+// workgroups a CU, so a launch is a number of rounds; a last one of at most a workgroup a CU takes 0.64 of a round, and a round
+// of 128 tokens 2 * 0.87 of one of 64.  Gate | up of the 4096-wide model, 64 and 128: 384 tokens 171 and 161 us, 512: 209 and 210,
+// 700: 289 and 301, 1001: 401 and 360.  Below a twentieth the estimate says nothing.
+static inline bool g8_four_tiles(uint64_t row_tiles, uint32_t n, uint32_t n_cu) {
+    auto rounds = [&](uint64_t workgroups) {
+        const uint64_t slots = 2ull * n_cu, rest = workgroups % slots;
+        return static_cast<double>(workgroups / slots) + (rest == 0 ? 0.0 : rest <= n_cu ? 0.64 : 1.0);
+    };
+    return 2 * 0.87 * rounds((n + 127) / 128 * row_tiles) < 0.95 * rounds((n + 63) / 64 * row_tiles);
 }

@@ -266,8 +266,8 @@ extern "C" __global__ __launch_bounds__(256) void cera_k_gemm_act_fp8(cera_k_gem
 extern "C" __global__ __launch_bounds__(256) void cera_k_gemm_act_f16(cera_k_gemm_act_f16_args a) {
     gemm_act_f16_body(reinterpret_cast<const uint4*>(a.quants), reinterpret_cast<uint4*>(a.out), a.n_words);
 }
-extern "C" __global__ __launch_bounds__(64 * G8_NW, 8 / G8_NW) void cera_k_gemm_q4_k(GemmArgs p) { gemm_q4k_fp8_body<false, false, G8_NW>(p); }
-extern "C" __global__ __launch_bounds__(64 * G8_NW, 8 / G8_NW) void cera_k_gemm_q4_k_swiglu(GemmArgs p) { gemm_q4k_fp8_body<true, false, G8_NW>(p); }
+extern "C" __global__ __launch_bounds__(64 * G8_NW, 2) void cera_k_gemm_q4_k(GemmArgs p) { gemm_q4k_fp8_body<false, false, 2>(p); }
+extern "C" __global__ __launch_bounds__(64 * G8_NW, 2) void cera_k_gemm_q4_k_swiglu(GemmArgs p) { gemm_q4k_fp8_body<true, false, 2>(p); }
 extern "C" __global__ __launch_bounds__(256, 2) void cera_k_gemm_q6_k(GemmArgs p) { gemm_q6k_f16_body<false>(p); }
 extern "C" __global__ __launch_bounds__(256, GemmQ4_0::WAVES_PER_SIMD) void cera_k_gemm_q4_0(GemmArgs p) { gemm_body<GemmQ4_0, false, false>(p); }
 extern "C" __global__ __launch_bounds__(256, GemmQ4_1::WAVES_PER_SIMD) void cera_k_gemm_q4_1(GemmArgs p) { gemm_body<GemmQ4_1, false, false>(p); }

@@ -180,7 +180,12 @@ cera_hip_status cera_launch_gemm(cera_hip_ctx* ctx, const cera_hip_dtensor* w, c
                  nullptr, nullptr, nullptr};
         CERA_TRY(cera_launch_i8(ctx, w->dtype, b, split));
     } else switch (w->dtype) {
-        case CERA_HIP_Q4_K: hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false>), grid, dim3(256), 0, ctx->stream, a); break;
+        case CERA_HIP_Q4_K:
+            if (g8_four_tiles(static_cast<uint64_t>(grid.y) * grid.z, n, ctx->n_cu)) {
+                grid.x = (n + 127) / 128;
+                hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false, 4>), grid, dim3(256), 0, ctx->stream, a);
+            } else hipLaunchKernelGGL((gemm_q4k_fp8_kernel<false, false>), grid, dim3(256), 0, ctx->stream, a);
+            break;
         case CERA_HIP_Q6_K:
             if (kq)
                 CERA_TRY(cera_launch_kq(ctx, KqArgs{a.w, a.w2, static_cast<const uint8_t*>(a.bh), bs, a.out, a.out2, a.m, a.m2, n, a.k, a.row_bytes, a.tiles1,
@@ -247,7 +252,9 @@ cera_hip_status cera_launch_gemm_swiglu(cera_hip_ctx* ctx, const cera_hip_dtenso
     if (i8) {
         I8Args b{a.w, a.w2, bq, bs, nullptr, nullptr, a.m, a.m, n, a.k, a.row_bytes, 0, a.k, 0, 0, 0, 0, nullptr, 1.0f, hq, hs, hbsum};
         CERA_TRY(cera_launch_i8_swiglu(ctx, gate->dtype, b));
-    } else if (fp8) hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false>), grid, dim3(256), 0, ctx->stream, a);
+    } else if (fp8 && g8_four_tiles(grid.y, n, ctx->n_cu))
+        hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false, 4>), dim3((n + 127) / 128, grid.y), dim3(256), 0, ctx->stream, a);
+    else if (fp8) hipLaunchKernelGGL((gemm_q4k_fp8_kernel<true, false>), grid, dim3(256), 0, ctx->stream, a);
     else hipLaunchKernelGGL((gemm_kernel<GemmQ4_1, true>), grid, dim3(256), 0, ctx->stream, a);
     HIP_TRY(ctx, hipGetLastError());
     *fused = true;

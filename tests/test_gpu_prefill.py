@@ -282,6 +282,27 @@ def test_gemm_swiglu_epilogue_matches_separate_kernels(hip, orc, dtype, m, k, n,
     assert np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k", [(12801, 449, 512), (12800, 512, 256), (12928, 511, 768)])
+def test_gemm_q4k_by_128_tokens(hip, orc, m, n, k):
+    """Q4_K launches that take workgroups of 128 tokens (two rounds of the chip by 64, one by 128): a last tile of 128 tokens with
+    nothing in its upper half, a whole one, a ragged one; whole and ragged tiles of rows.  A token's bits are those of a launch of
+    64 tokens, which takes 64 a workgroup (K is whole in both); the pair of halves and its SwiGLU launch agree byte for byte."""
+    _say(f"gemm Q4_K by 128 tokens m={m} n={n} k={k}")
+    w, _ = util.make_weights(Q4_K, m, k, seed=61)
+    x = util.rng(n + k).standard_normal((n, k)).astype(np.float32)
+    out = hip.gemm(Q4_K, w, x, m, n, k)
+    for a in (0, 64, (n - 1) // 64 * 64):
+        part = x[a:a + 64]
+        assert np.array_equal(out[:, a:a + 64].view(np.uint32), hip.gemm(Q4_K, w, part, m, len(part), k).view(np.uint32))
+    h, rb = m // 64 * 32, util.H.row_bytes(Q4_K, k)
+    wg, wu = w[:h * rb], w[h * rb:2 * h * rb]
+    g, u = hip.gemm_pair(Q4_K, wg, h, Q4_K, wu, h, x, n, k)
+    assert np.array_equal(g.T, out[:h]) and np.array_equal(u.T, out[h:2 * h])
+    q, sc, fused = hip.gemm_swiglu(Q4_K, wg, wu, h, x, n, k)
+    ref_s, ref_q = orc.quantize_q8_0(orc.silu_mul(g.reshape(-1), u.reshape(-1)))
+    assert fused and np.array_equal(q.reshape(-1), ref_q) and np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
 @pytest.mark.parametrize("m,k,n,want_fused", [(12288, 2048, 2, True), (12320, 2304, 5, True), (12288, 2048, 16, True), (12320, 2048, 17, True), (12288, 2048, 48, True), (96, 2048, 5, True), (4096, 2048, 48, False)])
 def test_gemm_swiglu_of_a_few_tokens(hip, orc, dtype, m, k, n, want_fused):
