@@ -6,14 +6,17 @@
 // ahead; the tokens, 64 of k at a time, straight from their quants, row by row, with one barrier.  Nothing is staged through
 // registers and a Q8_0 code needs no unpacking.  The sums start from 1.5 * 2^23 as an integer, so that the matrix core's result,
 // read as a float, is that number plus the dot: a subtraction in place of the conversion, which the vector ALU issues at half
-// the rate.  The product of the two scales is an outer product on the matrix core, two blocks an instruction.  A slice of K adds its
+// the rate.  The product of the two scales, f16 numbers both, is an outer product on the matrix core, two blocks an instruction, exact in
+// f32.  It is an f16 instruction with one of its four products in use: while one of f32 runs, no vector instruction of the SIMD does
+// (32 vector instructions of another wavefront beside them: 201 clocks with f32, 138 with f16, 134 alone).  Q8_0, hidden 3072, two layers: 300 tokens 524 -> 510 us, 1001
+// 992 -> 968, 2000 1714 -> 1676.  A slice of K adds its
 // blocks in the order of the kernel before it; the number of slices is i8_slices' own, so that sums in parts have another order.
 //
 // What bounds it: one subtraction and one FMA per output and block.  In 16384 x 3072 Q8_0 (gate | up) times 1001 tokens the vector
 // ALU is busy for 0.66 of the time and the matrix cores for 0.27, in turns; 28672 x 4096 times 2048 tokens 671 us, 717 TOP/s, before the order of the folds.  The kernel
 // before it (gemm.hip.h, which keeps Q4_1, rows of about 2^24 columns and more, the block dots and the code object's export)
 // unpacks into LDS, converts, and reads both operands through LDS.  Passes of two layers, before and now:
-//   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039 (986 with the folds in order)
+//   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039 (986 with the folds in order, 968 with the scales in f16)
 //   hidden 4096, Q4_0:  9 tokens 331 -> 300 us, 64: 440 -> 374, 128: 591 -> 477, 512: 1181 -> 947, 1001: 2055 -> 1673
 #include "f16_codes.hip.h"
 #include "gemm_i8.h"
@@ -25,6 +28,7 @@ namespace {
 typedef float f16x __attribute__((ext_vector_type(16)));
 typedef float f32x __attribute__((ext_vector_type(32)));
 typedef int i16x __attribute__((ext_vector_type(16)));
+typedef _Float16 h4x __attribute__((ext_vector_type(4)));
 typedef int i4x __attribute__((ext_vector_type(4)));
 
 constexpr int I8_WAVES = 4;
@@ -44,7 +48,8 @@ struct I8Q8_0 {
     static __device__ __forceinline__ i4x codes(const uint8_t* row, uint32_t z, uint32_t half) {
         return dwords(row, ((34 * z + 2) & ~3u) + 16 * half, z & 1);
     }
-    static __device__ __forceinline__ float scale(const uint8_t* row, uint32_t z) { return h2f(*reinterpret_cast<const uint16_t*>(row + 34 * z)); }
+    static __device__ __forceinline__ _Float16 scale(const uint8_t* row, uint32_t z) { return *reinterpret_cast<const _Float16*>(row + 34 * z); }
+    static __device__ __forceinline__ float dot(float f, float start) { return f - start; }
 };
 struct I8Q4_0 {
     static constexpr uint32_t SB = 144, PIECES = 5, START = 8;
@@ -56,7 +61,8 @@ struct I8Q4_0 {
         for (int i = 0; i < 4; ++i) q[i] = static_cast<int>(((static_cast<uint32_t>(q[i]) ^ 0x88888888u) << up) & 0xF0F0F0F0u);
         return q;
     }
-    static __device__ __forceinline__ float scale(const uint8_t* row, uint32_t z) { return h2f(*reinterpret_cast<const uint16_t*>(row + 18 * z)) * 0.0625f; }
+    static __device__ __forceinline__ _Float16 scale(const uint8_t* row, uint32_t z) { return *reinterpret_cast<const _Float16*>(row + 18 * z); }
+    static __device__ __forceinline__ float dot(float f, float start) { return fmaf(f, 0.0625f, -0.0625f * start); }   // the codes are sixteen times theirs; exact
 };
 
 // T: tiles of 32 tokens (4; 2 for up to 64).  SWIGLU: a wavefront's rows are sixteen of the gate matrix and the same sixteen of the up matrix
@@ -142,18 +148,19 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
         read(0);
 #pragma unroll
         for (int b = 0; b < 2; ++b) a[b] = W::codes(wr, z + b, half);
-        const float rs = W::scale(wr, z + half);
+        const h4x rs{W::scale(wr, z + half), 0, 0, 0};
         i16x r[2];
         f32x scale[2];
+        auto scales = [&](int t) { return __builtin_amdgcn_mfma_f32_32x32x4f16(rs, h4x{static_cast<_Float16>(ts[t & 1]), 0, 0, 0}, zero, 0, 0, 0); };
         __builtin_amdgcn_sched_barrier(0);
-        scale[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(rs, ts[0], zero, 0, 0, 0);
+        scale[0] = scales(0);
         r[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[0], x[0][0], start, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 2 * T; ++i) {   // block i & 1 of tile i >> 1; the products of the step behind it first
             const int t = i >> 1;
             if (i + 1 < 2 * T) {
-                if (i & 1) scale[(t + 1) & 1] = __builtin_amdgcn_mfma_f32_32x32x1f32(rs, ts[(t + 1) & 1], zero, 0, 0, 0);
+                if (i & 1) scale[(t + 1) & 1] = scales(t + 1);
                 r[(i + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[(i + 1) & 1], x[((i + 1) >> 1) & 1][(i + 1) & 1], start, 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -166,7 +173,7 @@ __global__ __launch_bounds__(64 * I8_WAVES, 2) void gemm_i8_kernel(I8Args p) {
             // Sixteen subtractions, then sixteen FMAs: an instruction that waits for the one before it costs its wavefront eight clocks, one that does
             // not five.  Q8_0, hidden 3072, two layers, 1001 tokens 1023 -> 986 us; 16384 x 3072 times 2048 tokens by itself 336 -> 310.
 #pragma unroll
-            for (int e = 0; e < 16; ++e) f[e] -= start_f;
+            for (int e = 0; e < 16; ++e) f[e] = W::dot(f[e], start_f);
             asm volatile("" : "+v"(f));
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[t][e] = fmaf(f[e], scale[t & 1][16 * (i & 1) + e], acc[t][e]);

@@ -186,6 +186,28 @@ def test_gemm_of_32_weight_blocks(hip, orc, dtype, bytes_, ma, mb, n, k):
 
 
 @pytest.mark.parametrize("dtype,bytes_", [(Q8_0, 34), (Q4_0, 18)])
+@pytest.mark.parametrize("n", [40, 130])
+def test_gemm_of_32_weight_blocks_with_subnormal_scales(hip, orc, dtype, bytes_, n):
+    """Weights' and tokens' scales below 2^-14, subnormal as f16, in the outer product on the matrix core: it keeps them, and a
+    product of two is exact in f32.  One row's scales are the smallest there are; bound as above."""
+    m, k = 132, 1024
+    _say(f"subnormal scales {util.NAMES[dtype]} n={n}")
+    r = util.rng(n)
+    w = r.integers(0, 256, (m, k // 32, bytes_), dtype=np.uint8)
+    d = (r.uniform(0.5, 2.0, (m, k // 32, 1)) * 1e-5).astype(np.float16)
+    d[0] = np.float16(2.0 ** -24)
+    w[:, :, :2] = d.view(np.uint8)
+    x = (r.standard_normal((n, k)) * 2.0 ** -10).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    assert 0 < xs.min() and xs.max() < 2.0 ** -14
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    wd = util.dequant_np(dtype, w.reshape(-1), m, k).astype(np.float64)
+    rms = np.sqrt((xd * xd).sum(1, keepdims=True) * (wd * wd).sum(1) / k)
+    got = hip.gemm(dtype, w.reshape(-1), x, m, n, k).reshape(m, n).T
+    assert (np.abs(got - xd @ wd.T) / rms).max() <= 2e-5
+
+
+@pytest.mark.parametrize("dtype,bytes_", [(Q8_0, 34), (Q4_0, 18)])
 def test_gemm_of_rows_of_16_million_columns(hip, orc, dtype, bytes_):
     """Rows that the kernel of the other Q8_0 and Q4_0 products has no offsets for.  A slice of K adds 2^16 blocks one after the other:
     roundings of at most 2^-24 of sums that grow as a random walk come to 2^-24 * sqrt(2^16 / 6) of the output's rms; 2.5 times that."""
