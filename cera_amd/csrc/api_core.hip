@@ -336,8 +336,8 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
     const uint64_t last_len = seq_len + n_queries - 1;
     if (seq_len == 0 || last_len > max_seq || max_seq > 0x7FFFFFFFull) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "attention: need 0 < seq_len <= max_seq < 2^31");
     // A batch of queries (prefill) runs the tiled MFMA kernel: a K/V tile is read once per 32
-    // queries instead of once per query.  Parts of 128 keys while the context is short, about
-    // eight parts per query block beyond that.
+    // queries instead of once per query.  Parts of at most 128 keys while the context is short, eight
+    // parts per query block or more beyond that.
     if (new_kv && n_queries != 1) return cera_fail(ctx, CERA_HIP_ERR_ARGUMENT, "attention: fused RoPE/append is for single-token decode");
     const bool batch = n_queries >= 16;
     if (batch && (reinterpret_cast<uintptr_t>(q) & 15)) return cera_fail(ctx, CERA_HIP_ERR_ARGUMENT, "attention: a query batch must be 16-byte aligned");
@@ -362,6 +362,14 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
     if (batch) {
         const uint64_t want = n_queries >= 1024 ? 4 : 8;   // many query blocks fill the chip with fewer parts
         part_keys = last_len <= 1024 ? 128u : static_cast<uint32_t>(((last_len + want - 1) / want + 31) / 32 * 32);
+        if (!ws) {
+            // Few query blocks: as many parts as give every CU a workgroup, down to a tile of 32 keys.  A part's tiles are a chain of
+            // loads, splits and products of about 3 us each, and a second workgroup a CU gains less than its sums cost the merge.
+            // Two layers, 32 / 8 heads of 128: 45 queries behind 700 keys (128 keys a part before, 64 now) 294 -> 289 us, behind 12000
+            // 490 -> 433, 30 behind 3000 294 -> 264; by two workgroups a CU 286, 427 and 275.  At most 64 parts: the merge adds them in order.
+            const uint64_t blocks = (n_queries + 31ull) / 32 * n_kv_heads, parts = std::min<uint64_t>((ctx->n_cu + blocks - 1) / blocks, 64);
+            part_keys = std::min(part_keys, static_cast<uint32_t>(((last_len + parts - 1) / parts + 31) / 32 * 32));
+        }
         n_parts = static_cast<uint32_t>((last_len + part_keys - 1) / part_keys);
     } else {
         // positions per chunk (8 S): one 8-key chunk per wavefront while the context is short (a single
@@ -381,7 +389,11 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
         // parts (wavefronts) per (query, kv head): enough to fill the chip ~4 waves per CU deep
         // (more parts make the partial kernel shorter but the merge longer: measured best from 2k
         // to 128k keys with an f32 cache), but at least one chunk each and at most ATTN_MAX_PARTS
-        const uint32_t waves_per_cu = kv_f16 ? 8 : 4;   // a half cache is nearer VALU-bound: more wavefronts help
+        // a half cache is nearer VALU-bound: more wavefronts help; from eight queries on all but the first find the rows in the
+        // L2, and the launch is a chain of loads (two layers, 32 / 8 heads of 128, 12 queries behind 900 keys: 275 -> 240 us, 8: 243 -> 228;
+        // five queries are level)
+        const bool shared_rows = n_queries >= 8;
+        const uint32_t waves_per_cu = shared_rows ? 12 : kv_f16 ? 8 : 4;
         uint32_t want_parts = n_splits ? n_splits : std::max(1u, ctx->n_cu * waves_per_cu / (n_kv_heads * n_queries));
         want_parts = std::min<uint32_t>(want_parts, ATTN_MAX_PARTS);
         chunks_per_part = std::max(1u, (n_chunks + want_parts - 1) / want_parts);
@@ -403,8 +415,8 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
                 if (cpp > first && parts * 4 < want_parts) break;
                 const uint64_t groups = (parts + 3) / 4 * n_kv_heads * subs * n_queries;   // workgroups
                 // workgroups a CU takes per round: two where the kernel is bound by its own instructions
-                // (an f16 cache, eight heads per kv head), one where it is bound by bytes
-                const uint64_t round = static_cast<uint64_t>(ctx->n_cu) * ((kv_f16 || G == 8) ? 2 : 1);
+                // (an f16 cache, eight heads per kv head), three where queries share rows, one where it is bound by bytes
+                const uint64_t round = static_cast<uint64_t>(ctx->n_cu) * (shared_rows ? 3 : (kv_f16 || G == 8) ? 2 : 1);
                 const uint64_t cost = cpp * ((groups + round - 1) / round);
                 if (cost < best || (kv_f16 && cost == best)) { best = cost; chunks_per_part = cpp; }
             }

@@ -1077,9 +1077,9 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(const float* __r
     attn_decode_merge_body<QUANT, HD>(part_acc, part_ml, n_parts, G, n_heads, out, scales, quants, bsum);
 }
 
-// Merge for a batch of queries (prefill): the same formula as above over the few parts a prefill
-// pass makes (8 at most), but eight (query, head) pairs per workgroup, 32 lanes each (a float4 of
-// the head's columns per lane), the parts walked in order by every lane.  The decode merge spends
+// Merge for a batch of queries (prefill): the same formula as above over the parts a prefill
+// pass makes (four to eight for many queries, up to 64 for a single block of them), but eight (query, head) pairs per workgroup, 32 lanes each (a float4 of
+// the head's columns per lane), the parts summed in order by every lane.  The decode merge spends
 // a 256-thread workgroup and two barriers on one pair, which for 512 queries x 32 heads x 4 parts
 // cost more than the attention itself.
 template <bool QUANT, int HD>
@@ -1096,18 +1096,32 @@ __device__ __forceinline__ void attn_prefill_merge_body(const float* __restrict_
     const uint64_t pbase = (static_cast<uint64_t>(qi) * n_kv + kvh) * n_parts;
     constexpr uint32_t C4 = HD / 4;
     const bool live = c < C4;
+    // each lane has the maximum and sum of one part of 32 at a time, and eight parts' columns are on their way at once
+    const float2* const ml = reinterpret_cast<const float2*>(part_ml) + pbase * G + hg;
+    const float4* const cols = reinterpret_cast<const float4*>(part_acc + (pbase * G + hg) * HD) + c;
     float M = -__builtin_inff();
-    for (uint32_t p = 0; p < n_parts; ++p) M = fmaxf(M, part_ml[((pbase + p) * G + hg) * 2]);
+    for (uint32_t p = c; p < n_parts; p += 32) M = fmaxf(M, ml[p * G].x);
+#pragma unroll
+    for (int o = 16; o; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 32));
     float L = 0.0f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t p = 0; p < n_parts; ++p) {
-        const float2 ml = *reinterpret_cast<const float2*>(part_ml + ((pbase + p) * G + hg) * 2);
-        const float w = cera_expf(ml.x - M);
-        L = fmaf(w, ml.y, L);
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (live) a = reinterpret_cast<const float4*>(part_acc + ((pbase + p) * G + hg) * HD)[c];
-        acc.x = fmaf(w, a.x, acc.x); acc.y = fmaf(w, a.y, acc.y);
-        acc.z = fmaf(w, a.z, acc.z); acc.w = fmaf(w, a.w, acc.w);
+    for (uint32_t p0 = 0; p0 < n_parts; p0 += 32) {
+        const float2 mine = p0 + c < n_parts ? ml[(p0 + c) * G] : make_float2(-__builtin_inff(), 0.0f);
+        const float weight = cera_expf(mine.x - M);
+        for (uint32_t p1 = p0; p1 < min(p0 + 32, n_parts); p1 += 8) {
+            float4 a[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i)
+                a[i] = live && p1 + i < n_parts ? cols[(p1 + i) * G * (HD / 4)] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                if (p1 + i >= n_parts) break;
+                const float w = __shfl(weight, (p1 + i) & 31, 32);
+                L = fmaf(w, __shfl(mine.y, (p1 + i) & 31, 32), L);
+                acc.x = fmaf(w, a[i].x, acc.x); acc.y = fmaf(w, a[i].y, acc.y);
+                acc.z = fmaf(w, a[i].z, acc.z); acc.w = fmaf(w, a[i].w, acc.w);
+            }
+        }
     }
     const float inv = 1.0f / L;
     const float4 o = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);

@@ -498,7 +498,7 @@ class Model:
                        v=m4(n * self.kv_dim * 4), attn=m4(n * self.q_dim * 4), gate=m4(n * self.ffn * 4), up=m4(n * self.ffn * 4),
                        xq=m4(n * maxk), xh=m4(n * maxk * 2), x8=m4(gemm_fp8_act_bytes(n, maxk)), xs=m4(n * (maxk // 32) * 4),
                        bsum=m4(n * (maxk // 32) * 4), tokens=m4(n * 4),
-                       acc=m4(n * self.nh * 8 * self.hd * 4), ml=m4(n * self.nh * 8 * 8))
+                       acc=m4(n * self.nh * 32 * self.hd * 4), ml=m4(n * self.nh * 32 * 8))   # at most 1024 keys in parts of 32
         self.pf_cap = n
 
     def _gemm(self, w, n, out, resid=None, staged=None):
@@ -533,7 +533,9 @@ class Model:
         self.L("cera_k_embed_rows", ((self.hs + 255) // 256, n), 256, EmbedRowsArgs(e["dev"], e["row_bytes"], P["tokens"], e["t"], self.hs, 1.0, P["hidden"]))
         scale = 1.0 / float(np.sqrt(np.float32(self.hd)))
         last_len = start_pos + n
-        part_keys = 128
+        blocks = (n + 31) // 32 * self.nkv   # a workgroup a CU where 128 keys a part are fewer
+        parts = min((self.n_cu + blocks - 1) // blocks, 64)
+        part_keys = min(128, ((last_len + parts - 1) // parts + 31) // 32 * 32)
         n_parts = (last_len + part_keys - 1) // part_keys
         for Ly in self.layers:
             st = {}

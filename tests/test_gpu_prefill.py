@@ -694,6 +694,28 @@ def test_attn_prefill_batch_vs_oracle(hip, orc, nh, nkv, start, n):
     assert np.isfinite(out).all()
 
 
+@pytest.mark.parametrize("kv_f16", [False, True])
+@pytest.mark.parametrize("nh,nkv,hd,start,n", [(32, 8, 128, 16, 16), (8, 1, 128, 5000, 20), (6, 2, 64, 2079, 33), (32, 8, 128, 900, 12), (8, 1, 64, 17, 8),
+                                               (64, 8, 128, 3000, 15)])
+def test_attn_of_few_queries_in_parts(hip, orc, nh, nkv, hd, start, n, kv_f16):
+    """16 and more queries whose blocks leave the chip idle: parts of one tile of 32 keys, the most parts that there are (64, two
+    rounds of the merge's lanes), a last part and a last block that are not whole; and 8 to 15 queries, which share the keys' rows.
+    Bound as for the accuracy of the split products below."""
+    _say(f"attn few queries nh={nh} nkv={nkv} hd={hd} start={start} n={n} f16={kv_f16}")
+    r = util.rng(n + start)
+    L = start + n
+    q = r.standard_normal((n, nh * hd), dtype=np.float32)
+    k, v = (r.standard_normal(L * nkv * hd, dtype=np.float32) for _ in range(2))
+    if kv_f16:
+        k, v = (x.astype(np.float16).astype(np.float32) for x in (k, v))
+    scale = 1.0 / np.sqrt(hd)
+    out = (hip.attn_f16kv if kv_f16 else hip.attn_prefill)(q, k, v, nh, nkv, hd, start, n, scale)
+    for i in sorted({0, n // 2, n - 1}):
+        Li = start + i + 1
+        ref = orc.decode_attention(q[i], k[:Li * nkv * hd], v[:Li * nkv * hd], nh, nkv, hd, scale, Li)
+        assert np.abs(out[i].astype(np.float64) - ref).max() <= 5e-5 * util.rms(ref), i
+
+
 @pytest.mark.parametrize("case", ["plain", "wide_range", "sink"])
 def test_attn_prefill_split_f16_keeps_f32_accuracy(hip, orc, case):
     """The batch kernel multiplies on the f16 matrix cores with every operand split into an f16
