@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "f16_codes.hip.h"
+#include "few_pairs.h"
 #include "gemv.hip.h"
 #include "gemm_few.h"
 #include "quantize.hip.h"
@@ -41,7 +42,7 @@ struct FewArgs {
     float *hs, *hbsum;
 };
 
-constexpr int FEW_WAVES = 8, FEW_ROWS = 16 * FEW_WAVES;
+constexpr uint32_t FEW_ROWS = 16 * FEW_WAVES;
 // LDS of one tile of 16 tokens and one super-block: a block's operand fragments (64 lanes x 16 bytes, the blocks 16 bytes
 // further apart than that, so that the eight blocks of a token do not share their banks when they are written), the block
 // scales, the mins' operand
@@ -250,9 +251,8 @@ struct FewQ6 {
     }
 };
 
-// T tiles of 16 tokens; S super-blocks a chunk, so that a chunk is up to four tiles and two of them fill at most half the LDS (Q6_K with one
-// tile two: 32000 x 4096 with 5 tokens 35.7 -> 34.6 us).  Four tiles of tokens would spill registers.
-template <typename W, int T> constexpr int FEW_CHUNK = T == 1 ? (W::MINS ? 4 : 2) : T == 2 ? 2 : 1;
+// T tiles of 16 tokens (four would spill registers)
+template <typename W, int T> constexpr int FEW_CHUNK = few_chunk(W::MINS, T);
 // Two super-blocks are on their way.  With four a slice of a few loads its last one up to four times again: 6144 x 4096 Q4_K in six
 // slices with 5 tokens 10.8 -> 8.6 us, 4096 x 14336 Q6_K in eight 19.6 -> 17.8, 28672 x 4096 in one 21.4 -> 21.6.
 constexpr int FEW_AHEAD = 2;
@@ -326,7 +326,7 @@ __device__ __forceinline__ void few_swiglu(const FewArgs& a, const f4v (&acc)[T]
 // the workgroup leaves silu(gate) * up as quants
 template <typename W, int T, bool COPY, bool SWIGLU = false>
 __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned char* lds) {
-    constexpr int S = FEW_CHUNK<W, T>, AHEAD = FEW_AHEAD, PAIRS = S * T * 128, NP = (PAIRS + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+    constexpr int S = FEW_CHUNK<W, T>, AHEAD = FEW_AHEAD, NP = few_rounds(S * T);
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nsb = a.k / 256;
     if (SWIGLU) second = wave >= FEW_WAVES / 2;
     const FewMat& M = second ? a.b : a.a;
@@ -334,24 +334,22 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
     const uint32_t sb0 = blockIdx.y * a.sb_per, sb1 = min(nsb, sb0 + a.sb_per);
     const uint8_t* const m0 = M.w;
     const typename W::At at = W::template at<COPY>(min(row0 + (lane & 15), M.m - 1) * M.row_bytes, lane >> 4, nsb);   // rows past the end: the last one again
-    // the tokens of a chunk: a thread takes the 32 quants of one block of one token (of three tiles some twice)
-    auto pair = [](int i) {
-        const uint32_t p = i * FEW_WAVES * 64 + threadIdx.x;
-        return p - (p >= PAIRS ? 128 : 0);
-    };
+    // the tokens of a chunk: a thread takes the 32 quants of one block of one token, block_of of token_of of the tile
+    auto tile = [&](int i) { return few_tile(S * T, i, wave); };
+    const uint32_t token_of = (threadIdx.x % FEW_TILE_PAIRS) >> 3, block_of = threadIdx.x & 7;
     uint4 q0[NP], q1[NP];
     float xs[NP], bs[NP];
     uint32_t oq[NP], os[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-        const uint32_t p = pair(i), tok = min((p >> 7) % T * 16 + ((p >> 3) & 15), a.n - 1);
-        oq[i] = tok * a.k + (p & 7) * 32;
-        os[i] = (tok * (a.k / 32) + (p & 7)) * 4;
+        const uint32_t tok = min(tile(i) % T * 16 + token_of, a.n - 1);
+        oq[i] = tok * a.k + block_of * 32;
+        os[i] = (tok * (a.k / 32) + block_of) * 4;
     }
     auto act_load = [&](uint32_t sb) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const uint32_t s = min(sb + min(i * (FEW_WAVES / 2) + (wave >> 1), S * T - 1u) / T, sb1 - 1);   // the super-block of the pair's tile
+            const uint32_t s = min(sb + tile(i) / T, sb1 - 1);
             const int8_t* const x = a.xq + s * 256;
             q0[i] = *reinterpret_cast<const uint4*>(x + oq[i]);
             q1[i] = *reinterpret_cast<const uint4*>(x + oq[i] + 16);
@@ -362,8 +360,8 @@ __device__ __forceinline__ void few_body(const FewArgs& a, bool second, unsigned
     auto act_store = [&](uint32_t buf) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const uint32_t p = pair(i), tok = (p >> 3) & 15, b = p & 7;
-            unsigned char* const t = lds + (buf * S * T + (p >> 7)) * FEW_TILE;
+            const uint32_t tok = token_of, b = block_of;
+            unsigned char* const t = lds + (buf * S * T + tile(i)) * FEW_TILE;
             const uint32_t q[8] = {q0[i].x, q0[i].y, q0[i].z, q0[i].w, q1[i].x, q1[i].y, q1[i].z, q1[i].w};
 #pragma unroll
             for (int g = 0; g < 4; ++g) {

@@ -343,6 +343,28 @@ def test_gemm_swiglu_of_a_few_tokens(hip, orc, dtype, m, k, n, want_fused):
     assert np.array_equal(q.reshape(-1), ref_q) and np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("n", [3, 5, 12, 16, 20, 45])
+def test_gemm_swiglu_of_a_few_tokens_with_long_rows(hip, orc, dtype, n):
+    """The whole of a long K in one workgroup, many chunks of tokens one after the other in the same two buffers, against the exact products
+    of the dequantized weights and quantized tokens.  A product is off by at most 2e-5 of its token's rms (test_gemm_pair_of_a_few_tokens),
+    |d silu / dg| <= 1.1 and |silu(g)| <= |g|; a quant is off by half a step d, d's f16 by 2^-11 of up to 127 steps."""
+    m, k, distinct = 12288, 14336, 96
+    _say(f"few gemm_swiglu, long rows {util.NAMES[dtype]} n={n}")
+    (wg, _), (wu, _) = (util.make_weights(dtype, distinct, k, seed=s) for s in (43, 44))
+    x = util.rng(n).standard_normal((n, k)).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    g, u = (xd @ util.dequant_np(dtype, w, distinct, k).astype(np.float64).T for w in (wg, wu))
+    h = g / (1 + np.exp(-g)) * u
+    off = 2e-5 * (1.1 * np.abs(u) * util.rms(g) + np.abs(g) * util.rms(u)) + 1e-6 * np.abs(h)
+    q, sc, fused = hip.gemm_swiglu(dtype, np.tile(wg, m // distinct), np.tile(wu, m // distinct), m, x, n, k)
+    assert fused
+    d = sc.reshape(n, m // distinct, distinct // 32, 1).astype(np.float64)
+    got = (q.reshape(n, m // distinct, distinct // 32, 32) * d).reshape(n, m // distinct, distinct)
+    assert (np.abs(got - h[:, None]) <= off[:, None] + (0.5 + 127 / 2048) * np.repeat(d, 32, 3).reshape(got.shape)).all()
+
+
 @pytest.mark.parametrize("dtype,m,k,n,want_fused", [(Q4_K, 2048, 512, 1040, True), (Q4_K, 1056, 256, 2000, True),
                                                       (Q4_K, 512, 256, 80, False), (Q4_0, 2048, 512, 1040, True)])
 def test_gemm_swiglu_f16_words_for_a_q6k_down_projection(hip, dtype, m, k, n, want_fused):
