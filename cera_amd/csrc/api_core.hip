@@ -3,6 +3,7 @@
 #include <cstring>
 
 #include "attention.hip.h"
+#include "attn_plan.h"
 #include "gemv_launch.hip.h"
 #include "gemv_nb.hip.h"
 #include "glue.hip.h"
@@ -302,6 +303,22 @@ static void attn_launch_partials(cera_hip_ctx* ctx, const AttnLaunch& a, const K
 static constexpr uint64_t ATTN_RECORDS_MIN_PAIRS = 448 * 1024;
 static constexpr uint64_t ATTN_RECORDS_MAX_BYTES = 128ull << 20;   // of the 512 MB that are kept free for workspaces
 
+// the context's room for parts' results, grown to so many bytes
+static cera_hip_status attn_partials(cera_hip_ctx* ctx, uint64_t acc_bytes, uint64_t ml_bytes) {
+    auto grow = [&](float*& p, uint64_t& held, uint64_t bytes) -> cera_hip_status {
+        if (held >= bytes) return CERA_HIP_OK;
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        if (p) HIP_TRY(ctx, hipFree(p));
+        p = nullptr;
+        held = 0;
+        HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&p), bytes));
+        held = bytes;
+        return CERA_HIP_OK;
+    };
+    CERA_TRY(grow(ctx->attn_acc, ctx->attn_acc_bytes, acc_bytes));
+    return grow(ctx->attn_ml, ctx->attn_ml_bytes, ml_bytes);
+}
+
 cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* kc, const void* vc,
                                  uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint64_t seq_len,
                                  uint64_t max_seq, float scale, uint32_t n_splits, uint32_t n_queries, float* out,
@@ -331,15 +348,14 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
         }
         return CERA_HIP_OK;
     }
-    uint32_t G = n_heads / n_kv_heads;
+    const uint32_t G = n_heads / n_kv_heads;
     // seq_len = keys visible to the first query; the last query sees seq_len + n_queries - 1
     const uint64_t last_len = seq_len + n_queries - 1;
     if (seq_len == 0 || last_len > max_seq || max_seq > 0x7FFFFFFFull) return cera_fail(ctx, CERA_HIP_ERR_SHAPE, "attention: need 0 < seq_len <= max_seq < 2^31");
     // A batch of queries (prefill) runs the tiled MFMA kernel: a K/V tile is read once per 32
-    // queries instead of once per query.  Parts of at most 128 keys while the context is short, eight
-    // parts per query block or more beyond that.
+    // queries instead of once per query.
     if (new_kv && n_queries != 1) return cera_fail(ctx, CERA_HIP_ERR_ARGUMENT, "attention: fused RoPE/append is for single-token decode");
-    const bool batch = n_queries >= 16;
+    const bool batch = attn_is_batch(n_queries);
     if (batch && (reinterpret_cast<uintptr_t>(q) & 15)) return cera_fail(ctx, CERA_HIP_ERR_ARGUMENT, "attention: a query batch must be 16-byte aligned");
     const AttnNewKV nk = new_kv ? *new_kv : AttnNewKV{};
     if (new_kv && out_quants && !out_bsum && n_splits == 0 && last_len <= attn_short_max_keys(head_dim)) {
@@ -356,100 +372,37 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
         HIP_TRY(ctx, hipGetLastError());
         return CERA_HIP_OK;
     }
-    uint32_t n_parts, part_keys = 0, chunks_per_part = 0;
-    uint32_t S = 1;
-    uint32_t Gw = G;   // decode: heads per wavefront
-    if (batch) {
-        const uint64_t want = n_queries >= 1024 ? 4 : 8;   // many query blocks fill the chip with fewer parts
-        part_keys = last_len <= 1024 ? 128u : static_cast<uint32_t>(((last_len + want - 1) / want + 31) / 32 * 32);
-        if (!ws) {
-            // Few query blocks: as many parts as give every CU a workgroup, down to a tile of 32 keys.  A part's tiles are a chain of
-            // loads, splits and products of about 3 us each, and a second workgroup a CU gains less than its sums cost the merge.
-            // Two layers, 32 / 8 heads of 128: 45 queries behind 700 keys (128 keys a part before, 64 now) 294 -> 289 us, behind 12000
-            // 490 -> 433, 30 behind 3000 294 -> 264; by two workgroups a CU 286, 427 and 275.  At most 64 parts: the merge adds them in order.
-            const uint64_t blocks = (n_queries + 31ull) / 32 * n_kv_heads, parts = std::min<uint64_t>((ctx->n_cu + blocks - 1) / blocks, 64);
-            part_keys = std::min(part_keys, static_cast<uint32_t>(((last_len + parts - 1) / parts + 31) / 32 * 32));
-        }
-        n_parts = static_cast<uint32_t>((last_len + part_keys - 1) / part_keys);
-    } else {
-        // positions per chunk (8 S): one 8-key chunk per wavefront while the context is short (a single
-        // memory round trip, many wavefronts), longer chunks once there is plenty of work.  Measured on
-        // the 32/8/128 shape over rotating caches; with a kv head's query heads split over two
-        // wavefronts (attn_launch_partials) 32-key chunks are best from 1024 keys up to where the split
-        // ends: 64-key chunks take one wavefront per SIMD (registers) and lose 2-3 us from 8k to 16k keys.
-        // heads per wavefront: attn_launch_partials has the reasons
-        if (G == 8 || (G == 4 && last_len < (kv_f16 ? 32768u : 16384u))) Gw = G / 2;
-        else if (G == 6) Gw = 2;
-        else if (G == 3 || G == 5 || G == 7) Gw = 1;
-        const bool split_heads = Gw != G;
-        if (split_heads) S = last_len >= ATTN_FUSED_NEW_KV_MAX_KEYS ? 4 : 1;
-        else S = last_len >= 8192 ? 8 : (last_len >= 2048 ? 4 : (last_len >= ATTN_FUSED_NEW_KV_MAX_KEYS ? 2 : 1));
-        if (Gw == 8 && S == 8) S = 4;   // eight heads x 64 positions per chunk does not fit the register file
-        uint32_t n_chunks = static_cast<uint32_t>((last_len + 8 * S - 1) / (8 * S));
-        // parts (wavefronts) per (query, kv head): enough to fill the chip ~4 waves per CU deep
-        // (more parts make the partial kernel shorter but the merge longer: measured best from 2k
-        // to 128k keys with an f32 cache), but at least one chunk each and at most ATTN_MAX_PARTS
-        // a half cache is nearer VALU-bound: more wavefronts help; from eight queries on all but the first find the rows in the
-        // L2, and the launch is a chain of loads (two layers, 32 / 8 heads of 128, 12 queries behind 900 keys: 275 -> 240 us, 8: 243 -> 228;
-        // five queries are level)
-        const bool shared_rows = n_queries >= 8;
-        const uint32_t waves_per_cu = shared_rows ? 12 : kv_f16 ? 8 : 4;
-        uint32_t want_parts = n_splits ? n_splits : std::max(1u, ctx->n_cu * waves_per_cu / (n_kv_heads * n_queries));
-        want_parts = std::min<uint32_t>(want_parts, ATTN_MAX_PARTS);
-        chunks_per_part = std::max(1u, (n_chunks + want_parts - 1) / want_parts);
-        if (!n_splits) {
-            // Between the lengths where that divides evenly the chip runs a ragged last round.  A
-            // wavefront's time goes with its chunks, the launch's with the rounds of workgroups a CU
-            // runs (one workgroup per CU and round with an f32 cache, which is bound by bytes; two with
-            // an f16 cache or eight heads per kv head): from the nominal count down to a quarter of it, take the parts that
-            // minimise chunks x rounds.  Of equals an f32 cache takes the one with more parts, an f16
-            // cache the one with fewer -- either way the one nearer two workgroups per CU.
-            // 9216 keys, f32: 31.2 -> 21.9 us together with the kernel's launch-index mapping, 13824:
-            // 37.2 -> 27.9; f16: 8192 keys 16.3 -> 13.9.  Within 4 % of the best (chunk, parts) pair
-            // of a sweep at every length from 1k to 16k keys (f32) and of a parts sweep (f16).
-            const uint32_t subs = G / Gw;
-            uint64_t best = ~0ull;
-            const uint32_t first = chunks_per_part;
-            for (uint32_t cpp = first; cpp <= n_chunks; ++cpp) {
-                const uint64_t parts = (n_chunks + cpp - 1) / cpp;
-                if (cpp > first && parts * 4 < want_parts) break;
-                const uint64_t groups = (parts + 3) / 4 * n_kv_heads * subs * n_queries;   // workgroups
-                // workgroups a CU takes per round: two where the kernel is bound by its own instructions
-                // (an f16 cache, eight heads per kv head), three where queries share rows, one where it is bound by bytes
-                const uint64_t round = static_cast<uint64_t>(ctx->n_cu) * (shared_rows ? 3 : (kv_f16 || G == 8) ? 2 : 1);
-                const uint64_t cost = cpp * ((groups + round - 1) / round);
-                if (cost < best || (kv_f16 && cost == best)) { best = cost; chunks_per_part = cpp; }
-            }
-        }
-        n_parts = (n_chunks + chunks_per_part - 1) / chunks_per_part;
-    }
-    uint64_t acc_bytes = static_cast<uint64_t>(n_queries) * n_kv_heads * n_parts * G * head_dim * sizeof(float);
-    uint64_t ml_bytes = static_cast<uint64_t>(n_queries) * n_kv_heads * n_parts * G * 2 * sizeof(float);
+    auto acc_bytes = [&](uint64_t parts) { return n_queries * parts * n_heads * head_dim * sizeof(float); };
+    auto ml_bytes = [&](uint64_t parts) { return n_queries * parts * n_heads * 2 * sizeof(float); };
+    cera_hip_status st = CERA_HIP_OK;
+    // more parts than the call needs: where the device has the memory, without giving up what is held
+    auto room = [&](uint32_t parts) {
+        const uint64_t a = acc_bytes(parts), l = ml_bytes(parts);
+        if (ws) return false;
+        if (a <= ctx->attn_acc_bytes && l <= ctx->attn_ml_bytes) return true;
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b + ctx->attn_acc_bytes + ctx->attn_ml_bytes < a + l) return false;
+        st = attn_partials(ctx, a, l);
+        if (st != CERA_HIP_ERR_OOM) return st == CERA_HIP_OK;
+        (void)hipGetLastError();   // or the next launch would report it
+        st = CERA_HIP_OK;
+        return false;
+    };
+    const AttnCut cut = attn_cut(n_heads, n_kv_heads, last_len, n_queries, n_splits, kv_f16, ctx->n_cu, room);
+    CERA_TRY(st);
+    const uint32_t n_parts = cut.n_parts;
     float *acc, *ml;
     if (ws) {
         // caller-provided workspace: nothing is allocated, a request that does not fit is refused
-        if (acc_bytes > ws->acc_bytes || ml_bytes > ws->ml_bytes)
+        if (acc_bytes(n_parts) > ws->acc_bytes || ml_bytes(n_parts) > ws->ml_bytes)
             return cera_fail(ctx, CERA_HIP_ERR_SHAPE,
-                             "attention: the split-K partials need " + std::to_string(acc_bytes) + " + " + std::to_string(ml_bytes) +
+                             "attention: the split-K partials need " + std::to_string(acc_bytes(n_parts)) + " + " + std::to_string(ml_bytes(n_parts)) +
                                  " bytes, the fixed workspace holds " + std::to_string(ws->acc_bytes) + " + " +
                                  std::to_string(ws->ml_bytes));
         acc = ws->acc;
         ml = ws->ml;
     } else {
-        if (ctx->attn_acc_bytes < acc_bytes) {
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            if (ctx->attn_acc) HIP_TRY(ctx, hipFree(ctx->attn_acc));
-            ctx->attn_acc = nullptr; ctx->attn_acc_bytes = 0;
-            HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_acc), acc_bytes));
-            ctx->attn_acc_bytes = acc_bytes;
-        }
-        if (ctx->attn_ml_bytes < ml_bytes) {
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            if (ctx->attn_ml) HIP_TRY(ctx, hipFree(ctx->attn_ml));
-            ctx->attn_ml = nullptr; ctx->attn_ml_bytes = 0;
-            HIP_TRY(ctx, hipMalloc(reinterpret_cast<void**>(&ctx->attn_ml), ml_bytes));
-            ctx->attn_ml_bytes = ml_bytes;
-        }
+        CERA_TRY(attn_partials(ctx, acc_bytes(n_parts), ml_bytes(n_parts)));
         acc = ctx->attn_acc;
         ml = ctx->attn_ml;
     }
@@ -465,7 +418,7 @@ cera_hip_status cera_launch_attn(cera_hip_ctx* ctx, const float* q, const void* 
         if (!records) CERA_TRY(cera_scratch_if_room(ctx, 13, rec_bytes, &records));
     }
     AttnLaunch a{q, static_cast<uint32_t>(seq_len), static_cast<uint32_t>(max_seq), scale, n_heads, n_kv_heads, n_queries,
-                 n_heads * head_dim, G, S, n_parts, part_keys, chunks_per_part, Gw, batch, new_kv != nullptr, nk, acc, ml,
+                 n_heads * head_dim, G, cut.S, n_parts, cut.part_keys, cut.chunks_per_part, cut.Gw, batch, new_kv != nullptr, nk, acc, ml,
                  static_cast<uint8_t*>(records)};
     const kv_half *kh = static_cast<const kv_half*>(kc), *vh = static_cast<const kv_half*>(vc);
     const float *kf = static_cast<const float*>(kc), *vf = static_cast<const float*>(vc);

@@ -2,6 +2,8 @@
 #pragma once
 #include <stdint.h>
 
+#define ATTN_MAX_PARTS 1024  // the merge kernel keeps one weight per part in LDS
+
 // The new token's own key and value, when the decode step lets the attention kernel do the
 // RoPE and the cache append: q arrives unrotated and is rotated on load; the wavefront whose
 // range holds the last position takes that position's K/V rows from the projection outputs
