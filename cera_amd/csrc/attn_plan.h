@@ -26,11 +26,14 @@ inline AttnCut attn_cut(uint32_t n_heads, uint32_t n_kv_heads, uint64_t last_len
         const uint64_t want = n_queries >= 1024 ? 4 : 8;   // many query blocks fill the chip with fewer parts
         c.part_keys = last_len <= 1024 ? 128u : static_cast<uint32_t>(((last_len + want - 1) / want + 31) / 32 * 32);
         c.n_parts = static_cast<uint32_t>((last_len + c.part_keys - 1) / c.part_keys);
-        // Few query blocks: as many parts as give every CU a workgroup, down to a tile of 32 keys.  A part's tiles are a chain of
+        // Few query blocks: as many parts as leave every CU at most one workgroup, down to a tile of 32 keys.  A part's tiles are a chain of
         // loads, splits and products of about 3 us each, and a second workgroup a CU gains less than its sums cost the merge.
         // Two layers, 32 / 8 heads of 128: 45 queries behind 700 keys (128 keys a part before, 64 now) 294 -> 289 us, behind 12000
-        // 490 -> 433, 30 behind 3000 294 -> 264; by two workgroups a CU 286, 427 and 275.  At most 64 parts: the merge adds them in order.
-        const uint64_t blocks = (n_queries + 31ull) / 32 * n_kv_heads, parts = std::min<uint64_t>((n_cu + blocks - 1) / blocks, 64);
+        // 490 -> 433, 30 behind 3000 294 -> 264; by two workgroups a CU 286, 427 and 275.  A few workgroups more than CUs are a second round of
+        // them: 160 queries behind 12000 keys, 32 / 4 heads of 128, 132 us a layer by the eight parts, 145 by 13 (260 workgroups), 111 by 12; 200
+        // queries 186 by ten, 139 by nine.  Over eight shapes, 16 to 257 queries behind 100 to 12000 keys, both caches, no slower than by the eight
+        // beyond noise, and 23 % less in the mean.  At most 64 parts: the merge adds them in order.
+        const uint64_t blocks = (n_queries + 31ull) / 32 * n_kv_heads, parts = std::min<uint64_t>(std::max<uint64_t>(n_cu / blocks, 1), 64);
         const uint32_t keys = std::min(c.part_keys, static_cast<uint32_t>(((last_len + parts - 1) / parts + 31) / 32 * 32));
         const uint32_t n = static_cast<uint32_t>((last_len + keys - 1) / keys);
         if (n > c.n_parts && room(n)) {

@@ -15,3 +15,7 @@ def _run(tmp_path, name):
 
 def test_more_parts_only_where_there_is_room(tmp_path):
     _run(tmp_path, "attn_plan_room")
+
+
+def test_more_parts_fill_the_chip_once(tmp_path):
+    _run(tmp_path, "attn_plan_rules")
