@@ -89,10 +89,15 @@ inline AttnCut attn_cut(uint32_t n_heads, uint32_t n_kv_heads, uint64_t last_len
     c.chunks_per_part = chunks(kv_f16 ? 8 : 4, kv_f16 || G == 8 ? 2 : 1);
     c.n_parts = (n_chunks + c.chunks_per_part - 1) / c.chunks_per_part;
     if (n_queries >= 8 && !n_splits) {
-        // From eight queries on all but the first find the rows in the L2, and the launch is a chain of loads: three workgroups a CU (two
-        // layers, 32 / 8 heads of 128, 12 queries behind 900 keys: 275 -> 240 us, 8: 243 -> 228; five queries are level)
+        // From eight queries on all but the first find the rows in the L2, and the launch is a chain of loads: three workgroups a CU,
+        // where that is far faster by an estimate, in keys: a part's, once for the launch's start and its end each and once for each
+        // workgroup of a CU, and 32.  The line is five thirds: 32 / 8 heads of 128, 12 queries behind 900 keys, f32, 35.2 -> 21.9 us a layer (the
+        // pass of two layers 275 -> 240); of 32 / 4 heads, 8 behind 3000, where it would be 22.8 -> 28.9, the cut stays.  Thirteen shapes of 1 to 32
+        // key heads, 8 to 15 queries behind 60 to 12000 keys, both caches: 5 % less time in the mean, up to 63 %, and none slower beyond noise; with
+        // three workgroups everywhere 7 % less, but up to 32 % more, and more than 3 % in a sixth of the shapes.  Five queries are level.
         const uint32_t more = chunks(12, 3), n = (n_chunks + more - 1) / more;
-        if (n <= c.n_parts || room(n)) {
+        auto cost = [&](uint32_t cpp) { return 32 + 8ull * c.S * cpp * (2 + (workgroups(cpp) + n_cu - 1) / n_cu); };
+        if (n > c.n_parts && cost(c.chunks_per_part) * 3 > cost(more) * 5 && room(n)) {
             c.chunks_per_part = more;
             c.n_parts = n;
         }
