@@ -336,6 +336,25 @@ def _launch3(host, name, grid, block, args):
              f"hipModuleLaunchKernel({name})")
 
 
+MAX_KEYS = 1024   # of a batched prefill of the host below
+
+
+def prefill_part_keys(n: int, last_len: int, n_kv: int, n_cu: int) -> int:
+    """Keys of a part for a batch of n queries whose last one sees last_len (at most MAX_KEYS) keys, as the library takes them: 128, or fewer,
+    in whole tiles of 32, as long as there is at most a workgroup a CU and 64 parts."""
+    parts = min(max(n_cu // ((n + 31) // 32 * n_kv), 1), 64)
+    return min(128, ((last_len + parts - 1) // parts + 31) // 32 * 32)
+
+
+def prefill_part_rows(n: int, max_len: int, n_kv: int, n_cu: int) -> int:
+    """The most queries times parts of a batch of up to n queries and max_len keys: rows of the parts' results a head."""
+    most = 0
+    for blocks in range(1, (n + 31) // 32 + 1):   # a block of 32 queries more has fewer parts
+        parts = max(min(max(n_cu // (blocks * n_kv), 1), 64), (max_len + 127) // 128)
+        most = max(most, min(32 * blocks, n) * min(parts, (max_len + 31) // 32))
+    return most
+
+
 class Model:
     """LlamaModel::forward / ::forward_prefill (cera/src/model/llama.rs:468-597, 738-1523) for a dense llama
     with Q4_K / Q6_K / Q4_0 / Q4_1 / Q8_0 projection matrices, driven from the code object alone: every
@@ -494,11 +513,11 @@ class Model:
         if self.pf_cap >= n:
             return
         m4, maxk = self.h.malloc, max(self.hs, self.ffn, self.q_dim)
+        rows = prefill_part_rows(n, min(self.max_seq, MAX_KEYS), self.nkv, self.n_cu)
         self.pf = dict(hidden=m4(n * self.hs * 4), normed=m4(n * self.hs * 4), q=m4(n * self.q_dim * 4), k=m4(n * self.kv_dim * 4),
                        v=m4(n * self.kv_dim * 4), attn=m4(n * self.q_dim * 4), gate=m4(n * self.ffn * 4), up=m4(n * self.ffn * 4),
                        xq=m4(n * maxk), xh=m4(n * maxk * 2), x8=m4(gemm_fp8_act_bytes(n, maxk)), xs=m4(n * (maxk // 32) * 4),
-                       bsum=m4(n * (maxk // 32) * 4), tokens=m4(n * 4),
-                       acc=m4(n * self.nh * 32 * self.hd * 4), ml=m4(n * self.nh * 32 * 8))   # at most 1024 keys in parts of 32
+                       bsum=m4(n * (maxk // 32) * 4), tokens=m4(n * 4), acc=m4(rows * self.nh * self.hd * 4), ml=m4(rows * self.nh * 8))
         self.pf_cap = n
 
     def _gemm(self, w, n, out, resid=None, staged=None):
@@ -523,7 +542,7 @@ class Model:
     def forward_prefill(self, tokens, start_pos: int) -> np.ndarray:
         """16 tokens or more at once (at most 1024 keys in all, hidden and ffn below 2048 so the tile GEMMs need no K split): logits of the last."""
         n = len(tokens)
-        assert n >= 16 and start_pos == self.seq_len and start_pos + n <= min(self.max_seq, 1024) and max(self.hs, self.ffn) < 2048
+        assert n >= 16 and start_pos == self.seq_len and start_pos + n <= min(self.max_seq, MAX_KEYS) and max(self.hs, self.ffn) < 2048
         self._pf_buffers(n)
         P, e, G = self.pf, self.embd, self.nh // self.nkv
         self.h._ck(self.h.hip.hipMemcpy(C.c_void_p(P["tokens"]), C.c_void_p(np.ascontiguousarray(tokens, np.uint32).ctypes.data),
@@ -533,9 +552,7 @@ class Model:
         self.L("cera_k_embed_rows", ((self.hs + 255) // 256, n), 256, EmbedRowsArgs(e["dev"], e["row_bytes"], P["tokens"], e["t"], self.hs, 1.0, P["hidden"]))
         scale = 1.0 / float(np.sqrt(np.float32(self.hd)))
         last_len = start_pos + n
-        blocks = (n + 31) // 32 * self.nkv   # a workgroup a CU where 128 keys a part are fewer
-        parts = min((self.n_cu + blocks - 1) // blocks, 64)
-        part_keys = min(128, ((last_len + parts - 1) // parts + 31) // 32 * 32)
+        part_keys = prefill_part_keys(n, last_len, self.nkv, self.n_cu)
         n_parts = (last_len + part_keys - 1) // part_keys
         for Ly in self.layers:
             st = {}

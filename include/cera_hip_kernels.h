@@ -274,7 +274,7 @@ typedef struct {
  * g = n_heads / n_kv_heads wavefronts.  The batch's own keys are already in the cache (rope_kv).
  *   first_len  keys visible to query 0; query i sees first_len + i
  *   part_keys  keys per part, a multiple of 32 (the library: 128 up to 1024 keys, else about an
- *              eighth of the keys; fewer, down to 32 and to 64 parts, where that gives the chip less than a
+ *              eighth of the keys; fewer, down to 32 and to 64 parts, as long as that is at most a
  *              workgroup a CU); n_parts = ceil((first_len + n_queries - 1) / part_keys) <= 1024
  *   q rows 16-byte aligned, q_stride floats apart
  * grid = (ceil(n_queries / 32), n_kv, n_parts) workgroups of 64 g.

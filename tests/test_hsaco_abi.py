@@ -154,3 +154,18 @@ def test_decode_copy_row_bytes_follow_the_header_macro():
         subprocess.run(["gcc", "-I", str(ROOT / "include"), str(c), "-o", str(Path(d) / "m")], check=True)
         out = subprocess.run([str(Path(d) / "m")], check=True, capture_output=True, text=True).stdout.split()
     assert [int(v) for v in out] == [hsaco_api.decode_copy_row_bytes(t, k) for t, k in cases]
+
+
+@pytest.mark.parametrize("n_kv", [1, 2, 3, 8, 20])
+def test_prefill_buffers_hold_the_parts_of_every_batch(n_kv):
+    """Room for the parts' results of any batch up to the capacity and any number of keys, and no more than one of them needs: eight parts of
+    1024 queries, not the 32 of a short batch."""
+    n_cu = 256
+    for cap in (16, 33, 100, 1000, 1024):
+        rows = hsaco_api.prefill_part_rows(cap, 1024, n_kv, n_cu)
+        need = 0
+        for n in {16, 31, 32, 33, 64, 65, 96, 97, 160, 300, 511, cap} | set(range(16, cap + 1, 32)):
+            for last in (n, 33, 100, 127, 128, 129, 500, 895, 897, 1000, 1023, 1024):
+                if n <= cap and last >= n:
+                    need = max(need, n * -(-last // hsaco_api.prefill_part_keys(n, last, n_kv, n_cu)))
+        assert need <= rows <= 1.4 * need, (cap, need, rows)
