@@ -441,7 +441,7 @@ static cera_hip_status gemm_swiglu_host(cera_hip_ctx* ctx, const cera_hip_tensor
         // (a Q4_K pair's epilogue writes the f16 words itself; every other route converts the quants afterwards)
         bool hh_in_epilogue = halves && wg->dtype == CERA_HIP_Q4_K;
         if (n <= FEW_MAX_TOKENS && cera_gemm_few_supports(wg, static_cast<uint32_t>(n)) && cera_gemm_few_supports(wu, static_cast<uint32_t>(n))) {
-            // as the forward pass does, whose matrices have decode copies
+            // the launch of a forward pass of three tokens and more (two take the multi-token GEMV there), whose matrices have decode copies
             CERA_TRY(cera_tensor_prepare_stream(ctx, wg));
             CERA_TRY(cera_tensor_prepare_stream(ctx, wu));
             CERA_TRY(cera_launch_gemm_few_swiglu(ctx, wg, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db), static_cast<uint32_t>(n),
@@ -451,7 +451,7 @@ static cera_hip_status gemm_swiglu_host(cera_hip_ctx* ctx, const cera_hip_tensor
         if (!fused) CERA_TRY(cera_launch_gemm_swiglu(ctx, wg, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
                                          static_cast<uint32_t>(n), static_cast<int8_t*>(hq), static_cast<float*>(hs),
                                          static_cast<float*>(hb), &fused, nullptr, nullptr, hh_in_epilogue ? hh : nullptr));
-        if (!fused) {   // the forward pass's other route: the two GEMMs, then the SwiGLU + quantize kernel
+        if (!fused) {   // the two GEMMs, then the SwiGLU + quantize kernel (a forward pass of a few tokens: the pair of cera_launch_gemm_few, then that)
             CERA_TRY(cera_launch_gemm(ctx, wg, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),
                                       static_cast<uint32_t>(n), static_cast<float*>(dg), 1, mm, nullptr, 1.0f));
             CERA_TRY(cera_launch_gemm(ctx, wu, static_cast<float*>(ds), static_cast<int8_t*>(dq), static_cast<float*>(db),

@@ -238,9 +238,11 @@ CERA_HIP_API cera_hip_status cera_hip_gemm_pair(cera_hip_ctx*, const cera_hip_te
  * cpu::silu_mul_inplace, cera/src/backend/cpu.rs:2570-2575, then quantize_columns for the down
  * projection, cera/src/model/transformer.rs:865-946): quants[n][m] / scales[n][m/32] =
  * Q8_0(silu(gate.x) * (up.x)) per token row, quantized in the GEMM's epilogue.  gate and up must
- * share a type with an int8 GEMM (not Q6_K), k and m, m a multiple of 32.  Small batches, which
- * need a K split to fill the chip, take the two GEMMs and the SwiGLU kernel instead (*fused = 0,
- * nullable); both routes give identical bytes. */
+ * share a type with an int8 GEMM, k and m, m a multiple of 32.  One launch (*fused = 1, nullable) serves
+ * batches that fill the chip (not of Q6_K), and 2 to 48 tokens of Q4_K and Q6_K rows of 2048 columns and more where it
+ * is estimated no slower than the pair.  It adds up the whole of K in order: its bytes are those of
+ * cera_hip_gemm_pair, where that has no slices of K, and of SwiGLU and Q8_0 behind it.  Everything else takes the
+ * two GEMMs, which may have slices of K, and the SwiGLU kernel (*fused = 0). */
 CERA_HIP_API cera_hip_status cera_hip_gemm_swiglu(cera_hip_ctx*, const cera_hip_tensor* gate, const cera_hip_tensor* up,
                                                   const float* x, uint64_t n, int8_t* quants, float* scales, int* fused);
 

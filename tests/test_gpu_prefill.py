@@ -325,6 +325,21 @@ def test_gemm_q4k_by_128_tokens(hip, orc, m, n, k):
     assert fused and np.array_equal(q.reshape(-1), ref_q) and np.array_equal(sc.reshape(-1).view(np.uint32), ref_s.view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [897, 900, 960])
+def test_gemm_q4k_by_128_tokens_in_parts_of_k(hip, orc, n):
+    """4096 x 4096 with 15 tiles of 64 tokens: two slices of K, two rounds of the chip by 64 tokens and one by 128.  Against the exact products
+    of the dequantized weights and quantized tokens; block results are whole numbers, and the bound is that of test_gemm_pair_of_a_few_tokens."""
+    m = k = 4096
+    _say(f"gemm Q4_K by 128 tokens in parts n={n}")
+    w, _ = util.make_weights(Q4_K, m, k, seed=62)
+    x = util.rng(n).standard_normal((n, k)).astype(np.float32)
+    xs, xq = orc.quantize_q8_0(x.reshape(-1))
+    xd = (xq.reshape(-1, 32).astype(np.float64) * xs.reshape(-1, 1)).reshape(n, k)
+    want = xd @ util.dequant_np(Q4_K, w, m, k).astype(np.float64).T
+    rms = np.sqrt(np.mean(want * want, axis=1, keepdims=True))
+    assert (np.abs(hip.gemm(Q4_K, w, x, m, n, k).T - want) / rms).max() <= 2e-5
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
 @pytest.mark.parametrize("m,k,n,want_fused", [(12288, 2048, 2, True), (12320, 2304, 5, True), (12288, 2048, 16, True), (12320, 2048, 17, True), (12288, 2048, 48, True), (96, 2048, 5, True), (4096, 2048, 48, False)])
 def test_gemm_swiglu_of_a_few_tokens(hip, orc, dtype, m, k, n, want_fused):
@@ -366,6 +381,7 @@ def test_gemm_swiglu_of_a_few_tokens_with_long_rows(hip, orc, dtype, n):
 
 
 @pytest.mark.parametrize("dtype,m,k,n,want_fused", [(Q4_K, 2048, 512, 1040, True), (Q4_K, 1056, 256, 2000, True),
+                                                      (Q4_K, 6400, 256, 449, True), (Q4_K, 6400, 256, 510, True),   # by 128 tokens
                                                       (Q4_K, 512, 256, 80, False), (Q4_0, 2048, 512, 1040, True)])
 def test_gemm_swiglu_f16_words_for_a_q6k_down_projection(hip, dtype, m, k, n, want_fused):
     """The f16 form of the SwiGLU quants that a Q6_K down projection reads: half words of the integer
