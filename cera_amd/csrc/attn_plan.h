@@ -94,7 +94,7 @@ inline AttnCut attn_cut(uint32_t n_heads, uint32_t n_kv_heads, uint64_t last_len
         // workgroup of a CU, and 32.  The line is five thirds: 32 / 8 heads of 128, 12 queries behind 900 keys, f32, 35.2 -> 21.9 us a layer (the
         // pass of two layers 275 -> 240); of 32 / 4 heads, 8 behind 3000, where it would be 22.8 -> 28.9, the cut stays.  Thirteen shapes of 1 to 32
         // key heads, 8 to 15 queries behind 60 to 12000 keys, both caches: 5 % less time in the mean, up to 63 %, and none slower beyond noise; with
-        // three workgroups everywhere 7 % less, but up to 32 % more, and more than 3 % in a sixth of the shapes.  Five queries are level.
+        // three workgroups everywhere 7 % less, but up to 32 % more, and more than 3 % in a sixth of 660 calls.  Five queries are level.
         const uint32_t more = chunks(12, 3), n = (n_chunks + more - 1) / more;
         auto cost = [&](uint32_t cpp) { return 32 + 8ull * c.S * cpp * (2 + (workgroups(cpp) + n_cu - 1) / n_cu); };
         if (n > c.n_parts && cost(c.chunks_per_part) * 3 > cost(more) * 5 && room(n)) {

@@ -12,9 +12,10 @@
 //
 // What bounds it: the instructions, about 140 (Q4_K) and 200 (Q6_K) per 16 rows x 256 weights to unpack and 40 per tile of 16 tokens.
 // A SIMD that has matrix instructions among them issues one in four clocks, whichever it is and however many wavefronts it
-// has: gate | up with 5 tokens takes 17 us without its loads, the loads alone 12, both 21.5 (3.1 TB/s).  Gate | up, 14336 x 4096 Q4_K
-// as a pair: 21.5 us at 5 tokens, 36.6 at 45; down, 4096 x 14336 Q6_K: 17.8 and 25.6 (22.3, 37.1, 19.8 and 25.8 with codes in the mantissa of
-// 1024, code and scale of a Q6_K weight put together and then rounded and split, and up to four super-blocks ahead).  The 64-token
+// has: gate | up with 5 tokens takes 17 us without its loads, the loads alone 12, both 21.5 (3.1 TB/s).  In a pass, gate | up of 14336 x 4096 Q4_K
+// with SwiGLU takes 21.9 us at 5 tokens and 36.5 at 45 (the pair 21.5 and 35.6, SwiGLU 4.6 and 5.1, with codes in the mantissa of 1024, code
+// and scale of a Q6_K weight put together and then rounded and split, and up to four super-blocks ahead); Q | K | V 11.0 and 16.9 (14.0, 17.2), down, 4096
+// x 14336 Q6_K, 16.8 and 23.4 (19.0, 23.7).  At 45 tokens the vector ALU is busy for half of gate | up, the matrix cores for 16 %.  The 64-token
 // tiles before it took 36 us for a down product and 50 for a pair, with a launch for the tokens' copy before and one for the sums
 // behind them; passes of the two-layer 8B shapes: 5 tokens 406 -> 262 us, 45 tokens 466 -> 294 (267 and 299 with SwiGLU in a launch of its own).
 #include <algorithm>

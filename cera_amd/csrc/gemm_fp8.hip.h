@@ -34,12 +34,11 @@
 // unpacked for twice as many products: 28672 x 4096 (gate | up) times 1001 tokens 401 us by 64, 360 by 128; two layers, 2048 tokens 3394 -> 3237; the
 // sums are the same.  g8_four_tiles says which a launch takes.
 //
-// What bounds it: on this chip the matrix core and the vector ALU of a SIMD do not run at the same
-// time in a kernel of this kind (matrix-core busy + vector-ALU busy = 100 % of the dispatch, here as
-// in the int8 kernel), so the cost of a 32 x 32 x 32 tile step is the SUM of its MFMA clocks (64 dot +
-// 32 scale tile + 12 min terms) and its vector instructions (16 FMAs + about 12 of unpacking and
-// scale decoding, ~3 clocks each).  Against the int8 form (32 + 32 + 32 MFMA clocks, 16 converts + 16
-// FMAs + staging) that sum is what the fp8 dot lowers.
+// What bounds it: a 32 x 32 x 32 tile step has 64 MFMA clocks for the dot, 32 for its share of the scale tile and 12 for the min terms, and 16 FMAs
+// with about 12 vector instructions of unpacking and scale decoding (half of them with 128 tokens), ~3 clocks each.  While the scale tile's f32 instruction
+// runs, the SIMD issues no vector instruction, and a wavefront's FMAs wait for its own dots; beside the fp8 and bf16 ones vector instructions of
+// the other wavefront run.  So the two overlap in part: matrix cores and vector ALU together are busy for 100 % of a long dispatch by 64 tokens (0.47 and
+// 0.53), and for 113 % by 128 (gate | up times 2048 tokens, 0.58 and 0.55).  The int8 form has 32 + 32 + 32 MFMA clocks, 16 converts, 16 FMAs and staging.
 #pragma once
 #include "gemm.hip.h"
 #include "gemm_q6k_f16.hip.h"
@@ -249,8 +248,7 @@ __device__ __forceinline__ void gemm_q4k_fp8_body(GemmArgs p) {
     // The K loop is software-pipelined inside the wavefront.  A step is one (pair g, token tile tn,
     // block jb of the pair): 8 TT per super-block.  Tick t issues the matrix-core work of step t+1, reads
     // the fragments of step t+3 from LDS and then runs the 16 FMAs of step t while that work
-    // executes: on this hardware a SIMD overlaps matrix-core and vector instructions of the SAME
-    // wavefront, not those of two different wavefronts.
+    // executes.
     //
     // Weight prefetch: a super-block's rows are copied to LDS one super-block ahead (behind the barrier
     // of tick T - 3) and read into registers at that tick of the super-block before theirs.

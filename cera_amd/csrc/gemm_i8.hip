@@ -13,7 +13,7 @@
 // blocks in the order of the kernel before it; the number of slices is i8_slices' own, so that sums in parts have another order.
 //
 // What bounds it: one subtraction and one FMA per output and block.  In 16384 x 3072 Q8_0 (gate | up) times 1001 tokens the vector
-// ALU is busy for 0.66 of the time and the matrix cores for 0.27, in turns; 28672 x 4096 times 2048 tokens 671 us, 717 TOP/s, before the order of the folds.  The kernel
+// ALU is busy for 0.76 of the time and the matrix cores for 0.30; 28672 x 4096 times 2048 tokens with SwiGLU 655 us, 734 TOP/s.  The kernel
 // before it (gemm.hip.h, which keeps Q4_1, rows of about 2^24 columns and more, the block dots and the code object's export)
 // unpacks into LDS, converts, and reads both operands through LDS.  Passes of two layers, before and now:
 //   hidden 3072, Q8_0:  9 tokens 263 -> 234 us, 64: 341 -> 294, 128: 453 -> 376, 512: 838 -> 605, 1001: 1320 -> 1039 (986 with the folds in order, 968 with the scales in f16)
