@@ -14,8 +14,8 @@
 //
 // 4096 x 14336 (with the tokens' operand and the sum of the slices): 512 tokens 172 -> 139 us, 2048 tokens 617 -> 440 us;
 // 4096 x 4096 with 512 tokens 66 -> 56 us, 128 tokens 33 -> 29 us.  What bounds it: the products of both parts, 193 us of the
-// 440 at the nominal rate, and the folds and the unpacking; the matrix cores are busy for 46 % of the time and the vector ALU
-// for 57 %, and the two take turns.
+// 440 at the nominal rate, and the folds and the unpacking; the matrix cores are busy for 44 % of the time and the vector ALU
+// for 55 %, and the two take turns.
 #include "f16_codes.hip.h"
 #include "gemm_kq.h"
 #include "gemv.hip.h"
